@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void k_obs_anom(int64_t m, int N, const double
 // values are exact in FP64, so the FP64 accumulation adds no FP32 error).
 // ---------------------------------------------------------------------------
 template <int NP, typename TS>
-__global__ __launch_bounds__(256) void k_gram(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
+__global__ __launch_bounds__(256, 2) void k_gram(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
                                               const int32_t* __restrict__ sel_idx,
                                               const double* __restrict__ sel_w, int64_t m,
                                               const double* __restrict__ rho,
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256) void k_eig(int64_t z0, const int32_t* __restri
 // Zones without observations get T = I exactly (Sa = Sf, rrsqrt.F90:326,371).
 // ---------------------------------------------------------------------------
 template <int NP>
-__global__ __launch_bounds__(256) void k_tmat(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
+__global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
                                               const double* __restrict__ ymat,
                                               double* __restrict__ mat,
                                               const double* __restrict__ vec) {

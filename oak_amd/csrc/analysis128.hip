@@ -158,7 +158,7 @@ __device__ __forceinline__ void gram128_wave(int64_t p0, int64_t p, const int32_
 }
 
 template <typename TS>
-__global__ __launch_bounds__(256) void k_gram128(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
+__global__ __launch_bounds__(256, 2) void k_gram128(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
                                                  const int32_t* __restrict__ sel_idx,
                                                  const double* __restrict__ sel_w, int64_t m,
                                                  const double* __restrict__ rho,
@@ -868,7 +868,7 @@ struct XformLdsF {
   double a[P128 + 2];  // a / scaling, then v.w~
 };
 
-__global__ __launch_bounds__(256) void k_xform128f(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
+__global__ __launch_bounds__(256, 2) void k_xform128f(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
                                                    const int64_t* __restrict__ zone_ptr,
                                                    const double* __restrict__ ymat,
                                                    const double* __restrict__ vec,

@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void k_obs_anom_f32(int64_t m, int N, const do
 // the transposed product (A = [T|a]^T from LDS, B = Sf^T) so that each
 // 16-row strip is stored as contiguous runs of the column-major Ea.
 template <int NP>
-__global__ __launch_bounds__(256) void k_update_f32(int64_t z0, const int32_t* __restrict__ zorder, int N,
+__global__ __launch_bounds__(256, 2) void k_update_f32(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ zone_ptr,
                                                     const double* __restrict__ mat,
                                                     const double* __restrict__ vec,

@@ -642,7 +642,7 @@ struct FormQ256Lds {
   double tau[2][16];
 };
 
-__global__ __launch_bounds__(256) void k_formq256(int64_t z0, const int32_t* __restrict__ zorder,
+__global__ __launch_bounds__(256, 2) void k_formq256(int64_t z0, const int32_t* __restrict__ zorder,
                                                   const int64_t* __restrict__ sel_ptr,
                                                   const double* __restrict__ qmat,
                                                   double* __restrict__ umat) {
@@ -774,7 +774,7 @@ struct FormQ64Lds {
   double tau[2][16];
 };
 
-__global__ __launch_bounds__(256) void k_formq64(int64_t z0, const int32_t* __restrict__ zorder,
+__global__ __launch_bounds__(256, 2) void k_formq64(int64_t z0, const int32_t* __restrict__ zorder,
                                                  const int64_t* __restrict__ sel_ptr,
                                                  double* __restrict__ qmat) {
   constexpr int NP = 64, NB = 4, LV = FormQ64Lds::LV;
@@ -906,7 +906,7 @@ void launch_tridiag_lower64(const ChunkArgs& A, hipStream_t st) {
 // the vectors of Omega, then T.  Zones without observations
 // get T = I.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_tmat256(int64_t z0, const int32_t* __restrict__ zorder,
+__global__ __launch_bounds__(256, 2) void k_tmat256(int64_t z0, const int32_t* __restrict__ zorder,
                                                  int N, const int64_t* __restrict__ sel_ptr,
                                                  const double* __restrict__ umat,
                                                  double* __restrict__ mat,
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(256) void k_tmat256(int64_t z0, const int32_t* __re
 // TE is the type of S and out (double, or float on the mixed path).
 // ---------------------------------------------------------------------------
 template <int MODE, typename TE>
-__global__ __launch_bounds__(256) void k_update256(int nzc, int64_t z0,
+__global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
                                                    const int32_t* __restrict__ zorder, int N,
                                                    const int64_t* __restrict__ zone_ptr,
                                                    const double* __restrict__ mat,
