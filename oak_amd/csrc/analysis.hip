@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __re
                                               const double* __restrict__ vec) {
   constexpr int NB = NP / 16;
   constexpr int LD = NP + 1;
-  __shared__ double Ys[NP * LD];
+  __shared__ double Ys[NP < 64 ? NP * LD : 1];
   __shared__ double T0[NP * LD];
   __shared__ double U[4][NP];
   const int zl = blockIdx.x;
@@ -526,11 +526,12 @@ __global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __re
   }
   const double* v = vec + (size_t)zl * 4 * NP + 2 * NP;
   const double* Yz = ymat + (size_t)zl * NP * NP;
-  for (int e = threadIdx.x; e < NP * NP; e += 256) Ys[(e / NP) * LD + e % NP] = Yz[e];
+  for (int e = threadIdx.x; e < NP * NP; e += 256) (NP < 64 ? Ys : T0)[(e / NP) * LD + e % NP] = Yz[e];
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int li = lane & 15, kk = lane >> 4;
-  for (int tile = wave; tile < NB * NB; tile += 4) {
+  // NP = 64: ymat holds M^-1/2 itself (staged straight into T0 above)
+  for (int tile = wave; NP < 64 && tile < NB * NB; tile += 4) {
     const int I = tile / NB, J = tile % NB;
     d4 acc = {0, 0, 0, 0};
 #pragma unroll 4
@@ -728,7 +729,9 @@ void launch_prep_ens(int NP, const PrepEnsArgs& A, hipStream_t st) {
 template <int NP>
 static void eig_t(const ChunkArgs& A, hipStream_t st) {
   constexpr int GPW = 64 / NP;
-  if (A.eig_method == 1) {
+  if (NP == 64 && A.eig_method == 1) {
+    launch_func(NP, A, false, st);
+  } else if (A.eig_method == 1) {
     launch_tql_pipeline(NP, A, st);
     // zones the QL could not finish fall back to Jacobi
     hipLaunchKernelGGL(k_eig<NP>, dim3(nblk(A.nzc, 4 * GPW)), dim3(256), 0, st, A.z0, A.zorder, A.nzc,
@@ -738,14 +741,7 @@ static void eig_t(const ChunkArgs& A, hipStream_t st) {
     hipLaunchKernelGGL(k_eig<NP>, dim3(nblk(A.nzc, 4 * GPW)), dim3(256), 0, st, A.z0, A.zorder, A.nzc,
                        A.N, A.sel_ptr, A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol,
                        A.max_sweeps, (const int32_t*)nullptr);
-  }
-}
-
-void launch_eig_small(int NP, const ChunkArgs& A, hipStream_t st) {
-  switch (NP) {
-    case 16: eig_t<16>(A, st); break;
-    case 32: eig_t<32>(A, st); break;
-    case 64: eig_t<64>(A, st); break;
+    if (NP == 64) launch_yyt(NP, A, st);
   }
 }
 

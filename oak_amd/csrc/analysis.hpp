@@ -159,10 +159,9 @@ void launch_chunk(int NP, const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 int persist_grid128();
 void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
-// eigensolver of a chunk for NP <= 64 (QL pipeline or Jacobi, with fallback)
-void launch_eig_small(int NP, const ChunkArgs& A, hipStream_t st);
 // zones with 1 <= p < 64 at NP = 128 in observation space (dual.hip): A has
-// the dual order and the NP = 64 buffers; ymat128/vec128/ampl receive W, a, v
+// the dual order and the NP = 64 buffers; ymat128/vec128/ampl receive M^-1/2,
+// a, v
 void launch_dual128(const ChunkArgs& A, int N, double* ymat128, double* vec128, double* ampl,
                     hipStream_t st, PhaseTimer* tm);
 void launch_chunk128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
@@ -172,14 +171,18 @@ void launch_tql_pipeline(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_ql256(const ChunkArgs& A, hipStream_t st);
 void launch_tridiag256_tail(const ChunkArgs& A, hipStream_t st);
-// NP = 128, OAKG_TUNE_TRIDIAG_SPLIT 3: steps 0..63 of the reduction on the
-// lower-triangle register tiles (wide256.hip)
-void launch_tridiag_lower128(const ChunkArgs& A, hipStream_t st);
-// OAKG_TUNE_TRIDIAG_SPLIT 4: steps 64..125 by the lower-triangle kernel at
-// NP = 64 on the trailing block (after launch_tridiag_lower128)
-void launch_tridiag_lower128_tail(const ChunkArgs& A, hipStream_t st);
-// NP = 64: reduction on the lower triangle and Q on MFMA (wide256.hip)
-void launch_tridiag_lower64(const ChunkArgs& A, hipStream_t st);
+// Householder reductions on the lower triangle (wide256.hip): d, e, the
+// reflectors, and Q^T b and Q^T 1_N (ones = N; -1: the vector in slot 2) in
+// place of b and slot 2 of vec
+void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st);
+void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st);
+// NP = 64, 128 (funcm.hip): the reduction, then M^-1/2 in ymat, a and v;
+// dual: the functions of I + G that dual.hip needs
+void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st);
+// the same M^-1/2 from the Jacobi option's eigenvectors
+void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
+// pole table of the current device
+hipError_t init_poles(int device);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
 void launch_update_f32(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_nll_adjoint(int NP, const ChunkArgs& A, hipStream_t st);

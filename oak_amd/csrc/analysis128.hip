@@ -10,7 +10,8 @@
 //              runs the 120 intra-block pairs of its blocks, then 7 block
 //              rounds (round-robin over the 8 blocks) of 16 cross-block rounds;
 //              blocks move between waves through the zone's scratch matrix
-//   k_xform128 T = (Y Y^T) Omega formed in LDS and the update Ea = xa + Sf T
+//   funcm.hip  M^-1/2, a and v from the tridiagonal form (default)
+//   k_xform128 T = M^-1/2 Omega formed in LDS and the update Ea = xa + Sf T
 //              run from it (FP64 MFMA; FP32 MFMA for FP32 members)
 #include <type_traits>
 
@@ -327,14 +328,12 @@ __global__ __launch_bounds__(256) void k_eig128(int64_t z0, const int32_t* __res
                                                 double* __restrict__ ampl,
                                                 int32_t* __restrict__ sweeps_out,
                                                 unsigned* __restrict__ err, double tol,
-                                                int max_sweeps,
-                                                const int32_t* __restrict__ only) {
+                                                int max_sweeps) {
   __shared__ Eig128Lds L;
   const int zl = blockIdx.x;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;  // the zone is solved by the other pipeline
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (only && !(only[zl] & 3)) return;
   double* V = vec + (size_t)zl * 4 * P128;
   if (sel_ptr[z + 1] == sel_ptr[z]) {
     if (tid < P128) V[P128 + tid] = 0.0;
@@ -584,17 +583,15 @@ __global__ __launch_bounds__(256) void k_eig128(int64_t z0, const int32_t* __res
 }
 
 // ---------------------------------------------------------------------------
-// Transform and update fused, NP = 128, FP64: T = (Y Y^T) Omega is formed in
+// Transform and update fused, NP = 128, FP64: T = M^-1/2 Omega is formed in
 // LDS and out = Sf_z T, xa = x0 + Sf_z a run from it, so T never goes through
 // HBM.  One workgroup per zone (the 128 x 128 block fills the LDS):
-//   1. Y -> LDS (row stride LDT: the MFMA operand reads, 16 rows x 4
+//   1. M^-1/2 -> LDS (row stride LDT: the MFMA operand reads, 16 rows x 4
 //      consecutive doubles per instruction, hit distinct banks)
-//   2. Y Y^T on v_mfma_f64_16x16x4f64, the 36 lower tiles (wave w owns tile
-//      rows w and 7 - w, 9 tiles each), stored mirrored over Y
-//   3. the Omega correction (the rank-structured formula of k_tmat in
+//   2. the Omega correction (the rank-structured formula of k_tmat in
 //      analysis.hip), applied in place; the buffer then holds X[s][r] = T[r][s]
-//   4. the update (Out^T strip = X Sf_strip^T) with the A operand X read
-//      from LDS and each wave's first strip of Sf loaded during steps 1-3
+//   3. the update (Out^T strip = X Sf_strip^T) with the A operand X read
+//      from LDS and each wave's first strip of Sf loaded during steps 1-2
 // ---------------------------------------------------------------------------
 constexpr int LDT = P128 + 2;
 
@@ -648,9 +645,6 @@ __global__ __launch_bounds__(512) void k_xform128(int64_t z0, const int32_t* __r
     }
   };
   const double* Vz = vec + (size_t)zl * 4 * P128;
-  // a zone solved in observation space (dual.hip) has -1 in its mu slot and
-  // W in place of Y: M^-1/2 = I - W W^T instead of Y Y^T
-  const bool dual = Vz[3 * P128] < 0.0;
   if (tid < P128) L.a[tid] = Vz[P128 + tid];
   else if (tid < 2 * P128) L.v[tid - P128] = tid - P128 < N ? Vz[2 * P128 + tid - P128] : 0.0;
   if (sel_ptr[z + 1] == sel_ptr[z]) {
@@ -659,73 +653,17 @@ __global__ __launch_bounds__(512) void k_xform128(int64_t z0, const int32_t* __r
     if (sz > 0) load_strip(16 * wave);
     lds_barrier();
   } else {
-    // Y is stored to LDS first, then the wave's first strip of Sf is
+    // M^-1/2 is stored to LDS first, then the wave's first strip of Sf is
     // loaded; the barriers of this kernel order LDS only, so the Sf loads
     // stay in flight while the transform is formed
-    const double2* Y2 = reinterpret_cast<const double2*>(ymat + (size_t)zl * P128 * P128);
+    const double2* R2 = reinterpret_cast<const double2*>(ymat + (size_t)zl * P128 * P128);
 #pragma unroll
     for (int it = 0; it < P128 * P128 / 1024; ++it) {
       const int e = tid + 512 * it;
-      *reinterpret_cast<double2*>(L.t + (e >> 6) * LDT + 2 * (e & 63)) = Y2[e];
+      *reinterpret_cast<double2*>(L.t + (e >> 6) * LDT + 2 * (e & 63)) = R2[e];
     }
     __builtin_amdgcn_sched_barrier(0);
     if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-    {
-      // 36 lower tiles over 8 waves: the pair of tile rows R0 = w % 4 and
-      // R1 = 7 - w % 4 has 9 tiles; wave w < 4 takes (R0, 0..R0) and
-      // (R1, 0..3-R0), wave w + 4 takes (R1, 4-R0..7-R0).
-      const int R0 = wave & 3, R1 = 7 - R0;
-      const bool hi = wave >= 4;
-      const int jlo = hi ? 4 - R0 : 0, jhi = hi ? 7 - R0 : 3 - R0;  // row R1 range
-      d4 acc0[4], acc1[4];
-#pragma unroll
-      for (int J = 0; J < 4; ++J) acc0[J] = acc1[J] = d4{0, 0, 0, 0};
-      const double* yr = L.t + li * LDT + 2 * kk;
-      for (int p = 0; p < P128 / 8; ++p) {
-        asm volatile("" ::: "memory");
-        const double2 y0 = *reinterpret_cast<const double2*>(yr + 16 * R0 * LDT + 8 * p);
-        const double2 y1 = *reinterpret_cast<const double2*>(yr + 16 * R1 * LDT + 8 * p);
-        // tile columns jlo + J (for the waves w < 4, jlo = 0: also the columns of row R0)
-        double2 yb[4];
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          yb[J] = *reinterpret_cast<const double2*>(yr + 16 * (jlo + J) * LDT + 8 * p);
-        if (!hi) {
-#pragma unroll
-          for (int J = 0; J < 4; ++J)
-            if (J <= R0) {
-              acc0[J] = mfma_f64(y0.x, yb[J].x, acc0[J]);
-              acc0[J] = mfma_f64(y0.y, yb[J].y, acc0[J]);
-            }
-        }
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          if (jlo + J <= jhi) {
-            acc1[J] = mfma_f64(y1.x, yb[J].x, acc1[J]);
-            acc1[J] = mfma_f64(y1.y, yb[J].y, acc1[J]);
-          }
-      }
-      lds_barrier();  // every wave has read Y
-      // D[16 I + lane / 16 + 4 r][16 J + lane % 16]; mirrored entries keep T symmetric
-      auto put = [&](int I, int J, const d4& acc) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = 16 * I + kk + 4 * r, n = 16 * J + li;
-          const double tv = dual ? (m == n ? 1.0 : 0.0) - acc[r] : acc[r];
-          L.t[m * LDT + n] = tv;
-          L.t[n * LDT + m] = tv;
-        }
-      };
-      if (!hi) {
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          if (J <= R0) put(R0, J, acc0[J]);
-      }
-#pragma unroll
-      for (int J = 0; J < 4; ++J)
-        if (jlo + J <= jhi) put(R1, jlo + J, acc1[J]);
-    }
     lds_barrier();
     // Omega = v w^T + P(v) P(w)^T (rrsqrt.F90:737-756, matoper.F90:509-535)
     // applied on the right of the symmetric T (as k_tmat in analysis.hip).
@@ -850,11 +788,11 @@ __global__ __launch_bounds__(512) void k_xform128(int64_t z0, const int32_t* __r
 }
 
 // ---------------------------------------------------------------------------
-// The same for FP32 members (mixed precision): Y is staged in LDS rounded to
-// FP32, Y Y^T runs on v_mfma_f32_16x16x4f32 and T Omega is kept in FP32, the
-// operand precision of the FP32 update that consumes it (the Omega row sums
-// and xa = x0 + Sf a stay in FP64).  The buffers take 78 KB, so two zones
-// share a CU; four waves per zone: wave w owns tile rows w and 7 - w.
+// The same for FP32 members (mixed precision): M^-1/2, rounded to FP32 where
+// it was formed, is staged in LDS and T Omega kept in FP32, the operand
+// precision of the FP32 update that consumes it (the Omega row sums and xa =
+// x0 + Sf a stay in FP64).  The buffers take 74 KB, so two zones share a CU;
+// four waves per zone.
 //   FP32 MFMA layout: A (16x4) lane l holds A[l % 16][l / 16], B (4x16)
 //   B[l / 16][l % 16], D (16x16) register r holds D[4 (l / 16) + r][l % 16].
 // ---------------------------------------------------------------------------
@@ -900,7 +838,6 @@ __global__ __launch_bounds__(256, 2) void k_xform128f(int64_t z0, const int32_t*
     }
   };
   const double* Vz = vec + (size_t)zl * 4 * P128;
-  const bool dual = Vz[3 * P128] < 0.0;  // T = (I - W W^T) Omega (dual.hip)
   if (tid < P128) L.a[tid] = Vz[P128 + tid] / scaling;
   else L.v[tid - P128] = tid - P128 < N ? Vz[2 * P128 + tid - P128] : 0.0;
   if (sel_ptr[z + 1] == sel_ptr[z]) {
@@ -910,68 +847,18 @@ __global__ __launch_bounds__(256, 2) void k_xform128f(int64_t z0, const int32_t*
     if (sz > 0) load_strip(16 * wave);
     lds_barrier();
   } else {
-    const double2* Y2 = reinterpret_cast<const double2*>(ymat + (size_t)zl * P128 * P128);
+    // M^-1/2 as k_func and k_dual_lift leave it for this path, in FP32
+    const float4* R4 = reinterpret_cast<const float4*>(ymat + (size_t)zl * P128 * P128);
+    float4 rv[16];
 #pragma unroll
-    for (int it0 = 0; it0 < P128 * P128 / 512; it0 += 16) {
-      double2 yv[16];
+    for (int u = 0; u < 16; ++u) rv[u] = R4[tid + 256 * u];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) yv[u] = Y2[tid + 256 * (it0 + u)];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = tid + 256 * (it0 + u);
-        *reinterpret_cast<float2*>(L.t + (e >> 6) * LDF + 2 * (e & 63)) =
-            make_float2((float)yv[u].x, (float)yv[u].y);
-      }
+    for (int u = 0; u < 16; ++u) {
+      const int e = tid + 256 * u;
+      *reinterpret_cast<float4*>(L.t + (e >> 5) * LDF + 4 * (e & 31)) = rv[u];
     }
     __builtin_amdgcn_sched_barrier(0);
     if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-    {
-      const int R0 = wave, R1 = 7 - wave;  // tiles (R0, 0..R0) and (R1, 0..R1)
-      f4 acc0[4], acc1[8];
-#pragma unroll
-      for (int J = 0; J < 4; ++J) acc0[J] = f4{0, 0, 0, 0};
-#pragma unroll
-      for (int J = 0; J < 8; ++J) acc1[J] = f4{0, 0, 0, 0};
-      const float* yr = L.t + li * LDF + 2 * kk;
-#pragma unroll 1
-      for (int p = 0; p < P128 / 8; ++p) {
-        const float2 y0 = *reinterpret_cast<const float2*>(yr + 16 * R0 * LDF + 8 * p);
-        const float2 y1 = *reinterpret_cast<const float2*>(yr + 16 * R1 * LDF + 8 * p);
-        float2 yb[8];
-#pragma unroll
-        for (int J = 0; J < 8; ++J) yb[J] = *reinterpret_cast<const float2*>(yr + 16 * J * LDF + 8 * p);
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          if (J <= R0) {
-            acc0[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(y0.x, yb[J].x, acc0[J], 0, 0, 0);
-            acc0[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(y0.y, yb[J].y, acc0[J], 0, 0, 0);
-          }
-#pragma unroll
-        for (int J = 0; J < 8; ++J)
-          if (J <= R1) {
-            acc1[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(y1.x, yb[J].x, acc1[J], 0, 0, 0);
-            acc1[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(y1.y, yb[J].y, acc1[J], 0, 0, 0);
-          }
-      }
-      lds_barrier();  // every wave has read Y
-      // D[16 I + 4 (lane / 16) + r][16 J + lane % 16]; mirrored entries keep T symmetric
-      auto put = [&](int I, int J, const f4& acc) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = 16 * I + 4 * kk + r, n = 16 * J + li;
-          const float tv = dual ? (m == n ? 1.0f : 0.0f) - acc[r] : acc[r];
-          L.t[m * LDF + n] = tv;
-          L.t[n * LDF + m] = tv;
-        }
-      };
-#pragma unroll
-      for (int J = 0; J < 4; ++J)
-        if (J <= R0) put(R0, J, acc0[J]);
-#pragma unroll
-      for (int J = 0; J < 8; ++J)
-        if (J <= R1) put(R1, J, acc1[J]);
-    }
     lds_barrier();
     // Omega on the right of the symmetric T, as in k_xform128 (row sums read
     // as column sums, accumulated in FP64)
@@ -1118,14 +1005,11 @@ void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
                        A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, A.err);
   if (tm) tm->mark(PH_EIG);
   if (A.eig_method == 1) {
-    launch_tql_pipeline(128, A, st);
-    hipLaunchKernelGGL(k_eig128, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.nzc, A.N, A.sel_ptr,
-                       A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol, A.max_sweeps,
-                       (const int32_t*)A.tql_status);
+    launch_func(128, A, false, st);
   } else {
     hipLaunchKernelGGL(k_eig128, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.nzc, A.N, A.sel_ptr,
-                       A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol, A.max_sweeps,
-                       (const int32_t*)nullptr);
+                       A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol, A.max_sweeps);
+    launch_yyt(128, A, st);
   }
 }
 

@@ -463,10 +463,11 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   // interleaved in groups of 4 records over the 64 zones of a QL wave)
   // (about 1.1 N^2 records for typical zones; 2 N^2 + 8 N leaves room for slow ones)
   const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
-  const bool ql = c->eig_method == 1 || NP == 256;  // N > 128: QL only
+  const bool func = c->eig_method == 1 && (NP == 64 || NP == 128);  // funcm.hip
+  const bool ql = (c->eig_method == 1 && NP <= 32) || NP == 256;  // N > 128: QL only
   // zones with 1 <= p < dual_lt in observation space (dual.hip): N > 64, the
   // analysis modes (not the likelihood), not in a no-allocation call
-  const int dual_lt = (NP == 128 && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
+  const int dual_lt = (NP == 128 && func && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
   constexpr int PD = 64;
   const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP) +
                           (ql ? (size_t)cap * 16 + 4 : 0) +
@@ -499,12 +500,15 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   double *dvec = nullptr, *evec = nullptr;
   char* rlog = nullptr;
   int32_t* tst = nullptr;
-  if (ql) {
+  if (ql || func) {
     dvec = (double*)wsget(c, Workspace::DVEC, sizeof(double) * (size_t)NP * zs);
     evec = (double*)wsget(c, Workspace::EVEC, sizeof(double) * (size_t)NP * zs);
+    if (!dvec || !evec) check(c, hipErrorOutOfMemory, "workspace");
+  }
+  if (ql) {
     rlog = (char*)wsget(c, Workspace::RLOG, (size_t)16 * cap * zs);
     tst = (int32_t*)wsget(c, Workspace::TQL_STATUS, sizeof(int32_t) * zs);
-    if (!dvec || !evec || !rlog || !tst) check(c, hipErrorOutOfMemory, "workspace");
+    if (!rlog || !tst) check(c, hipErrorOutOfMemory, "workspace");
   }
   // zone order (not in a no-allocation call: its scratch is sized without it)
   const bool order = c->tune_order == 1 && !c->arena && nz > 1 && nz <= INT32_MAX;
@@ -567,7 +571,7 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     kk.cap = cap;
     kk.NP = NP;
     kk.nslot = nslot;
-    kk.ql = ql;
+    kk.ql = ql + 2 * func;
     kk.ql_zw = c->tune_ql_zw;
     kk.order = order;
     kk.tri_split = c->tune_tri_split;
@@ -605,7 +609,7 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
       }
     }
   } guard{s0, use_graph};
-  if (ql) fill_i32(sweeps_all, nz, 0, s0);
+  if (ql || func) fill_i32(sweeps_all, nz, 0, s0);
   if (order) {
     hipLaunchKernelGGL(k_zone_order, dim3(1), dim3(1024), 0, s0, nz, nchunk, base.sel_ptr, zorder);
     check(c, hipGetLastError(), "zone order");
@@ -640,9 +644,9 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     A.vec = vec + zo * 4 * NP;
     A.umat = umat ? umat + zo * NP * NP : nullptr;
     A.sweeps = sweeps_all + z0;
-    A.eig_method = ql ? 1 : 0;
-    A.dvec = ql ? dvec + zo * NP : nullptr;
-    A.evec = ql ? evec + zo * NP : nullptr;
+    A.eig_method = ql || func ? 1 : 0;
+    A.dvec = dvec ? dvec + zo * NP : nullptr;
+    A.evec = evec ? evec + zo * NP : nullptr;
     A.rlog = ql ? (void*)(rlog + (size_t)16 * cap * zo) : nullptr;
     A.rlog_cap = cap;
     A.tql_status = ql ? tst + zo : nullptr;
@@ -1537,7 +1541,7 @@ size_t noalloc_fixed_bytes(int64_t m, int NP, int64_t nz) {
 size_t noalloc_zone_bytes(int NP, bool ql) {
   const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
   return sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP) +
-         (ql || NP == 256 ? (size_t)cap * 16 + 4 : 0);
+         ((ql && NP <= 32) || NP == 256 ? (size_t)cap * 16 + 4 : 0);
 }
 
 // For the duration of a no-allocation call: the arena over the scratch, the
@@ -1581,6 +1585,7 @@ int oakg_create(oakg_ctx** out, int device, int precision) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || device < 0 || device >= ndev) return OAKG_EHIP;
   if (hipSetDevice(device) != hipSuccess) return OAKG_EHIP;
+  if (init_poles(device) != hipSuccess) return OAKG_EHIP;
   oakg_ctx* c = new (std::nothrow) oakg_ctx;
   if (!c) return OAKG_ENOMEM;
   c->device = device;

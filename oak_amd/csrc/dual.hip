@@ -5,25 +5,25 @@
 // b = S~^T d~.  Its N - p eigenvalues beyond the rank of S~ are exactly 1,
 // and every output of analysisIncrement is a matrix function of M, so it
 // follows from the p x p matrix G = S~ S~^T = U diag(lambda) U^T
-// (mu = max(1 + lambda, 1), as rrsqrt.F90:137 clamps):
+// (mu = 1 + lambda):
 //
-//   a        = M^-1 b        = S~^T U diag(1/mu) U^T d~
-//   M^-1/2                   = I - W W^T,  W = S~^T U diag(1/sqrt(mu^1/2 (1 + mu^1/2)))
-//   M^1/2 1_N                = 1_N + S~^T U diag(1/(1 + mu^1/2)) U^T S~ 1_N
+//   a        = M^-1 b        = S~^T (I + G)^-1 d~
+//   M^-1/2                   = I - S~^T f(I + G) S~,  f(x) = 1 / (x + sqrt x)
+//   M^1/2 1_N                = 1_N + S~^T h(I + G) S~ 1_N,  h(x) = 1 / (1 + sqrt x)
 //
-// (M^-1/2 - I and M^1/2 - I restricted to the range of S~^T; the weights are
-// (mu^-1/2 - 1)/lambda and (mu^1/2 - 1)/lambda written without the
-// cancellation at lambda -> 0).  The p x p eigenproblem runs through the
-// NP = 64 kernels of tridiag.hip (Householder, QL, the eigenvector epilogue
-// with its refinement of (I + G)^-1 d~); k_dual_lift then writes a, the
-// normalised M^1/2 1_N and W into the zone's NP = 128 slots, with a flag
-// (mu[0] = -1) that tells the transform kernels to form T = (I - W W^T) Omega
-// instead of (Y Y^T) Omega.  The work per zone drops from that of a 128 x 128
-// eigensolve to a 64 x 64 one plus two 128 x 64 x 64 products.
+// (M^-1/2 - I and M^1/2 - I restricted to the range of S~^T; f and h are
+// (1 - x^-1/2) / (x - 1) and (x^1/2 - 1) / (x - 1) written without the
+// cancellation at x -> 1).  I + G runs through the NP = 64 reduction and
+// k_func with the weights of f and h (funcm.hip), and k_dual_lift writes a,
+// the normalised M^1/2 1_N and M^-1/2 into the zone's NP = 128 slots, as
+// k_func leaves them for the other zones.  The work per zone drops from that
+// of a 128 x 128 reduction to a 64 x 64 one plus two products of 128 x p with
+// p x p and p x 128.
 //
-//   k_dual_gram   M_d = I + G (64 x 64), b_d = d~ (p rows of HS gathered and
-//                 scaled in LDS, 4 x 4 register blocks of G per thread)
-//   k_dual_lift   a, M^1/2 1_N, W from U diag(mu^-1/4), mu, a_d
+//   k_dual_gram   M_d = I + G (64 x 64), b_d = d~, S~ 1_N (p rows of HS
+//                 gathered and scaled in LDS, 4 x 4 register blocks of G per
+//                 thread)
+//   k_dual_lift   a, M^1/2 1_N, M^-1/2 from f(I + G) and the two vectors
 #include "analysis.hpp"
 #include "common.hpp"
 
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void k_dual_gram(int64_t z0, const int32_t* __
                                                    const double* __restrict__ innov,
                                                    const TS* __restrict__ HS,
                                                    double* __restrict__ mat_d,
-                                                   double* __restrict__ vec_d,
+                                                   double* __restrict__ vec_d, int N,
                                                    unsigned* __restrict__ err) {
   __shared__ double s[PD][LDS_S];
   __shared__ double dq[PD], sr[PD];
@@ -125,87 +125,88 @@ __global__ __launch_bounds__(256) void k_dual_gram(int64_t z0, const int32_t* __
       const int q = 4 * qb + i, k = 4 * kb + j;
       Md[q * PD + k] = acc[i][j] + (q == k ? 1.0 : 0.0);
     }
-  if (tid < PD) vec_d[(size_t)zl * 4 * PD + tid] = dq[tid];
+  if (tid < PD) {
+    double a = 0.0;
+    for (int c = 0; c < N; ++c) a += s[tid][c];
+    vec_d[(size_t)zl * 4 * PD + tid] = dq[tid];
+    vec_d[(size_t)zl * 4 * PD + 2 * PD + tid] = a;
+  }
 }
 
+// M^-1/2 = I - S~^T (f S~) on v_mfma_f64_16x16x4f64: wave w forms tile columns
+// w and w + 4 of Z = f S~ (its accumulators are the B operands of the second
+// product), with the zone's p rows only.  TS is the type of S and of M^-1/2.
 template <typename TS>
-__global__ __launch_bounds__(256) void k_dual_lift(int64_t z0, const int32_t* __restrict__ zorder,
-                                                   int N, const int64_t* __restrict__ sel_ptr,
-                                                   const int32_t* __restrict__ sel_idx,
-                                                   const double* __restrict__ sel_w, int64_t m,
-                                                   const double* __restrict__ rho,
-                                                   const double* __restrict__ innov,
-                                                   const TS* __restrict__ HS,
-                                                   const double* __restrict__ ymat_d,
-                                                   const double* __restrict__ vec_d,
-                                                   double* __restrict__ ymat,
-                                                   double* __restrict__ vec,
-                                                   double* __restrict__ ampl,
-                                                   unsigned* __restrict__ err) {
+__global__ __launch_bounds__(256, 2) void k_dual_lift(int64_t z0, const int32_t* __restrict__ zorder,
+                                                      int N, const int64_t* __restrict__ sel_ptr,
+                                                      const int32_t* __restrict__ sel_idx,
+                                                      const double* __restrict__ sel_w, int64_t m,
+                                                      const double* __restrict__ rho,
+                                                      const double* __restrict__ innov,
+                                                      const TS* __restrict__ HS,
+                                                      const double* __restrict__ ymat_d,
+                                                      const double* __restrict__ vec_d,
+                                                      double* __restrict__ ymat,
+                                                      double* __restrict__ vec,
+                                                      double* __restrict__ ampl,
+                                                      unsigned* __restrict__ err) {
   __shared__ double s[PD][LDS_S];
-  __shared__ double dq[PD], sr[PD], ad[PD], q2[PD], t1[PD], t4[PD], red[4];
+  __shared__ double dq[PD], sr[PD], red[4];
   const int zl = blockIdx.x;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
   const int64_t p0 = sel_ptr[z];
   const int64_t p = sel_ptr[z + 1] - p0;
-  const int tid = threadIdx.x;
-  const double* Yd = ymat_d + (size_t)zl * PD * PD;  // U diag(mu^-1/4)
-  const double* Vd = vec_d + (size_t)zl * 4 * PD;     // [PD..2PD) a_d, [3PD..4PD) mu
-  if (tid < PD) {
-    q2[tid] = sqrt(Vd[3 * PD + tid]);  // mu^1/2
-    ad[tid] = Vd[PD + tid];
-  }
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lr = lane >> 4, lc = lane & 15;
+  const double* F = ymat_d + (size_t)zl * PD * PD;
+  const double* Vd = vec_d + (size_t)zl * 4 * PD;  // [PD..2PD) (I+G)^-1 d~, [2PD..3PD) h S~ 1
   load_rows<TS>(s, dq, p0, p, sel_idx, sel_w, m, rho, innov, HS, err, sr);
-  // t1 = S~ 1_N
-  if (tid < PD) {
-    double a = 0.0;
-    for (int c = 0; c < N; ++c) a += s[tid][c];
-    t1[tid] = a;
-  }
-  lds_barrier();
-  // t4 = U diag(1/(1 + mu^1/2)) U^T t1 = Yd diag(mu^1/2 / (1 + mu^1/2)) Yd^T t1
-  if (tid < PD) {
-    double a = 0.0;
-    for (int q = 0; q < PD; ++q) a = fma(Yd[q * PD + tid], t1[q], a);
-    dq[tid] = a * (q2[tid] / (1.0 + q2[tid]));  // dq is free after load_rows
-  }
-  lds_barrier();
-  if (tid < PD) {
-    double a = 0.0;
-    for (int j = 0; j < PD; ++j) a = fma(Yd[tid * PD + j], dq[j], a);
-    t4[tid] = a;
-  }
-  // W = S~^T Yd diag(c), c_j = 1/sqrt(1 + mu_j^1/2): thread (column j, block
-  // of 32 rows); the rows of S~ are read as LDS broadcasts, Yd as coalesced
-  // rows from global memory
-  {
-    const int j = tid & 63, ib = tid >> 6;
-    const double cj = 1.0 / sqrt(1.0 + q2[j]);
-    double acc[32];
+  const int ni = ((int)p + 15) >> 4, nk = ((int)p + 3) >> 2;  // row tiles, k-steps (p < 64)
+  d4 zt[2][4];
 #pragma unroll
-    for (int ii = 0; ii < 32; ++ii) acc[ii] = 0.0;
-    for (int q = 0; q < p; ++q) {
-      const double wq = Yd[q * PD + j] * cj;
+  for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-      for (int ii = 0; ii < 32; ++ii) acc[ii] = fma(s[q][32 * ib + ii], wq, acc[ii]);
-    }
-    double* Y = ymat + (size_t)zl * NPP * NPP;
+    for (int I = 0; I < 4; ++I) zt[jj][I] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int k = 0; k < nk; ++k) {
+    const double b0 = s[4 * k + lr][16 * wave + lc], b1 = s[4 * k + lr][16 * (wave + 4) + lc];
 #pragma unroll
-    for (int ii = 0; ii < 32; ++ii) {
-      Y[(size_t)(32 * ib + ii) * NPP + j] = acc[ii];
-      Y[(size_t)(32 * ib + ii) * NPP + PD + j] = 0.0;
+    for (int I = 0; I < 4; ++I)
+      if (I < ni) {
+        const double fv = F[(16 * I + lc) * PD + 4 * k + lr];
+        zt[0][I] = mfma_f64(fv, b0, zt[0][I]);
+        zt[1][I] = mfma_f64(fv, b1, zt[1][I]);
+      }
+  }
+  TS* R = reinterpret_cast<TS*>(ymat + (size_t)zl * NPP * NPP);
+#pragma unroll 1
+  for (int I = 0; I < 8; ++I) {
+    d4 x0 = {0.0, 0.0, 0.0, 0.0}, x1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int K = 0; K < 4; ++K)
+      if (K < ni) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double av = s[16 * K + 4 * q + lr][16 * I + lc];
+          x0 = mfma_f64(av, zt[0][K][q], x0);
+          x1 = mfma_f64(av, zt[1][K][q], x1);
+        }
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * I + lr + 4 * r, c0 = 16 * wave + lc, c1 = c0 + 64;
+      R[(size_t)row * NPP + c0] = (TS)((row == c0 ? 1.0 : 0.0) - x0[r]);
+      R[(size_t)row * NPP + c1] = (TS)((row == c1 ? 1.0 : 0.0) - x1[r]);
     }
   }
-  lds_barrier();  // t4
   double* V = vec + (size_t)zl * 4 * NPP;
   // a, M^1/2 1_N (rows i < 128, threads 0..127; the other waves add zeros)
   const int i = tid;
   double vr = 0.0, ar = 0.0;
   if (tid < NPP) {
     for (int q = 0; q < p; ++q) {
-      ar = fma(s[q][i], ad[q], ar);
-      vr = fma(s[q][i], t4[q], vr);
+      ar = fma(s[q][i], Vd[PD + q], ar);
+      vr = fma(s[q][i], Vd[2 * PD + q], vr);
     }
     vr += i < N ? 1.0 : 0.0;
   }
@@ -217,7 +218,6 @@ __global__ __launch_bounds__(256) void k_dual_lift(int64_t z0, const int32_t* __
     V[i] = 0.0;
     V[NPP + i] = ar;
     V[2 * NPP + i] = vr / sqrt(nv);
-    V[3 * NPP + i] = i == 0 ? -1.0 : 0.0;  // dual flag for the transform kernels
     if (ampl && i < N) ampl[(size_t)z * N + i] = ar;
     if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
   }
@@ -228,12 +228,12 @@ void launch_dual128(const ChunkArgs& A, int N, double* ymat128, double* vec128, 
   if (tm) tm->mark(PH_GRAM);
   if (A.prec == 1)
     hipLaunchKernelGGL(k_dual_gram<float>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.mat, A.vec, A.err);
+                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.mat, A.vec, N, A.err);
   else
     hipLaunchKernelGGL(k_dual_gram<double>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, A.err);
+                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, N, A.err);
   if (tm) tm->mark(PH_EIG);
-  launch_eig_small(PD, A, st);
+  launch_func(PD, A, true, st);
   if (A.prec == 1)
     hipLaunchKernelGGL(k_dual_lift<float>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, N,
                        A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.ymat, A.vec,

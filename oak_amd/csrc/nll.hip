@@ -79,7 +79,8 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
   for (int c = 0; c < KPL; ++c) {
     const int k = lane + 64 * c;
     ak[c] = k < NP ? V[NP + k] : 0.0;
-    wk[c] = k < NP ? 1.0 / sqrt(V[3 * NP + k]) : 0.0;  // mu_k^-1/2
+    // NP >= 64: Y is M^-1/2, u = |M^-1/2 s|^2; else u = sum_k mu_k^-1/2 (Y^T s)_k^2
+    wk[c] = NP >= 64 ? 1.0 : (k < NP ? 1.0 / sqrt(V[3 * NP + k]) : 0.0);
   }
   const double Lz = corr[z];
   double accL = 0.0, accR = 0.0, accLog = 0.0;
@@ -131,16 +132,16 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
     // (padding entries have mu = 1, a = b = 0)
     double slog = 0, sinv = 0, aa = 0, ba = 0;
     for (int k = lane; k < NP; k += 64) {
-      const double mu = V[3 * NP + k], ak2 = V[NP + k];
+      const double mu = NP >= 64 ? 1.0 : V[3 * NP + k], ak2 = V[NP + k];
       slog += log(mu);
       sinv += 1.0 - 1.0 / mu;
       aa = fma(ak2, ak2, aa);
       ba = fma(V[k], ak2, ba);
     }
-    slog = nll_wave_sum(slog);
-    sinv = nll_wave_sum(sinv);
+    slog = NP >= 64 ? V[3 * NP] : nll_wave_sum(slog);
+    sinv = NP >= 64 ? V[3 * NP + 1] : nll_wave_sum(sinv);
     aa = nll_wave_sum(aa);
-    ba = nll_wave_sum(ba);
+    ba = NP >= 64 ? V[3 * NP + 2] : nll_wave_sum(ba);
     if (lane == 0) {
       const double sL = ((red[0][0] + red[1][0]) + red[2][0]) + red[3][0];
       const double sR = ((red[0][1] + red[1][1]) + red[2][1]) + red[3][1];

@@ -520,153 +520,6 @@ __global__ __launch_bounds__(256) void k_tridiag(int64_t z0, const int32_t* __re
 }
 
 // ---------------------------------------------------------------------------
-// Q = H_0 H_1 ... H_125 for NP = 128 from the reflectors k_tridiag leaves in
-// the rows of qmat (row k: v_k, with tau_k in its otherwise zero entry k),
-// accumulated backwards in blocks of 16 reflectors in compact WY form
-// (LAPACK dlarft / dlarfb): H_k0 ... H_k0+15 = I - Vb Tb Vb^T with Tb upper
-// triangular, and Q <- Q - Vb (Tb (Vb^T Q)), all products on
-// v_mfma_f64_16x16x4f64.  Q stays in the accumulators: wave w holds tile
-// columns w and 7 - w (8 tiles of 16 x 16 each, so the waves get similar
-// work as the active block grows); block b touches only tiles (I, J) with
-// I, J >= b.  The D register kk of a tile is the B operand of the k-step
-// over its rows 4 kk .. 4 kk + 3, so the three products chain in registers.
-// The next block's reflectors are loaded while a block is applied.  Q is
-// written with its columns reversed, as k_tridiag writes it for NP < 128.
-// ---------------------------------------------------------------------------
-struct FormQLds {
-  // padded row of Vb and Tb: with 18 doubles the MFMA operand reads of 64
-  // lanes (16 rows x 4, or 16 columns x 4) and the staging writes below fall
-  // on distinct bank pairs as far as 64 lanes allow
-  static constexpr int LV = 18;
-  double vb[2][128 * LV];        // Vb[r][j]: row r of reflector k0 + j
-  double tb[2][16 * LV];         // Tb
-  double g[16 * LV];             // Vb^T Vb
-  double tau[2][16];
-};
-
-__global__ __launch_bounds__(256, 2) void k_formq128(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
-                                                  double* __restrict__ qmat) {
-  constexpr int NP = 128, NB = 8, LV = FormQLds::LV;
-  __shared__ FormQLds S;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;  // the zone is solved by the other pipeline
-  if (sel_ptr[z + 1] == sel_ptr[z]) return;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int lr = lane >> 4, lc = lane & 15;
-  double* V = qmat + (size_t)zl * NP * NP;
-  const int J0 = wave, J1 = 7 - wave;
-  d4 q[2][8];
-#pragma unroll
-  for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-    for (int I = 0; I < 8; ++I)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        q[jj][I][r] = (I == (jj ? J1 : J0) && lr + 4 * r == lc) ? 1.0 : 0.0;
-  // thread t moves reflector pj = t / 16 of a block, rows pr + 16 e (e < 8):
-  // 16 threads read 16 consecutive values of a reflector row, and their
-  // LDS stores (row stride LV) spread over the banks
-  const int pj = t >> 4, pr = t & 15;
-  double pf[8];
-  auto load_block = [&](int b) {
-    const int k = 16 * b + pj;
-    if (k < NP - 2) {
-      const double* src = V + (size_t)k * NP + pr;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) pf[e] = src[16 * e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) pf[e] = 0.0;
-    }
-  };
-  load_block(NB - 1);
-  for (int b = NB - 1; b >= 0; --b) {
-    const int buf = b & 1;
-    double* vb = S.vb[buf];
-    double* tb = S.tb[buf];
-    {
-      const int k = 16 * b + pj;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int r = pr + 16 * e;
-        vb[r * LV + pj] = r <= k ? 0.0 : pf[e];  // v_k is zero above row k + 1
-        if (r == k) S.tau[buf][pj] = pf[e];
-      }
-    }
-    if (b > 0) load_block(b - 1);
-    lds_barrier();
-    // (1) wave 0: G = Vb^T Vb (rows >= 16 b), then Tb column by column:
-    //     Tb[j][j] = tau_j, Tb[0:j, j] = -tau_j Tb[0:j, 0:j] G[0:j, j]
-    if (wave == 0) {
-      d4 g = {0.0, 0.0, 0.0, 0.0};
-      for (int kk = 4 * b; kk < 32; ++kk) {
-        const double x = vb[(4 * kk + lr) * LV + lc];
-        g = mfma_f64(x, x, g);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S.g[(lr + 4 * r) * LV + lc] = g[r];
-      __builtin_amdgcn_wave_barrier();
-      if (lane < 16) {
-        double tr[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          asm volatile("" ::: "memory");  // G column by column, not all loads at once
-          double s = 0.0;
-#pragma unroll
-          for (int k = 0; k < j; ++k) s = fma(tr[k], S.g[k * LV + j], s);
-          const double tj = S.tau[buf][j];
-          tr[j] = lane < j ? -tj * s : (lane == j ? tj : 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) tb[lane * LV + j] = tr[j];
-      }
-    }
-    // (2) W_J = Vb^T Q[:, J] for the wave's tile columns J >= b
-    d4 w[2];
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      w[jj] = d4{0.0, 0.0, 0.0, 0.0};
-      if ((jj ? J1 : J0) >= b) {
-#pragma unroll
-        for (int I = 0; I < 8; ++I)
-          if (I >= b) {
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-              w[jj] = mfma_f64(vb[(16 * I + 4 * kk + lr) * LV + lc], q[jj][I][kk], w[jj]);
-          }
-      }
-    }
-    lds_barrier();  // Tb
-    // (3) W'_J = -Tb W_J;  Q[I][J] += Vb[I rows] W'_J
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      if ((jj ? J1 : J0) >= b) {
-        d4 wp = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) wp = mfma_f64(-tb[lc * LV + 4 * kk + lr], w[jj][kk], wp);
-#pragma unroll
-        for (int I = 0; I < 8; ++I)
-          if (I >= b) {
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-              q[jj][I] = mfma_f64(vb[(16 * I + lc) * LV + 4 * kk + lr], wp[kk], q[jj][I]);
-          }
-      }
-    }
-  }
-  // every reflector row was read before the last barrier
-#pragma unroll
-  for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-    for (int I = 0; I < 8; ++I)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        V[(size_t)(16 * I + lr + 4 * r) * NP + (NP - 1 - (16 * (jj ? J1 : J0) + lc))] = q[jj][I][r];
-}
-
-
-
 // Implicit QL with Wilkinson shifts on (d, e), one lane per zone (EISPACK
 // tql2 ordering: eigenvalue l converges at the top of the block l..m).  The
 // end m of the unreduced block is carried from one sweep to the next: the
@@ -914,92 +767,6 @@ __global__ __launch_bounds__(NP < 64 ? 64 : NP) void k_tql_apply(int64_t z0, con
 }
 
 // ---------------------------------------------------------------------------
-// U = Q Z for NP = 64 with the rows in registers: thread r holds row r of Q
-// whole (64 values), so a chain needs no other thread; it runs in unrolled,
-// branch-free segments of 16 positions with the identity (1, 0) outside the
-// chain, the (c, s) of each position from a table in LDS (the scheme of
-// k_tql_apply128's groups).  The operations on a row are those of
-// k_tql_apply.  One wave per zone.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_tql_apply64(int64_t z0, const int32_t* __restrict__ zorder,
-                                                     const int64_t* __restrict__ sel_ptr,
-                                                     double* __restrict__ qmat,
-                                                     const double2* __restrict__ rlog,
-                                                     int64_t cap,
-                                                     const int32_t* __restrict__ status) {
-  constexpr int NP = 64;
-  __shared__ double2 buf[2][NP + 12];
-  __shared__ double2 pr[NP];
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;  // the zone is solved by the other pipeline
-  if (sel_ptr[z + 1] == sel_ptr[z]) return;
-  const int stz = status[zl];
-  if (stz & 3) return;  // failed zone: solved again by the fallback
-  const int tid = threadIdx.x;
-  double* Qr = qmat + (size_t)zl * NP * NP + (size_t)tid * NP;
-  double x[NP];
-  {
-    const double2* q2 = reinterpret_cast<const double2*>(Qr);
-#pragma unroll
-    for (int c = 0; c < NP / 2; ++c) {
-      const double2 v = q2[c];
-      x[2 * c] = v.x;
-      x[2 * c + 1] = v.y;
-    }
-  }
-  const int64_t len = stz >> 2;
-  const double2* lg = rlog + rlog_off(zl, cap);
-  if (tid < len) buf[0][tid] = lg[rlog_rec(tid)];
-  __syncthreads();
-  int64_t pos = 0;
-  int b = 0;
-  while (pos < len) {
-    const double2 hd = buf[b][0];
-    const int m = __builtin_amdgcn_readfirstlane(((int)hd.x) >> 16);
-    const int cnt = __builtin_amdgcn_readfirstlane((int)hd.y);
-    const int l = m - cnt;
-    const int64_t nxt = pos + 1 + cnt;
-    const bool pf = nxt + tid < len;
-    double2 pv = make_double2(0.0, 0.0);
-    if (pf) pv = lg[rlog_rec(nxt + tid)];
-    // positions m-1 .. l: rotation of columns P and P+1 with the record of
-    // position P
-    pr[tid] = (tid >= l && tid <= m - 1) ? buf[b][1 + (m - 1 - tid)] : make_double2(1.0, 0.0);
-    auto segment = [&](auto top) {
-      constexpr int T = decltype(top)::value;
-      if (m - 1 < T - 15 || l > T) return;
-      double2 qv[16];
-#pragma unroll
-      for (int t = 0; t < 16; ++t)
-        if (T - t >= 0) qv[t] = pr[T - t];
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const int J = T - t;
-        if (J >= 0) {
-          const double hh = x[J + 1], zj = x[J];
-          x[J + 1] = fma(qv[t].y, zj, qv[t].x * hh);
-          x[J] = fma(qv[t].x, zj, -qv[t].y * hh);
-        }
-      }
-    };
-    segment(std::integral_constant<int, 62>{});
-    segment(std::integral_constant<int, 46>{});
-    segment(std::integral_constant<int, 30>{});
-    segment(std::integral_constant<int, 14>{});
-    if (pf) buf[b ^ 1][tid] = pv;
-    __syncthreads();
-    pos = nxt;
-    b ^= 1;
-  }
-  {
-    double2* q2 = reinterpret_cast<double2*>(Qr);
-#pragma unroll
-    for (int c = 0; c < NP / 2; ++c) q2[c] = make_double2(x[2 * c], x[2 * c + 1]);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // U = Q Z for NP = 256 with the rows in registers, the scheme of
 // k_tql_apply128 (below) at twice the width: workgroup y takes rows
 // 128 y .. 128 y + 127, row r's columns 0..127 in thread r (waves 0-1, the
@@ -1176,349 +943,6 @@ __global__ __launch_bounds__(256) void k_tql_apply256(int64_t z0, const int32_t*
 }
 
 // ---------------------------------------------------------------------------
-// U = Q Z for NP = 128 with the rows in registers.  A chain (one QL sweep,
-// from its first position m-1 down to l) runs as unrolled, branch-free
-// segments of 16 positions, each segment it meets with the identity at the
-// positions it does not cover (a jump into the middle of an unrolled sequence
-// is not structured control flow, and the compiler's rewriting of it copies
-// the registers around); the (c, s) of a segment come from a per-wave,
-// position-indexed table in LDS.  The arithmetic of every rotation is that of
-// k_tql_apply.  The LDS of the rotation phase is reused by the load of Q and
-// by the epilogue, to stage a half of U for its column sums.
-// ---------------------------------------------------------------------------
-// k_tql_apply128 (N > 64): the logged rotations applied to the rows of Q,
-// then the epilogue of k_eigvec_epi.  Each row of Q is split over two
-// threads, row r's columns 0..63 in thread r (waves 0-1, the lower group) and
-// columns 64..127 in thread 128 + r (waves 2-3, the upper group): 64 values a
-// thread, all in VGPRs.  A chain of rotations (positions m-1 down to l) acts
-// on the upper columns (positions >= 64), couples columns 63 and 64 (position
-// 63), then acts on the lower columns (positions <= 62).  The groups run one
-// chain apart: in step t the upper group applies chain t while the lower
-// group applies chain t-1, both after the coupling rotation of chain t-1,
-// which each group computes from its own column and the other group's column
-// published at the end of step t-1 (same inputs and operations in both
-// groups, so the two copies agree bit for bit).  The records of chains t+1,
-// t and t-1 are in three buffers.
-struct Apply128Lds {
-  union {
-    double z[8 + 128 * 65];  // a staged half of U, row stride 65 (load and epilogue)
-    struct {
-      double2 buf[3][128 + 12];  // records of chains t+1, t, t-1
-      double2 pr[4][64];         // per wave: (c, s) of its group's positions
-      double xc[2][2][128];      // [step parity][0: column 63, 1: column 64] per row
-    } r;
-  };
-  double ev[5][128];    // epilogue vectors
-  double part[2][4][64];  // partial column sums of four row quarters
-  double hd[2][2][128];   // [0: x, 1: y][group] partial row products
-};
-
-__global__ __launch_bounds__(256) void k_tql_apply128(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
-                                                       const double* __restrict__ mat,
-                                                       double* __restrict__ qmat,
-                                                       const double2* __restrict__ rlog,
-                                                       int64_t cap,
-                                                       const int32_t* __restrict__ status,
-                                                       const double* __restrict__ dvec, int nzc,
-                                                       double* __restrict__ vec,
-                                                       double* __restrict__ ampl,
-                                                       unsigned* __restrict__ err, int refine) {
-  constexpr int NP = 128, H = 64, LD = 65;
-  __shared__ Apply128Lds S;
-  double* Z = S.z + 8;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;  // the zone is solved by the other pipeline
-  const int tid = threadIdx.x;
-  const int g = tid >> 7, r = tid & 127, w = tid >> 6, lane = tid & 63;
-  if (sel_ptr[z + 1] == sel_ptr[z]) {  // no observations: a = 0
-    if (tid < NP) vec[(size_t)zl * 4 * NP + NP + tid] = 0.0;
-    return;
-  }
-  const int stz = status[zl];
-  if (stz & 3) return;  // failed zone: solved again by the fallback
-  double* Q = qmat + (size_t)zl * NP * NP;
-  double x[H];  // row r, columns 64 g .. 64 g + 63
-  copy_batched<16>(tid, NP * H, 256, [&](int e) { return Q[(e >> 6) * NP + H + (e & 63)]; },
-                   [&](int e, double v) { Z[(e >> 6) * LD + (e & 63)] = v; });
-  __syncthreads();
-  if (g == 1) {
-#pragma unroll
-    for (int c = 0; c < H; ++c) x[c] = Z[r * LD + c];
-  }
-  __syncthreads();
-  copy_batched<16>(tid, NP * H, 256, [&](int e) { return Q[(e >> 6) * NP + (e & 63)]; },
-                   [&](int e, double v) { Z[(e >> 6) * LD + (e & 63)] = v; });
-  __syncthreads();
-  if (g == 0) {
-#pragma unroll
-    for (int c = 0; c < H; ++c) x[c] = Z[r * LD + c];
-  }
-  __syncthreads();  // Z is now reused by the record buffers
-  const int64_t len = stz >> 2;
-  const double2* lg = rlog + rlog_off(zl, cap);
-  if (tid < len && tid < NP) S.r.buf[0][tid] = lg[rlog_rec(tid)];
-  __syncthreads();
-  int64_t pos = 0;
-  int bt = 0, bp = 2, par = 0;
-  bool has_prev = false;
-  int m_prev = 0, l_prev = 0;
-  double2* pr = S.r.pr[w];
-  while (true) {
-    const bool has_cur = pos < len;
-    if (!has_cur && !has_prev) break;
-    int m = 0, l = 0;
-    int64_t nxt = pos;
-    if (has_cur) {
-      const double2 hd = S.r.buf[bt][0];
-      m = __builtin_amdgcn_readfirstlane(((int)hd.x) >> 16);
-      const int cnt = __builtin_amdgcn_readfirstlane((int)hd.y);
-      l = m - cnt;
-      nxt = pos + 1 + cnt;
-    }
-    const int bn = bt == 2 ? 0 : bt + 1;
-    const bool pf = has_cur && tid < NP && nxt + tid < len;
-    double2 pv = make_double2(0.0, 0.0);
-    if (pf) pv = lg[rlog_rec(nxt + tid)];
-    // coupling rotation (position 63) of chain t-1
-    if (has_prev && l_prev <= H - 1 && m_prev - 1 >= H - 1) {
-      const double2 q = S.r.buf[bp][1 + (m_prev - 1) - (H - 1)];
-      const double c64 = g == 1 ? x[0] : S.r.xc[par ^ 1][1][r];
-      const double c63 = g == 0 ? x[H - 1] : S.r.xc[par ^ 1][0][r];
-      const double n64 = fma(q.y, c63, q.x * c64);
-      const double n63 = fma(q.x, c63, -q.y * c64);
-      if (g == 1) x[0] = n64;
-      else x[H - 1] = n63;
-    }
-    if (g == 1) {
-      if (has_cur && m - 1 >= H) {
-        // chain t on columns 64..127: positions 126..64 in four unrolled
-        // segments of 16 with the identity (1, 0) outside l..m-1
-        {
-          const int P = H + lane;
-          pr[lane] = (P >= l && P <= m - 1) ? S.r.buf[bt][1 + (m - 1 - P)] : make_double2(1.0, 0.0);
-        }
-        auto segment = [&](auto top) {
-          constexpr int T = decltype(top)::value;
-          if (m - 1 < T - 15 || l > T) return;
-          double2 qv[16];
-#pragma unroll
-          for (int t = 0; t < 16; ++t)
-            if (T - t >= H) qv[t] = pr[T - t - H];
-#pragma unroll
-          for (int t = 0; t < 16; ++t) {
-            const int J = T - t;
-            if (J >= H) {
-              const double hh = x[J + 1 - H], zj = x[J - H];
-              x[J + 1 - H] = fma(qv[t].y, zj, qv[t].x * hh);
-              x[J - H] = fma(qv[t].x, zj, -qv[t].y * hh);
-            }
-          }
-        };
-        segment(std::integral_constant<int, 126>{});
-        segment(std::integral_constant<int, 110>{});
-        segment(std::integral_constant<int, 94>{});
-        segment(std::integral_constant<int, 78>{});
-      }
-      S.r.xc[par][1][r] = x[0];
-    } else {
-      if (has_prev && l_prev <= H - 2) {
-        // chain t-1 on columns 0..63: positions 62..l
-        const int mp = m_prev, lp = l_prev;
-        pr[lane] = (lane >= lp && lane <= mp - 1 && lane <= H - 2) ? S.r.buf[bp][1 + (mp - 1 - lane)]
-                                                                   : make_double2(1.0, 0.0);
-        auto segment_lo = [&](auto top) {
-          constexpr int T = decltype(top)::value;
-          if (mp - 1 < T - 15 || lp > T) return;
-          double2 qv[16];
-#pragma unroll
-          for (int t = 0; t < 16; ++t)
-            if (T - t >= 0) qv[t] = pr[T - t];
-#pragma unroll
-          for (int t = 0; t < 16; ++t) {
-            const int J = T - t;
-            if (J >= 0) {
-              const double hh = x[J + 1], zj = x[J];
-              x[J + 1] = fma(qv[t].y, zj, qv[t].x * hh);
-              x[J] = fma(qv[t].x, zj, -qv[t].y * hh);
-            }
-          }
-        };
-        segment_lo(std::integral_constant<int, 62>{});
-        segment_lo(std::integral_constant<int, 46>{});
-        segment_lo(std::integral_constant<int, 30>{});
-        segment_lo(std::integral_constant<int, 14>{});
-      }
-      S.r.xc[par][0][r] = x[H - 1];
-    }
-    if (pf) S.r.buf[bn][tid] = pv;
-    __syncthreads();
-    has_prev = has_cur;
-    m_prev = m;
-    l_prev = l;
-    bp = bt;
-    bt = bn;
-    pos = nxt;
-    par ^= 1;
-  }
-  // ---- epilogue: the quantities of k_eigvec_epi from the half rows in hand ----
-  double* mu = S.ev[0];  // mu_j = max(lambda_j, 1) of column j
-  double* bv = S.ev[1];  // b
-  double* xv = S.ev[2];  // U^T b / mu, then U^T (b - M a0) / mu
-  double* yv = S.ev[3];  // U^T 1_N sqrt(mu), then mu^-1/4
-  double* av = S.ev[4];  // a0, then b - M a0, then vr^2
-  double* V = vec + (size_t)zl * 4 * NP;
-  if (tid < NP) {
-    mu[tid] = fmax(dvec[(size_t)tid * nzc + zl], 1.0);
-    bv[tid] = V[tid];
-  }
-  const int cc = tid & 63, q4 = tid >> 6;
-  auto stage = [&](int grp) {
-    if (g == grp) {
-#pragma unroll
-      for (int c = 0; c < H; ++c) Z[r * LD + c] = x[c];
-    }
-    __syncthreads();
-  };
-  // U^T b and U^T 1_N over the staged half (column offset co), rows in quarters
-  auto colsum2 = [&](int co) {
-    double s1[4] = {0, 0, 0, 0}, s2[4] = {0, 0, 0, 0};
-#pragma unroll 2
-    for (int r0 = 32 * q4; r0 < 32 * q4 + 32; r0 += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int rr = r0 + u;
-        const double zz = Z[rr * LD + cc];
-        s1[u] = fma(zz, bv[rr], s1[u]);
-        s2[u] += rr < N ? zz : 0.0;
-      }
-    }
-    S.part[0][q4][cc] = (s1[0] + s1[1]) + (s1[2] + s1[3]);
-    S.part[1][q4][cc] = (s2[0] + s2[1]) + (s2[2] + s2[3]);
-    __syncthreads();
-    if (tid < 64) {
-      const double c1 = (S.part[0][0][tid] + S.part[0][1][tid]) + (S.part[0][2][tid] + S.part[0][3][tid]);
-      const double c2 = (S.part[1][0][tid] + S.part[1][1][tid]) + (S.part[1][2][tid] + S.part[1][3][tid]);
-      xv[co + tid] = c1 / mu[co + tid];
-      yv[co + tid] = c2 * sqrt(mu[co + tid]);
-    }
-    __syncthreads();
-  };
-  auto colsum1 = [&](int co) {
-    double s1[4] = {0, 0, 0, 0};
-#pragma unroll 2
-    for (int r0 = 32 * q4; r0 < 32 * q4 + 32; r0 += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) s1[u] = fma(Z[(r0 + u) * LD + cc], av[r0 + u], s1[u]);
-    }
-    S.part[0][q4][cc] = (s1[0] + s1[1]) + (s1[2] + s1[3]);
-    __syncthreads();
-    if (tid < 64)
-      xv[co + tid] = ((S.part[0][0][tid] + S.part[0][1][tid]) + (S.part[0][2][tid] + S.part[0][3][tid])) /
-                     mu[co + tid];
-    __syncthreads();
-  };
-  // half-row products (U x)_r over the group's columns, into hd[.][g][r]
-  auto rowdot_h = [&](const double* xa, const double* ya) {
-    double tx = 0, ty = 0;
-#pragma unroll
-    for (int c0 = 0; c0 < H; c0 += 16) {
-      double2 xx[8], yy[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        xx[u] = reinterpret_cast<const double2*>(xa + H * g + c0)[u];
-        if (ya) yy[u] = reinterpret_cast<const double2*>(ya + H * g + c0)[u];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        tx = fma(x[c0 + 2 * u], xx[u].x, tx);
-        tx = fma(x[c0 + 2 * u + 1], xx[u].y, tx);
-        if (ya) {
-          ty = fma(x[c0 + 2 * u], yy[u].x, ty);
-          ty = fma(x[c0 + 2 * u + 1], yy[u].y, ty);
-        }
-      }
-    }
-    S.hd[0][g][r] = tx;
-    if (ya) S.hd[1][g][r] = ty;
-  };
-  stage(0);
-  colsum2(0);
-  stage(1);
-  colsum2(H);  // the upper half stays staged
-  rowdot_h(xv, yv);
-  __syncthreads();
-  double a0 = 0, vr = 0;
-  if (tid < NP) {
-    a0 = S.hd[0][0][tid] + S.hd[0][1][tid];
-    vr = S.hd[1][0][tid] + S.hd[1][1][tid];
-    av[tid] = a0;
-  }
-  __syncthreads();
-  // refinement a = a0 + U diag(1/mu) U^T (b - M a0) (FP64 path; the mixed
-  // path's bound of 1e-4 is far above the cross-talk it removes); M
-  // symmetric: row r of M a0 from column r, half of the columns per group
-  // (32 loads in flight)
-  double ar = a0;
-  if (refine) {
-    {
-      const double* M = mat + (size_t)zl * NP * NP;
-      double mq[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int c0 = 0; c0 < H; c0 += 32) {
-        double mv[32];
-#pragma unroll
-        for (int u = 0; u < 32; ++u) mv[u] = M[(size_t)(H * g + c0 + u) * NP + r];
-#pragma unroll
-        for (int u = 0; u < 32; ++u) mq[u & 7] = fma(mv[u], av[H * g + c0 + u], mq[u & 7]);
-      }
-      S.hd[0][g][r] = ((mq[0] + mq[1]) + (mq[2] + mq[3])) + ((mq[4] + mq[5]) + (mq[6] + mq[7]));
-    }
-    __syncthreads();
-    if (tid < NP) av[tid] = bv[tid] - (S.hd[0][0][tid] + S.hd[0][1][tid]);
-    __syncthreads();
-    colsum1(H);  // upper half still staged
-    stage(0);
-    colsum1(0);
-    rowdot_h(xv, nullptr);
-    __syncthreads();
-    if (tid < NP) ar = a0 + (S.hd[0][0][tid] + S.hd[0][1][tid]);
-  } else {
-    stage(0);  // the lower half, for Y below
-  }
-  if (tid < NP) {
-    av[tid] = vr * vr;
-    yv[tid] = 1.0 / sqrt(sqrt(mu[tid]));
-  }
-  __syncthreads();
-  if (tid < NP) {
-    double nq[4] = {0, 0, 0, 0};
-#pragma unroll 8
-    for (int q = 0; q < NP; q += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) nq[u] += av[q + u];
-    }
-    const double nv = (nq[0] + nq[1]) + (nq[2] + nq[3]);
-    const double vn = vr / sqrt(nv);
-    V[NP + tid] = ar;
-    V[2 * NP + tid] = vn;
-    V[3 * NP + tid] = mu[tid];
-    if (ampl && tid < N) ampl[(size_t)z * N + tid] = ar;
-    if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
-  }
-  // Y = U diag(mu^-1/4): the lower half is staged, then the upper half
-  for (int e = tid; e < NP * H; e += 256)
-    Q[(e >> 6) * NP + (e & 63)] = Z[(e >> 6) * LD + (e & 63)] * yv[e & 63];
-  __syncthreads();
-  if (g == 1) {
-#pragma unroll
-    for (int c = 0; c < H; ++c) Z[r * LD + c] = x[c] * yv[H + c];
-  }
-  __syncthreads();
-  for (int e = tid; e < NP * H; e += 256) Q[(e >> 6) * NP + H + (e & 63)] = Z[(e >> 6) * LD + (e & 63)];
-}
-
-// ---------------------------------------------------------------------------
 // Epilogue from eigenvectors U (rows in global memory) and eigenvalues d.
 // ---------------------------------------------------------------------------
 template <int NP, int BS = 256>
@@ -1617,39 +1041,8 @@ __global__ __launch_bounds__(BS) void k_eigvec_epi(int64_t z0, const int32_t* __
 // ---------------------------------------------------------------------------
 template <int NP>
 static void tql_pipeline_t(const ChunkArgs& A, hipStream_t st) {
-  int split = 0;
-  if constexpr (NP == 128) split = A.tri_split;
-  if (split == 2) {
-    hipLaunchKernelGGL((k_tridiag<128, 3>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-    hipLaunchKernelGGL((k_tridiag<128, 4>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-    hipLaunchKernelGGL((k_tridiag<128, 2>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-  } else if (split == 4) {
-    // steps 0..63 on the lower triangle only, then the trailing block by the
-    // lower-triangle kernel at NP = 64, one wave per zone (wide256.hip)
-    launch_tridiag_lower128(A, st);
-    launch_tridiag_lower128_tail(A, st);
-  } else if (split == 3) {
-    // steps 0..63 on the lower triangle only (wide256.hip), then as split 1
-    launch_tridiag_lower128(A, st);
-    hipLaunchKernelGGL((k_tridiag<128, 2>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-  } else if (split == 1) {
-    hipLaunchKernelGGL((k_tridiag<128, 1>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-    hipLaunchKernelGGL((k_tridiag<128, 2>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-  } else if (NP == 64) {
-    // the lower-triangle reduction on one wave per zone, Q on MFMA
-    launch_tridiag_lower64(A, st);
-  } else {
-    hipLaunchKernelGGL((k_tridiag<NP, 0>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-  }
-  if constexpr (NP == 128)
-    hipLaunchKernelGGL(k_formq128, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr, A.ymat);
+  hipLaunchKernelGGL((k_tridiag<NP, 0>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
+                     A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
   // zones per QL wave: a tuning knob (the rotation log layout groups 64
   // zones whatever the wave width)
   // (the deflation test: absolute for the mixed path, relative outside the
@@ -1674,21 +1067,10 @@ static void tql_pipeline_t(const ChunkArgs& A, hipStream_t st) {
   else
     OAK_TQL(16);
 #undef OAK_TQL
-  if constexpr (NP == 128) {  // the epilogue runs at the end of the apply kernel
-    hipLaunchKernelGGL(k_tql_apply128, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.mat,
-                       A.ymat, (const double2*)A.rlog, A.rlog_cap, A.tql_status, A.dvec, A.nzc,
-                       A.vec, A.ampl, A.err, A.prec == 1 ? 0 : 1);
-  } else {
-    if constexpr (NP == 64)
-      hipLaunchKernelGGL(k_tql_apply64, dim3(A.nzc), dim3(64), 0, st, A.z0, A.zorder, A.sel_ptr,
-                         A.ymat, (const double2*)A.rlog, A.rlog_cap, A.tql_status);
-    else
-      hipLaunchKernelGGL(k_tql_apply<NP>, dim3(A.nzc), dim3(NP < 64 ? 64 : NP), 0, st, A.z0,
-                         A.zorder, A.sel_ptr, A.ymat, (const double2*)A.rlog, A.rlog_cap,
-                         A.tql_status);
-    hipLaunchKernelGGL(k_eigvec_epi<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                       A.mat, A.ymat, A.dvec, A.nzc, A.vec, A.ampl, A.err);
-  }
+  hipLaunchKernelGGL(k_tql_apply<NP>, dim3(A.nzc), dim3(NP < 64 ? 64 : NP), 0, st, A.z0, A.zorder,
+                     A.sel_ptr, A.ymat, (const double2*)A.rlog, A.rlog_cap, A.tql_status);
+  hipLaunchKernelGGL(k_eigvec_epi<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                     A.mat, A.ymat, A.dvec, A.nzc, A.vec, A.ampl, A.err);
 }
 
 // NP = 256, steps 128..253 of the Householder reduction: the trailing
@@ -1741,8 +1123,6 @@ void launch_tql_pipeline(int NP, const ChunkArgs& A, hipStream_t st) {
   switch (NP) {
     case 16: tql_pipeline_t<16>(A, st); break;
     case 32: tql_pipeline_t<32>(A, st); break;
-    case 64: tql_pipeline_t<64>(A, st); break;
-    case 128: tql_pipeline_t<128>(A, st); break;
   }
 }
 

@@ -329,21 +329,42 @@ struct TriLowerLds {
 // dimensions of M and of the reflector rows (NP for a zone's own block; the
 // N = 128 trailing block, reduced by k_tridiag_lower<64, true>, sits in rows
 // 64.. of the zone's NP = 128 block).
+// vecs (NULL: none): the zone's vectors (stride zvec) to which the reflectors
+// are applied as they are formed, entries 0 .. NP-1 (b, giving Q^T b) and
+// c1 .. c1 + NP-1 (1_N for ones >= 0: row r < ones is 1; else as found).
+struct TriArgs {
+  int64_t z0;
+  const int32_t* zorder;
+  const int64_t* sel_ptr;
+  const double* mat;
+  double* qmat;
+  int64_t zstride;
+  int ldm, ldv;
+  // d_i of zone zl at dvec[zl dz + d0 + i dstep], e_i at evec[zl dz + e0 + i dstep]
+  double *dvec, *evec;
+  int64_t dz, d0, e0, dstep;
+  double* vecs;
+  int zvec, c1, ones;
+};
+
 template <int NP, bool FULL = false>
-__global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tridiag_lower(
-    int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
-    const double* __restrict__ mat, double* __restrict__ qmat, double* __restrict__ dvec,
-    double* __restrict__ evec, int nzc, int64_t zstride, int ldm, int ldv) {
+__global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tridiag_lower(TriArgs A) {
+  const double* __restrict__ mat = A.mat;
+  double* __restrict__ qmat = A.qmat;
+  const int64_t zstride = A.zstride;
+  const int ldm = A.ldm, ldv = A.ldv;
   using L = TriLowerLds<NP>;
   constexpr int NH = NP / 64, PR = L::PR, H = NP / 2, NB = NP / 8;
   constexpr int NT = (NB - 1) * NB / 2;  // register tiles (tile columns 1..NB-1)
   constexpr int BS = 64 * L::NW;         // threads
   __shared__ L S;
   const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
+  const int64_t z = zone_at(A.zorder, A.z0 + zl);
   if (z < 0) return;
-  if (sel_ptr[z + 1] == sel_ptr[z]) return;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  if (A.sel_ptr[z + 1] == A.sel_ptr[z]) return;
+  double* dv = A.dvec + (size_t)zl * A.dz + A.d0;
+  double* ev = A.evec + (size_t)zl * A.dz + A.e0;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const bool own = t < NT;
   int tr = NB - 1, tc = NB - 1;
   if (own) {  // ring s = NB - 1 - tc holds the s + 1 tiles of tile column tc
@@ -371,6 +392,22 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   double x[NH];
 #pragma unroll
   for (int h = 0; h < NH; ++h) x[h] = M[(size_t)(lane + 64 * h) * ldm];  // column 0 (M symmetric)
+  // the vectors: vector q in the registers of wave q % NW (one wave: both)
+  constexpr int NV = L::NW > 1 ? 1 : 2;
+  double u[NV][NH];
+  double* uz = A.vecs ? A.vecs + (size_t)zl * A.zvec : nullptr;
+  const bool has_u = A.vecs && wave < 2;
+  if (has_u) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      const bool second = (NV == 2 ? q : wave) == 1;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        const int r = lane + 64 * h;
+        u[q][h] = second && A.ones >= 0 ? (r < A.ones ? 1.0 : 0.0) : uz[(second ? A.c1 : 0) + r];
+      }
+    }
+  }
   __syncthreads();
   auto pick = [&](int h) {
     double v = x[0];
@@ -431,8 +468,19 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
           V[(size_t)i * ldv + r] = r == i ? tau : v[h];
         }
         if (lane == 0) {
-          dvec[(size_t)(NP - 1 - i) * nzc + zl] = di;
-          evec[(size_t)(NP - 2 - i) * nzc + zl] = beta;
+          dv[i * A.dstep] = di;
+          ev[i * A.dstep] = beta;
+        }
+      }
+      if (has_u) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+          double su = 0.0;
+#pragma unroll
+          for (int h = 0; h < NH; ++h) su = fma(v[h], u[q][h], su);
+          su = tau * wave_sum_d(su);
+#pragma unroll
+          for (int h = 0; h < NH; ++h) u[q][h] = fma(-su, v[h], u[q][h]);
         }
       }
     }
@@ -573,11 +621,18 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   // kernels reduce (launch_tridiag256_tail); NP = 128, as row r, column
   // c - H of rows H.. (the layout k_tridiag<128, 1> leaves for
   // k_tridiag<128, 2>)
+  if (has_u) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+        uz[((NV == 2 ? q : wave) == 1 ? A.c1 : 0) + lane + 64 * h] = u[q][h];
+  }
   if constexpr (FULL) {
     if (t == 0) {  // tile (NB-1, NB-1): the trailing 2 x 2 block, rows NP-2, NP-1
-      dvec[(size_t)1 * nzc + zl] = a[6][6];
-      evec[(size_t)0 * nzc + zl] = a[7][6];
-      dvec[(size_t)0 * nzc + zl] = a[7][7];
+      dv[(NP - 2) * A.dstep] = a[6][6];
+      ev[(NP - 2) * A.dstep] = a[7][6];
+      dv[(NP - 1) * A.dstep] = a[7][7];
     }
     return;
   }
@@ -592,37 +647,28 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
         if (tr != tc) blk[(size_t)(c0 - H + jj) * LDO + (r0 - H + ii)] = a[ii][jj];
       }
   }
-  if (NP == 256 && t == 0) evec[(size_t)(NP - 1) * nzc + zl] = 0.0;
+  if (NP == 256 && t == 0) ev[-A.dstep] = 0.0;  // e_255 of the reversed order
 }
 
-// e_{NP-1} = 0 of every zone of a chunk (NP = 128)
-__global__ void k_fill_elast128(double* __restrict__ evec, int nzc) {
-  const int zl = blockIdx.x * 256 + threadIdx.x;
-  if (zl < nzc) evec[(size_t)127 * nzc + zl] = 0.0;
+// NP = 128: steps 0..63 on the lower-triangle tiles (two waves, four zones
+// per CU); then the trailing 64 x 64 block (rows 64.., columns 0..63 of the
+// zone's reflector block) in full by k_tridiag_lower<64> (one wave per zone,
+// eight zones per CU): its reflectors go to columns 64..127 of the same rows
+// (their columns 0..63 keep the block's values, which k_func masks: a
+// reflector is zero up to its own index), its d, e and vector entries to
+// 64..127.  As one kernel on full 8 x 8 tiles (four waves, two zones per CU)
+// the reduction of 64 800 zones took 20.5 ms, like this 14.4 ms.
+void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st) {
+  TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)128 * 128, 128, 128,
+            A.dvec, A.evec, 128, 0, 0, 1, A.vec, 4 * 128, 2 * 128, ones};
+  hipLaunchKernelGGL((k_tridiag_lower<128>), dim3(A.nzc), dim3(128), 0, st, T);
+  T.mat = A.ymat + 64 * 128;
+  T.qmat = A.ymat + 64 * 128 + 64;
+  T.d0 = T.e0 = 64;
+  T.vecs = A.vec + 64;
+  T.ones = -1;
+  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
 }
-
-// NP = 128, tri_split 3: steps 0..63 on the lower-triangle tiles (two waves,
-// four zones per CU), then k_tridiag<128, 2> from the trailing block
-void launch_tridiag_lower128(const ChunkArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((k_tridiag_lower<128>), dim3(A.nzc), dim3(128), 0, st, A.z0, A.zorder,
-                     A.sel_ptr, A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)128 * 128, 128, 128);
-}
-
-// tri_split 4: the trailing 64 x 64 block (rows 64.., columns 0..63 of the
-// zone's reflector block) reduced in full by k_tridiag_lower<64> (one wave
-// per zone, eight zones per CU): its reflectors go to columns 64..127 of the
-// same rows (their columns 0..63 keep the block's values, which k_formq128
-// does not read: entries below a reflector's own index are zero by
-// definition), its d and e to entries 0..63 and 0..62 of the reversed
-// tridiagonal, as steps 64..125 of the whole reduction would write them;
-// e_127 = 0 is written here
-void launch_tridiag_lower128_tail(const ChunkArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, A.z0, A.zorder,
-                     A.sel_ptr, A.ymat + 64 * 128, A.ymat + 64 * 128 + 64, A.dvec, A.evec, A.nzc,
-                     (int64_t)128 * 128, 128, 128);
-  hipLaunchKernelGGL(k_fill_elast128, dim3((A.nzc + 255) / 256), dim3(256), 0, st, A.evec, A.nzc);
-}
-
 
 // ---------------------------------------------------------------------------
 // Q = H_0 H_1 ... H_253 from the reflectors in the rows of qmat (row k: v_k,
@@ -759,142 +805,12 @@ __global__ __launch_bounds__(256, 2) void k_formq256(int64_t z0, const int32_t* 
       U[(size_t)(16 * I + lr + 4 * r) * NP + (NP - 1 - (16 * J + lc))] = q[I][r];
 }
 
-// ---------------------------------------------------------------------------
-// Q = H_0 ... H_61 for NP = 64 (the reflectors k_tridiag_lower<64, true>
-// leaves in the rows of qmat), the scheme of k_formq256 with one workgroup
-// per zone: wave w holds tile column w of Q (4 tiles), blocks of 16
-// reflectors in compact WY form on MFMA.  Every reflector is read before Q
-// is written over them (in place, columns reversed as the QL kernels expect).
-// ---------------------------------------------------------------------------
-struct FormQ64Lds {
-  static constexpr int LV = 17;
-  double vb[2][64 * LV];
-  double tb[2][16 * LV];
-  double g[16 * LV];
-  double tau[2][16];
-};
-
-__global__ __launch_bounds__(256, 2) void k_formq64(int64_t z0, const int32_t* __restrict__ zorder,
-                                                 const int64_t* __restrict__ sel_ptr,
-                                                 double* __restrict__ qmat) {
-  constexpr int NP = 64, NB = 4, LV = FormQ64Lds::LV;
-  __shared__ FormQ64Lds S;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;
-  if (sel_ptr[z + 1] == sel_ptr[z]) return;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int lr = lane >> 4, lc = lane & 15;
-  double* V = qmat + (size_t)zl * NP * NP;
-  const int J = wave;
-  d4 q[NB];
-#pragma unroll
-  for (int I = 0; I < NB; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) q[I][r] = (I == J && lr + 4 * r == lc) ? 1.0 : 0.0;
-  // thread t moves reflector pj = t / 16 of a block, rows pr + 16 e (e < 4)
-  const int pj = t >> 4, pr = t & 15;
-  double pf[4];
-  auto load_block = [&](int b) {
-    const int k = 16 * b + pj;
-    if (k < NP - 2) {
-      const double* src = V + (size_t)k * NP + pr;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pf[e] = src[16 * e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pf[e] = 0.0;
-    }
-  };
-  load_block(NB - 1);
-  for (int b = NB - 1; b >= 0; --b) {
-    const int buf = b & 1;
-    double* vb = S.vb[buf];
-    double* tb = S.tb[buf];
-    {
-      const int k = 16 * b + pj;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = pr + 16 * e;
-        vb[r * LV + pj] = r <= k ? 0.0 : pf[e];  // v_k is zero above row k + 1
-        if (r == k) S.tau[buf][pj] = pf[e];
-      }
-    }
-    if (b > 0) load_block(b - 1);
-    lds_barrier();
-    // wave 0: G = Vb^T Vb (rows >= 16 b), then Tb column by column:
-    // Tb[j][j] = tau_j, Tb[0:j, j] = -tau_j Tb[0:j, 0:j] G[0:j, j]
-    if (wave == 0) {
-      d4 g = {0.0, 0.0, 0.0, 0.0};
-      for (int kk = 4 * b; kk < 16; ++kk) {
-        const double xv = vb[(4 * kk + lr) * LV + lc];
-        g = mfma_f64(xv, xv, g);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S.g[(lr + 4 * r) * LV + lc] = g[r];
-      __builtin_amdgcn_wave_barrier();
-      if (lane < 16) {
-        double trr[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          asm volatile("" ::: "memory");  // G column by column, not all loads at once
-          double s = 0.0;
-#pragma unroll
-          for (int k = 0; k < j; ++k) s = fma(trr[k], S.g[k * LV + j], s);
-          const double tj = S.tau[buf][j];
-          trr[j] = lane < j ? -tj * s : (lane == j ? tj : 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) tb[lane * LV + j] = trr[j];
-      }
-    }
-    // W = Vb^T Q[:, J]
-    d4 w = {0.0, 0.0, 0.0, 0.0};
-    if (J >= b) {
-#pragma unroll
-      for (int I = 0; I < NB; ++I)
-        if (I >= b) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk)
-            w = mfma_f64(vb[(16 * I + 4 * kk + lr) * LV + lc], q[I][kk], w);
-        }
-    }
-    lds_barrier();  // Tb
-    // W' = -Tb W;  Q[I][J] += Vb[I rows] W'
-    if (J >= b) {
-      d4 wp = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) wp = mfma_f64(-tb[lc * LV + 4 * kk + lr], w[kk], wp);
-#pragma unroll
-      for (int I = 0; I < NB; ++I)
-        if (I >= b) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk)
-            q[I] = mfma_f64(vb[(16 * I + lc) * LV + 4 * kk + lr], wp[kk], q[I]);
-        }
-    }
-  }
-  // every reflector row was read before the last barrier
-#pragma unroll
-  for (int I = 0; I < NB; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      V[(size_t)(16 * I + lr + 4 * r) * NP + (NP - 1 - (16 * J + lc))] = q[I][r];
-}
-
 // NP = 64 (33 <= N <= 64, and the observation-space zones of N = 128): the
-// reduction on the lower triangle in full (one wave per zone), e_63 = 0,
-// then Q by k_formq64
-__global__ void k_fill_elast64(double* __restrict__ evec, int nzc) {
-  const int zl = blockIdx.x * 256 + threadIdx.x;
-  if (zl < nzc) evec[(size_t)63 * nzc + zl] = 0.0;
-}
-
-void launch_tridiag_lower64(const ChunkArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, A.z0, A.zorder,
-                     A.sel_ptr, A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)64 * 64, 64, 64);
-  hipLaunchKernelGGL(k_fill_elast64, dim3((A.nzc + 255) / 256), dim3(256), 0, st, A.evec, A.nzc);
-  hipLaunchKernelGGL(k_formq64, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr, A.ymat);
+// whole reduction on one wave per zone.
+void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st) {
+  const TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)64 * 64, 64, 64,
+                  A.dvec, A.evec, 64, 0, 0, 1, A.vec, 4 * 64, 2 * 64, ones};
+  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
 }
 
 // ---------------------------------------------------------------------------
@@ -1141,8 +1057,10 @@ void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
                        A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec,
                        A.err);
   if (tm) tm->mark(PH_EIG);
-  hipLaunchKernelGGL((k_tridiag_lower<256>), dim3(A.nzc), dim3(512), 0, st, A.z0, A.zorder,
-                     A.sel_ptr, A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)256 * 256, 256, 256);
+  const TriArgs tri{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)256 * 256, 256, 256,
+                    A.dvec, A.evec, 1, (int64_t)255 * A.nzc, (int64_t)254 * A.nzc, -(int64_t)A.nzc,
+                    nullptr, 0, 0, 0};
+  hipLaunchKernelGGL((k_tridiag_lower<256>), dim3(A.nzc), dim3(512), 0, st, tri);
   launch_tridiag256_tail(A, st);
   hipLaunchKernelGGL(k_formq256, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
                      A.ymat, A.umat);
