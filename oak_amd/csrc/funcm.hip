@@ -15,20 +15,25 @@
 //
 //   T^-1/2 = sum_j w_j (T + s_j)^-1,  T^1/2 c = sum_j w_j (c - s_j (T + s_j)^-1 c)
 //
-// and each (T + s)^-1 is semiseparable: with the pivots gamma_0 = d_0 + s,
-// gamma_i = d_i + s - e_{i-1}^2 / gamma_{i-1} and rho_i = -e_i / gamma_i,
+// and each G = (T + s)^-1 is semiseparable.  Eliminating from both ends to the
+// middle row h = NP/2 - 1, with the pivots gamma_0 = d_0 + s, gamma_i = d_i + s
+// - e_{i-1}^2 / gamma_{i-1} above it, the same from the bottom below it, and
+// tau_i = -e / gamma_i (e the coupling of row i towards the middle),
 //
-//   G_kk = 1/gamma_k + rho_k^2 G_{k+1,k+1},   G_ik = rho_i G_{i+1,k}  (i < k).
+//   G_hh = 1 / (gamma_h - e_h^2 / gamma_{h+1}),  and outwards
+//   G_ii = 1/gamma_i + tau_i^2 G_mm,  G_ik = tau_i G_mk
 //
+// for m the neighbour of i towards the middle and every k at or beyond m.
 // T >= I (M is I plus a positive semidefinite matrix), so every exact pivot is
 // at least 1 + s: a pivot that rounding leaves below is set to it, as
-// rrsqrt.F90:137 clamps the eigenvalues.  One lane per pole runs the two
-// recurrences (about 60 cycles a row); a QL iteration with its ~1.1 N^2 plane
-// rotations on the rows of Q, which this replaces, took 22 of the 45 ms of
-// the eigensolve of 64 800 zones at N = 128.
+// rrsqrt.F90:137 clamps the eigenvalues.  One lane per pole and half runs the
+// recurrences, NP/2 rows in and NP/2 rows out; a QL iteration with its ~1.1
+// N^2 plane rotations on the rows of Q, which this replaces, took 22 of the 45
+// ms of the eigensolve of 64 800 zones at N = 128.
 #include <math.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "analysis.hpp"
 #include "common.hpp"
@@ -120,70 +125,78 @@ hipError_t init_poles(int device) {
 }
 
 // ---------------------------------------------------------------------------
-// R, a and v of a zone, one workgroup (4 waves) per zone:
+// R, a and v of a zone, one workgroup per zone, NP/16 waves:
 //   1. wave 0, one lane per pole: pivots, the diagonal of (T + s)^-1 and the
-//      solves with Q^T b (s = 0) and Q^T 1, top down then bottom up; waves
-//      1..3 meanwhile form the triangular factors T_b of the reflector
+//      solves with Q^T b (s = 0) and Q^T 1, top down then bottom up; the other
+//      waves meanwhile form the triangular factors T_b of the reflector
 //      blocks (H_k0 ... H_k0+15 = I - V T_b V^T, compact WY, LAPACK dlarft)
-//   2. F = T^-1/2 in 16 x 16 tiles in the accumulators, wave w holding tile
-//      columns w (and NP/16 - 1 - w): the tiles off the diagonal are products
-//      over the poles (MFMA, 8 steps) of row and column factors of the
-//      semiseparable form relative to the tile edges; the diagonal tiles run
-//      the recurrence
+//   2. F = T^-1/2 in 16 x 16 tiles in the accumulators, each wave holding a
+//      tile column: the tiles off the diagonal are products over the poles
+//      (MFMA, 8 steps) of row and column factors of the semiseparable form
+//      relative to the tile edges; the diagonal tiles run the recurrence
 //   3. R = Q F Q^T, block by block from the last reflectors: with X = F V,
 //      S = V^T X and P = T_b^T V^T,
 //        F <- F - V T_b (X^T - S P) - X P,
-//      each wave on its own tile columns (X through LDS), and [a, v] = Q [x, y]
+//      each wave on its own tile column (X through LDS), and [a, v] = Q [x, y]
 //      along the way.  F stays symmetric; it is kept whole, since the MFMA
 //      contracts over a tile's rows and the lower half alone would need the
 //      transposed tiles.
 // The MFMAs of step 3 are the bound (3456 of 16 x 16 x 4 per zone at NP = 128,
-// 14.9 us on a CU); two zones share a CU (80 KB of LDS), three at NP = 64, so
-// that one zone's pole recurrences run under another's MFMAs.
+// 23 us on a CU at 2.4 GHz); two zones of 8 waves share a CU (79 KB of LDS,
+// 128 registers a lane), four at NP = 64, so that one zone's pole recurrences
+// and barriers run under another's MFMAs.  Measured 60 us per zone and CU at
+// NP = 128, 15 us at NP = 64 (8192 zones); two tile columns on each of four
+// waves (256 registers) spilled and took 79 us, pivots from one end 66 us.
 // DUAL (observation-space zones, dual.hip): F with the weights w / (1 + s),
 // i.e. x -> 1 / (x + sqrt x), and y with w s / (1 + s), x -> 1 / (1 + sqrt x);
-// v is left as Q y.  TR is the type R is stored in (float for the FP32 update
+// v is left as Q y.  LIKE: also log det M, sum (1 - 1/mu) and b^T a (slot 3 of
+// vec) for the likelihood.  TR is the type R is stored in (float for the FP32 update
 // of the mixed path).
 // ---------------------------------------------------------------------------
 template <int NP>
 struct FuncLds {
   static constexpr int NB = NP / 16, LV = 18;
   union {
+    // rows in the order of the elimination: the upper half downwards, then the
+    // lower half upwards (step_row)
     struct {
-      double a[NP * 32];  // rho, then the row factors alpha
-      double g[NP * 32];  // G_kk, then the column factors beta
+      double a[NP * 32];  // tau, then alpha
+      double g[NP * 32];  // G_ii, then beta
+      double d[NP];       // d; then G_hh of the poles
+      double e[NP];       // coupling towards the middle
+      double c[2][NP];    // Q^T b, Q^T 1; then x, y
     } p;
     struct {
       double vb[2][NP * LV];  // V[r][j]: row r of reflector 16 b + j
       double x[NP * LV];      // X = F V
-      double s[4][16 * 17];   // each wave's share of S = V^T X
+      double s[NB][136];      // each wave's share of S = V^T X, packed
+      double sf[16 * 17];     // S
       double g[2][16];        // V^T [x, y]
-      double t[4][2][16];     // T_b V^T [x, y], per wave
+      double t[2][16];        // T_b V^T [x, y]
     } m;
   };
   double tp[NB * 136];  // T_b, packed by columns (upper triangles)
-  union {
-    double dia[4][136];  // each wave's diagonal tile
-    struct {
-      double d[NP], e[NP];
-      double gs[3][136];  // V^T V of waves 1..3
-    } c;
-  } w;
-  double c[2][NP];  // Q^T b, Q^T 1; then x, y; then a, v
+  double c[2][NP];      // x, y; then a, v
   int bucket;
 };
 
-// position of pole j of row r: 16-byte pairs swapped within the row, so that
+// place of row r in the elimination order, and back
+template <int NP>
+__device__ __forceinline__ int step_row(int r) {
+  return r < NP / 2 ? r : NP / 2 + NP - 1 - r;
+}
+
+// position of pole j of row r (of that order): 16-byte pairs swapped within the row, so that
 // the operand reads (16 rows x 4 pairs) spread over the banks
 __device__ __forceinline__ int pole_at(int r, int j) {
   return r * 32 + ((((j >> 1) ^ r) & 15) << 1) + (j & 1);
 }
 
-// eight consecutive poles 8 kk .. 8 kk + 7 of row r
-__device__ __forceinline__ void load_poles(const double* arr, int r, int kk, double (&o)[8]) {
+// four consecutive poles 4 k4 .. 4 k4 + 3 of row r
+__device__ __forceinline__ void load_poles4(const double* arr, int r, int k4, double (&o)[4]) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const double2 v = *reinterpret_cast<const double2*>(arr + r * 32 + ((((4 * kk + c) ^ r) & 15) << 1));
+  for (int c = 0; c < 2; ++c) {
+    const double2 v = *reinterpret_cast<const double2*>(arr + r * 32 + ((((2 * k4 + c) ^ r) & 15) << 1));
     o[2 * c] = v.x;
     o[2 * c + 1] = v.y;
   }
@@ -197,16 +210,30 @@ __device__ __forceinline__ double row_sum16(double v) {
   return v;
 }
 
-template <int NP, bool DUAL, typename TR>
-__global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
-                                                 const int64_t* __restrict__ sel_ptr,
-                                                 double* __restrict__ qmat,
-                                                 const double* __restrict__ dvec,
-                                                 const double* __restrict__ evec,
-                                                 double* __restrict__ vec, double* __restrict__ ampl,
-                                                 unsigned* __restrict__ err, int likelihood) {
+// Sum of a lane's value and that of the lane 16 (32) away, by a row swap in
+// registers (a ds_bpermute costs an LDS round trip).
+__device__ __forceinline__ double sum_xor16(double v) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double sum_xor32(double v) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+template <int NP, bool DUAL, bool LIKE, typename TR>
+__global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                    const int64_t* __restrict__ sel_ptr,
+                                                    double* __restrict__ qmat,
+                                                    const double* __restrict__ dvec,
+                                                    const double* __restrict__ evec,
+                                                    double* __restrict__ vec, double* __restrict__ ampl,
+                                                    unsigned* __restrict__ err) {
   using L = FuncLds<NP>;
-  constexpr int NB = L::NB, LV = L::LV, TC = NB / 4, ER = NP / 16;
+  constexpr int NB = L::NB, LV = L::LV;
+  constexpr int TPR = NP / 4, ER = 4;  // threads per reflector of a block, rows of each
   __shared__ L S;
   const int zl = blockIdx.x;
   const int64_t z = zone_at(zorder, z0 + zl);
@@ -220,10 +247,11 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
   }
   double* V = qmat + (size_t)zl * NP * NP;
   if (tid < NP) {
-    S.w.c.d[tid] = dvec[(size_t)zl * NP + tid];
-    S.w.c.e[tid] = tid < NP - 1 ? evec[(size_t)zl * NP + tid] : 0.0;
-    S.c[0][tid] = Vz[tid];
-    S.c[1][tid] = Vz[2 * NP + tid];
+    const int k = step_row<NP>(tid);
+    S.p.d[k] = dvec[(size_t)zl * NP + tid];
+    S.p.e[k] = evec[(size_t)zl * NP + (tid < NP / 2 ? tid : tid - 1)];
+    S.p.c[0][k] = Vz[tid];
+    S.p.c[1][k] = Vz[2 * NP + tid];
   }
   lds_barrier();
   if (wave == 0) {
@@ -231,85 +259,127 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
     double nt = 0.0;  // Gershgorin bound of T
 #pragma unroll
     for (int h = 0; h < NP / 64; ++h) {
-      const int r = lane + 64 * h;
-      nt = fmax(nt, fabs(S.w.c.d[r]) + fabs(S.w.c.e[r]) + (r > 0 ? fabs(S.w.c.e[r - 1]) : 0.0));
+      const int k = lane + 64 * h;  // k's outer neighbour couples through e of k - 1
+      nt = fmax(nt, fabs(S.p.d[k]) + fabs(S.p.e[k]) + (k % (NP / 2) ? fabs(S.p.e[k - 1]) : 0.0));
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
-    // smallest kappa = 4^(bucket+1) >= nt (nt < 2^ex)
+    // smallest kappa = 4^(bucket+1) >= nt (nt < 2^ex); any nt gives a row of the table
     const int ex = (__double2hiint(nt) >> 20) - 1022;
     int bk = ((ex + 1) >> 1) - 1;
     bk = bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk);
     bk = __builtin_amdgcn_readfirstlane(bk);
     if (lane == 0) S.bucket = bk;
-    if (lane < 32) {
-      const double s = g_poles[bk][0][lane], sp1 = 1.0 + s;
-      double wj = g_poles[bk][1][lane];
-      if (DUAL) wj = wj * s / sp1;
-      const double* cc = S.c[lane == 31 ? 0 : 1];
-      double rho = 0.0, z1 = 0.0, ep = 0.0;
+    // lanes 0..31 rows 0 .. NP/2 - 1 downwards, lanes 32..63 the rest upwards
+    const int j = lane & 31;
+    const bool bot = lane >= 32;
+    const double s = g_poles[bk][0][j], sp1 = 1.0 + s;
+    double wj = g_poles[bk][1][j];
+    if (DUAL) wj = wj * s / sp1;
+    const int h0 = bot ? NP / 2 : 0;
+    const double* dd = S.p.d + h0;
+    const double* ee = S.p.e + h0;
+    double* cc = S.p.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
+    double* c1 = S.p.c[1] + h0;
+    double* aa = S.p.a + h0 * 32;
+    double* gg = S.p.g + h0 * 32;
+    // position of the lane's pole in the row of step 16 t + i (i constant)
+    auto at = [&](int t, int i) { return (16 * t + i) * 32 + ((j & ~1) ^ (2 * i)) + (j & 1); };
+    double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
 #pragma unroll 1
-      for (int t = 0; t < NB; ++t) {
-        double dv[16], ev[16], cv[16];
+    for (int t = 0; t < NB / 2; ++t) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          dv[i] = S.w.c.d[16 * t + i];
-          ev[i] = S.w.c.e[16 * t + i];
-          cv[i] = cc[16 * t + i];
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const double gam = fmax(fma(ep, rho, dv[i] + s), sp1);
-          const double inv = rcp_acc(gam);
-          z1 = fma(rho, z1, cv[i]);
-          const int at = pole_at(16 * t + i, lane);
-          S.p.a[at] = inv;
-          S.p.g[at] = z1 * inv;
-          rho = -ev[i] * inv;
-          ep = ev[i];
-        }
-      }
-      double x = 0.0, G = 0.0, slog = 0.0, sinv = 0.0, sba = 0.0;
-#pragma unroll 1
-      for (int t = NB - 1; t >= 0; --t) {
-        double iv[16], zi[16], ev[16], tv[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int at = pole_at(16 * t + i, lane);
-          iv[i] = S.p.a[at];
-          zi[i] = S.p.g[at];
-          ev[i] = S.w.c.e[16 * t + i];
-          tv[i] = S.c[1][16 * t + i];
-        }
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-          const double r = -ev[i] * iv[i];
-          G = fma(r * r, G, iv[i]);
-          x = fma(r, x, zi[i]);
-          const int at = pole_at(16 * t + i, lane);
-          S.p.a[at] = r;
-          S.p.g[at] = G;
-          tv[i] = DUAL ? wj * x : wj * fma(-s, x, tv[i]);
-          if (likelihood) {
-            slog -= log(iv[i]);
-            sinv += 1.0 - G;
-            sba = fma(S.c[0][16 * t + i], x, sba);
-          }
-          if (lane == 31) S.c[0][16 * t + i] = x;
-        }
-        // sums over the poles: lanes 0..15 keep rows 0..7, lanes 16..31 rows 8..15
-        const bool up = lane >= 16;
+      for (int h = 0; h < 2; ++h) {
+        asm volatile("" ::: "memory");  // the reads of eight rows at a time
+        double dv[8], ev[8], cv[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const double give = up ? tv[i] : tv[i + 8], keep = up ? tv[i + 8] : tv[i];
+          const int k = 16 * t + 8 * h + i;
+          dv[i] = dd[k];
+          ev[i] = ee[k];
+          cv[i] = cc[k];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
+          z1 = fma(tau, z1, cv[i]);
+          aa[at(t, 8 * h + i)] = q;
+          gg[at(t, 8 * h + i)] = z1 * q;
+          tau = -ev[i] * q;
+          e2 = ev[i] * ev[i];
+        }
+      }
+    }
+    // the middle: q, z1 of rows h (top lanes) and h + 1 (bottom lanes);
+    // 1 / G_hh = gamma_h - e_h^2 / gamma_{h+1}, x_h = G_hh (z_h + tau_{h+1} z_{h+1})
+    double G, x;
+    {
+      const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+      const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+      const double eh = S.p.e[NP / 2 - 1];
+      G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+      x = G * fma(-eh * qb, zb, zh);
+      if (!bot) S.p.d[j] = G;
+    }
+    double slog = LIKE && !bot ? -log(G) : 0.0, sinv = 0.0, sba = 0.0;
+#pragma unroll 1
+    for (int t = NB / 2 - 1; t >= 0; --t) {
+#pragma unroll
+      for (int h = 1; h >= 0; --h) {
+        asm volatile("" ::: "memory");
+        double iv[8], zi[8], ev[8], tv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int k = 16 * t + 8 * h + i;
+          iv[i] = aa[at(t, 8 * h + i)];
+          zi[i] = gg[at(t, 8 * h + i)];
+          ev[i] = ee[k];
+          tv[i] = c1[k];
+        }
+#pragma unroll
+        for (int i = 7; i >= 0; --i) {
+          double r = -ev[i] * iv[i];
+          const double gn = fma(r * r, G, iv[i]), xn = fma(r, x, zi[i]);
+          if (h == 1 && i == 7) {
+            // row h itself: G and x as they are, and 1 for tau
+            const bool mid = !bot && t == NB / 2 - 1;
+            if (LIKE) slog -= mid ? 0.0 : log(iv[i]);
+            G = mid ? G : gn;
+            x = mid ? x : xn;
+            r = mid ? 1.0 : r;
+          } else {
+            if (LIKE) slog -= log(iv[i]);
+            G = gn;
+            x = xn;
+          }
+          aa[at(t, 8 * h + i)] = r;
+          gg[at(t, 8 * h + i)] = G;
+          tv[i] = DUAL ? wj * x : wj * fma(-s, x, tv[i]);
+          if (LIKE) {
+            sinv += 1.0 - G;
+            sba = fma(S.p.c[0][h0 + 16 * t + 8 * h + i], x, sba);
+          }
+          if (j == 31) cc[16 * t + 8 * h + i] = x;
+        }
+        // sums over the poles: of each 32 lanes the lower 16 keep steps 0..3
+        // of the eight, the upper 16 steps 4..7
+        const bool up = (lane & 16) != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
           tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
         }
         if (lc == 0) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) S.c[1][16 * t + (up ? 8 : 0) + i] = tv[i];
+          for (int i = 0; i < 4; ++i) c1[16 * t + 8 * h + (up ? 4 : 0) + i] = tv[i];
         }
       }
-      if (likelihood && lane == 31) {  // log det M, sum (1 - 1/mu) and b^T a
+    }
+    if (LIKE) {  // log det M, sum (1 - 1/mu) and b^T a
+      slog += shfl_xor_d(slog, 32);
+      sinv += shfl_xor_d(sinv, 32);
+      sba += shfl_xor_d(sba, 32);
+      if (lane == 31) {
         Vz[3 * NP] = slog;
         Vz[3 * NP + 1] = sinv;
         Vz[3 * NP + 2] = sba;
@@ -317,27 +387,29 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
     }
   } else {
     // ---- T_b of the reflector blocks ----
-    for (int b = wave - 1; b < NB; b += 3) {
+    for (int b = wave - 1; b < NB; b += NB - 1) {
       const int k = 16 * b + lc;
       const double* src = V + (size_t)k * NP;
       d4 g = {0.0, 0.0, 0.0, 0.0};
       for (int k0 = 4 * b; k0 < NP / 4; k0 += 4) {
         double xv[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int r = 4 * (k0 + u) + lr;
-          xv[u] = (k < NP - 2 && r > k) ? src[r] : 0.0;
-        }
+        for (int u = 0; u < 4; ++u) xv[u] = src[4 * (k0 + u) + lr];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) g = mfma_f64(xv[u], xv[u], g);
+        for (int u = 0; u < 4; ++u) {
+          const double xm = (k < NP - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
+          g = mfma_f64(xm, xm, g);
+        }
       }
-      const double tau = (lane < 16 && k < NP - 2) ? src[k] : 0.0;
-      double* gs = S.w.c.gs[wave - 1];
+      const double tk = src[k];
+      const double tau = k < NP - 2 ? tk : 0.0;
+      // V^T V packed into the block's place, then column by column replaced:
+      // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j]
+      double* gs = S.tp + b * 136;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (lr + 4 * r <= lc) gs[lc * (lc + 1) / 2 + lr + 4 * r] = g[r];
       __builtin_amdgcn_wave_barrier();
-      // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j]
       double tr[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -347,59 +419,80 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
         for (int q = 0; q < j; ++q) sm = fma(tr[q], gs[j * (j + 1) / 2 + q], sm);
         const double tj = readlane_d(tau, j);
         tr[j] = lane < j ? -tj * sm : (lane == j ? tj : 0.0);
-        if (lane <= j) S.tp[b * 136 + j * (j + 1) / 2 + lane] = tr[j];
+        __builtin_amdgcn_wave_barrier();
+        if (lane <= j) gs[j * (j + 1) / 2 + lane] = tr[j];
       }
       __builtin_amdgcn_wave_barrier();
     }
   }
   lds_barrier();
-  // ---- F = T^-1/2 ----
-  const int J0 = wave, J1 = NB - 1 - wave;  // tile columns (TC = 1: J0 only)
-  d4 f[TC][NB];
-  double wq[8];
-  {
+  // ---- F = T^-1/2, tile column J (waves w and w + 4 share a SIMD: the
+  // columns J and NB - 1 - J, whose updates add up alike).  The columns of the
+  // lower half see the rows mirrored: f[I] is tile row I or NB - 1 - I, so that
+  // I < Js lie outside the wave's own tile, Js < I < NB/2 towards the middle
+  // and the rest beyond it ----
+  const int J = wave < NB / 2 ? wave : NB + NB / 2 - 1 - wave;
+  const bool low = J >= NB / 2;
+  const int Js = low ? NB - 1 - J : J;
+  auto row_of = [&](int I) { return low ? NB - 1 - I : I; };
+  // place of tile row r in the pole arrays (elimination order)
+  auto tile_of = [&](int r) { return r < NB / 2 ? r : NB / 2 + NB - 1 - r; };
+  d4 f[NB];
+  // column lc of tile J from arr, times the weights of the lane's eight poles
+  auto column_factors = [&](const double* arr, double (&o)[8]) {
     const int bk = S.bucket;
+    const int row = 16 * tile_of(J) + (low ? 15 - lc : lc);
+    load_poles4(arr, row, 2 * lr, reinterpret_cast<double(&)[4]>(o[0]));
+    load_poles4(arr, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(o[4]));
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      wq[q] = g_poles[bk][1][8 * lr + q];
-      if (DUAL) wq[q] = wq[q] / (1.0 + g_poles[bk][0][8 * lr + q]);
+      double w = g_poles[bk][1][8 * lr + q];
+      if (DUAL) w = w / (1.0 + g_poles[bk][0][8 * lr + q]);
+      o[q] *= w;
     }
-  }
-  // diagonal tiles: lane (lr, lc) runs column lc up from its diagonal entry
-  // for its eight poles
-#pragma unroll
-  for (int jj = 0; jj < TC; ++jj) {
-    const int J = jj ? J1 : J0;
+  };
+  d4 fd = {0.0, 0.0, 0.0, 0.0};  // the diagonal tile
+  {
+    // lane (lr, lc) runs column lc outwards from its diagonal entry for its
+    // eight poles; the sums over the poles reach every lr, which keeps rows
+    // lr + 4 r of that triangle (i: the rows in elimination order)
     double g[8];
-    load_poles(S.p.g, 16 * J + lc, lr, g);
+    column_factors(S.p.g, g);
+    d4 us;
+    const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) g[q] *= wq[q];
-    double* dia = S.w.dia[wave];
-#pragma unroll 1
     for (int i = 15; i >= 0; --i) {
-      double r[8];
-      load_poles(S.p.a, 16 * J + i, lr, r);
+      if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
 #pragma unroll
-      for (int q = 0; q < 8; ++q) g[q] *= i < lc ? r[q] : 1.0;
-      double sm = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
-      sm += shfl_xor_d(sm, 16);
-      sm += shfl_xor_d(sm, 32);
-      if (lr == 0 && i <= lc) dia[lc * (lc + 1) / 2 + i] = sm;
+      for (int h = 0; h < 2; ++h) {
+        double r[4];
+        load_poles4(S.p.a, 16 * tile_of(J) + i, 2 * lr + h, r);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? r[q] : 1.0;
+      }
+      const double sm =
+          sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+      if (i % 4 == 3) us[i / 4] = 0.0;
+      us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
     }
-    __builtin_amdgcn_wave_barrier();
-    d4 fd;
+    // the other triangle: the transpose by a product with the identity (exact)
+    d4 ut;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = lr + 4 * r, hi = i > lc ? i : lc, lo = i > lc ? lc : i;
-      fd[r] = dia[hi * (hi + 1) / 2 + lo];
+      ut[r] = low ? us[3 - r] : us[r];
+      fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
     }
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
-      if (I == J) f[jj][I] = fd;
-    __builtin_amdgcn_wave_barrier();
+    for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+  }
+  if (tid < NP) {
+    const int k = step_row<NP>(tid);
+    S.c[0][tid] = S.p.c[0][k];
+    S.c[1][tid] = S.p.c[1][k];
   }
   lds_barrier();
-  // alpha_i = rho_i ... rho_{last row of the tile}, beta_k = G_kk rho_{first} ... rho_{k-1}
+  // towards the middle edge of a row's tile: alpha = tau_i ... (row i to the
+  // edge), beta = G_ii times the tau between the outer edge and row i
   if (tid < 32 * NB) {
     const int t = tid >> 5, j = tid & 31;
     double r[16], g[16];
@@ -425,115 +518,111 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
     }
   }
   lds_barrier();
+  // off the diagonal: rows from arr, columns in B, both relative to the tile
+  // edges (alpha of a tile's outermost row is the tile's whole product); four
+  // poles at a time keep the operands few
+  auto tile = [&](const double* arr, int I, double (&B)[8]) {
+    const int rI = row_of(I), t16 = 16 * tile_of(rI);
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      double av[4], edge[4];
+      load_poles4(arr, t16 + (rI < NB / 2 ? lc : 15 - lc), 2 * lr + h, av);
+      load_poles4(S.p.a, t16, 2 * lr + h, edge);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        acc = mfma_f64(av[q], B[4 * h + q], acc);
+        B[4 * h + q] *= edge[q];
+      }
+      asm volatile("" ::: "memory");
+    }
+    return acc;
+  };
   {
-    double B[TC][8];
+    double B[8];
+    column_factors(S.p.g, B);
 #pragma unroll
-    for (int jj = 0; jj < TC; ++jj) {  // tiles above the diagonal, upwards
-      load_poles(S.p.g, 16 * (jj ? J1 : J0) + lc, lr, B[jj]);
+    for (int I = NB / 2 - 2; I >= 0; --I)  // outside
+      if (I < Js) f[I] = tile(S.p.a, I, B);
+    column_factors(S.p.a, B);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) B[jj][q] *= wq[q];
+    for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
+      if (I == NB / 2) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) B[q] *= S.p.d[8 * lr + q];
+      }
+      if (I > Js) f[I] = tile(I < NB / 2 ? S.p.g : S.p.a, I, B);
     }
 #pragma unroll
-    for (int I = NB - 2; I >= 0; --I) {
-      asm volatile("" ::: "memory");
-      double al[8], edge[8];
-      load_poles(S.p.a, 16 * I + lc, lr, al);
-      load_poles(S.p.a, 16 * I, lr, edge);
-#pragma unroll
-      for (int jj = 0; jj < TC; ++jj)
-        if (I < (jj ? J1 : J0)) {
-          d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            acc = mfma_f64(al[q], B[jj][q], acc);
-            B[jj][q] *= edge[q];
-          }
-          f[jj][I] = acc;
-        }
-    }
-#pragma unroll
-    for (int jj = 0; jj < TC; ++jj) {  // tiles below the diagonal, downwards
-      load_poles(S.p.a, 16 * (jj ? J1 : J0) + lc, lr, B[jj]);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) B[jj][q] *= wq[q];
-    }
-#pragma unroll
-    for (int I = 1; I < NB; ++I) {
-      asm volatile("" ::: "memory");
-      double be[8], edge[8];
-      load_poles(S.p.g, 16 * I + lc, lr, be);
-      load_poles(S.p.a, 16 * I, lr, edge);
-#pragma unroll
-      for (int jj = 0; jj < TC; ++jj)
-        if (I > (jj ? J1 : J0)) {
-          d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            acc = mfma_f64(be[q], B[jj][q], acc);
-            B[jj][q] *= edge[q];
-          }
-          f[jj][I] = acc;
-        }
-    }
+    for (int I = 0; I < NB / 2; ++I)
+      if (I == Js) f[I] = fd;
   }
   // ---- R = Q F Q^T, [a, v] = Q [x, y] ----
-  // thread t moves reflector pj = t / 16 of a block, rows pr + 16 e
-  const int pj = tid >> 4, pr = tid & 15;
+  // thread t moves reflector pj of a block, rows pr + TPR e (loaded whole,
+  // masked when stored: a load under a condition is waited for alone)
   double pf[ER];
-  auto load_block = [&](int b) {
-    const int k = 16 * b + pj;
-    const double* src = V + (size_t)k * NP + pr;
+  auto load_block = [&](int b, int pj, int pr) {
+    const double* src = V + (size_t)(16 * b + pj) * NP + pr;
 #pragma unroll
-    for (int e = 0; e < ER; ++e) pf[e] = (k < NP - 2 && pr + 16 * e > k) ? src[16 * e] : 0.0;
+    for (int e = 0; e < ER; ++e) pf[e] = src[TPR * e];
   };
-  load_block(NB - 1);
+  load_block(NB - 1, tid / TPR, tid % TPR);
   lds_barrier();  // the pole arrays are read
 #pragma unroll 1
   for (int b = NB - 1; b >= 0; --b) {
+    // the thread index made opaque in each pass: left visible, the addresses
+    // and predicates made from it are computed ahead of the loop, and spill
+    int tq = threadIdx.x;
+    asm volatile("" : "+v"(tq));
+    const int tid = tq, lr = (tq >> 4) & 3, lc = tq & 15, pj = tq / TPR, pr = tq % TPR;
     double* vb = S.m.vb[b & 1];
+    const int k = 16 * b + pj;  // the reflector: zero up to row k (none past NP - 3)
 #pragma unroll
-    for (int e = 0; e < ER; ++e) vb[(pr + 16 * e) * LV + pj] = pf[e];
-    if (b > 0) load_block(b - 1);
-    lds_barrier();
-    {  // V^T [x, y]
-      double g0 = 0.0, g1 = 0.0;
-#pragma unroll
-      for (int e = 0; e < ER; ++e) {
-        const int r = pr + 16 * e;
-        const double vv = vb[r * LV + pj];
-        g0 = fma(vv, S.c[0][r], g0);
-        g1 = fma(vv, S.c[1][r], g1);
-      }
-      g0 = row_sum16(g0);
-      g1 = row_sum16(g1);
-      if (pr == 0) {
-        S.m.g[0][pj] = g0;
-        S.m.g[1][pj] = g1;
-      }
+    for (int e = 0; e < ER; ++e) {
+      const int r = pr + TPR * e;
+      pf[e] = (k < NP - 2 && r > k) ? pf[e] : 0.0;
+      vb[r * LV + pj] = pf[e];
     }
-    d4 y[TC], sp = {0.0, 0.0, 0.0, 0.0};
+    lds_barrier();
+    double g0 = 0.0, g1 = 0.0;  // V^T [x, y]
 #pragma unroll
-    for (int jj = 0; jj < TC; ++jj) y[jj] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int e = 0; e < ER; ++e) {
+      const int r = pr + TPR * e;
+      g0 = fma(pf[e], S.c[0][r], g0);
+      g1 = fma(pf[e], S.c[1][r], g1);
+    }
+    g0 = row_sum16(g0);
+    g1 = row_sum16(g1);
+    if (TPR == 32) {
+      g0 = sum_xor16(g0);
+      g1 = sum_xor16(g1);
+    }
+    if (pr == 0) {
+      S.m.g[0][pj] = g0;
+      S.m.g[1][pj] = g1;
+    }
+    // X^T = V^T F on the tile rows I >= b
+    d4 y = {0.0, 0.0, 0.0, 0.0};
+    {
+      const double* vp = vb + lr * LV + lc;
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
-      if (I >= b) {
+      for (int I = 0; I < NB; ++I) {
+        asm volatile("" ::: "memory");  // the reads of later rows stay below
+        const int rI = row_of(I);
+        if (rI >= b) {
+          double va[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const double vv = vb[(16 * I + 4 * q + lr) * LV + lc];
+          for (int q = 0; q < 4; ++q) va[q] = vp[(16 * rI + 4 * q) * LV];
 #pragma unroll
-          for (int jj = 0; jj < TC; ++jj) y[jj] = mfma_f64(vv, f[jj][I][q], y[jj]);
+          for (int q = 0; q < 4; ++q) y = mfma_f64(va[q], f[I][q], y);
         }
       }
-#pragma unroll
-    for (int jj = 0; jj < TC; ++jj) {
-      const int J = jj ? J1 : J0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S.m.x[(16 * J + lc) * LV + lr + 4 * r] = y[jj][r];
     }
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int jj = 0; jj < TC; ++jj) {
-      const int J = jj ? J1 : J0;
+    for (int r = 0; r < 4; ++r) S.m.x[(16 * J + lc) * LV + lr + 4 * r] = y[r];
+    __builtin_amdgcn_wave_barrier();
+    {
+      d4 sp = {0.0, 0.0, 0.0, 0.0};
       if (J >= b) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -541,93 +630,104 @@ __global__ __launch_bounds__(256, 2) void k_func(int64_t z0, const int32_t* __re
           sp = mfma_f64(S.m.x[at], vb[at], sp);
         }
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (lr + 4 * r <= lc) S.m.s[wave][lc * (lc + 1) / 2 + lr + 4 * r] = sp[r];
+    }
+    const double* tp = S.tp + b * 136;
+    // position of (lc, 4 q + lr) and its transpose in a packed triangle
+    auto packed = [&](int q) {
+      const int kk = 4 * q + lr, hi = kk > lc ? kk : lc, lo = kk > lc ? lc : kk;
+      return hi * (hi + 1) / 2 + lo;
+    };
+    d4 pv = {0.0, 0.0, 0.0, 0.0};  // P
+    if (J >= b) {
+      const double* vr = vb + (16 * J + lc) * LV + lr;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        pv = mfma_f64(4 * q + lr <= lc ? tp[packed(q)] : 0.0, vr[4 * q], pv);
+    }
+    lds_barrier();
+    if (b > 0) load_block(b - 1, pj, pr);
+    if (tid < 256) {  // S, T_b V^T [x, y]
+      const int i = tid >> 4, hi = i > lc ? i : lc, lo = i > lc ? lc : i, at = hi * (hi + 1) / 2 + lo;
+      double sm = S.m.s[0][at];
+#pragma unroll
+      for (int w = 1; w < NB; ++w) sm += S.m.s[w][at];
+      S.m.sf[i * 17 + lc] = sm;
+      const double tv = i <= lc ? tp[at] : 0.0;
+      const double t0 = row_sum16(tv * S.m.g[0][lc]), t1 = row_sum16(tv * S.m.g[1][lc]);
+      if (lc == 0) {
+        S.m.t[0][i] = t0;
+        S.m.t[1][i] = t1;
+      }
+    }
+    lds_barrier();
+    d4 qv = {0.0, 0.0, 0.0, 0.0};
+    if (J >= b) {
+      d4 s2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s2 = mfma_f64(S.m.sf[lc * 17 + 4 * q + lr], pv[q], s2);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) y[q] -= s2[q];
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S.m.s[wave][(lr + 4 * r) * 17 + lc] = sp[r];
-    lds_barrier();
-    const double* tp = S.tp + b * 136;
-    double tt[4], tn[4], sa[4];  // T_b^T, T_b and S as A operands
+    for (int q = 0; q < 4; ++q) qv = mfma_f64(lc <= 4 * q + lr ? tp[packed(q)] : 0.0, y[q], qv);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int k = 4 * q + lr, hi = k > lc ? k : lc, lo = k > lc ? lc : k;
-      const double tv = tp[hi * (hi + 1) / 2 + lo];
-      tt[q] = k <= lc ? tv : 0.0;
-      tn[q] = lc <= k ? tv : 0.0;
-      const int at = lc * 17 + k;
-      sa[q] = (S.m.s[0][at] + S.m.s[1][at]) + (S.m.s[2][at] + S.m.s[3][at]);
+      qv[q] = -qv[q];
+      pv[q] = -pv[q];
     }
-    d4 qv[TC], pv[TC];
+    if (tid < 2 * NP) {  // [x, y] <- [x, y] - V (T_b V^T [x, y])
+      const int vq = tid / NP, r = tid % NP;
+      const double2* v2 = reinterpret_cast<const double2*>(vb + r * LV);
+      const double2* t2 = reinterpret_cast<const double2*>(S.m.t[vq]);
+      double s0 = S.c[vq][r], s1 = 0.0;
 #pragma unroll
-    for (int jj = 0; jj < TC; ++jj) {
-      const int J = jj ? J1 : J0;
-      pv[jj] = d4{0.0, 0.0, 0.0, 0.0};
+      for (int c = 0; c < 8; ++c) {
+        const double2 vv = v2[c], tv = t2[c];
+        s0 = fma(-vv.x, tv.x, s0);
+        s1 = fma(-vv.y, tv.y, s1);
+      }
+      S.c[vq][r] = s0 + s1;
+    }
+    // F <- F - V qv - X pv, the second term for the tile columns J >= b (two
+    // conditions without an else: with one, the tiles of both branches stay
+    // live and spill)
+    {
+      const double* vp = vb + lc * LV + lr;
+      const double* xp = S.m.x + lc * LV + lr;
+#pragma unroll
+      for (int I = 0; I < NB; ++I) {
+        asm volatile("" ::: "memory");  // the reads of later rows stay below
+        const int rI = row_of(I);
+        if (rI >= b) {
+          double vv[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) vv[q] = vp[16 * rI * LV + 4 * q];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) f[I] = mfma_f64(vv[q], qv[q], f[I]);
+        }
+      }
       if (J >= b) {
-        d4 s2 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) pv[jj] = mfma_f64(tt[q], vb[(16 * J + lc) * LV + 4 * q + lr], pv[jj]);
+        for (int I = 0; I < NB; ++I) {
+          asm volatile("" ::: "memory");
+          double xv[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s2 = mfma_f64(sa[q], pv[jj][q], s2);
+          for (int q = 0; q < 4; ++q) xv[q] = xp[16 * row_of(I) * LV + 4 * q];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) y[jj][q] -= s2[q];
-      }
-      qv[jj] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) qv[jj] = mfma_f64(tn[q], y[jj][q], qv[jj]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        qv[jj][q] = -qv[jj][q];
-        pv[jj][q] = -pv[jj][q];
-      }
-    }
-    {  // [x, y] <- [x, y] - V (T_b V^T [x, y])
-      double* tw = S.m.t[wave][0];
-      if (lane < 32) {
-        double sm = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const double tv = tp[k * (k + 1) / 2 + (lc <= k ? lc : k)];
-          sm = fma(lc <= k ? tv : 0.0, S.m.g[lr][k], sm);
-        }
-        tw[lane] = sm;
-      }
-      __builtin_amdgcn_wave_barrier();
-      if (tid < 2 * NP) {
-        const int vq = tid / NP, r = tid % NP;
-        double sm = S.c[vq][r];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) sm = fma(-vb[r * LV + k], tw[16 * vq + k], sm);
-        S.c[vq][r] = sm;
-      }
-    }
-#pragma unroll
-    for (int I = 0; I < NB; ++I) {
-      if (I >= b) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const double vv = vb[(16 * I + lc) * LV + 4 * q + lr];
-#pragma unroll
-          for (int jj = 0; jj < TC; ++jj) f[jj][I] = mfma_f64(vv, qv[jj][q], f[jj][I]);
-        }
-      }
-      if ((TC > 1 ? J1 > J0 ? J1 : J0 : J0) >= b) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const double xv = S.m.x[(16 * I + lc) * LV + 4 * q + lr];
-#pragma unroll
-          for (int jj = 0; jj < TC; ++jj)
-            if ((jj ? J1 : J0) >= b) f[jj][I] = mfma_f64(xv, pv[jj][q], f[jj][I]);
+          for (int q = 0; q < 4; ++q) f[I] = mfma_f64(xv[q], pv[q], f[I]);
         }
       }
     }
   }
   TR* R = reinterpret_cast<TR*>(V);  // every reflector was read before the last barrier
 #pragma unroll
-  for (int jj = 0; jj < TC; ++jj)
+  for (int I = 0; I < NB; ++I)
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        R[(size_t)(16 * I + lr + 4 * r) * NP + 16 * (jj ? J1 : J0) + lc] = (TR)f[jj][I][r];
+    for (int r = 0; r < 4; ++r)
+      R[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = (TR)f[I][r];
   lds_barrier();
   if (tid < NP) {
     double nv = 0.0;
@@ -695,23 +795,25 @@ __global__ __launch_bounds__(256) void k_yyt(int64_t z0, const int32_t* __restri
 // The reduction (wide256.hip) and the functions of T for a chunk at NP = 64
 // or 128 (dual: the observation-space zones).
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
-  const dim3 g(A.nzc), b(256);
-  const int like = A.mode == 2;
-#define OAK_FUNC(P, D, TR)                                                                      \
-  hipLaunchKernelGGL((k_func<P, D, TR>), g, b, 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,   \
-                     A.dvec, A.evec, A.vec, A.ampl, A.err, like)
+#define OAK_FUNC(P, D, LK, TR)                                                                     \
+  hipLaunchKernelGGL((k_func<P, D, LK, TR>), dim3(A.nzc), dim3(4 * P), 0, st, A.z0, A.zorder, A.N, \
+                     A.sel_ptr, A.ymat, A.dvec, A.evec, A.vec, A.ampl, A.err)
   if (NP == 64) {
     launch_tridiag_lower64(A, dual ? -1 : A.N, st);
     if (dual)
-      OAK_FUNC(64, true, double);
+      OAK_FUNC(64, true, false, double);
+    else if (A.mode == 2)
+      OAK_FUNC(64, false, true, double);
     else
-      OAK_FUNC(64, false, double);
+      OAK_FUNC(64, false, false, double);
   } else {
     launch_tridiag_lower128(A, A.N, st);
     if (A.prec == 1)
-      OAK_FUNC(128, false, float);
+      OAK_FUNC(128, false, false, float);
+    else if (A.mode == 2)
+      OAK_FUNC(128, false, true, double);
     else
-      OAK_FUNC(128, false, double);
+      OAK_FUNC(128, false, false, double);
   }
 #undef OAK_FUNC
 }
