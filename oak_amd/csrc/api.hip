@@ -1311,42 +1311,25 @@ int obs_operator_impl(oakg_ctx* c, int32_t nvar, const oakg_grid* grids, int64_t
       if (m > 0 && !pos[d]) arg_fail(c, "observation coordinate missing for a grid's dimension");
   begin_call(c);
   const int stride = 1 << nmax;
-  // host side: trees and simplex tables, concatenated over the variables
-  std::vector<BoxDev> boxes;
-  std::vector<int64_t> box0(nvar), tet0(nvar);
+  // search levels and simplex tables; the tables concatenated over the
+  // variables, the bounds of one variable's boxes at a time
+  std::vector<BoxLevels> levels(nvar);
+  std::vector<int64_t> tet0(nvar);
   std::vector<double> tets;
+  int64_t nbound = 1;
   for (int v = 0; v < nvar; ++v) {
     const oakg_grid& g = grids[v];
-    GridHost gh{};
-    gh.n = g.ndim;
-    std::vector<std::vector<double>> hc(g.ndim);
-    for (int d = 0; d < 4; ++d) gh.shape[d] = d < g.ndim ? g.shape[d] : 1;
-    for (int d = 0; d < g.ndim; ++d) {
-      if (dev) {
-        hc[d].resize(nodes[v]);
-        check(c, hipMemcpy(hc[d].data(), g.coord[d], sizeof(double) * nodes[v], hipMemcpyDeviceToHost),
-              "D2H grid");
-        gh.coord[d] = hc[d].data();
-      } else {
-        gh.coord[d] = g.coord[d];
-      }
-    }
-    // each variable's tree keeps its own box numbering; its launch gets the
-    // address of its first box
-    std::vector<BoxDev> b = build_box_tree(gh);
-    box0[v] = (int64_t)boxes.size();
-    boxes.insert(boxes.end(), b.begin(), b.end());
-    if ((int64_t)boxes.size() > INT32_MAX) arg_fail(c, "grid trees above 2^31 boxes");
+    int64_t shape[4];
+    for (int d = 0; d < g.ndim; ++d) shape[d] = g.shape[d];
+    levels[v] = box_levels(g.ndim, shape);
+    nbound = std::max(nbound, 2 * g.ndim * levels[v].total);
     std::vector<double> t = tet_table(g.ndim);
     tet0[v] = (int64_t)tets.size();
     tets.insert(tets.end(), t.begin(), t.end());
   }
-  BoxDev* dbox = (BoxDev*)wsget(c, Workspace::OP_BOXES, sizeof(BoxDev) * std::max<size_t>(boxes.size(), 1));
+  double* dbox = (double*)wsget(c, Workspace::OP_BOXES, sizeof(double) * nbound);
   double* dtet = (double*)wsget(c, Workspace::OP_TET, sizeof(double) * std::max<size_t>(tets.size(), 1));
   if (!dbox || !dtet) check(c, hipErrorOutOfMemory, "workspace");
-  if (!boxes.empty())
-    check(c, hipMemcpyAsync(dbox, boxes.data(), sizeof(BoxDev) * boxes.size(), hipMemcpyHostToDevice,
-                            c->stream), "H2D boxes");
   if (!tets.empty())
     check(c, hipMemcpyAsync(dtet, tets.data(), sizeof(double) * tets.size(), hipMemcpyHostToDevice,
                             c->stream), "H2D tetrahedra");
@@ -1414,7 +1397,7 @@ int obs_operator_impl(oakg_ctx* c, int32_t nvar, const oakg_grid* grids, int64_t
       }
     }
     if (m > 0)
-      launch_obs_interp(g.ndim, m, v, gd, dbox + box0[v], dtet + tet0[v], tet_count(g.ndim), o, stride,
+      launch_obs_interp(g.ndim, m, v, gd, levels[v], dbox, dtet + tet0[v], tet_count(g.ndim), o, stride,
                         slotc, slotw, cnt, dvalid, status, c->stream);
     check(c, hipGetLastError(), "interp launch");
   }
@@ -1426,10 +1409,6 @@ int obs_operator_impl(oakg_ctx* c, int32_t nvar, const oakg_grid* grids, int64_t
   check(c, hipStreamSynchronize(c->stream), "sync");
   if (hst & 1u) {
     c->err = "an observation's cell has degenerate simplices (|det| <= 1e-8, OAK's SVD branch): not supported";
-    return OAKG_EUNSUP;
-  }
-  if (hst & 2u) {
-    c->err = "grid search deeper than 48 levels";
     return OAKG_EUNSUP;
   }
   *nnz = tot;

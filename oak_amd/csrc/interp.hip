@@ -5,10 +5,11 @@
 // (assimilation.F90:4132-4208) and the zone permutation of the state columns
 // (assimilation.F90:2404-2409).
 //
-// One thread per observation: a depth-first walk of the grid's box tree
-// (built once on the host, flattened), the cell test of the candidate
-// leaves (InCube: the first simplex of the cell's split that holds the
-// point), then the 2^n corner weights of the cell.  The arithmetic of the
+// One thread per observation: a depth-first walk of the grid's box tree, the
+// cell test of the candidate leaves (InCube: the first simplex of the cell's
+// split that holds the point) with the 2^n corner weights of the cell.  The
+// tree is never stored as one: its boxes follow from the grid's shape, and
+// only the bounds of the boxes above the cells are computed, on the device.  The arithmetic of the
 // simplex test and weights runs in the same order as the host restatement
 // (sums in index order, LU with partial pivoting, no contraction), so
 // indices and weights are reproducible bit for bit.
@@ -73,116 +74,36 @@ std::vector<double> tet_table(int n) {
   return tc;
 }
 
-// The box tree of locate_databox: box [imin, imax] of node indices with the
-// bounds of its nodes' coordinates; a box with a side above 1 has the
-// sub-boxes (im = (imin + imax) / 2; bit d of m - 1 set: [imin, im] along d,
-// else [im, imax]) with a side >= 1, stored contiguously in m order; a box
-// with no side above 1 is a cell.  Bounds come up from the leaves (the
-// sub-boxes cover their parent's nodes).
-struct TreeBuilder {
-  const GridHost& g;
-  std::vector<BoxDev>& boxes;
-  int64_t lin(const int64_t* p) const {
-    int64_t l = 0, off = 1;
-    for (int d = 0; d < g.n; ++d) {
-      l += p[d] * off;
-      off *= g.shape[d];
-    }
-    return l;
+// The box tree of locate_databox: a box is a range of node indices per dim; a
+// box with a side above 1 is split in every dim at im = (imin + imax) / 2 (bit
+// d of the child's number set: [imin, im], else [im, imax]); a box with no
+// side above 1 is a cell.  A side of 1 gives itself and then the point
+// [imin, imin], a point itself twice, so that a tree over a grid whose sides
+// differ holds each cell many times (2^(n depth) boxes; built and uploaded by
+// the host, 2 million boxes and 290 ms for 120 x 90 x 20 nodes; the whole call
+// with the levels below: 1.1 ms).
+//
+// Only the order of the cells in the walk and each cell's own bounds decide
+// the result: a box's bounds hold its cells' bounds, so tests above the cells
+// only prune.  A box with a point in some dim comes after the box that has the
+// side itself in its place and whose cells, with wider bounds, include its
+// own: it gives no hit that the walk has not had.  So the walk splits only the
+// sides above 1, and level k has per dim the 2^k intervals of level k, or the
+// cells once every interval is one.
+BoxLevels box_levels(int n, const int64_t* shape) {
+  BoxLevels b{};
+  for (int d = 0; d < n; ++d) {
+    b.cells[d] = (int32_t)(shape[d] - 1);
+    while (((int64_t)1 << b.dim_depth[d]) < b.cells[d]) ++b.dim_depth[d];
+    b.depth = std::max(b.depth, b.dim_depth[d]);
   }
-  void build(int64_t id) {
-    const int n = g.n;
-    int64_t imin[4], imax[4];
-    for (int d = 0; d < 4; ++d) {
-      imin[d] = boxes[id].imin[d];
-      imax[d] = boxes[id].imax[d];
-    }
-    bool split = false;
-    for (int d = 0; d < n; ++d) split |= imax[d] - imin[d] > 1;
-    if (!split) {
-      double lo[4], hi[4];
-      for (int d = 0; d < n; ++d) {
-        lo[d] = HUGE_VAL;
-        hi[d] = -HUGE_VAL;
-      }
-      int64_t cnt[4], tot = 1;
-      for (int d = 0; d < n; ++d) {
-        cnt[d] = imax[d] - imin[d] + 1;
-        tot *= cnt[d];
-      }
-      for (int64_t q = 0; q < tot; ++q) {
-        int64_t p[4], r = q;
-        for (int d = 0; d < n; ++d) {
-          p[d] = imin[d] + r % cnt[d];
-          r /= cnt[d];
-        }
-        const int64_t l = lin(p);
-        for (int d = 0; d < n; ++d) {
-          const double x = g.coord[d][l];
-          if (x < lo[d]) lo[d] = x;
-          if (x > hi[d]) hi[d] = x;
-        }
-      }
-      for (int d = 0; d < n; ++d) {
-        boxes[id].xmin[d] = lo[d];
-        boxes[id].xmax[d] = hi[d];
-      }
-      boxes[id].child0 = -1;
-      boxes[id].nchild = 0;
-      return;
-    }
-    int64_t im[4];
-    for (int d = 0; d < n; ++d) im[d] = (imin[d] + imax[d]) / 2;
-    const int64_t first = (int64_t)boxes.size();
-    int nk = 0;
-    for (int q = 0; q < (1 << n); ++q) {
-      BoxDev b{};
-      bool keep = false;
-      for (int d = 0; d < 4; ++d) {
-        if (d >= n) {
-          b.imin[d] = b.imax[d] = 0;
-          continue;
-        }
-        if ((q >> d) & 1) {
-          b.imin[d] = (int32_t)imin[d];
-          b.imax[d] = (int32_t)im[d];
-        } else {
-          b.imin[d] = (int32_t)im[d];
-          b.imax[d] = (int32_t)imax[d];
-        }
-        keep |= b.imax[d] - b.imin[d] >= 1;
-      }
-      if (!keep) continue;
-      boxes.push_back(b);
-      ++nk;
-    }
-    boxes[id].child0 = (int32_t)first;
-    boxes[id].nchild = nk;
-    for (int q = 0; q < nk; ++q) build(first + q);
-    for (int d = 0; d < n; ++d) {
-      double lo = HUGE_VAL, hi = -HUGE_VAL;
-      for (int q = 0; q < nk; ++q) {
-        const BoxDev& c = boxes[first + q];
-        if (c.xmin[d] < lo) lo = c.xmin[d];
-        if (c.xmax[d] > hi) hi = c.xmax[d];
-      }
-      boxes[id].xmin[d] = lo;
-      boxes[id].xmax[d] = hi;
-    }
+  for (int k = 0; k < b.depth; ++k) {
+    int64_t c = 1;
+    for (int d = 0; d < n; ++d) c *= k < b.dim_depth[d] ? (int64_t)1 << k : b.cells[d];
+    b.off[k] = b.total;
+    b.total += c;
   }
-};
-
-std::vector<BoxDev> build_box_tree(const GridHost& g) {
-  std::vector<BoxDev> boxes;
-  BoxDev root{};
-  for (int d = 0; d < 4; ++d) {
-    root.imin[d] = 0;
-    root.imax[d] = d < g.n ? (int32_t)(g.shape[d] - 1) : 0;
-  }
-  boxes.push_back(root);
-  TreeBuilder tb{g, boxes};
-  tb.build(0);
-  return boxes;
+  return b;
 }
 
 // ---------------------------------------------------------------------------
@@ -329,26 +250,141 @@ __device__ void cell_corners(const GridDev& g, const int32_t* ind, double* px, i
   }
 }
 
+// The interval [lo, hi] with number id of a dim at level k (all intervals are
+// one cell after kd splits): its child `bit` one level down; an interval of
+// one cell has itself (bit 0).  Numbers count a level's intervals, from kd on
+// the cells.
+__device__ __forceinline__ void child_interval(int k, int kd, int bit, int32_t& lo, int32_t& hi,
+                                               int32_t& id) {
+  const int32_t im = lo + (hi - lo) / 2;
+  if (bit)
+    hi = im;
+  else
+    lo = im;
+  id = k + 1 < kd ? 2 * id + 1 - bit : lo;
+}
+
+// Bounds of the boxes of level k: from the nodes (the lowest level, sides of
+// at most 2) or from the level below.  Comparisons that fail for NaN leave it
+// out.  One thread per box; a grid of 120 x 90 x 20 nodes has 1e5 boxes in all.
+template <int N, bool NODES>
+__global__ __launch_bounds__(256) void k_box_bounds(GridDev g, BoxLevels bl, int k, int64_t count,
+                                                    double* __restrict__ bounds) {
+  constexpr int TWON = 1 << N;
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= count) return;
+  double mn[N], mx[N];
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    mn[d] = HUGE_VAL;
+    mx[d] = -HUGE_VAL;
+  }
+  int64_t r = b;
+  int32_t lo[N], hi[N], id[N];
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    const int kd = bl.dim_depth[d];
+    const int64_t c = k < kd ? (int64_t)1 << k : bl.cells[d];
+    id[d] = (int32_t)(r % c);
+    r /= c;
+    if (k < kd) {
+      lo[d] = 0;
+      hi[d] = bl.cells[d];
+      for (int i = k - 1; i >= 0; --i) {
+        const int32_t im = lo[d] + (hi[d] - lo[d]) / 2;
+        if ((id[d] >> i) & 1)
+          lo[d] = im;
+        else
+          hi[d] = im;
+      }
+    } else {
+      lo[d] = id[d];
+      hi[d] = id[d] + 1;
+    }
+  }
+  if (NODES) {
+    int32_t p[N];
+#pragma unroll
+    for (int d = 0; d < N; ++d) p[d] = lo[d];
+    for (;;) {
+      int64_t l = 0, off = 1;
+#pragma unroll
+      for (int d = 0; d < N; ++d) {
+        l += p[d] * off;
+        off *= g.shape[d];
+      }
+#pragma unroll
+      for (int d = 0; d < N; ++d) {
+        const double x = g.coord[d][l];
+        if (x < mn[d]) mn[d] = x;
+        if (x > mx[d]) mx[d] = x;
+      }
+      bool more = false;
+#pragma unroll
+      for (int d = 0; d < N; ++d)
+        if (!more) {
+          if (p[d] < hi[d]) {
+            ++p[d];
+            more = true;
+          } else {
+            p[d] = lo[d];
+          }
+        }
+      if (!more) break;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < TWON; ++q) {
+      int64_t l = 0, off = 1;
+#pragma unroll
+      for (int d = 0; d < N; ++d) {
+        const int kd = bl.dim_depth[d];
+        int32_t clo = lo[d], chi = hi[d], cid = id[d];
+        child_interval(k, kd, hi[d] - lo[d] > 1 ? (q >> d) & 1 : 0, clo, chi, cid);
+        l += cid * off;
+        off *= k + 1 < kd ? (int64_t)1 << (k + 1) : bl.cells[d];
+      }
+      const double* c = bounds + 2 * N * (bl.off[k + 1] + l);
+#pragma unroll
+      for (int d = 0; d < N; ++d) {
+        if (c[d] < mn[d]) mn[d] = c[d];
+        if (c[N + d] > mx[d]) mx[d] = c[N + d];
+      }
+    }
+  }
+  double* o = bounds + 2 * N * (bl.off[k] + b);
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    o[d] = mn[d];
+    o[N + d] = mx[d];
+  }
+}
+
 // Pass 1: per observation of variable var, the cell (depth-first search of
 // the box tree), the corner weights, and the entries of its row of H in the
 // slots [stride l, stride l + 2^n): state column (or -1: no entry) and
 // weight (the slots of every observation start out as -1).
 // counts[l] = number of entries, valid[l] = validobs, status bit 1 for a
-// degenerate cell (OAKG_EUNSUP) and bit 2 for a search deeper than the stack.
+// degenerate cell (OAKG_EUNSUP).
+//
+// Bound by latency (one chain of dependent loads and divisions per thread), so
+// waves of one workgroup each, and the bounds of a box's 2^n children are
+// loaded together: the walk keeps, per level, the children still to visit as
+// a mask, and rebuilds a box from the masks when it comes back to it.
 template <int N>
-__global__ __launch_bounds__(256) void k_obs_interp(int64_t m, int var, GridDev g,
-                                                    const BoxDev* __restrict__ boxes,
-                                                    const double* __restrict__ tc, int nbth,
-                                                    const int32_t* __restrict__ obs_var,
-                                                    const double* __restrict__ ox,
-                                                    const double* __restrict__ oy,
-                                                    const double* __restrict__ oz,
-                                                    const double* __restrict__ ot, int stride,
-                                                    int32_t* __restrict__ slot_col,
-                                                    double* __restrict__ slot_w,
-                                                    int64_t* __restrict__ counts,
-                                                    uint8_t* __restrict__ valid,
-                                                    unsigned* __restrict__ status) {
+__global__ __launch_bounds__(64) void k_obs_interp(int64_t m, int var, GridDev g, BoxLevels bl,
+                                                   const double* __restrict__ bounds,
+                                                   const double* __restrict__ tc, int nbth,
+                                                   const int32_t* __restrict__ obs_var,
+                                                   const double* __restrict__ ox,
+                                                   const double* __restrict__ oy,
+                                                   const double* __restrict__ oz,
+                                                   const double* __restrict__ ot, int stride,
+                                                   int32_t* __restrict__ slot_col,
+                                                   double* __restrict__ slot_w,
+                                                   int64_t* __restrict__ counts,
+                                                   uint8_t* __restrict__ valid,
+                                                   unsigned* __restrict__ status) {
   constexpr int TWON = 1 << N;
   const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (l >= m) return;
@@ -357,104 +393,139 @@ __global__ __launch_bounds__(256) void k_obs_interp(int64_t m, int var, GridDev 
   const double* oc[4] = {ox, oy, oz, ot};
 #pragma unroll
   for (int d = 0; d < N; ++d) xi[d] = oc[d][l];
-  // depth-first search: stack of (box, next child)
-  constexpr int kDepth = 48;
-  int32_t st_box[kDepth];
-  int32_t st_next[kDepth];
-  int depth = -1;
-  int32_t found[4] = {0, 0, 0, 0};
   bool hit = false;
-  auto inside_bounds = [&](const BoxDev& b) {
+  int64_t node[TWON];
+  double w[TWON];
+  // the cell with lower corner lo.  0: holds xi (its nodes and weights are
+  // set), 1: does not, 2: degenerate
+  auto test_cell = [&](const int32_t* lo) -> int {
+    double px[N * TWON];
+    cell_corners<N>(g, lo, px, node);
     bool in = true;
 #pragma unroll
-    for (int d = 0; d < N; ++d) in = in && !(xi[d] < b.xmin[d] || xi[d] > b.xmax[d]);
-    return in;
-  };
-  auto test_cell = [&](const BoxDev& b) -> int {
-    double px[N * TWON];
-    int32_t ind[N];
+    for (int d = 0; d < N; ++d) {
+      double mn = HUGE_VAL, mx = -HUGE_VAL;
 #pragma unroll
-    for (int d = 0; d < N; ++d) ind[d] = b.imin[d];
-    cell_corners<N>(g, ind, px, nullptr);
-    return cube_coeff<N>(tc, nbth, px, xi, nullptr);
+      for (int j = 0; j < TWON; ++j) {
+        const double x = px[d + N * j];
+        if (x < mn) mn = x;
+        if (x > mx) mx = x;
+      }
+      in = in && !(xi[d] < mn || xi[d] > mx);
+    }
+    return in ? cube_coeff<N>(tc, nbth, px, xi, w) : 1;
   };
-  {
-    const BoxDev root = boxes[0];
-    if (inside_bounds(root)) {
-      if (root.nchild == 0) {
-        const int r = test_cell(root);
-        if (r == 2) atomicOr(status, 1u);
-        if (r == 0) {
-          hit = true;
+  // the box of the walk at level k and the mask of its children to visit
+  uint16_t todo[32];
+  int32_t lo[N], hi[N], id[N];
+  int k = 0;
+  auto to_root = [&]() {
 #pragma unroll
-          for (int d = 0; d < N; ++d) found[d] = root.imin[d];
+    for (int d = 0; d < N; ++d) {
+      lo[d] = 0;
+      hi[d] = bl.cells[d];
+      id[d] = bl.dim_depth[d] > 0 ? 0 : lo[d];
+    }
+  };
+  auto children = [&]() -> unsigned {
+    unsigned mask = 0;
+#pragma unroll
+    for (int q = 0; q < TWON; ++q) {
+      bool leaf = true, copy = false;
+      int64_t at = 0, off = 1;
+#pragma unroll
+      for (int d = 0; d < N; ++d) {
+        const int kd = bl.dim_depth[d], bit = (q >> d) & 1;
+        copy = copy || (bit && hi[d] - lo[d] <= 1);
+        int32_t a = lo[d], b = hi[d], c = id[d];
+        child_interval(k, kd, bit, a, b, c);
+        leaf = leaf && b - a <= 1;
+        at += c * off;
+        off *= k + 1 < kd ? (int64_t)1 << (k + 1) : bl.cells[d];
+      }
+      bool in = true;
+      if (!leaf) {
+        const double* c = bounds + 2 * N * (bl.off[k + 1] + at);
+#pragma unroll
+        for (int d = 0; d < N; ++d) in = in && !(xi[d] < c[d] || xi[d] > c[N + d]);
+      }
+      mask |= (unsigned)(in && !copy) << q;
+    }
+    return mask;
+  };
+  to_root();
+  if (bl.depth == 0) {
+    const int r = test_cell(lo);
+    if (r == 2) atomicOr(status, 1u);
+    hit = r == 0;
+  } else {
+    bool in = true;
+#pragma unroll
+    for (int d = 0; d < N; ++d) in = in && !(xi[d] < bounds[d] || xi[d] > bounds[N + d]);
+    todo[0] = in ? children() : 0;
+    for (;;) {
+      if (todo[k] == 0) {
+        // back to the box above, rebuilt from the children taken
+        if (k == 0) break;
+        const int up = k - 1;
+        to_root();
+        for (k = 0; k < up; ++k) {
+          const int q = __ffs(todo[k]) - 1;
+#pragma unroll
+          for (int d = 0; d < N; ++d)
+            child_interval(k, bl.dim_depth[d], (q >> d) & 1, lo[d], hi[d], id[d]);
         }
-      } else {
-        depth = 0;
-        st_box[0] = 0;
-        st_next[0] = 0;
+        todo[k] &= todo[k] - 1;
+        continue;
       }
-    }
-  }
-  while (depth >= 0 && !hit) {
-    const BoxDev& parent = boxes[st_box[depth]];
-    if (st_next[depth] >= parent.nchild) {
-      --depth;
-      continue;
-    }
-    const int32_t cid = parent.child0 + st_next[depth]++;
-    const BoxDev child = boxes[cid];
-    if (!inside_bounds(child)) continue;
-    if (child.nchild == 0) {
-      const int r = test_cell(child);
-      if (r == 2) {
-        atomicOr(status, 1u);
-        depth = -1;
-        break;
-      }
-      if (r == 0) {
-        hit = true;
+      const int q = __ffs(todo[k]) - 1;
+      int32_t a[N], b[N], c[N];
+      bool leaf = true;
 #pragma unroll
-        for (int d = 0; d < N; ++d) found[d] = child.imin[d];
+      for (int d = 0; d < N; ++d) {
+        a[d] = lo[d];
+        b[d] = hi[d];
+        c[d] = id[d];
+        child_interval(k, bl.dim_depth[d], (q >> d) & 1, a[d], b[d], c[d]);
+        leaf = leaf && b[d] - a[d] <= 1;
       }
-      continue;
+      if (leaf) {
+        const int r = test_cell(a);
+        if (r == 2) atomicOr(status, 1u);
+        hit = r == 0;
+        if (r != 1) break;
+        todo[k] &= todo[k] - 1;
+      } else {
+#pragma unroll
+        for (int d = 0; d < N; ++d) {
+          lo[d] = a[d];
+          hi[d] = b[d];
+          id[d] = c[d];
+        }
+        ++k;
+        todo[k] = children();
+      }
     }
-    if (depth + 1 >= kDepth) {
-      atomicOr(status, 2u);
-      depth = -1;
-      break;
-    }
-    ++depth;
-    st_box[depth] = cid;
-    st_next[depth] = 0;
   }
   int64_t cnt = 0;
   uint8_t ok = 0;
   if (hit) {
     // cinterp: masked corners put the point out of the grid
-    double px[N * TWON], w[TWON];
-    int64_t node[TWON];
-    cell_corners<N>(g, found, px, node);
     bool masked = false;
     if (g.mask)
 #pragma unroll
       for (int j = 0; j < TWON; ++j) masked = masked || g.mask[node[j]] != 0;
-    if (!masked) {
-      const int r = cube_coeff<N>(tc, nbth, px, xi, w);
-      if (r == 2) atomicOr(status, 1u);
-      if (r == 0) {
-        // packSparseMatrix: entries of nodes outside the state are dropped;
-        // validobs is the validity of the observation's last entry
+    // packSparseMatrix: entries of nodes outside the state are dropped;
+    // validobs is the validity of the observation's last entry
+    if (!masked)
 #pragma unroll
-        for (int j = 0; j < TWON; ++j) {
-          const int64_t s = g.state ? g.state[node[j]] : node[j];
-          slot_col[l * stride + j] = s >= 0 ? (int32_t)s : -1;
-          slot_w[l * stride + j] = w[j];
-          cnt += s >= 0;
-          ok = s >= 0;
-        }
+      for (int j = 0; j < TWON; ++j) {
+        const int64_t s = g.state ? g.state[node[j]] : node[j];
+        slot_col[l * stride + j] = s >= 0 ? (int32_t)s : -1;
+        slot_w[l * stride + j] = w[j];
+        cnt += s >= 0;
+        ok = s >= 0;
       }
-    }
   }
   if (!(hit && cnt > 0)) {
 #pragma unroll
@@ -482,14 +553,33 @@ __global__ void k_obs_compact(int64_t m, int stride, const int64_t* __restrict__
   }
 }
 
-void launch_obs_interp(int n, int64_t m, int var, const GridDev& g, const BoxDev* boxes,
-                       const double* tc, int nbth, const ObsPosDev& o, int slot_stride,
-                       int32_t* slot_col, double* slot_w, int64_t* counts, uint8_t* valid,
-                       unsigned* status, hipStream_t st) {
-  const dim3 grid((unsigned)((m + 255) / 256)), blk(256);
-#define OAK_INTERP(NN)                                                                            \
-  hipLaunchKernelGGL(k_obs_interp<NN>, grid, blk, 0, st, m, var, g, boxes, tc, nbth, o.var, o.x, \
-                     o.y, o.z, o.t, slot_stride, slot_col, slot_w, counts, valid, status)
+template <int N>
+static void obs_interp_t(int64_t m, int var, const GridDev& g, const BoxLevels& bl, double* bounds,
+                         const double* tc, int nbth, const ObsPosDev& o, int slot_stride,
+                         int32_t* slot_col, double* slot_w, int64_t* counts, uint8_t* valid,
+                         unsigned* status, hipStream_t st) {
+  for (int k = bl.depth - 1; k >= 0; --k) {
+    const int64_t c = (k + 1 < bl.depth ? bl.off[k + 1] : bl.total) - bl.off[k];
+    const dim3 grid((unsigned)((c + 255) / 256)), blk(256);
+    if (k == bl.depth - 1)
+      hipLaunchKernelGGL((k_box_bounds<N, true>), grid, blk, 0, st, g, bl, k, c, bounds);
+    else
+      hipLaunchKernelGGL((k_box_bounds<N, false>), grid, blk, 0, st, g, bl, k, c, bounds);
+  }
+  hipLaunchKernelGGL(k_obs_interp<N>, dim3((unsigned)((m + 63) / 64)), dim3(64), 0, st, m, var, g,
+                     bl, bounds, tc, nbth, o.var, o.x, o.y, o.z, o.t, slot_stride, slot_col, slot_w,
+                     counts, valid, status);
+}
+
+// Computes the grid's bounds into `bounds` (2 n bl.total doubles), then one
+// pass over the observations.
+void launch_obs_interp(int n, int64_t m, int var, const GridDev& g, const BoxLevels& bl,
+                       double* bounds, const double* tc, int nbth, const ObsPosDev& o,
+                       int slot_stride, int32_t* slot_col, double* slot_w, int64_t* counts,
+                       uint8_t* valid, unsigned* status, hipStream_t st) {
+#define OAK_INTERP(NN)                                                                           \
+  obs_interp_t<NN>(m, var, g, bl, bounds, tc, nbth, o, slot_stride, slot_col, slot_w, counts,    \
+                   valid, status, st)
   switch (n) {
     case 1: OAK_INTERP(1); break;
     case 2: OAK_INTERP(2); break;
