@@ -731,6 +731,8 @@ static void eig_t(const ChunkArgs& A, hipStream_t st) {
   constexpr int GPW = 64 / NP;
   if (NP == 64 && A.eig_method == 1) {
     launch_func(NP, A, false, st);
+  } else if (A.eig_method == 1 && A.mode != 2) {
+    launch_func_small(NP, A, st);
   } else if (A.eig_method == 1) {
     launch_tql_pipeline(NP, A, st);
     // zones the QL could not finish fall back to Jacobi
@@ -763,7 +765,8 @@ static void chunk_t(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
     return;
   }
   if (tm) tm->mark(PH_TMAT);
-  hipLaunchKernelGGL(k_tmat<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,
+  if (NP == 64 || A.eig_method != 1)
+    hipLaunchKernelGGL(k_tmat<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,
                      A.mat, A.vec);
   if (tm) tm->mark(PH_UPDATE);
   if (A.prec == 1)

@@ -179,6 +179,8 @@ void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st);
 // NP = 64, 128 (funcm.hip): the reduction, then M^-1/2 in ymat, a and v;
 // dual: the functions of I + G that dual.hip needs
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st);
+// NP = 16, 32: the same, and T = R Omega in place of M (no k_tmat)
+void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st);
 // the same M^-1/2 from the Jacobi option's eigenvectors
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
 // pole table of the current device

@@ -463,8 +463,9 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   // interleaved in groups of 4 records over the 64 zones of a QL wave)
   // (about 1.1 N^2 records for typical zones; 2 N^2 + 8 N leaves room for slow ones)
   const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
-  const bool func = c->eig_method == 1 && (NP == 64 || NP == 128);  // funcm.hip
-  const bool ql = (c->eig_method == 1 && NP <= 32) || NP == 256;  // N > 128: QL only
+  // funcm.hip, else QL (the likelihood at N <= 32; N > 128 with either method)
+  const bool func = c->eig_method == 1 && (NP == 64 || NP == 128 || (NP <= 32 && base.mode != 2));
+  const bool ql = (c->eig_method == 1 && NP <= 32 && base.mode == 2) || NP == 256;
   // zones with 1 <= p < dual_lt in observation space (dual.hip): N > 64, the
   // analysis modes (not the likelihood), not in a no-allocation call
   const int dual_lt = (NP == 128 && func && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
@@ -1517,10 +1518,10 @@ size_t noalloc_fixed_bytes(int64_t m, int NP, int64_t nz) {
 }
 
 // Bytes of the zone-chunk workspace per zone (as run_zones sizes it).
-size_t noalloc_zone_bytes(int NP, bool ql) {
+size_t noalloc_zone_bytes(int NP) {
   const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
   return sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP) +
-         ((ql && NP <= 32) || NP == 256 ? (size_t)cap * 16 + 4 : 0);
+         (NP == 256 ? (size_t)cap * 16 + 4 : 0);
 }
 
 // For the duration of a no-allocation call: the arena over the scratch, the
@@ -1754,7 +1755,7 @@ int oakg_local_analysis_csr_noalloc(oakg_ctx* c, int64_t nzones, const int64_t* 
     const int NP = padded_n(N);
     if (nzones < 0 || obs->m < 0) arg_fail(c, "negative nzones or m");
     const size_t need = noalloc_fixed_bytes(obs->m, NP, nzones) +
-                        64 * noalloc_zone_bytes(NP, c->eig_method == 1) + 8 * 256;
+                        64 * noalloc_zone_bytes(NP) + 8 * 256;
     if (need > kScratchBytes)
       arg_fail(c, "oakg_local_analysis_csr_noalloc: m = " + std::to_string(obs->m) + ", N = " +
                       std::to_string(N) + " and " + std::to_string(nzones) + " zones need " +

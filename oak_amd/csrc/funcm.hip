@@ -34,6 +34,7 @@
 
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include "analysis.hpp"
 #include "common.hpp"
@@ -221,6 +222,13 @@ __device__ __forceinline__ double sum_xor32(double v) {
   const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
   const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
   return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Orders a wave's own LDS accesses (they complete in order; the compiler must
+// not move them across).
+__device__ __forceinline__ void lds_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
 }
 
 template <int NP, bool DUAL, bool LIKE, typename TR>
@@ -745,6 +753,550 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
   }
 }
 
+// ===========================================================================
+// N <= 32: the reduction, then R, a, v and the transform itself, a wave per
+// zone (or for several) and no workgroup barrier
+// ===========================================================================
+
+// Lane c of each 16-lane row, to the row (c constant after unrolling).
+__device__ __forceinline__ double row_bcast(double v, int c) {
+#define OAK_BC(C) \
+  case C: return __builtin_amdgcn_update_dpp(v, v, 0x150 + C, 0xF, 0xF, false);
+  switch (c & 15) {
+    OAK_BC(0) OAK_BC(1) OAK_BC(2) OAK_BC(3) OAK_BC(4) OAK_BC(5) OAK_BC(6) OAK_BC(7)
+    OAK_BC(8) OAK_BC(9) OAK_BC(10) OAK_BC(11) OAK_BC(12) OAK_BC(13) OAK_BC(14)
+    default: return __builtin_amdgcn_update_dpp(v, v, 0x15F, 0xF, 0xF, false);
+  }
+#undef OAK_BC
+}
+
+template <typename F, int... K>
+__device__ __forceinline__ void run_steps(F& f, std::integer_sequence<int, K...>) {
+  (void)(f(std::integral_constant<int, K>()) && ...);
+}
+
+// The two 16-lane halves of each 32 lanes of v, each to both halves.
+__device__ __forceinline__ void split16(double v, double& lo, double& hi) {
+  const unsigned l = (unsigned)__double2loint(v), h = (unsigned)__double2hiint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+  lo = __hiloint2double((int)b[0], (int)a[0]);
+  hi = __hiloint2double((int)b[1], (int)a[1]);
+}
+
+// M = Q T Q^T as launch_tridiag_lower64 leaves it (reflectors by rows with tau
+// on the diagonal, rows N-2 and up not written; d, e; Q^T b, Q^T 1).  64 / NP
+// zones share a wave: lane r of a zone holds row r of M in registers, the
+// entries of v and w that the products need come from the other lanes by DPP
+// row broadcasts, and the sums over rows by DPP, so that a step has neither an
+// LDS access nor a barrier.  Bound by the issue of FP64 instructions: 16 N^2/2
+// broadcasts and FMAs per zone and the four reductions of each step.  At N = 16
+// 4096 zones take 10 us, 16384 zones 15 us (the reduction with the row vectors
+// in LDS: 36 and 70 us).
+template <int NP>
+__global__ __launch_bounds__(64, 3) void k_tridiag_small(int64_t z0, const int32_t* __restrict__ zorder,
+                                                         int nzc, int N,
+                                                         const int64_t* __restrict__ sel_ptr,
+                                                         const double* __restrict__ mat,
+                                                         double* __restrict__ qmat,
+                                                         double* __restrict__ dvec,
+                                                         double* __restrict__ evec,
+                                                         double* __restrict__ vec) {
+  static_assert(NP == 16 || NP == 32, "");
+  const int lane = threadIdx.x, r = lane % NP;
+  const int zw = blockIdx.x * (64 / NP) + lane / NP;
+  const int zl = zw < nzc ? zw : nzc - 1;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  const bool active = zw < nzc && z >= 0 && sel_ptr[z < 0 ? 1 : z + 1] > sel_ptr[z < 0 ? 1 : z];
+  if (__ballot(active) == 0) return;
+  double* V = qmat + (size_t)zl * NP * NP;
+  double* Vz = vec + (size_t)zl * 4 * NP;
+  double x[NP];
+  {
+    const double2* row = reinterpret_cast<const double2*>(mat + (size_t)zl * NP * NP + (size_t)r * NP);
+#pragma unroll
+    for (int c = 0; c < NP / 2; ++c) {
+      const double2 t = row[c];
+      x[2 * c] = t.x;
+      x[2 * c + 1] = t.y;
+    }
+  }
+  double u0 = Vz[r], u1 = r < N ? 1.0 : 0.0;
+  auto zone_sum = [](double s) {
+    s = row_sum16(s);
+    return NP == 32 ? sum_xor16(s) : s;
+  };
+  // step k as a constant: every register index and broadcast lane is one
+  auto step = [&](auto kc) -> bool {
+    constexpr int k = decltype(kc)::value;
+    if (k >= N - 2) return false;
+    // H = I - tau v v^T with H x = beta e_1, x = M[k+1.., k] (as in wide256.hip)
+    const double sg = zone_sum(r > k + 1 ? x[k] * x[k] : 0.0);
+    double lo = x[k], hi = x[k];
+    if (NP == 32) split16(x[k], lo, hi);
+    const double alpha = row_bcast(k + 1 < 16 ? lo : hi, k + 1);
+    double tau = 0.0, scal = 0.0, beta = alpha;
+    if (sg > 0x1p-900) {  // below: entries under 2^-450 of an M >= I, no reflection
+      const double hh = fma(alpha, alpha, sg), aa = fabs(alpha);
+      const double rn = rsqrt_acc(hh), nrm = hh * rn;
+      beta = alpha >= 0.0 ? -nrm : nrm;
+      tau = fma(aa, rn, 1.0);
+      const double rd = rcp_acc(aa + nrm);
+      scal = alpha >= 0.0 ? rd : -rd;
+    }
+    const double v = r > k + 1 ? x[k] * scal : (r == k + 1 ? 1.0 : 0.0);
+    if (active) V[k * NP + r] = r == k ? tau : v;
+    lo = hi = v;
+    if (NP == 32) split16(v, lo, hi);
+    double p0 = 0.0, p1 = 0.0;
+#pragma unroll
+    for (int c = k + 1; c < NP; ++c) {
+      const double vc = row_bcast(c < 16 ? lo : hi, c);
+      if (c & 1)
+        p1 = fma(vc, x[c], p1);
+      else
+        p0 = fma(vc, x[c], p0);
+    }
+    const double p = p0 + p1;
+    const double pv = zone_sum(v * p), s0 = zone_sum(v * u0), s1 = zone_sum(v * u1);
+    const double w = r > k ? fma(-0.5 * tau * tau * pv, v, tau * p) : 0.0;
+    u0 = fma(-tau * s0, v, u0);
+    u1 = fma(-tau * s1, v, u1);
+    x[k + 1] = r == k ? beta : x[k + 1];
+    double wlo = w, whi = w;
+    if (NP == 32) split16(w, wlo, whi);
+#pragma unroll
+    for (int c = k + 1; c < NP; ++c) {
+      const double vc = row_bcast(c < 16 ? lo : hi, c), wc = row_bcast(c < 16 ? wlo : whi, c);
+      x[c] = fma(-v, wc, fma(-w, vc, x[c]));
+    }
+    return true;
+  };
+  run_steps(step, std::make_integer_sequence<int, NP - 2>());
+  // the diagonals: lane r's x[r] and x[r + 1]
+  double d = x[0], e = x[1];
+#pragma unroll
+  for (int c = 1; c < NP; ++c) {
+    d = r == c ? x[c] : d;
+    if (c + 1 < NP) e = r == c ? x[c + 1] : e;
+  }
+  if (active) {
+    dvec[(size_t)zl * NP + r] = d;
+    if (r < NP - 1) evec[(size_t)zl * NP + r] = e;
+    Vz[r] = u0;
+    Vz[2 * NP + r] = u1;
+  }
+}
+
+// R, a, v as k_func, and T = R Omega (analysis.hip) in place of M, for a zone
+// per wave.  NP = 32: the two tiles on the diagonal are the halves of the
+// elimination; NP = 16: one tile holds both halves.  In either case the
+// entries that couple the halves are F_ik = sum_j w_j G_hh alpha_i alpha_k
+// (alpha_i the product of the tau from row i to the middle).  With a wave
+// holding the whole of F, X^T = V^T F is at once, in the accumulator layout,
+// the A operand of X, and S that of S, so that only one transpose of X goes
+// through the LDS.
+// Bound by the chain of its phases at few zones (10 us for 64 zones of N = 16),
+// by FP64 issue and the MFMAs (28 of 64 cycles per zone at NP = 16, 132 at
+// NP = 32, for R) at many: 17 us for 4096 zones, 30 us for 16384.  QL sweeps,
+// rotations, epilogue and k_tmat took 118 and 160 us.
+template <int NP>
+struct FuncSmallLds {
+  static constexpr int NB = NP / 16;
+  union {
+    struct {
+      double a[NP * 32];  // tau, then alpha
+      double g[NP * 32];  // G_ii
+      double d[NP], e[NP], c[2][NP];
+    } p;
+    struct {
+      double x[NP * 18];
+      double t[NB][16 * 17];  // V^T V, then T_b
+      double v[NP];
+    } m;
+  };
+};
+
+template <int NP>
+__global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                      const int64_t* __restrict__ sel_ptr,
+                                                      const double* __restrict__ qmat,
+                                                      const double* __restrict__ dvec,
+                                                      const double* __restrict__ evec,
+                                                      double* __restrict__ mat, double* __restrict__ vec,
+                                                      double* __restrict__ ampl, unsigned* __restrict__ err) {
+  using L = FuncSmallLds<NP>;
+  constexpr int NB = L::NB, H = NP / 2;
+  __shared__ L S;
+  const int zl = blockIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  if (z < 0) return;
+  const int lane = threadIdx.x, lr = lane >> 4, lc = lane & 15;
+  double* Vz = vec + (size_t)zl * 4 * NP;
+  double* M = mat + (size_t)zl * NP * NP;
+  if (sel_ptr[z + 1] == sel_ptr[z]) {  // no observations: T = I, a = 0
+    if (lane < NP) Vz[NP + lane] = 0.0;
+    for (int e = lane; e < NP * NP; e += 64) M[e] = (e / NP == e % NP) ? 1.0 : 0.0;
+    return;
+  }
+  const double* V = qmat + (size_t)zl * NP * NP;
+  if (lane < NP) {
+    const int k = step_row<NP>(lane);
+    S.p.d[k] = dvec[(size_t)zl * NP + lane];
+    S.p.e[k] = evec[(size_t)zl * NP + (lane < H ? lane : lane - 1)];
+    S.p.c[0][k] = Vz[lane];
+    S.p.c[1][k] = Vz[2 * NP + lane];
+  }
+  // reflector 16 b + lc, rows 4 q + lr (zero up to row k, none past N - 3)
+  double va[NB][NP / 4], tau[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const double* src = V + (size_t)(16 * b + lc) * NP;
+    tau[b] = src[16 * b + lc];
+#pragma unroll
+    for (int q = 0; q < NP / 4; ++q) va[b][q] = src[4 * q + lr];
+  }
+  lds_fence();
+  // ---- pivots and solves: lanes 0..31 rows 0 .. H-1 downwards, one pole
+  // each, lanes 32..63 the rest upwards ----
+  double nt = 0.0;  // Gershgorin bound of T
+  if (lane < NP)
+    nt = fabs(S.p.d[lane]) + fabs(S.p.e[lane]) + (lane % H ? fabs(S.p.e[lane - 1]) : 0.0);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
+  const int ex = (__double2hiint(nt) >> 20) - 1022;
+  int bk = ((ex + 1) >> 1) - 1;
+  bk = __builtin_amdgcn_readfirstlane(bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk));
+  double alpha[H], gh;  // alpha of the lane's rows and pole; G_hh
+  const int j = lane & 31;
+  const bool bot = lane >= 32;
+  const int h0 = bot ? H : 0;
+  double* aa = S.p.a + h0 * 32;
+  double* gg = S.p.g + h0 * 32;
+  const int jx = (j & ~1) ^ (H == 8 && bot ? 16 : 0);
+  auto at = [&](int i) { return i * 32 + (jx ^ (2 * i)) + (j & 1); };
+  {
+    const double s = g_poles[bk][0][j], sp1 = 1.0 + s, wj = g_poles[bk][1][j];
+    double* cc = S.p.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
+    double* c1 = S.p.c[1] + h0;
+    double qv[H], zv[H], ev[H];
+    double q = 0.0, z1 = 0.0, t = 0.0, e2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      ev[i] = S.p.e[h0 + i];
+      q = rcp_acc(fmax(fma(-e2, q, S.p.d[h0 + i] + s), sp1));
+      z1 = fma(t, z1, cc[i]);
+      qv[i] = q;
+      zv[i] = z1 * q;
+      t = -ev[i] * q;
+      e2 = ev[i] * ev[i];
+    }
+    const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+    const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+    const double eh = S.p.e[H - 1];
+    double G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+    double x = G * fma(-eh * qb, zb, zh), al = 1.0;
+    gh = G;
+    double tv[H];
+#pragma unroll
+    for (int i = H - 1; i >= 0; --i) {
+      double rr = -ev[i] * qv[i];
+      const double gn = fma(rr * rr, G, qv[i]), xn = fma(rr, x, zv[i]);
+      const bool mid = i == H - 1 && !bot;  // row h itself
+      G = mid ? G : gn;
+      x = mid ? x : xn;
+      rr = mid ? 1.0 : rr;
+      al *= rr;
+      alpha[i] = al;
+      aa[at(i)] = rr;
+      gg[at(i)] = G;
+      tv[i] = wj * fma(-s, x, c1[i]);
+      if (j == 31) cc[i] = x;
+    }
+    // sums over the poles: of each 32 lanes the lower 16 keep the first half
+    // of the rows, the upper 16 the second
+    const bool up = (lane & 16) != 0;
+#pragma unroll
+    for (int i = 0; i < H / 2; ++i) {
+      const double give = up ? tv[i] : tv[i + H / 2], keep = up ? tv[i + H / 2] : tv[i];
+      tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
+    }
+    if (lc == 0) {
+#pragma unroll
+      for (int i = 0; i < H / 2; ++i) c1[(up ? H / 2 : 0) + i] = tv[i];
+    }
+  }
+  lds_fence();
+  // [x, y] as columns 0 and 1 of a tile per 16 rows
+  d4 c[NB];
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double t = S.p.c[lc & 1][step_row<NP>(16 * I + lr + 4 * r)];
+      c[I][r] = lc < 2 ? t : 0.0;
+    }
+  // ---- F = T^-1/2: each half's triangle outwards from its diagonal entries,
+  // eight poles a lane, the other one by a product with the identity ----
+  double w8[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) w8[q] = g_poles[bk][1][8 * lr + q];
+  d4 f[NB][NB];
+#pragma unroll
+  for (int J = 0; J < NB; ++J) {
+    // column 16 J + lc is row lcs (elimination order) of half hb
+    const bool hb = NP == 32 ? J == 1 : lc >= 8;
+    const int lcs = hb ? 15 - lc : lc, base = NP == 32 ? 16 * J : (hb ? 8 : 0);
+    double g[8];
+    load_poles4(S.p.g, base + lcs, 2 * lr, reinterpret_cast<double(&)[4]>(g[0]));
+    load_poles4(S.p.g, base + lcs, 2 * lr + 1, reinterpret_cast<double(&)[4]>(g[4]));
+#pragma unroll
+    for (int q = 0; q < 8; ++q) g[q] *= w8[q];
+    const int lrs = hb ? 3 - lr : lr;
+    d4 us = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = H - 1; i >= 0; --i) {
+      if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        double rr[4];
+        load_poles4(S.p.a, base + i, 2 * lr + h, rr);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? rr[q] : 1.0;
+      }
+      const double sm =
+          sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+      us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+    }
+    d4 ut, fd;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      ut[r] = hb ? us[3 - r] : us[r];
+      fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+    f[J][J] = fd;
+  }
+  // the entries between the halves
+  lds_fence();
+#pragma unroll
+  for (int i = 0; i < H; ++i) aa[at(i)] = alpha[i];
+  // G_hh of the poles 8 lr + q (lanes 0..31 hold them)
+  double w8g[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) w8g[q] = w8[q] * shfl_d(gh, 8 * lr + q);
+  lds_fence();
+  {
+    double av[NB][8];
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+      const int row = step_row<NP>(16 * I + lc);
+      load_poles4(S.p.a, row, 2 * lr, reinterpret_cast<double(&)[4]>(av[I][0]));
+      load_poles4(S.p.a, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(av[I][4]));
+    }
+    if (NP == 32) {
+      f[0][NB - 1] = d4{0.0, 0.0, 0.0, 0.0};
+      f[NB - 1][0] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        f[0][NB - 1] = mfma_f64(av[0][q], av[NB - 1][q] * w8g[q], f[0][NB - 1]);
+        f[NB - 1][0] = mfma_f64(av[NB - 1][q], av[0][q] * w8g[q], f[NB - 1][0]);
+      }
+    } else {
+      d4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 8; ++q) x = mfma_f64(av[0][q], av[0][q] * w8g[q], x);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f[0][0][r] = (lc < 8) == (r < 2) ? f[0][0][r] : x[r];
+    }
+  }
+  lds_fence();
+  // ---- T_b of the reflector blocks: lane i of row b of the wave has row i;
+  // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j] ----
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int k = 16 * b + lc;
+#pragma unroll
+    for (int q = 0; q < NP / 4; ++q) va[b][q] = (k < N - 2 && 4 * q + lr > k) ? va[b][q] : 0.0;
+    tau[b] = k < N - 2 ? tau[b] : 0.0;
+    d4 g = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 4 * b; q < NP / 4; ++q) g = mfma_f64(va[b][q], va[b][q], g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S.m.t[b][(lr + 4 * r) * 17 + lc] = g[r];
+  }
+  lds_fence();
+  {
+    const int b = NB == 2 ? (lr & 1) : 0;
+    const double tb = NB == 2 && b ? tau[NB - 1] : tau[0];
+    double gr[16], sm[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      gr[q] = S.m.t[b][q * 17 + lc];
+      sm[q] = 0.0;
+    }
+    lds_fence();
+#pragma unroll
+    for (int jj = 0; jj < 16; ++jj) {
+      const double tj = row_bcast(tb, jj);
+      const double tr = lc < jj ? -tj * sm[jj] : (lc == jj ? tj : 0.0);
+      S.m.t[b][lc * 17 + jj] = tr;
+#pragma unroll
+      for (int q = jj + 1; q < 16; ++q) sm[q] = fma(row_bcast(gr[q], jj), tr, sm[q]);
+    }
+  }
+  lds_fence();
+  // ---- R = Q F Q^T, [a, v] = Q [x, y] ----
+#pragma unroll
+  for (int b = NB - 1; b >= 0; --b) {
+    // V[16 I + lc][4 q + lr] of the block (the other operand form)
+    double vt[NB][4], tA[4], tB[4];
+#pragma unroll
+    for (int I = b; I < NB; ++I)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = 16 * b + 4 * q + lr;
+        const double t = V[(size_t)k * NP + 16 * I + lc];
+        vt[I][q] = (k < N - 2 && 16 * I + lc > k) ? t : 0.0;
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      tA[q] = S.m.t[b][(4 * q + lr) * 17 + lc];
+      tB[q] = S.m.t[b][lc * 17 + 4 * q + lr];
+    }
+    d4 y[NB], x[NB], pv[NB];
+#pragma unroll
+    for (int J = 0; J < NB; ++J) {
+      y[J] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int I = b; I < NB; ++I)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[J] = mfma_f64(va[b][4 * I + q], f[I][J][q], y[J]);
+      x[J] = y[J];  // as an A operand: X, rows of tile J
+      if (J >= b) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S.m.x[(16 * J + lc) * 18 + lr + 4 * r] = y[J][r];
+      }
+    }
+    lds_fence();
+    d4 s = {0.0, 0.0, 0.0, 0.0};  // S = X^T V
+    d4 zc = {0.0, 0.0, 0.0, 0.0}, z2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int J = b; J < NB; ++J)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        s = mfma_f64(S.m.x[(16 * J + 4 * q + lr) * 18 + lc], va[b][4 * J + q], s);
+        zc = mfma_f64(va[b][4 * J + q], c[J][q], zc);
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) z2 = mfma_f64(tB[q], zc[q], z2);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) z2[q] = -z2[q];
+#pragma unroll
+    for (int J = b; J < NB; ++J) {
+      pv[J] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        pv[J] = mfma_f64(tA[q], vt[J][q], pv[J]);
+        c[J] = mfma_f64(vt[J][q], z2[q], c[J]);
+      }
+    }
+#pragma unroll
+    for (int J = 0; J < NB; ++J) {
+      if (J >= b) {
+        d4 s2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s2 = mfma_f64(s[q], pv[J][q], s2);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[J][q] -= s2[q];
+      }
+      d4 qv = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) qv = mfma_f64(tB[q], y[J][q], qv);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        qv[q] = -qv[q];
+        if (J >= b) pv[J][q] = -pv[J][q];
+      }
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (I >= b) f[I][J] = mfma_f64(vt[I][q], qv[q], f[I][J]);
+          if (J >= b) f[I][J] = mfma_f64(x[I][q], pv[J][q], f[I][J]);
+        }
+    }
+    lds_fence();
+  }
+  // ---- a, v, and T = R Omega (k_tmat's formula) ----
+  double vr[NB][4], nv = 0.0;
+  bool nan = false;
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double ar = row_bcast(c[I][r], 0);
+      const int row = 16 * I + lr + 4 * r;
+      vr[I][r] = row_bcast(c[I][r], 1);
+      nv = fma(vr[I][r], vr[I][r], nv);
+      nan = nan || ar != ar;
+      if (lc == 0) {
+        Vz[NP + row] = ar;
+        if (ampl && row < N) ampl[(size_t)z * N + row] = ar;
+      }
+    }
+  if (__ballot(nan) != 0 && lane == 0) atomicOr(err, OAKG_DERR_NAN);
+  nv = 1.0 / sqrt(sum_xor32(sum_xor16(nv)));
+  double vs = 0.0;
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      vr[I][r] *= nv;
+      if (lc == 0) S.m.v[16 * I + lr + 4 * r] = vr[I][r];
+      vs += 16 * I + lr + 4 * r < N - 1 ? vr[I][r] : 0.0;
+    }
+  vs = sum_xor32(sum_xor16(vs));
+  lds_fence();
+  const double wN = 1.0 / sqrt((double)N);
+  const double vN = S.m.v[N - 1], sgv = vN >= 0 ? 1.0 : -1.0;
+  const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0), vw = vs * wN;
+  // U = R [v, w~, z_v]
+  d4 B[NB], U[NB];
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * I + lr + 4 * r;
+      const double zv = vr[I][r] + (row == N - 1 ? sgv : 0.0);
+      const double wt = row < N - 1 ? wN : 0.0;
+      B[I][r] = lc == 0 ? vr[I][r] : (lc == 1 ? wt : (lc == 2 ? zv : 0.0));
+    }
+#pragma unroll
+  for (int I = 0; I < NB; ++I) {
+    U[I] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int K = 0; K < NB; ++K)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) U[I] = mfma_f64(f[K][I][q], B[K][q], U[I]);
+  }
+#pragma unroll
+  for (int J = 0; J < NB; ++J) {
+    const int s = 16 * J + lc;
+    const double zw = wN + (s == N - 1 ? 1.0 : 0.0), vt = s < N - 1 ? S.m.v[s] : 0.0;
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double u1 = row_bcast(U[I][r], 0), u2 = row_bcast(U[I][r], 1), u3 = row_bcast(U[I][r], 2);
+        double t = s == N - 1 ? 0.0 : f[I][J][r];
+        if (s < N) t += u1 * wN + alw * u2 * zw + alv * u3 * vt + alv * alw * vw * u3 * zw;
+        M[(size_t)(16 * I + lr + 4 * r) * NP + s] = t;
+      }
+  }
+}
+
 // R = Y Y^T (and the likelihood's log det M, sum (1 - 1/mu) and b^T a) from
 // the Y = U diag(mu^-1/4) and mu of the Jacobi option, so that one form
 // reaches the transform.
@@ -816,6 +1368,23 @@ void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
       OAK_FUNC(128, false, false, double);
   }
 #undef OAK_FUNC
+}
+
+// NP = 16, 32: M and b of a chunk to T = R Omega (in place of M), a and v.
+void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st) {
+#define OAK_SMALL(P)                                                                               \
+  do {                                                                                             \
+    hipLaunchKernelGGL(k_tridiag_small<P>, dim3((A.nzc + 64 / P - 1) / (64 / P)), dim3(64), 0, st, \
+                       A.z0, A.zorder, A.nzc, A.N, A.sel_ptr, A.mat, A.ymat, A.dvec, A.evec,       \
+                       A.vec);                                                                     \
+    hipLaunchKernelGGL(k_func_small<P>, dim3(A.nzc), dim3(64), 0, st, A.z0, A.zorder, A.N,         \
+                       A.sel_ptr, A.ymat, A.dvec, A.evec, A.mat, A.vec, A.ampl, A.err);            \
+  } while (0)
+  if (NP == 16)
+    OAK_SMALL(16);
+  else
+    OAK_SMALL(32);
+#undef OAK_SMALL
 }
 
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {
