@@ -729,16 +729,11 @@ void launch_prep_ens(int NP, const PrepEnsArgs& A, hipStream_t st) {
 template <int NP>
 static void eig_t(const ChunkArgs& A, hipStream_t st) {
   constexpr int GPW = 64 / NP;
-  if (NP == 64 && A.eig_method == 1) {
-    launch_func(NP, A, false, st);
-  } else if (A.eig_method == 1 && A.mode != 2) {
-    launch_func_small(NP, A, st);
-  } else if (A.eig_method == 1) {
-    launch_tql_pipeline(NP, A, st);
-    // zones the QL could not finish fall back to Jacobi
-    hipLaunchKernelGGL(k_eig<NP>, dim3(nblk(A.nzc, 4 * GPW)), dim3(256), 0, st, A.z0, A.zorder, A.nzc,
-                       A.N, A.sel_ptr, A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol,
-                       A.max_sweeps, (const int32_t*)A.tql_status);
+  if (A.eig_method == 1) {
+    if (NP == 64)
+      launch_func(NP, A, false, st);
+    else
+      launch_func_small(NP, A, st);
   } else {
     hipLaunchKernelGGL(k_eig<NP>, dim3(nblk(A.nzc, 4 * GPW)), dim3(256), 0, st, A.z0, A.zorder, A.nzc,
                        A.N, A.sel_ptr, A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol,
@@ -749,6 +744,12 @@ static void eig_t(const ChunkArgs& A, hipStream_t st) {
 
 template <int NP>
 static void chunk_t(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
+  if (A.mode == 2) {  // innovation likelihood and its adjoint
+    if (tm) tm->mark(PH_EIG);
+    launch_nll_chol(NP, A, st);
+    if (tm) tm->mark(PH_END);
+    return;
+  }
   if (tm) tm->mark(PH_GRAM);
   if (A.prec == 1)
     hipLaunchKernelGGL((k_gram<NP, float>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
@@ -758,12 +759,6 @@ static void chunk_t(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
                        A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, A.err);
   if (tm) tm->mark(PH_EIG);
   eig_t<NP>(A, st);
-  if (A.mode == 2) {  // innovation likelihood: adjoint instead of transform + update
-    if (tm) tm->mark(PH_UPDATE);
-    launch_nll_adjoint(NP, A, st);
-    if (tm) tm->mark(PH_END);
-    return;
-  }
   if (tm) tm->mark(PH_TMAT);
   if (NP == 64 || A.eig_method != 1)
     hipLaunchKernelGGL(k_tmat<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,

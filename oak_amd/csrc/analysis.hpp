@@ -165,7 +165,6 @@ void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_dual128(const ChunkArgs& A, int N, double* ymat128, double* vec128, double* ampl,
                     hipStream_t st, PhaseTimer* tm);
 void launch_chunk128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
-void launch_tql_pipeline(int NP, const ChunkArgs& A, hipStream_t st);
 // NP = 256 (wide256.hip): the whole chunk; QL, rotations and epilogue of
 // its eigensolver (tridiag.hip)
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
@@ -187,6 +186,8 @@ void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
 hipError_t init_poles(int device);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
 void launch_update_f32(int NP, const ChunkArgs& A, hipStream_t st);
+// N <= 64: Gram, factor and adjoint in one; N > 64: the adjoint after the eigensolve
+void launch_nll_chol(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_nll_adjoint(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_report(int NP, const ReportArgs& A, hipStream_t st);
 void launch_nll_totals(int64_t nz, const double* Jz, const double* gA, double* out,

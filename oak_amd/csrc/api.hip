@@ -463,14 +463,17 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   // interleaved in groups of 4 records over the 64 zones of a QL wave)
   // (about 1.1 N^2 records for typical zones; 2 N^2 + 8 N leaves room for slow ones)
   const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
-  // funcm.hip, else QL (the likelihood at N <= 32; N > 128 with either method)
-  const bool func = c->eig_method == 1 && (NP == 64 || NP == 128 || (NP <= 32 && base.mode != 2));
-  const bool ql = (c->eig_method == 1 && NP <= 32 && base.mode == 2) || NP == 256;
+  // the likelihood at N <= 64 keeps nothing per zone (nll.hip); else funcm.hip,
+  // or QL for N > 128 with either method
+  const bool chol = base.mode == 2 && NP <= 64;
+  const bool func = c->eig_method == 1 && NP <= 128 && !chol;
+  const bool ql = NP == 256;
+  const int MP = chol ? 1 : NP;  // matrices MP x MP and vectors of MP entries per zone
   // zones with 1 <= p < dual_lt in observation space (dual.hip): N > 64, the
   // analysis modes (not the likelihood), not in a no-allocation call
   const int dual_lt = (NP == 128 && func && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
   constexpr int PD = 64;
-  const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP) +
+  const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * MP * MP + 6 * MP) +
                           (ql ? (size_t)cap * 16 + 4 : 0) +
                           (dual_lt ? sizeof(double) * ((size_t)2 * PD * PD + 4 * PD) : 0);
   const size_t budget = c->ws_budget;
@@ -492,9 +495,9 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     }
   }
   const int64_t zs = zc * nslot;
-  double* mat = (double*)wsget(c, Workspace::MAT, sizeof(double) * (size_t)NP * NP * zs);
-  double* ymat = (double*)wsget(c, Workspace::YMAT, sizeof(double) * (size_t)NP * NP * zs);
-  double* vec = (double*)wsget(c, Workspace::VEC, sizeof(double) * (size_t)4 * NP * zs);
+  double* mat = (double*)wsget(c, Workspace::MAT, sizeof(double) * (size_t)MP * MP * zs);
+  double* ymat = (double*)wsget(c, Workspace::YMAT, sizeof(double) * (size_t)MP * MP * zs);
+  double* vec = (double*)wsget(c, Workspace::VEC, sizeof(double) * (size_t)4 * MP * zs);
   double* umat = nullptr;  // NP = 256: Q, U, Y (the reflectors stay in ymat)
   if (NP == 256) umat = (double*)wsget(c, Workspace::UMAT, sizeof(double) * (size_t)NP * NP * zs);
   if (!mat || !ymat || !vec || (NP == 256 && !umat)) check(c, hipErrorOutOfMemory, "workspace");
@@ -610,7 +613,7 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
       }
     }
   } guard{s0, use_graph};
-  if (ql || func) fill_i32(sweeps_all, nz, 0, s0);
+  if (ql || func || chol) fill_i32(sweeps_all, nz, 0, s0);
   if (order) {
     hipLaunchKernelGGL(k_zone_order, dim3(1), dim3(1024), 0, s0, nz, nchunk, base.sel_ptr, zorder);
     check(c, hipGetLastError(), "zone order");
@@ -640,9 +643,9 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     A.z0 = z0;
     A.zorder = zorder;
     A.nzc = (int)(order ? oq + (k < orr ? 1 : 0) : std::min<int64_t>(zc, nz - z0));
-    A.mat = mat + zo * NP * NP;
-    A.ymat = ymat + zo * NP * NP;
-    A.vec = vec + zo * 4 * NP;
+    A.mat = mat + zo * MP * MP;
+    A.ymat = ymat + zo * MP * MP;
+    A.vec = vec + zo * 4 * MP;
     A.umat = umat ? umat + zo * NP * NP : nullptr;
     A.sweeps = sweeps_all + z0;
     A.eig_method = ql || func ? 1 : 0;

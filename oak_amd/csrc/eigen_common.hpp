@@ -1,4 +1,4 @@
-// Device helpers shared by the eigensolver kernels (tridiag.hip, wide256.hip).
+// Device helpers shared by the kernels of the zones' matrix functions.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,6 +22,47 @@ __device__ __forceinline__ double rcp_acc(double x) {
   const double y = __builtin_amdgcn_rcp(x);
   const double e = fma(-x, y, 1.0);
   return fma(fma(e, e, e), y, y);
+}
+
+// Sum over each 16-lane row of a wave, to its lanes.
+__device__ __forceinline__ double row_sum16(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x124>(v);
+  v += dpp_d<0x128>(v);
+  return v;
+}
+
+// Sum of a lane's value and that of the lane 16 (32) away, by a row swap in
+// registers (a ds_bpermute costs an LDS round trip).
+__device__ __forceinline__ double sum_xor16(double v) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double sum_xor32(double v) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Lane c of each 16-lane row, to the row (c constant after unrolling).
+__device__ __forceinline__ double row_bcast(double v, int c) {
+#define OAK_BC(C) \
+  case C: return __builtin_amdgcn_update_dpp(v, v, 0x150 + C, 0xF, 0xF, false);
+  switch (c & 15) {
+    OAK_BC(0) OAK_BC(1) OAK_BC(2) OAK_BC(3) OAK_BC(4) OAK_BC(5) OAK_BC(6) OAK_BC(7)
+    OAK_BC(8) OAK_BC(9) OAK_BC(10) OAK_BC(11) OAK_BC(12) OAK_BC(13) OAK_BC(14)
+    default: return __builtin_amdgcn_update_dpp(v, v, 0x15F, 0xF, 0xF, false);
+  }
+#undef OAK_BC
+}
+
+// Orders a wave's own LDS accesses (they complete in order; the compiler must
+// not move them across).
+__device__ __forceinline__ void lds_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // Padded index of row r in the LDS row vectors of the Householder

@@ -203,34 +203,6 @@ __device__ __forceinline__ void load_poles4(const double* arr, int r, int k4, do
   }
 }
 
-__device__ __forceinline__ double row_sum16(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x124>(v);
-  v += dpp_d<0x128>(v);
-  return v;
-}
-
-// Sum of a lane's value and that of the lane 16 (32) away, by a row swap in
-// registers (a ds_bpermute costs an LDS round trip).
-__device__ __forceinline__ double sum_xor16(double v) {
-  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
-  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-__device__ __forceinline__ double sum_xor32(double v) {
-  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
-  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-
-// Orders a wave's own LDS accesses (they complete in order; the compiler must
-// not move them across).
-__device__ __forceinline__ void lds_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <int NP, bool DUAL, bool LIKE, typename TR>
 __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ sel_ptr,
@@ -757,18 +729,6 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
 // N <= 32: the reduction, then R, a, v and the transform itself, a wave per
 // zone (or for several) and no workgroup barrier
 // ===========================================================================
-
-// Lane c of each 16-lane row, to the row (c constant after unrolling).
-__device__ __forceinline__ double row_bcast(double v, int c) {
-#define OAK_BC(C) \
-  case C: return __builtin_amdgcn_update_dpp(v, v, 0x150 + C, 0xF, 0xF, false);
-  switch (c & 15) {
-    OAK_BC(0) OAK_BC(1) OAK_BC(2) OAK_BC(3) OAK_BC(4) OAK_BC(5) OAK_BC(6) OAK_BC(7)
-    OAK_BC(8) OAK_BC(9) OAK_BC(10) OAK_BC(11) OAK_BC(12) OAK_BC(13) OAK_BC(14)
-    default: return __builtin_amdgcn_update_dpp(v, v, 0x15F, 0xF, 0xF, false);
-  }
-#undef OAK_BC
-}
 
 template <typename F, int... K>
 __device__ __forceinline__ void run_steps(F& f, std::integer_sequence<int, K...>) {
@@ -1354,8 +1314,6 @@ void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
     launch_tridiag_lower64(A, dual ? -1 : A.N, st);
     if (dual)
       OAK_FUNC(64, true, false, double);
-    else if (A.mode == 2)
-      OAK_FUNC(64, false, true, double);
     else
       OAK_FUNC(64, false, false, double);
   } else {

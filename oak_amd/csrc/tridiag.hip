@@ -1039,40 +1039,6 @@ __global__ __launch_bounds__(BS) void k_eigvec_epi(int64_t z0, const int32_t* __
 }
 
 // ---------------------------------------------------------------------------
-template <int NP>
-static void tql_pipeline_t(const ChunkArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((k_tridiag<NP, 0>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                     A.mat, A.ymat, A.dvec, A.evec, A.nzc, (int64_t)NP * NP, 1);
-  // zones per QL wave: a tuning knob (the rotation log layout groups 64
-  // zones whatever the wave width)
-  // (the deflation test: absolute for the mixed path, relative outside the
-  // unit eigenvalue cluster for FP64)
-#define OAK_TQL(ZW)                                                                                       \
-  do {                                                                                                    \
-    if (A.prec == 1)                                                                                      \
-      hipLaunchKernelGGL((k_tql<NP, ZW, true>), dim3((A.nzc + ZW - 1) / ZW), dim3(64), 0, st, A.nzc,     \
-                         A.z0, A.zorder, A.sel_ptr, A.dvec, A.evec, (double2*)A.rlog, A.rlog_cap,         \
-                         A.tql_status, A.err);                                                            \
-    else                                                                                                  \
-      hipLaunchKernelGGL((k_tql<NP, ZW, false>), dim3((A.nzc + ZW - 1) / ZW), dim3(64), 0, st, A.nzc,    \
-                         A.z0, A.zorder, A.sel_ptr, A.dvec, A.evec, (double2*)A.rlog, A.rlog_cap,         \
-                         A.tql_status, A.err);                                                            \
-  } while (0)
-  if (A.ql_zw == 4)
-    OAK_TQL(4);
-  else if (A.ql_zw == 8)
-    OAK_TQL(8);
-  else if (A.ql_zw == 32)
-    OAK_TQL(32);
-  else
-    OAK_TQL(16);
-#undef OAK_TQL
-  hipLaunchKernelGGL(k_tql_apply<NP>, dim3(A.nzc), dim3(NP < 64 ? 64 : NP), 0, st, A.z0, A.zorder,
-                     A.sel_ptr, A.ymat, (const double2*)A.rlog, A.rlog_cap, A.tql_status);
-  hipLaunchKernelGGL(k_eigvec_epi<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                     A.mat, A.ymat, A.dvec, A.nzc, A.vec, A.ampl, A.err);
-}
-
 // NP = 256, steps 128..253 of the Householder reduction: the trailing
 // 128 x 128 block that k_tridiag_lower<256> leaves in rows 128..191 of each zone's
 // reflector block, reduced by the NP = 128 kernels in two launches (their
@@ -1117,13 +1083,6 @@ void launch_ql256(const ChunkArgs& A, hipStream_t st) {
                      A.umat, (const double2*)A.rlog, A.rlog_cap, A.tql_status, A.err);
   hipLaunchKernelGGL((k_eigvec_epi<NP, 1024>), dim3(A.nzc), dim3(1024), 0, st, A.z0, A.zorder, A.N,
                      A.sel_ptr, A.mat, A.umat, A.dvec, A.nzc, A.vec, A.ampl, A.err);
-}
-
-void launch_tql_pipeline(int NP, const ChunkArgs& A, hipStream_t st) {
-  switch (NP) {
-    case 16: tql_pipeline_t<16>(A, st); break;
-    case 32: tql_pipeline_t<32>(A, st); break;
-  }
 }
 
 }  // namespace oakg
