@@ -59,7 +59,7 @@ struct oakg_ctx {
   // last call, for the lazily copied per-zone counts
   int64_t last_nz = 0;
   const int64_t* last_sel_ptr = nullptr;
-  int64_t* d_stats = nullptr;  // device: error word + reduced statistics
+  int64_t* pinned = nullptr;  // host memory the device writes small results to
   bool counts_ready = true;
   // internal streams of the chunk pipeline (default priority) and their events
   hipStream_t aux[OAKG_PIPE_SLOTS - 1] = {};
@@ -100,39 +100,45 @@ __global__ void k_fill_f64(double* p, int64_t n, double v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-// Per-call statistics reduced on the device: [0] error bits, [1] zones with
-// p > 0, [2] sum p, [3] max p, [4] max sweeps, [5] zones the QL eigensolver
-// handed to the Jacobi fallback.  One block.
-__global__ __launch_bounds__(1024) void k_call_stats(int64_t nz, const int64_t* __restrict__ sel_ptr,
-                                                     const int32_t* __restrict__ sweeps,
-                                                     const unsigned* __restrict__ err,
-                                                     int64_t* __restrict__ out) {
-  __shared__ int64_t sh[3][1024];
+// Per-call statistics to the host (pinned memory, read after a
+// synchronisation): [0] error bits, [1] zones with p > 0, [2] sum p, [3] max
+// p, [4] max sweeps, [5] zones handed to a fallback.  The workgroups add up in
+// the error block (integers, so in any order); the last one publishes.
+__global__ __launch_bounds__(256) void k_call_stats(int64_t nz, const int64_t* __restrict__ sel_ptr,
+                                                    const int32_t* __restrict__ sweeps, unsigned* err,
+                                                    int64_t* __restrict__ out) {
+  unsigned long long* sums = (unsigned long long*)(err + kSyncSums);
   int64_t na = 0, pm = 0, sm = 0;
-  for (int64_t z = threadIdx.x; z < nz; z += blockDim.x) {
+  for (int64_t z = (int64_t)blockIdx.x * 256 + threadIdx.x; z < nz; z += (int64_t)gridDim.x * 256) {
     const int64_t p = sel_ptr[z + 1] - sel_ptr[z];
     na += p > 0;
     pm = p > pm ? p : pm;
     if (sweeps) sm = sweeps[z] > sm ? sweeps[z] : sm;
   }
-  const int t = threadIdx.x;
-  sh[0][t] = na; sh[1][t] = pm; sh[2][t] = sm;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (t < s) {
-      sh[0][t] += sh[0][t + s];
-      sh[1][t] = sh[1][t] > sh[1][t + s] ? sh[1][t] : sh[1][t + s];
-      sh[2][t] = sh[2][t] > sh[2][t + s] ? sh[2][t] : sh[2][t + s];
-    }
-    __syncthreads();
+  for (int o = 32; o > 0; o >>= 1) {
+    na += __shfl_xor(na, o, 64);
+    pm = max(pm, (int64_t)__shfl_xor(pm, o, 64));
+    sm = max(sm, (int64_t)__shfl_xor(sm, o, 64));
   }
-  if (t == 0) {
-    out[0] = (int64_t)err[0];
-    out[5] = (int64_t)err[1];
-    out[1] = sh[0][0];
+  if ((threadIdx.x & 63) == 0 && nz > 0) {
+    atomicAdd(sums, (unsigned long long)na);
+    atomicMax(sums + 1, (unsigned long long)pm);
+    if (sm > 0) atomicMax(sums + 2, (unsigned long long)sm);
+    __threadfence();  // this wave's sums before its workgroup's arrival
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(err + kSyncStats, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+          gridDim.x - 1) {
+    auto get = [](unsigned long long* p) {
+      return (int64_t)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    out[0] = (int64_t)__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    out[5] = (int64_t)__hip_atomic_load(err + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    out[1] = get(sums);
     out[2] = nz > 0 ? sel_ptr[nz] - sel_ptr[0] : 0;
-    out[3] = sh[1][0];
-    out[4] = sh[2][0];
+    out[3] = get(sums + 1);
+    out[4] = get(sums + 2);
   }
 }
 
@@ -374,33 +380,34 @@ void begin_call(oakg_ctx* c) {
   c->err.clear();
   check(c, hipSetDevice(c->device), "hipSetDevice");
   if (c->arena) {
-    // no-allocation call: the error word and the statistics come first in
-    // the scratch (NoallocCall swaps them in); no events are created
+    // no-allocation call: the error block comes first in the scratch
+    // (NoallocCall swaps it in); no events are created
   } else {
     if (!c->d_err) {
-      check(c, hipMalloc(&c->d_err, 2 * sizeof(unsigned)), "hipMalloc");
-      check(c, hipMalloc(&c->d_stats, 8 * sizeof(int64_t)), "hipMalloc");
+      check(c, hipMalloc(&c->d_err, kSyncWords * sizeof(unsigned)), "hipMalloc");
     }
     if (!c->ev_t0) check(c, hipEventCreate(&c->ev_t0), "event");
     if (!c->ev_t1) check(c, hipEventCreate(&c->ev_t1), "event");
   }
-  fill_u32(c->d_err, 2, 0u, c->stream);  // [0] error bits, [1] eigensolver fallbacks
+  fill_u32(c->d_err, kSyncWords, 0u, c->stream);
   memset(&c->stats, 0, sizeof c->stats);
   c->counts_ready = true;
   c->counts.clear();
   if (c->timing) c->timer.reset(c->stream);
 }
 
-// Ends a call: reduces the statistics on the device, brings them back with
-// the error word in one copy, synchronizes, and turns device errors into
+// Ends a call: reduces the statistics on the device, which writes them and
+// the error word to the context's pinned memory, synchronizes, and turns device errors into
 // return codes.  sel_ptr may be NULL (no zone loop in the call).
 void finish_call(oakg_ctx* c, int64_t nz, const int64_t* sel_ptr, const int32_t* sweeps) {
-  int64_t h[6] = {0, 0, 0, 0, 0, 0};
-  hipLaunchKernelGGL(k_call_stats, dim3(1), dim3(1024), 0, c->stream, sel_ptr ? nz : 0,
-                     sel_ptr, sweeps, c->d_err, c->d_stats);
+  const int64_t n = sel_ptr ? nz : 0;
+  const unsigned blocks = (unsigned)std::min<int64_t>(64, std::max<int64_t>(1, (n + 1023) / 1024));
+  hipLaunchKernelGGL(k_call_stats, dim3(blocks), dim3(256), 0, c->stream, n, sel_ptr, sweeps, c->d_err,
+                     c->pinned);
   check(c, hipGetLastError(), "stats launch");
-  check(c, hipMemcpyAsync(h, c->d_stats, sizeof h, hipMemcpyDeviceToHost, c->stream), "D2H stats");
   check(c, hipStreamSynchronize(c->stream), "sync");
+  int64_t h[6];
+  for (int i = 0; i < 6; ++i) h[i] = ((volatile int64_t*)c->pinned)[i];
   c->stats.zones_analysed = h[1];
   c->stats.obs_selected = h[2];
   c->stats.pmax = h[3];
@@ -458,7 +465,8 @@ void materialize_counts(oakg_ctx* c) {
 // its slowest zones, above all) overlaps the next chunks' work.  The streams are
 // joined by events before the call continues.  With phase timing the chunks
 // run in order on the caller's stream (the timer's events are on that stream).
-void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_all) {
+// Returns whether the zones' Jacobi sweeps are in sweeps_all.
+bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_all) {
   // QL rotation log: records of 16 B per zone, a multiple of 4 (the log is
   // interleaved in groups of 4 records over the 64 zones of a QL wave)
   // (about 1.1 N^2 records for typical zones; 2 N^2 + 8 N leaves room for slow ones)
@@ -597,7 +605,7 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
       ++c->graph_replays;
       check(c, hipEventRecord(c->ev_cap_out, c->cap_stream), "event");
       check(c, hipStreamWaitEvent(c->stream, c->ev_cap_out, 0), "stream wait");
-      return;
+      return !(func || ql || chol);
     }
     check(c, hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal), "capture");
   }
@@ -613,7 +621,6 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
       }
     }
   } guard{s0, use_graph};
-  if (ql || func || chol) fill_i32(sweeps_all, nz, 0, s0);
   if (order) {
     hipLaunchKernelGGL(k_zone_order, dim3(1), dim3(1024), 0, s0, nz, nchunk, base.sel_ptr, zorder);
     check(c, hipGetLastError(), "zone order");
@@ -701,6 +708,7 @@ void run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     check(c, hipEventRecord(c->ev_cap_out, c->cap_stream), "event");
     check(c, hipStreamWaitEvent(c->stream, c->ev_cap_out, 0), "stream wait");
   }
+  return !(func || ql || chol);
 }
 
 template <typename F>
@@ -804,7 +812,7 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
     sel.w = stage(c, Workspace::U_SEL_W, sel_w_in, tot, dev);
     total = tot;
   } else {
-    check(c, run_selection(c->ws, g.zd, g.od, localise, c->stream, c->d_err, sel, &total),
+    check(c, run_selection(c->ws, g.zd, g.od, localise, c->stream, c->d_err, c->pinned, sel, &total),
           "selection");
   }
 
@@ -845,10 +853,10 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
   A.scaling = 1.0;
   A.infl = 1.0;
   A.maxcorr = HUGE_VAL;
-  run_zones(c, NP, A, nz, sweeps);
+  const bool swept = run_zones(c, NP, A, nz, sweeps);
   if (c->timing) c->timer.mark(PH_END);
   if (!c->arena) check(c, hipEventRecord(c->ev_t1, c->stream), "event");
-  finish_call(c, nz, sel.ptr, sweeps);
+  finish_call(c, nz, sel.ptr, swept ? sweeps : nullptr);
   float ms = 0;
   if (!c->arena) (void)hipEventElapsedTime(&ms, c->ev_t0, c->ev_t1);
   collect_stats(c, nz, sel.ptr, ms);
@@ -912,7 +920,7 @@ int local_nll_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, in
   if (c->timing) c->timer.mark(PH_SELECT);
   SelDev sel{};
   int64_t total = 0;
-  check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, sel, &total), "selection");
+  check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, &total), "selection");
   int32_t* sweeps = (int32_t*)wsget(c, Workspace::SWEEPS, sizeof(int32_t) * std::max<int64_t>(nz, 1));
   if (!sweeps) check(c, hipErrorOutOfMemory, "workspace");
   ChunkArgs A{};
@@ -935,12 +943,12 @@ int local_nll_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, in
   A.nll_gL = gLz;
   A.nll_gA = gAz;
   A.nll_gth = gth;
-  run_zones(c, NP, A, nz, sweeps);
+  const bool swept = run_zones(c, NP, A, nz, sweeps);
   launch_nll_totals(nz, Jz, gAz, tot, c->stream);
   check(c, hipGetLastError(), "totals");
   if (c->timing) c->timer.mark(PH_END);
   check(c, hipEventRecord(c->ev_t1, c->stream), "event");
-  finish_call(c, nz, sel.ptr, sweeps);
+  finish_call(c, nz, sel.ptr, swept ? sweeps : nullptr);
   float ms = 0;
   (void)hipEventElapsedTime(&ms, c->ev_t0, c->ev_t1);
   collect_stats(c, nz, sel.ptr, ms);
@@ -1050,7 +1058,7 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     if (c->timing) c->timer.mark(PH_SELECT);
     SelDev sel{};
     int64_t total = 0;
-    check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, sel, &total), "selection");
+    check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, &total), "selection");
     T* dEa = dev ? Ea : (T*)wsget(c, Workspace::OUT_S, sizeof(T) * std::max<int64_t>(n, 1) * N);
     const int64_t ld_ea = dev ? ldEa : n;
     int32_t* sweeps = (int32_t*)wsget(c, Workspace::SWEEPS, sizeof(int32_t) * std::max<int64_t>(nz, 1));
@@ -1087,10 +1095,10 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     A.infl = inflation;
     A.maxcorr = max_correction;
     A.maxcorr_v = dmc;
-    run_zones(c, NP, A, nz, sweeps);
+    const bool swept = run_zones(c, NP, A, nz, sweeps);
     if (c->timing) c->timer.mark(PH_END);
     check(c, hipEventRecord(c->ev_t1, c->stream), "event");
-    finish_call(c, nz, sel.ptr, sweeps);
+    finish_call(c, nz, sel.ptr, swept ? sweeps : nullptr);
     float ms = 0;
     (void)hipEventElapsedTime(&ms, c->ev_t0, c->ev_t1);
     collect_stats(c, nz, sel.ptr, ms);
@@ -1528,29 +1536,25 @@ size_t noalloc_zone_bytes(int NP) {
 }
 
 // For the duration of a no-allocation call: the arena over the scratch, the
-// error word and statistics at its head, no phase timing.
+// error block at its head, no phase timing.
 struct NoallocCall {
   oakg_ctx* c;
   Arena arena;
   unsigned* save_err;
-  int64_t* save_stats;
   bool save_timing;
   NoallocCall(oakg_ctx* cc, void* base) : c(cc) {
     arena.base = (char*)base;
     arena.cap = kScratchBytes;
     save_err = c->d_err;
-    save_stats = c->d_stats;
     save_timing = c->timing;
     char* head = (char*)arena.get(256);
-    c->d_err = (unsigned*)head;               // [0] error bits, [1] eigensolver fallbacks
-    c->d_stats = (int64_t*)(head + 64);       // 8 statistics
+    c->d_err = (unsigned*)head;
     c->timing = false;
     c->arena = &arena;
   }
   ~NoallocCall() {
     c->arena = nullptr;
     c->d_err = save_err;
-    c->d_stats = save_stats;
     c->timing = save_timing;
   }
 };
@@ -1573,6 +1577,10 @@ int oakg_create(oakg_ctx** out, int device, int precision) {
   if (!c) return OAKG_ENOMEM;
   c->device = device;
   c->precision = precision;
+  if (hipHostMalloc((void**)&c->pinned, 64, hipHostMallocDefault) != hipSuccess) {
+    delete c;
+    return OAKG_ENOMEM;
+  }
   // chunk workspace: a quarter of the device memory, between 8 and 64 GiB
   // (larger chunks leave fewer part-filled rounds of workgroups at the end
   // of each kernel; 64 GiB holds config 2's 64 800 zones of N = 128)
@@ -1611,7 +1619,7 @@ int oakg_destroy(oakg_ctx* c) {
   if (c->ev_t0) (void)hipEventDestroy(c->ev_t0);
   if (c->ev_t1) (void)hipEventDestroy(c->ev_t1);
   if (c->d_err) (void)hipFree(c->d_err);
-  if (c->d_stats) (void)hipFree(c->d_stats);
+  if (c->pinned) (void)hipHostFree(c->pinned);
   c->ws.release();
   delete c;
   return OAKG_OK;
@@ -1784,7 +1792,7 @@ int oakg_select_observations(oakg_ctx* c, const oakg_zones* zones, const oakg_ob
     Geo g = stage_geo(c, zones, obs, dev, true);
     SelDev sel{};
     int64_t tot = 0;
-    check(c, run_selection(c->ws, g.zd, g.od, localise_obs, c->stream, c->d_err, sel, &tot),
+    check(c, run_selection(c->ws, g.zd, g.od, localise_obs, c->stream, c->d_err, c->pinned, sel, &tot),
           "selection");
     finish_call(c, zones->nzones, sel.ptr, nullptr);
     const int64_t nz = zones->nzones;

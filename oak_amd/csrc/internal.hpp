@@ -12,6 +12,11 @@ namespace oakg {
 
 constexpr int kMaxCells = 1 << 22;  // cap of the observation bin grid
 
+// Words of a context's error block, all zero at the start of a call: [0] error
+// bits, [1] eigensolver fallbacks, the arrival counters of the kernels whose
+// last workgroup joins the parts, and their sums (int64, from kSyncSums on).
+constexpr int kSyncGeo = 2, kSyncStats = 3, kSyncSums = 4, kSyncWords = 10;
+
 
 // Device views of the call's inputs (all device pointers).
 struct ZonesDev {
@@ -43,8 +48,8 @@ class Workspace {
  public:
   enum Slot {
     // internal buffers
-    COUNTS, SEL_PTR, SEL_IDX, SEL_W, ZORDER, ZORDER_P, ZORDER_D, PERSIST_WQ, MAT_D, YMAT_D, VEC_D, GRID, KEY, KEY2, IDX, SIDX, CELL_CNT, CELL_PTR, SX, SY,
-    SORT_TMP, SCAN_TMP, SCAN_TMP2, HS, INNOV, RHO, XBAR, HEC, MAT, YMAT, VEC, SWEEPS, DVEC, EVEC, RLOG, UMAT, TQL_STATUS, HS32, NLL_Z, NLL_GTH,
+    COUNTS, SEL_PTR, SEL_IDX, SEL_W, ZORDER, ZORDER_P, ZORDER_D, PERSIST_WQ, MAT_D, YMAT_D, VEC_D, GRID, KEY, KEY2, IDX, SIDX, CELL_PTR, SX, SY,
+    SORT_TMP, SCAN_TMP, HS, INNOV, RHO, XBAR, HEC, MAT, YMAT, VEC, SWEEPS, DVEC, EVEC, RLOG, UMAT, TQL_STATUS, HS32, NLL_Z, NLL_GTH,
     // staged copies of host inputs and outputs
     Z_PTR, Z_POS, Z_CORR, Z_MAXLEN, O_X, O_Y, O_Z, O_T, O_YO, O_RMSE2, O_EXCL, IN_S, IN_HSF,
     IN_XF, IN_HXF, H_RP, H_COL, H_VAL, H_SHIFT, OUT_XA, OUT_S, OUT_AMPL, U_SEL_PTR, U_SEL_IDX,
@@ -78,7 +83,8 @@ class Workspace {
 };
 
 hipError_t run_selection(Workspace& ws, const ZonesDev& zd, const ObsDev& od, int localise,
-                         hipStream_t st, unsigned* d_err, SelDev& sel, int64_t* total);
+                         hipStream_t st, unsigned* d_err, int64_t* pinned, SelDev& sel,
+                         int64_t* total);
 hipError_t scan_counts(Workspace& ws, const int64_t* counts, int64_t* sel_ptr, int64_t nz,
                        hipStream_t st);
 
