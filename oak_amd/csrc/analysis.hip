@@ -15,6 +15,7 @@
 //             assimilation.F90:3299-3320)
 #include "analysis.hpp"
 #include "common.hpp"
+#include "spmm.hpp"
 
 namespace oakg {
 
@@ -86,26 +87,6 @@ __global__ void k_state_mean_x2(int64_t n2, int N, const double2* __restrict__ E
 
 // Ensemble mode, HE(:,k) = H.x.E(:,k) + Hshift (assimilation.F90:3112-3114;
 // COO accumulation order of matoper_inc.F90:238-240 kept within each row).
-__global__ void k_spmm_obs(int64_t m, int64_t n, int N, const int64_t* __restrict__ row_ptr,
-                           const int32_t* __restrict__ col, const double* __restrict__ val,
-                           const double* __restrict__ E, int64_t ld,
-                           const double* __restrict__ Hshift, double* __restrict__ HEc,
-                           unsigned* __restrict__ err) {
-#pragma clang fp contract(off)
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y;
-  if (l >= m) return;
-  const double* Ek = E + (int64_t)k * ld;
-  double s = 0;
-  for (int64_t e = row_ptr[l]; e < row_ptr[l + 1]; ++e) {
-    int32_t j = col[e];
-    if (j < 0 || j >= n) { atomicOr(err, OAKG_DERR_IDX); continue; }
-    double t = val[e] * Ek[j];
-    s = s + t;
-  }
-  HEc[l + (int64_t)k * m] = s + Hshift[l];
-}
-
 // Ensemble mode, observation anomalies: ybar = sum(HE,2)/N, HSf = (HE - ybar)/sqrt(N-1)
 // (assimilation.F90:3128-3134), written row-major m x NP; innov = yo - ybar.
 template <int NP, int TR = (NP > 64 ? 32 : 64)>
@@ -703,7 +684,7 @@ static void prep_ens_t(const PrepEnsArgs& A, hipStream_t st) {
                          A.ldE, A.xbar);
   }
   if (A.m == 0) return;
-  hipLaunchKernelGGL(k_spmm_obs, dim3(nblk(A.m, 256), A.N), dim3(256), 0, st, A.m, A.n, A.N,
+  hipLaunchKernelGGL(k_spmm_obs<double>, dim3(spmm_blocks(A.m, A.N)), dim3(256), 0, st, A.m, A.n, A.N,
                      A.row_ptr, A.col, A.val, A.E, A.ldE, A.Hshift, A.HEc, A.err);
   constexpr int TR = NP > 128 ? 16 : (NP > 64 ? 32 : 64);
   hipLaunchKernelGGL((k_obs_anom<NP, TR>), dim3(nblk(A.m, TR)), dim3(256), 0, st, A.m, A.N, A.HEc, A.yo,

@@ -6,7 +6,7 @@
 // the innovation scaling and the accumulation of S^T R^-1 S stay in FP64.
 //
 //   k_state_mean_f32   xbar (FP64 sums of FP32 members)
-//   k_spmm_obs_f32     HE = H E + Hshift (FP64 accumulation)
+//   k_spmm_obs<float>  HE = H E + Hshift (FP64 accumulation)
 //   k_obs_anom_f32     HS = (HE - ybar)/sqrt(N-1) stored FP32, innov/rho FP64
 //   k_gram<NP, float>  (analysis.hip / analysis128.hip) M = I + S^T diag(r) S
 //                      from the FP32 S on FP64 MFMA: products of FP32 values
@@ -23,6 +23,7 @@
 //                      (the FP32 sum of N terms Sf_k a_k cancels strongly)
 #include "analysis.hpp"
 #include "common.hpp"
+#include "spmm.hpp"
 
 namespace oakg {
 
@@ -62,24 +63,6 @@ __global__ void k_state_mean_f32x4(int64_t n4, int N, const float4* __restrict__
   double2* x2 = reinterpret_cast<double2*>(xbar + 4 * i);
   x2[0] = make_double2(s0 / N, s1 / N);
   x2[1] = make_double2(s2 / N, s3 / N);
-}
-
-__global__ void k_spmm_obs_f32(int64_t m, int64_t n, int N, const int64_t* __restrict__ row_ptr,
-                               const int32_t* __restrict__ col, const double* __restrict__ val,
-                               const float* __restrict__ E, int64_t ld,
-                               const float* __restrict__ Hshift, double* __restrict__ HEc,
-                               unsigned* __restrict__ err) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y;
-  if (l >= m) return;
-  const float* Ek = E + (int64_t)k * ld;
-  double s = 0;
-  for (int64_t e = row_ptr[l]; e < row_ptr[l + 1]; ++e) {
-    int32_t j = col[e];
-    if (j < 0 || j >= n) { atomicOr(err, OAKG_DERR_IDX); continue; }
-    s = fma(val[e], (double)Ek[j], s);
-  }
-  HEc[l + (int64_t)k * m] = s + (double)Hshift[l];
 }
 
 template <int NP, int TR>
@@ -209,7 +192,7 @@ static void prep_ens_f32_t(const PrepEnsArgs& A, hipStream_t st) {
                          A.E32, A.ldE, A.xbar);
   }
   if (A.m == 0) return;
-  hipLaunchKernelGGL(k_spmm_obs_f32, dim3(nblk32(A.m, 256), A.N), dim3(256), 0, st, A.m, A.n, A.N,
+  hipLaunchKernelGGL(k_spmm_obs<float>, dim3(spmm_blocks(A.m, A.N)), dim3(256), 0, st, A.m, A.n, A.N,
                      A.row_ptr, A.col, A.val, A.E32, A.ldE, A.Hshift32, A.HEc, A.err);
   constexpr int TR = NP > 128 ? 16 : (NP > 64 ? 32 : 64);
   hipLaunchKernelGGL((k_obs_anom_f32<NP, TR>), dim3(nblk32(A.m, TR)), dim3(256), 0, st, A.m, A.N,
