@@ -10,9 +10,7 @@
 //             Y = X diag(mu^-5/4) with Y Y^T = (I+C)^-1/2
 //   k_tmat    T = (I+C)^-1/2 Omega, Omega = RotateVector(w, v) (rrsqrt.F90:185,
 //             737-745; perpSpace matoper.F90:509-535) as identity + rank-5 terms
-//   k_update  [xa - xf | Sa] = Sf_z [a | T] on MFMA, with the ensemble-mode
-//             epilogue (inflation, maxCorrection, Ea = xa + sqrt(N-1) Sa;
-//             assimilation.F90:3299-3320)
+// The Householder path and the update (Sf T, Sf a) are in funcm.hip and update.hip.
 #include "analysis.hpp"
 #include "common.hpp"
 #include "spmm.hpp"
@@ -480,6 +478,7 @@ __global__ __launch_bounds__(256) void k_eig(int64_t z0, const int32_t* __restri
 }
 
 // ---------------------------------------------------------------------------
+// After the Jacobi option at N <= 32 (the eigensolver's T otherwise):
 // T = (Y Y^T) Omega, Omega = RotateVector(w, v) = v w^T + P(v) P(w)^T with
 // P(u) = [I; 0] + alpha_u (u + sign(u_N) e_N) u(1:N-1)^T, alpha_u = -1/(|u_N|+1):
 //   Omega = I - e e^T + v w^T + alpha_w w~ z_w^T + alpha_v z_v v~^T
@@ -488,13 +487,13 @@ __global__ __launch_bounds__(256) void k_eig(int64_t z0, const int32_t* __restri
 // Zones without observations get T = I exactly (Sa = Sf, rrsqrt.F90:326,371).
 // ---------------------------------------------------------------------------
 template <int NP>
-__global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
+__global__ __launch_bounds__(256) void k_tmat(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
                                               const double* __restrict__ ymat,
                                               double* __restrict__ mat,
                                               const double* __restrict__ vec) {
   constexpr int NB = NP / 16;
   constexpr int LD = NP + 1;
-  __shared__ double Ys[NP < 64 ? NP * LD : 1];
+  __shared__ double Ys[NP * LD];
   __shared__ double T0[NP * LD];
   __shared__ double U[4][NP];
   const int zl = blockIdx.x;
@@ -507,12 +506,11 @@ __global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __re
   }
   const double* v = vec + (size_t)zl * 4 * NP + 2 * NP;
   const double* Yz = ymat + (size_t)zl * NP * NP;
-  for (int e = threadIdx.x; e < NP * NP; e += 256) (NP < 64 ? Ys : T0)[(e / NP) * LD + e % NP] = Yz[e];
+  for (int e = threadIdx.x; e < NP * NP; e += 256) Ys[(e / NP) * LD + e % NP] = Yz[e];
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int li = lane & 15, kk = lane >> 4;
-  // NP = 64: ymat holds M^-1/2 itself (staged straight into T0 above)
-  for (int tile = wave; NP < 64 && tile < NB * NB; tile += 4) {
+  for (int tile = wave; tile < NB * NB; tile += 4) {
     const int I = tile / NB, J = tile % NB;
     d4 acc = {0, 0, 0, 0};
 #pragma unroll 4
@@ -560,92 +558,6 @@ __global__ __launch_bounds__(256, 2) void k_tmat(int64_t z0, const int32_t* __re
       t += U[1][r] * ws + alw * U[2][r] * zw + alv * U[3][r] * vt + alv * alw * vw * U[3][r] * zw;
     }
     M[e] = t;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Update: out = Sf_z [T | a] for the zone's rows.  Computed transposed on the
-// MFMA (A = [T|a]^T from LDS, B = Sf_z^T from global) so that the stores of
-// each 16-row strip are contiguous in the column-major outputs.
-//   MODE_LOC: xa = xf + Sf a, Sa = Sf T            (rrsqrt.F90:151,185,463)
-//   MODE_ENS: Sf = (E - xbar)/sqrt(N-1) on the fly; xa = xbar + clamp(Sf a);
-//             Ea = xa + sqrt(N-1) * (inflation * Sf T)  (assimilation.F90:3301-3320)
-// ---------------------------------------------------------------------------
-template <int NP, int MODE>
-__global__ __launch_bounds__(256) void k_update(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ zone_ptr,
-                                                const double* __restrict__ mat,
-                                                const double* __restrict__ vec,
-                                                const double* __restrict__ X0,  // xf or xbar
-                                                const double* __restrict__ S, int64_t ldS,  // Sf or E
-                                                double* __restrict__ xa, double* __restrict__ Out,
-                                                int64_t ldO, double scaling, double infl,
-                                                double maxcorr,
-                                                const double* __restrict__ maxcorr_v) {
-#pragma clang fp contract(off)
-  constexpr int NB = NP / 16;
-  constexpr int LDW = NP + 17;
-  __shared__ double Ws[NP * LDW];
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  const int64_t i0 = zone_ptr[z];
-  const int64_t sz = zone_ptr[z + 1] - i0;
-  const double* T = mat + (size_t)zl * NP * NP;
-  const double* a = vec + (size_t)zl * 4 * NP + NP;
-  for (int e = threadIdx.x; e < NP * (NP + 16); e += 256) {
-    const int k = e / (NP + 16), c = e % (NP + 16);
-    double v = 0.0;
-    if (c < NP) v = T[k * NP + c];
-    else if (c == NP) v = a[k];
-    Ws[k * LDW + c] = v;
-  }
-  __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int li = lane & 15, kk = lane >> 4;
-  for (int64_t rb = 16 * wave; rb < sz; rb += 64) {
-    d4 acc[NB + 1];
-#pragma unroll
-    for (int J = 0; J <= NB; ++J) acc[J] = d4{0, 0, 0, 0};
-    const int64_t row = rb + li;
-    const bool rok = row < sz;
-    const double xb = (MODE == 1 && rok) ? X0[i0 + row] : 0.0;
-    for (int k0 = 0; k0 < NP; k0 += 4) {
-      const int kc = k0 + kk;
-      double bval = 0.0;
-      if (rok && kc < N) {
-        const double sv = S[(i0 + row) + (int64_t)kc * ldS];
-        bval = (MODE == 1) ? (sv - xb) / scaling : sv;
-      }
-#pragma unroll
-      for (int J = 0; J <= NB; ++J) acc[J] = mfma_f64(Ws[kc * LDW + 16 * J + li], bval, acc[J]);
-    }
-    // xa - xf of row (rb + li) is column 0 of the last tile: lanes 0..15, register 0
-    const double dx = shfl_d(acc[NB][0], li);
-    double xar = 0.0;
-    if (rok) {
-      const double x0 = X0[i0 + row];
-      xar = x0 + dx;
-      if (MODE == 1) {
-        const double mc = maxcorr_v ? maxcorr_v[i0 + row] : maxcorr;
-        if (xar - mc > x0) xar = x0 + mc;
-        if (xar < x0 - mc) xar = x0 - mc;
-      }
-      if (MODE == 0 && kk == 0) xa[i0 + row] = xar;
-    }
-#pragma unroll
-    for (int J = 0; J < NB; ++J) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = 16 * J + kk + 4 * r;
-        if (rok && col < N) {
-          double o = acc[J][r];
-          if (MODE == 1) {
-            double sa = (infl != 1.0) ? infl * o : o;
-            o = xar + sa * scaling;
-          }
-          Out[(i0 + row) + (int64_t)col * ldO] = o;
-        }
-      }
-    }
   }
 }
 
@@ -740,21 +652,13 @@ static void chunk_t(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
                        A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, A.err);
   if (tm) tm->mark(PH_EIG);
   eig_t<NP>(A, st);
-  if (tm) tm->mark(PH_TMAT);
-  if (NP == 64 || A.eig_method != 1)
-    hipLaunchKernelGGL(k_tmat<NP>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,
-                     A.mat, A.vec);
+  if (NP < 64 && A.eig_method != 1) {
+    if (tm) tm->mark(PH_TMAT);
+    hipLaunchKernelGGL(k_tmat<(NP < 64 ? NP : 32)>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N,
+                       A.sel_ptr, A.ymat, A.mat, A.vec);
+  }
   if (tm) tm->mark(PH_UPDATE);
-  if (A.prec == 1)
-    launch_update_f32(NP, A, st);
-  else if (A.mode == 0)
-    hipLaunchKernelGGL((k_update<NP, 0>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.zone_ptr,
-                       A.mat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out, A.ldO, A.scaling, A.infl,
-                       A.maxcorr, A.maxcorr_v);
-  else
-    hipLaunchKernelGGL((k_update<NP, 1>), dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.zone_ptr,
-                       A.mat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out, A.ldO, A.scaling, A.infl,
-                       A.maxcorr, A.maxcorr_v);
+  launch_update(NP, A, st);
   if (tm) tm->mark(PH_END);
 }
 

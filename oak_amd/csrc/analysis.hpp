@@ -107,7 +107,8 @@ struct ChunkArgs {
   unsigned* err;
   double tol;
   int max_sweeps;
-  const double* X0;  // xf (mode 0) or xbar (mode 1)
+  int zone_rows;     // mean rows of a zone
+  const double* X0;  // xf (mode 0) or xbar (mode 1, N > 64)
   const double* S;   // Sf (mode 0) or E (mode 1)
   int64_t ldS;
   double* xa;   // mode 0
@@ -185,7 +186,8 @@ void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
 // pole table of the current device
 hipError_t init_poles(int device);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
-void launch_update_f32(int NP, const ChunkArgs& A, hipStream_t st);
+// N <= 64 (update.hip): T from mat (N <= 32) or M^-1/2 from ymat
+void launch_update(int NP, const ChunkArgs& A, hipStream_t st);
 // N <= 64: Gram, factor and adjoint in one; N > 64: the adjoint after the eigensolve
 void launch_nll_chol(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_nll_adjoint(int NP, const ChunkArgs& A, hipStream_t st);

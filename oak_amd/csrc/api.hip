@@ -853,6 +853,7 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
   A.scaling = 1.0;
   A.infl = 1.0;
   A.maxcorr = HUGE_VAL;
+  A.zone_rows = (int)std::min<int64_t>(n / std::max<int64_t>(nz, 1), INT32_MAX);
   const bool swept = run_zones(c, NP, A, nz, sweeps);
   if (c->timing) c->timer.mark(PH_END);
   if (!c->arena) check(c, hipEventRecord(c->ev_t1, c->stream), "event");
@@ -1014,7 +1015,10 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     const double* dval = stage(c, Workspace::H_VAL, H->val, H->nnz, dev);
     const T* dHs = stage(c, Workspace::H_SHIFT, Hshift, m, dev);
     const double* dmc = stage(c, Workspace::MAXCORR, maxc_elem, n, dev);
-    double* xbar = (double*)wsget(c, Workspace::XBAR, sizeof(double) * std::max<int64_t>(n, 1));
+    // the mean of the state: the update of N <= 64 forms it from its own rows
+    const bool own_mean = NP <= 64;
+    double* xbar = own_mean ? nullptr
+                            : (double*)wsget(c, Workspace::XBAR, sizeof(double) * std::max<int64_t>(n, 1));
     double* HEc = (double*)wsget(c, Workspace::HEC, sizeof(double) * std::max<int64_t>(m, 1) * N);
     double* HS = nullptr;
     float* HS32 = nullptr;
@@ -1024,7 +1028,7 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
       HS = (double*)wsget(c, Workspace::HS, sizeof(double) * std::max<int64_t>(m, 1) * NP);
     double* innov = (double*)wsget(c, Workspace::INNOV, sizeof(double) * std::max<int64_t>(m, 1));
     double* rho = (double*)wsget(c, Workspace::RHO, sizeof(double) * std::max<int64_t>(m, 1));
-    if (!xbar || !HEc || !(mixed ? (void*)HS32 : (void*)HS) || !innov || !rho)
+    if ((!own_mean && !xbar) || !HEc || !(mixed ? (void*)HS32 : (void*)HS) || !innov || !rho)
       check(c, hipErrorOutOfMemory, "workspace");
     const double scaling = sqrt((double)N - 1.0);
     PrepEnsArgs P{};
@@ -1095,7 +1099,8 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     A.infl = inflation;
     A.maxcorr = max_correction;
     A.maxcorr_v = dmc;
-    const bool swept = run_zones(c, NP, A, nz, sweeps);
+    A.zone_rows = (int)std::min<int64_t>(n / std::max<int64_t>(nz, 1), INT32_MAX);
+  const bool swept = run_zones(c, NP, A, nz, sweeps);
     if (c->timing) c->timer.mark(PH_END);
     check(c, hipEventRecord(c->ev_t1, c->stream), "event");
     finish_call(c, nz, sel.ptr, swept ? sweeps : nullptr);

@@ -17,8 +17,7 @@
 //                      spread (T ~ I); with |C| up to ~1e5 (precise SSH
 //                      observations) that is ~1e-3 of the spread.  Rounding
 //                      S itself perturbs those directions only at second order.
-//   k_update_f32       (N <= 64; analysis128.hip's k_xform128f for NP = 128)
-//                      Ea = xa + sqrt(N-1) infl (Sf T) on v_mfma_f32_16x16x4f32
+//   update             (update.hip for N <= 64; k_xform128f for NP = 128) Ea = xa + sqrt(N-1) infl (Sf T) on v_mfma_f32_16x16x4f32
 //                      with T rounded to FP32; xa = xbar + clamp(Sf a) in FP64
 //                      (the FP32 sum of N terms Sf_k a_k cancels strongly)
 #include "analysis.hpp"
@@ -26,15 +25,6 @@
 #include "spmm.hpp"
 
 namespace oakg {
-
-// v_mfma_f32_16x16x4f32 operand layout on gfx950 (checked on the device):
-//   A (16x4):  lane l holds A[l % 16][l / 16]
-//   B (4x16):  lane l holds B[l / 16][l % 16]
-//   D (16x16): lane l, register r holds D[4 (l / 16) + r][l % 16]
-// (the FP64 instruction places D rows at l / 16 + 4 r instead)
-__device__ __forceinline__ f4 mfma_f32(float a, float b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 __global__ void k_state_mean_f32(int64_t n, int N, const float* __restrict__ E, int64_t ld,
                                  double* __restrict__ xbar) {
@@ -106,79 +96,6 @@ __global__ __launch_bounds__(256) void k_obs_anom_f32(int64_t m, int N, const do
   }
 }
 
-// Ensemble update for FP32 members: Sf = (E - xbar)/sqrt(N-1) on the fly,
-// xa = xbar + clamp(Sf a), Ea = xa + sqrt(N-1) infl (Sf T).  The MFMA computes
-// the transposed product (A = [T|a]^T from LDS, B = Sf^T) so that each
-// 16-row strip is stored as contiguous runs of the column-major Ea.
-template <int NP>
-__global__ __launch_bounds__(256, 2) void k_update_f32(int64_t z0, const int32_t* __restrict__ zorder, int N,
-                                                    const int64_t* __restrict__ zone_ptr,
-                                                    const double* __restrict__ mat,
-                                                    const double* __restrict__ vec,
-                                                    const double* __restrict__ xbar,
-                                                    const float* __restrict__ E, int64_t ldE,
-                                                    float* __restrict__ Out, int64_t ldO,
-                                                    double scaling, double infl, double maxcorr,
-                                                    const double* __restrict__ maxcorr_v) {
-  constexpr int NB = NP / 16;
-  constexpr int LDW = NP + 17;  // the 4 k-rows of one MFMA step land on distinct banks
-  __shared__ float Ws[NP * LDW];
-  __shared__ double as[NP];
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  const int64_t i0 = zone_ptr[z];
-  const int64_t sz = zone_ptr[z + 1] - i0;
-  const double* T = mat + (size_t)zl * NP * NP;
-  const double* a = vec + (size_t)zl * 4 * NP + NP;
-  for (int e = threadIdx.x; e < NP * NP; e += 256) Ws[(e / NP) * LDW + e % NP] = (float)T[e];
-  if (threadIdx.x < NP) as[threadIdx.x] = a[threadIdx.x] / scaling;
-  __syncthreads();
-  const float inv = (float)(1.0 / scaling);
-  const double sc_infl = scaling * infl;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int li = lane & 15, kk = lane >> 4;
-  for (int64_t rb = 16 * wave; rb < sz; rb += 64) {
-    f4 acc[NB];
-#pragma unroll
-    for (int J = 0; J < NB; ++J) acc[J] = f4{0, 0, 0, 0};
-    const int64_t row = rb + li;
-    const bool rok = row < sz;
-    const double xbd = rok ? xbar[i0 + row] : 0.0;
-    const float xb = (float)xbd;
-    const float* Er = E + (i0 + (rok ? row : 0));
-    double dxp = 0.0;  // (E - xbar) a / sqrt(N-1) over this lane's members, FP64
-#pragma unroll 4
-    for (int k0 = 0; k0 < NP; k0 += 4) {
-      const int kc = k0 + kk;
-      float bval = 0.0f;
-      if (rok && kc < N) {
-        const float ev = Er[(int64_t)kc * ldE];
-        bval = (ev - xb) * inv;
-        dxp = fma((double)ev - xbd, as[kc], dxp);
-      }
-#pragma unroll
-      for (int J = 0; J < NB; ++J) acc[J] = mfma_f32(Ws[kc * LDW + 16 * J + li], bval, acc[J]);
-    }
-    dxp += __shfl_xor(dxp, 16, 64);
-    dxp += __shfl_xor(dxp, 32, 64);
-    if (rok) {
-      double xar = xbd + dxp;
-      const double mc = maxcorr_v ? maxcorr_v[i0 + row] : maxcorr;
-      if (xar - mc > xbd) xar = xbd + mc;
-      if (xar < xbd - mc) xar = xbd - mc;
-      float* Orow = Out + (i0 + row);
-#pragma unroll
-      for (int J = 0; J < NB; ++J) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int col = 16 * J + 4 * kk + r;
-          if (col < N) Orow[(int64_t)col * ldO] = (float)(xar + sc_infl * (double)acc[J][r]);
-        }
-      }
-    }
-  }
-}
-
 static inline unsigned nblk32(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 template <int NP>
@@ -207,19 +124,6 @@ void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st) {
     case 128: prep_ens_f32_t<128>(A, st); break;
     case 256: prep_ens_f32_t<256>(A, st); break;
   }
-}
-
-void launch_update_f32(int NP, const ChunkArgs& A, hipStream_t st) {
-#define OAK_UPD32(P)                                                                             \
-  hipLaunchKernelGGL(k_update_f32<P>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.zone_ptr, A.mat, \
-                     A.vec, A.X0, A.S32, A.ldS, A.Out32, A.ldO, A.scaling, A.infl, A.maxcorr, \
-                     A.maxcorr_v)
-  switch (NP) {
-    case 16: OAK_UPD32(16); break;
-    case 32: OAK_UPD32(32); break;
-    case 64: OAK_UPD32(64); break;
-  }
-#undef OAK_UPD32
 }
 
 }  // namespace oakg

@@ -1,0 +1,299 @@
+// The update of a zone's rows for N <= 64:
+//   MODE 0 (locAnalysis): xa = xf + Sf a, Sa = Sf T   (rrsqrt.F90:151,185,463)
+//   MODE 1 (ensemble): Sf = (E - xbar)/sqrt(N-1) with xbar the members' mean;
+//     xa = xbar + clamp(Sf a); Ea = xa + sqrt(N-1) (inflation Sf T)
+//     (assimilation.F90:3301-3320).  The factors sqrt(N-1) cancel in Sf T and
+//     go to a in Sf a, so that E - xbar is used as it is.
+// Computed transposed on the MFMA (A = T^T, B = Sf^T) so that the loads and
+// stores of each 16-row strip are 16 consecutive rows of four members.  A
+// strip's members are all in registers before the product: the mean of the
+// state needs no pass of its own over the ensemble.  FP32 members: E - xbar
+// and T rounded to FP32 for v_mfma_f32_16x16x4f32, Sf a in FP64 (the sum of N
+// terms Sf_k a_k cancels strongly).
+#include <type_traits>
+
+#include "analysis.hpp"
+#include "common.hpp"
+#include "eigen_common.hpp"
+
+namespace oakg {
+
+namespace {
+
+template <typename T>
+using vec4 = typename std::conditional<sizeof(T) == 4, f4, d4>::type;
+// D row of register r in lane group kk (the two instructions differ)
+template <typename T>
+__device__ __forceinline__ constexpr int drow(int kk, int r) {
+  return sizeof(T) == 4 ? 4 * kk + r : kk + 4 * r;
+}
+__device__ __forceinline__ d4 mfma(double a, double b, d4 c) { return mfma_f64(a, b, c); }
+__device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// What the rows of a strip share: the row's mean (or xf), the clamp and the
+// column of the increment.  b: the lane's members k(q) of row `row`, replaced
+// by the anomalies; as: a (MODE 0) or a / sqrt(N-1).  Returns xa.
+template <int Q, int MODE, typename TE, typename K, typename As>
+__device__ __forceinline__ double strip_head(TE (&b)[Q], int N, K k, As as, bool rok, int64_t row,
+                                             const double* __restrict__ X0, double maxcorr,
+                                             const double* __restrict__ maxcorr_v) {
+#pragma clang fp contract(off)
+  double x0 = 0.0, dx = 0.0;
+  if (MODE == 1) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) x0 += k(q) < N ? (double)b[q] : 0.0;
+    x0 = sum_xor32(sum_xor16(x0)) / N;
+  } else {
+    x0 = X0[row];
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    double d = MODE == 1 ? (double)b[q] - x0 : (double)b[q];
+    d = rok && k(q) < N ? d : 0.0;
+    dx = fma(d, as(q), dx);
+    b[q] = (TE)d;
+  }
+  double xar = x0 + sum_xor32(sum_xor16(dx));
+  if (MODE == 1) {
+    const double mc = maxcorr_v ? maxcorr_v[row] : maxcorr;
+    if (xar - mc > x0) xar = x0 + mc;
+    if (xar < x0 - mc) xar = x0 - mc;
+  }
+  return xar;
+}
+
+template <int MODE, typename TE>
+__device__ __forceinline__ TE out_value(TE o, double xar, double infl) {
+#pragma clang fp contract(off)
+  if (MODE == 0) return o;
+  const double d = infl != 1.0 ? infl * (double)o : (double)o;
+  return (TE)(xar + d);
+}
+
+}  // namespace
+
+// N <= 32: T (left in mat by the eigensolve) in registers, no LDS, no
+// barrier; `wpz` waves share a zone's strips, the next strip's members are
+// loaded before the current one's product.
+template <int NP, int MODE, typename TE>
+__global__ __launch_bounds__(256, NP == 32 ? 3 : 4) void k_update_small(int64_t z0, const int32_t* __restrict__ zorder,
+                                                         int nzc, int wpz, int N,
+                                                         const int64_t* __restrict__ zone_ptr,
+                                                         const double* __restrict__ mat,
+                                                         const double* __restrict__ vec,
+                                                         const double* __restrict__ X0,
+                                                         const TE* __restrict__ S, int64_t ldS,
+                                                         double* __restrict__ xa,
+                                                         TE* __restrict__ Out, int64_t ldO,
+                                                         double scaling, double infl, double maxcorr,
+                                                         const double* __restrict__ maxcorr_v) {
+  constexpr int NB = NP / 16, Q = NP / 4;
+  const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), zl = wave / wpz, sub = wave % wpz;
+  if (zl >= nzc) return;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  const int64_t i0 = zone_ptr[z], sz = zone_ptr[z + 1] - i0;
+  if (16 * (int64_t)sub >= sz) return;
+  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
+  TE b[Q], nb[Q];
+  auto load = [&](int64_t rb, TE (&v)[Q]) {
+    const int64_t row = i0 + (rb + li < sz ? rb + li : 0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) v[q] = S[row + (int64_t)(4 * q + kk < N ? 4 * q + kk : 0) * ldS];
+  };
+  load(16 * sub, b);
+  const double* T = mat + (size_t)zl * NP * NP;
+  const double* a = vec + (size_t)zl * 4 * NP + NP;
+  TE t[NB][Q];
+  double as[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    as[q] = MODE == 1 ? a[4 * q + kk] / scaling : a[4 * q + kk];
+#pragma unroll
+    for (int J = 0; J < NB; ++J) t[J][q] = (TE)T[(4 * q + kk) * NP + 16 * J + li];
+  }
+  for (int64_t rb = 16 * sub; rb < sz; rb += 16 * wpz) {
+    const bool more = rb + 16 * wpz < sz;
+    if (more) load(rb + 16 * wpz, nb);
+    const bool rok = rb + li < sz;
+    const int64_t row = i0 + (rok ? rb + li : 0);
+    const double xar = strip_head<Q, MODE>(b, N, [&](int q) { return 4 * q + kk; },
+                                           [&](int q) { return as[q]; }, rok, row, X0, maxcorr, maxcorr_v);
+    if (MODE == 0 && rok && kk == 0) xa[row] = xar;
+    vec4<TE> acc[NB];
+#pragma unroll
+    for (int J = 0; J < NB; ++J) acc[J] = vec4<TE>{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int J = 0; J < NB; ++J) acc[J] = mfma(t[J][q], b[q], acc[J]);
+#pragma unroll
+    for (int J = 0; J < NB; ++J)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = 16 * J + drow<TE>(kk, r);
+        if (rok && col < N) Out[row + (int64_t)col * ldO] = out_value<MODE, TE>(acc[J][r], xar, infl);
+      }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) b[q] = nb[q];
+  }
+}
+
+// 33 <= N <= 64: a workgroup per zone forms T = R Omega from M^-1/2 (in ymat)
+// in LDS - R is symmetric, so that Omega is applied to its columns and row s
+// holds column s of T - and its four waves take the strips in turn.  The k
+// index of the MFMA steps is permuted within pairs (lane group kk covers k =
+// 8 p + 2 kk and the next), so that one LDS read of two entries serves two
+//  Bound by the reads and writes of the ensemble: 64 800 zones of 121 rows,
+// N = 64, 8.0 GB and 2.1 GB of M^-1/2, 2.67 ms.  With T from a kernel of its own,
+// a spilling product that waited for each load and the mean in a pass before,
+// these took 1.6, 10.5 and 0.7 ms.
+template <int MODE, typename TE>
+__global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                     const int64_t* __restrict__ sel_ptr,
+                                                     const int64_t* __restrict__ zone_ptr,
+                                                     const double* __restrict__ ymat,
+                                                     const double* __restrict__ vec,
+                                                     const double* __restrict__ X0,
+                                                     const TE* __restrict__ S, int64_t ldS,
+                                                     double* __restrict__ xa, TE* __restrict__ Out,
+                                                     int64_t ldO, double scaling, double infl,
+                                                     double maxcorr,
+                                                     const double* __restrict__ maxcorr_v) {
+  constexpr int NP = 64, NB = NP / 16, Q = NP / 4;
+  constexpr int LD = sizeof(TE) == 4 ? NP + 4 : NP + 2;  // reads of 16 rows on distinct banks
+  typedef TE TE2 __attribute__((ext_vector_type(2)));
+  __shared__ __attribute__((aligned(16))) TE L[NP * LD];
+  __shared__ double u[4][NP], w[4][NP], v[NP], as[NP], vws;
+  const int zl = blockIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  const int64_t i0 = zone_ptr[z], sz = zone_ptr[z + 1] - i0;
+  if (sz <= 0) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, kk = lane >> 4;
+  const double* Vz = vec + (size_t)zl * 4 * NP;
+  auto k_of = [&](int q) { return 8 * (q >> 1) + 2 * kk + (q & 1); };
+  TE b[Q];
+  auto load = [&](int64_t rb) {
+    const int64_t row = i0 + (rb + li < sz ? rb + li : 0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) b[q] = S[row + (int64_t)(k_of(q) < N ? k_of(q) : 0) * ldS];
+  };
+  if (sel_ptr[z + 1] == sel_ptr[z]) {  // no observations: T = I, a = 0
+    load(16 * wave);
+    for (int e = tid; e < NP * NP; e += 256) L[(e / NP) * LD + e % NP] = e / NP == e % NP ? 1 : 0;
+    if (tid < NP) as[tid] = 0.0;
+    lds_barrier();
+  } else {
+    // thread (h, r): rows s = 4 i + h of column r (M^-1/2 is symmetric)
+    const int r = tid & 63, h = tid >> 6;
+    const double* R = ymat + (size_t)zl * NP * NP;
+    double x[NP / 4];
+#pragma unroll
+    for (int i = 0; i < NP / 4; ++i) x[i] = R[(4 * i + h) * NP + r];
+    if (tid < NP) {
+      as[tid] = MODE == 1 ? Vz[NP + tid] / scaling : Vz[NP + tid];
+      v[tid] = tid < N ? Vz[2 * NP + tid] : 0.0;
+    }
+    lds_barrier();
+    // (analysis.hip's k_tmat): with zw = w + e_{N-1}, vt = v but 0 at N - 1,
+    // T[r][s] = R[r][s] (0 at s = N-1) + u1 w + (alpha_w u2 + alpha_v alpha_w
+    // (v.w~) u3) zw_s + alpha_v u3 vt_s, u1 = (R v)_r, u2 = (R w~)_r, u3 = u1 +
+    // sign(v_N) R[r][N-1]
+    double su = 0.0, sw = 0.0;
+#pragma unroll
+    for (int i = 0; i < NP / 4; ++i) {
+      const int s = 4 * i + h;
+      su = fma(x[i], v[s], su);
+      sw += s < N - 1 ? x[i] : 0.0;
+    }
+    u[h][r] = su;
+    w[h][r] = sw;
+    const double wN = 1.0 / sqrt((double)N), vN = v[N - 1], sgv = vN >= 0 ? 1.0 : -1.0;
+    const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0);
+    if (wave == 0) {
+      const double s = wave_sum_fast(lane < N - 1 ? v[lane] * wN : 0.0);
+      if (lane == 0) vws = s;
+    }
+    load(16 * wave);  // in flight while T is finished (LDS barriers only)
+    lds_barrier();
+    const double u0 = R[(size_t)(N - 1) * NP + r];
+    const double u1 = (u[0][r] + u[1][r]) + (u[2][r] + u[3][r]);
+    const double u2 = wN * ((w[0][r] + w[1][r]) + (w[2][r] + w[3][r]));
+    const double u3 = fma(sgv, u0, u1);
+    const double c1 = u1 * wN, c2 = alw * u2 + alv * alw * vws * u3, c3 = alv * u3;
+#pragma unroll
+    for (int i = 0; i < NP / 4; ++i) {
+      const int s = 4 * i + h;
+      const double zw = s == N - 1 ? wN + 1.0 : wN, vt = s < N - 1 ? v[s] : 0.0;
+      const double t = s == N - 1 ? 0.0 : x[i];
+      L[s * LD + r] = (TE)(s < N ? t + (c1 + c2 * zw + c3 * vt) : x[i]);
+    }
+    lds_barrier();
+  }
+  const TE* lt = L + li * LD + 2 * kk;
+  for (int64_t rb = 16 * wave; rb < sz; rb += 64) {
+    if (rb != 16 * wave) load(rb);
+    const bool rok = rb + li < sz;
+    const int64_t row = i0 + (rok ? rb + li : 0);
+    const double xar = strip_head<Q, MODE>(b, N, k_of, [&](int q) { return as[k_of(q)]; }, rok, row, X0,
+                                           maxcorr, maxcorr_v);
+    if (MODE == 0 && rok && kk == 0) xa[row] = xar;
+    vec4<TE> acc[NB];
+#pragma unroll
+    for (int J = 0; J < NB; ++J) acc[J] = vec4<TE>{0, 0, 0, 0};
+#pragma unroll
+    for (int p = 0; p < Q / 2; ++p) {
+      asm volatile("" ::: "memory");  // the reads of later pairs stay below
+      TE2 A[NB];
+#pragma unroll
+      for (int J = 0; J < NB; ++J) A[J] = *reinterpret_cast<const TE2*>(lt + 16 * J * LD + 8 * p);
+#pragma unroll
+      for (int J = 0; J < NB; ++J) acc[J] = mfma(A[J].x, b[2 * p], acc[J]);
+#pragma unroll
+      for (int J = 0; J < NB; ++J) acc[J] = mfma(A[J].y, b[2 * p + 1], acc[J]);
+    }
+#pragma unroll
+    for (int J = 0; J < NB; ++J)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = 16 * J + drow<TE>(kk, r);
+        if (rok && col < N) Out[row + (int64_t)col * ldO] = out_value<MODE, TE>(acc[J][r], xar, infl);
+      }
+  }
+}
+
+// Waves per zone at N <= 32: one for every 32 rows of a mean zone, at most
+// the four of a workgroup (a wave reads the whole of T).
+void launch_update(int NP, const ChunkArgs& A, hipStream_t st) {
+  const int wpz = A.zone_rows > 64 ? 4 : (A.zone_rows > 32 ? 2 : 1);
+  const dim3 small((unsigned)(((int64_t)A.nzc * wpz + 3) / 4)), blk(256);
+#define OAK_UPD(MODE, TE, SRC, DST)                                                                   \
+  switch (NP) {                                                                                       \
+    case 16:                                                                                          \
+      hipLaunchKernelGGL((k_update_small<16, MODE, TE>), small, blk, 0, st, A.z0, A.zorder, A.nzc, wpz, \
+                         A.N, A.zone_ptr, A.mat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO, A.scaling, \
+                         A.infl, A.maxcorr, A.maxcorr_v);                                             \
+      break;                                                                                          \
+    case 32:                                                                                          \
+      hipLaunchKernelGGL((k_update_small<32, MODE, TE>), small, blk, 0, st, A.z0, A.zorder, A.nzc, wpz, \
+                         A.N, A.zone_ptr, A.mat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO, A.scaling, \
+                         A.infl, A.maxcorr, A.maxcorr_v);                                             \
+      break;                                                                                          \
+    case 64:                                                                                          \
+      hipLaunchKernelGGL((k_update64<MODE, TE>), dim3(A.nzc), blk, 0, st, A.z0, A.zorder, A.N,        \
+                         A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,    \
+                         A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                  \
+      break;                                                                                          \
+  }
+  if (A.prec == 1) {
+    OAK_UPD(1, float, A.S32, A.Out32)
+  } else if (A.mode == 0) {
+    OAK_UPD(0, double, A.S, A.Out)
+  } else {
+    OAK_UPD(1, double, A.S, A.Out)
+  }
+#undef OAK_UPD
+}
+
+}  // namespace oakg
