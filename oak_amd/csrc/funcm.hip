@@ -226,6 +226,10 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     return;
   }
   double* V = qmat + (size_t)zl * NP * NP;
+  // order of M (the rest is the identity): the tiles and reflector blocks that
+  // reach it take part
+  const int n = DUAL ? (int)(sel_ptr[z + 1] - sel_ptr[z]) : N;
+  const int nt = (n + 15) >> 4, nblk = n > 2 ? (n + 13) >> 4 : 0;
   if (tid < NP) {
     const int k = step_row<NP>(tid);
     S.p.d[k] = dvec[(size_t)zl * NP + tid];
@@ -367,22 +371,22 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     }
   } else {
     // ---- T_b of the reflector blocks ----
-    for (int b = wave - 1; b < NB; b += NB - 1) {
+    for (int b = wave - 1; b < nblk; b += NB - 1) {
       const int k = 16 * b + lc;
       const double* src = V + (size_t)k * NP;
       d4 g = {0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 4 * b; k0 < NP / 4; k0 += 4) {
+      for (int k0 = 4 * b; k0 < 4 * nt; k0 += 4) {
         double xv[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) xv[u] = src[4 * (k0 + u) + lr];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const double xm = (k < NP - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
+          const double xm = (k < n - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
           g = mfma_f64(xm, xm, g);
         }
       }
       const double tk = src[k];
-      const double tau = k < NP - 2 ? tk : 0.0;
+      const double tau = k < n - 2 ? tk : 0.0;
       // V^T V packed into the block's place, then column by column replaced:
       // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j]
       double* gs = S.tp + b * 136;
@@ -523,7 +527,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     column_factors(S.p.g, B);
 #pragma unroll
     for (int I = NB / 2 - 2; I >= 0; --I)  // outside
-      if (I < Js) f[I] = tile(S.p.a, I, B);
+      if (I < Js) f[I] = J < nt && row_of(I) < nt ? tile(S.p.a, I, B) : d4{0.0, 0.0, 0.0, 0.0};
     column_factors(S.p.a, B);
 #pragma unroll
     for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
@@ -531,7 +535,9 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
 #pragma unroll
         for (int q = 0; q < 8; ++q) B[q] *= S.p.d[8 * lr + q];
       }
-      if (I > Js) f[I] = tile(I < NB / 2 ? S.p.g : S.p.a, I, B);
+      if (I > Js)
+        f[I] = J < nt && row_of(I) < nt ? tile(I < NB / 2 ? S.p.g : S.p.a, I, B)
+                                        : d4{0.0, 0.0, 0.0, 0.0};
     }
 #pragma unroll
     for (int I = 0; I < NB / 2; ++I)
@@ -546,21 +552,21 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
 #pragma unroll
     for (int e = 0; e < ER; ++e) pf[e] = src[TPR * e];
   };
-  load_block(NB - 1, tid / TPR, tid % TPR);
+  load_block(nblk > 0 ? nblk - 1 : 0, tid / TPR, tid % TPR);
   lds_barrier();  // the pole arrays are read
 #pragma unroll 1
-  for (int b = NB - 1; b >= 0; --b) {
+  for (int b = nblk - 1; b >= 0; --b) {
     // the thread index made opaque in each pass: left visible, the addresses
     // and predicates made from it are computed ahead of the loop, and spill
     int tq = threadIdx.x;
     asm volatile("" : "+v"(tq));
     const int tid = tq, lr = (tq >> 4) & 3, lc = tq & 15, pj = tq / TPR, pr = tq % TPR;
     double* vb = S.m.vb[b & 1];
-    const int k = 16 * b + pj;  // the reflector: zero up to row k (none past NP - 3)
+    const int k = 16 * b + pj;  // the reflector: zero up to row k (none past n - 3)
 #pragma unroll
     for (int e = 0; e < ER; ++e) {
       const int r = pr + TPR * e;
-      pf[e] = (k < NP - 2 && r > k) ? pf[e] : 0.0;
+      pf[e] = (k < n - 2 && r > k) ? pf[e] : 0.0;
       vb[r * LV + pj] = pf[e];
     }
     lds_barrier();
@@ -589,7 +595,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
       for (int I = 0; I < NB; ++I) {
         asm volatile("" ::: "memory");  // the reads of later rows stay below
         const int rI = row_of(I);
-        if (rI >= b) {
+        if (rI >= b && rI < nt && J < nt) {
           double va[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) va[q] = vp[(16 * rI + 4 * q) * LV];
@@ -603,7 +609,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     __builtin_amdgcn_wave_barrier();
     {
       d4 sp = {0.0, 0.0, 0.0, 0.0};
-      if (J >= b) {
+      if (J >= b && J < nt) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int at = (16 * J + 4 * q + lr) * LV + lc;
@@ -621,7 +627,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
       return hi * (hi + 1) / 2 + lo;
     };
     d4 pv = {0.0, 0.0, 0.0, 0.0};  // P
-    if (J >= b) {
+    if (J >= b && J < nt) {
       const double* vr = vb + (16 * J + lc) * LV + lr;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -644,7 +650,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     }
     lds_barrier();
     d4 qv = {0.0, 0.0, 0.0, 0.0};
-    if (J >= b) {
+    if (J >= b && J < nt) {
       d4 s2 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int q = 0; q < 4; ++q) s2 = mfma_f64(S.m.sf[lc * 17 + 4 * q + lr], pv[q], s2);
@@ -681,7 +687,7 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
       for (int I = 0; I < NB; ++I) {
         asm volatile("" ::: "memory");  // the reads of later rows stay below
         const int rI = row_of(I);
-        if (rI >= b) {
+        if (rI >= b && rI < nt && J < nt) {
           double vv[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) vv[q] = vp[16 * rI * LV + 4 * q];
@@ -689,15 +695,16 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
           for (int q = 0; q < 4; ++q) f[I] = mfma_f64(vv[q], qv[q], f[I]);
         }
       }
-      if (J >= b) {
+      if (J >= b && J < nt) {
 #pragma unroll
         for (int I = 0; I < NB; ++I) {
           asm volatile("" ::: "memory");
           double xv[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) xv[q] = xp[16 * row_of(I) * LV + 4 * q];
+          if (row_of(I) < nt)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) f[I] = mfma_f64(xv[q], pv[q], f[I]);
+            for (int q = 0; q < 4; ++q) f[I] = mfma_f64(xv[q], pv[q], f[I]);
         }
       }
     }

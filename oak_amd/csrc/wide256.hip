@@ -345,6 +345,9 @@ struct TriArgs {
   int64_t dz, d0, e0, dstep;
   double* vecs;
   int zvec, c1, ones;
+  // FULL: order of the matrix (the rows from it on are the identity's); -1: the
+  // zone's observation count
+  int n;
 };
 
 template <int NP, bool FULL = false>
@@ -416,7 +419,8 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
     return v;
   };
   double* col = S.colw[wave];
-  for (int i = 0; i < (FULL ? NP - 2 : H); ++i) {
+  const int n = FULL ? (A.n >= 0 ? A.n : (int)(A.sel_ptr[z + 1] - A.sel_ptr[z])) : NP;
+  for (int i = 0; i < (FULL ? n - 2 : H); ++i) {
     const int b = i & 1;
     double* pw = S.pw[b];
     double* pub = S.pub[b];
@@ -629,11 +633,21 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
         uz[((NV == 2 ? q : wave) == 1 ? A.c1 : 0) + lane + 64 * h] = u[q][h];
   }
   if constexpr (FULL) {
-    if (t == 0) {  // tile (NB-1, NB-1): the trailing 2 x 2 block, rows NP-2, NP-1
-      dv[(NP - 2) * A.dstep] = a[6][6];
-      ev[(NP - 2) * A.dstep] = a[7][6];
-      dv[(NP - 1) * A.dstep] = a[7][7];
+    // rows n - 2 and n - 1 (x: column n - 2), then the identity's
+    static_assert(!FULL || NP == 64, "one wave: lane r has row r");
+    if (lane == n - 2) dv[lane * A.dstep] = x[0];
+    if (lane == n - 1) {
+      if (n >= 2) ev[(n - 2) * A.dstep] = x[0];
+      if (n <= 8) dv[lane * A.dstep] = S.l0[lane][lane];
     }
+    if (n > 8 && own && tr == tc && tc == (n - 1) >> 3) {
+      double dn = a[0][0];
+#pragma unroll
+      for (int jj = 1; jj < 8; ++jj) dn = jj == ((n - 1) & 7) ? a[jj][jj] : dn;
+      dv[(n - 1) * A.dstep] = dn;
+    }
+    if (lane >= n) dv[lane * A.dstep] = 1.0;
+    if (lane >= n - 1 && lane < NP - 1) ev[lane * A.dstep] = 0.0;
     return;
   }
   constexpr int LDO = NP == 256 ? H : NP;
@@ -660,13 +674,14 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
 // the reduction of 64 800 zones took 20.5 ms, like this 14.4 ms.
 void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st) {
   TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)128 * 128, 128, 128,
-            A.dvec, A.evec, 128, 0, 0, 1, A.vec, 4 * 128, 2 * 128, ones};
+            A.dvec, A.evec, 128, 0, 0, 1, A.vec, 4 * 128, 2 * 128, ones, 128};
   hipLaunchKernelGGL((k_tridiag_lower<128>), dim3(A.nzc), dim3(128), 0, st, T);
   T.mat = A.ymat + 64 * 128;
   T.qmat = A.ymat + 64 * 128 + 64;
   T.d0 = T.e0 = 64;
   T.vecs = A.vec + 64;
   T.ones = -1;
+  T.n = ones - 64;
   hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
 }
 
@@ -805,11 +820,12 @@ __global__ __launch_bounds__(256, 2) void k_formq256(int64_t z0, const int32_t* 
       U[(size_t)(16 * I + lr + 4 * r) * NP + (NP - 1 - (16 * J + lc))] = q[I][r];
 }
 
-// NP = 64 (33 <= N <= 64, and the observation-space zones of N = 128): the
-// whole reduction on one wave per zone.
+// NP = 64 (33 <= N <= 64, and the observation-space zones of N = 128: ones =
+// -1): the whole reduction on one wave per zone, of the steps that the order
+// (N, or the zone's observations) has.
 void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st) {
   const TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)64 * 64, 64, 64,
-                  A.dvec, A.evec, 64, 0, 0, 1, A.vec, 4 * 64, 2 * 64, ones};
+                  A.dvec, A.evec, 64, 0, 0, 1, A.vec, 4 * 64, 2 * 64, ones, ones};
   hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
 }
 
