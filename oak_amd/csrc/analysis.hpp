@@ -90,25 +90,20 @@ struct ChunkArgs {
   const double* sel_w;
   const double *rho, *innov, *HS;
   double *mat, *ymat, *vec, *ampl;
-  double* umat;  // NP = 256: Q, then U, then Y (mat: M then T; ymat: the reflectors)
+  double* umat;  // NP = 256: the pole arrays, then T^T (mat: M, then Q F; ymat: the reflectors)
   int32_t* sweeps;
-  // eigensolver: 0 = one-sided Jacobi, 1 = Householder tridiagonalisation + implicit QL
+  // 0 = one-sided Jacobi, 1 = Householder tridiagonalisation + functions of T
   int eig_method;
-  int ql_zw;                // zones per wave of the QL kernel (4, 8, 16 or 32)
-  int tri_split;            // NP = 128: the Householder reduction as two launches
   unsigned* persist_wq;     // NP = 128: work counter of the persistent Gram (NULL: one
                             // workgroup per zone)
   int persist_item;         // its scheduling: 1 a zone per workgroup, 0 each wave its quarter
   int persist_grid;         // its workgroups (persist_grid128)
-  double *dvec, *evec;      // tridiagonal / eigenvalues, NP x nzc
-  void* rlog;               // QL rotation log, rlog_cap records of 16 B per zone
-  int64_t rlog_cap;
-  int32_t* tql_status;      // per zone: bit0 log overflow, bit1 no convergence, >>2 log length
+  double *dvec, *evec;      // tridiagonal, NP per zone
   unsigned* err;
   double tol;
   int max_sweeps;
   int zone_rows;     // mean rows of a zone
-  const double* X0;  // xf (mode 0) or xbar (mode 1, N > 64)
+  const double* X0;  // xf (mode 0) or xbar (mode 1, N = 65..128)
   const double* S;   // Sf (mode 0) or E (mode 1)
   int64_t ldS;
   double* xa;   // mode 0
@@ -166,11 +161,9 @@ void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_dual128(const ChunkArgs& A, int N, double* ymat128, double* vec128, double* ampl,
                     hipStream_t st, PhaseTimer* tm);
 void launch_chunk128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
-// NP = 256 (wide256.hip): the whole chunk; QL, rotations and epilogue of
-// its eigensolver (tridiag.hip)
+// NP = 256 (wide256.hip): the whole chunk
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
-void launch_ql256(const ChunkArgs& A, hipStream_t st);
-void launch_tridiag256_tail(const ChunkArgs& A, hipStream_t st);
+void launch_pole256(const ChunkArgs& A, hipStream_t st);
 // Householder reductions on the lower triangle (wide256.hip): d, e, the
 // reflectors, and Q^T b and Q^T 1_N (ones = N; -1: the vector in slot 2) in
 // place of b and slot 2 of vec

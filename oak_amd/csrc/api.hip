@@ -416,10 +416,6 @@ void finish_call(oakg_ctx* c, int64_t nz, const int64_t* sel_ptr, const int32_t*
   const unsigned herr = (unsigned)h[0];
   if (herr & OAKG_DERR_RMSE) arg_fail(c, "observation error variance rmse^2 <= 0 or not finite");
   if (herr & OAKG_DERR_IDX) arg_fail(c, "index out of range in H or in the selection");
-  if (herr & OAKG_DERR_NOCONV) {
-    c->err = "the QL iteration did not finish a zone (no fallback above N = 128)";
-    throw Fail{OAKG_ECONV};
-  }
   if (herr & OAKG_DERR_NAN) {
     c->err = "NaN in the analysis amplitudes (rrsqrt.F90:145-149)";
     throw Fail{OAKG_ENAN};
@@ -467,22 +463,16 @@ void materialize_counts(oakg_ctx* c) {
 // run in order on the caller's stream (the timer's events are on that stream).
 // Returns whether the zones' Jacobi sweeps are in sweeps_all.
 bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_all) {
-  // QL rotation log: records of 16 B per zone, a multiple of 4 (the log is
-  // interleaved in groups of 4 records over the 64 zones of a QL wave)
-  // (about 1.1 N^2 records for typical zones; 2 N^2 + 8 N leaves room for slow ones)
-  const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
-  // the likelihood at N <= 64 keeps nothing per zone (nll.hip); else funcm.hip,
-  // or QL for N > 128 with either method
+  // the likelihood at N <= 64 keeps nothing per zone (nll.hip); else the
+  // functions of T (N > 128 with either method) or the Jacobi option
   const bool chol = base.mode == 2 && NP <= 64;
-  const bool func = c->eig_method == 1 && NP <= 128 && !chol;
-  const bool ql = NP == 256;
+  const bool func = (c->eig_method == 1 || NP == 256) && !chol;
   const int MP = chol ? 1 : NP;  // matrices MP x MP and vectors of MP entries per zone
   // zones with 1 <= p < dual_lt in observation space (dual.hip): N > 64, the
   // analysis modes (not the likelihood), not in a no-allocation call
   const int dual_lt = (NP == 128 && func && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
   constexpr int PD = 64;
   const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * MP * MP + 6 * MP) +
-                          (ql ? (size_t)cap * 16 + 4 : 0) +
                           (dual_lt ? sizeof(double) * ((size_t)2 * PD * PD + 4 * PD) : 0);
   const size_t budget = c->ws_budget;
   const int nslot = (!c->timing && !c->arena && nz >= 4096) ? c->tune_slots : 1;
@@ -490,10 +480,10 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   zc = std::min<int64_t>(zc, 1 << 20);
   if (nslot > 1) zc = std::min<int64_t>(zc, (nz + nslot - 1) / nslot);  // a chunk per slot
   zc = std::min<int64_t>(zc, nz);
-  zc = (zc + 63) & ~(int64_t)63;  // slots start on 64-zone groups of the rotation log
+  zc = (zc + 63) & ~(int64_t)63;  // whole groups of 64 zones
   if (c->arena) {
     // chunks of what is left of the scratch (7 buffers of up to 255 bytes of
-    // alignment), in whole 64-zone groups of the rotation log
+    // alignment), in whole groups of 64 zones
     const size_t left = c->arena->left();
     const int64_t fit = left > 8 * 256 ? (int64_t)((left - 8 * 256) / per_zone) : 0;
     zc = std::min<int64_t>(zc, fit & ~(int64_t)63);
@@ -510,17 +500,10 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   if (NP == 256) umat = (double*)wsget(c, Workspace::UMAT, sizeof(double) * (size_t)NP * NP * zs);
   if (!mat || !ymat || !vec || (NP == 256 && !umat)) check(c, hipErrorOutOfMemory, "workspace");
   double *dvec = nullptr, *evec = nullptr;
-  char* rlog = nullptr;
-  int32_t* tst = nullptr;
-  if (ql || func) {
+  if (func) {
     dvec = (double*)wsget(c, Workspace::DVEC, sizeof(double) * (size_t)NP * zs);
     evec = (double*)wsget(c, Workspace::EVEC, sizeof(double) * (size_t)NP * zs);
     if (!dvec || !evec) check(c, hipErrorOutOfMemory, "workspace");
-  }
-  if (ql) {
-    rlog = (char*)wsget(c, Workspace::RLOG, (size_t)16 * cap * zs);
-    tst = (int32_t*)wsget(c, Workspace::TQL_STATUS, sizeof(int32_t) * zs);
-    if (!rlog || !tst) check(c, hipErrorOutOfMemory, "workspace");
   }
   // zone order (not in a no-allocation call: its scratch is sized without it)
   const bool order = c->tune_order == 1 && !c->arena && nz > 1 && nz <= INT32_MAX;
@@ -571,8 +554,8 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   if (use_graph) {
     struct Key {
       ChunkArgs base;
-      int64_t nz, zc, cap;
-      int NP, nslot, ql, ql_zw, order, tri_split, dual_lt, persist;
+      int64_t nz, zc;
+      int NP, nslot, func, order, dual_lt, persist;
       const void* buf[16];
       hipStream_t stream;
     } kk;
@@ -580,16 +563,13 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     kk.base = base;
     kk.nz = nz;
     kk.zc = zc;
-    kk.cap = cap;
     kk.NP = NP;
     kk.nslot = nslot;
-    kk.ql = ql + 2 * func;
-    kk.ql_zw = c->tune_ql_zw;
+    kk.func = func;
     kk.order = order;
-    kk.tri_split = c->tune_tri_split;
     kk.dual_lt = dual_lt;
     kk.persist = persist ? 1 + persist_item : 0;
-    const void* bufs[16] = {mat,  ymat,   vec,    dvec,   evec,  rlog,  tst,   sweeps_all,
+    const void* bufs[16] = {mat,  ymat,   vec,    dvec,   evec,  sweeps_all,
                             zorder, zord_p, zord_d, mat_d, ymat_d, vec_d, wq,  umat};
     memcpy(kk.buf, bufs, sizeof bufs);
     kk.stream = c->stream;
@@ -605,7 +585,7 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
       ++c->graph_replays;
       check(c, hipEventRecord(c->ev_cap_out, c->cap_stream), "event");
       check(c, hipStreamWaitEvent(c->stream, c->ev_cap_out, 0), "stream wait");
-      return !(func || ql || chol);
+      return !(func || chol);
     }
     check(c, hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal), "capture");
   }
@@ -655,14 +635,9 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     A.vec = vec + zo * 4 * MP;
     A.umat = umat ? umat + zo * NP * NP : nullptr;
     A.sweeps = sweeps_all + z0;
-    A.eig_method = ql || func ? 1 : 0;
+    A.eig_method = func ? 1 : 0;
     A.dvec = dvec ? dvec + zo * NP : nullptr;
     A.evec = evec ? evec + zo * NP : nullptr;
-    A.rlog = ql ? (void*)(rlog + (size_t)16 * cap * zo) : nullptr;
-    A.rlog_cap = cap;
-    A.tql_status = ql ? tst + zo : nullptr;
-    A.ql_zw = c->tune_ql_zw;
-    A.tri_split = c->tune_tri_split;
     A.persist_wq = persist ? wq + (size_t)64 * sl : nullptr;
     A.persist_item = persist_item;
     A.persist_grid = persist_grid;
@@ -708,7 +683,7 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     check(c, hipEventRecord(c->ev_cap_out, c->cap_stream), "event");
     check(c, hipStreamWaitEvent(c->stream, c->ev_cap_out, 0), "stream wait");
   }
-  return !(func || ql || chol);
+  return !(func || chol);
 }
 
 template <typename F>
@@ -1015,8 +990,8 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     const double* dval = stage(c, Workspace::H_VAL, H->val, H->nnz, dev);
     const T* dHs = stage(c, Workspace::H_SHIFT, Hshift, m, dev);
     const double* dmc = stage(c, Workspace::MAXCORR, maxc_elem, n, dev);
-    // the mean of the state: the update of N <= 64 forms it from its own rows
-    const bool own_mean = NP <= 64;
+    // the mean of the state: the update forms it from its own rows but for N = 65..128
+    const bool own_mean = NP <= 64 || NP == 256;
     double* xbar = own_mean ? nullptr
                             : (double*)wsget(c, Workspace::XBAR, sizeof(double) * std::max<int64_t>(n, 1));
     double* HEc = (double*)wsget(c, Workspace::HEC, sizeof(double) * std::max<int64_t>(m, 1) * N);
@@ -1535,9 +1510,7 @@ size_t noalloc_fixed_bytes(int64_t m, int NP, int64_t nz) {
 
 // Bytes of the zone-chunk workspace per zone (as run_zones sizes it).
 size_t noalloc_zone_bytes(int NP) {
-  const int64_t cap = (((int64_t)2 * NP * NP + 8 * NP) + 3) & ~(int64_t)3;
-  return sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP) +
-         (NP == 256 ? (size_t)cap * 16 + 4 : 0);
+  return sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * NP * NP + 6 * NP);
 }
 
 // For the duration of a no-allocation call: the arena over the scratch, the

@@ -69,16 +69,12 @@ __device__ __forceinline__ void lds_fence() {
 // reductions: one pad entry per 8 rows (register tiles start every 8 rows).
 __host__ __device__ constexpr int tri_rx(int r) { return r + (r >> 3); }
 
-// ---------------------------------------------------------------------------
-// Rotation log.  The zones of one 64-zone group share cap * 64 records; record
-// k of the zone in lane l sits at (k / 4) * 256 + 4 l + (k % 4), so that one
-// store instruction of the QL wave stays within a few KB.  A chain (one QL
-// sweep on rows l..m) starts with a header {l + 65536 m, count} followed by
-// `count` records {c, s} for the rotation indices i = m-1, m-2, ...
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ size_t rlog_off(int zl, int64_t cap) {
-  return (size_t)(zl >> 6) * (size_t)cap * 64 + (size_t)(zl & 63) * 4;
+// Entry r of reflector k (zero up to row k, tau_k in entry k) as the N = 256
+// reduction leaves them in the zone's block V: rows 0..127 in full, then those
+// of the trailing 128 rows in a 128 x 128 block from row 192 (their entries
+// below row 128 do not exist: some entry of the block stands in).
+__device__ __forceinline__ const double* reflector256(const double* V, int k, int r) {
+  return k < 128 ? V + k * 256 + r : V + 192 * 256 + (k - 128) * 128 + (r < 128 ? 0 : r - 128);
 }
-__device__ __forceinline__ size_t rlog_rec(int64_t k) { return (size_t)(k >> 2) * 256 + (size_t)(k & 3); }
 
 }  // namespace oakg

@@ -1264,6 +1264,266 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
   }
 }
 
+// ===========================================================================
+// N > 128: a zone's F is 512 KB, so the steps of k_func are kernels of their
+// own (the others are in wide256.hip).
+// ===========================================================================
+
+// Pivots and solves as in k_func (wave 0), T_b of the reflector blocks (waves
+// 1 to 3), then a = Q x and v = Q y / |Q y|.  For the products that form F, per
+// row (in elimination order) and pole: tau and G_ii (the tiles on the
+// diagonal), and alpha and beta relative to the tile edges; `poles` has these
+// four arrays, then the weights and G_hh.  The recurrence
+// leaves 1/gamma and z/gamma of the way in where tau and G go on the way out.
+template <int NP>
+struct PoleLds {
+  double d[NP], e[NP], c[2][NP];  // c: Q^T b, Q^T 1, then x, y (elimination order)
+  double v[2][NP];                // x, y; then a, v
+  double tp[NP / 16 * 136];       // T_b, packed
+  double g[2][16], t[2][16], red[4];
+};
+
+__global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                    const int64_t* __restrict__ sel_ptr,
+                                                    const double* __restrict__ qmat,
+                                                    const double* __restrict__ dvec,
+                                                    const double* __restrict__ evec, double* poles,
+                                                    double* __restrict__ tblk,
+                                                    double* __restrict__ vec, double* __restrict__ ampl,
+                                                    unsigned* __restrict__ err) {
+  constexpr int NP = 256, H = NP / 2;
+  __shared__ PoleLds<NP> S;
+  const int zl = blockIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  if (z < 0) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lr = lane >> 4, lc = lane & 15;
+  double* Vz = vec + (size_t)zl * 4 * NP;
+  if (sel_ptr[z + 1] == sel_ptr[z]) {  // no observations: a = 0
+    Vz[NP + tid] = 0.0;
+    return;
+  }
+  const double* V = qmat + (size_t)zl * NP * NP;
+  const int nblk = N > 2 ? (N + 13) >> 4 : 0;
+  {
+    const int k = step_row<NP>(tid);
+    S.d[k] = dvec[(size_t)zl * NP + tid];
+    S.e[k] = evec[(size_t)zl * NP + (tid < H ? tid : tid - 1)];
+    S.c[0][k] = Vz[tid];
+    S.c[1][k] = Vz[2 * NP + tid];
+  }
+  lds_barrier();
+  if (wave == 0) {
+    double nt = 0.0;  // Gershgorin bound of T
+#pragma unroll
+    for (int h = 0; h < NP / 64; ++h) {
+      const int k = lane + 64 * h;
+      nt = fmax(nt, fabs(S.d[k]) + fabs(S.e[k]) + (k % H ? fabs(S.e[k - 1]) : 0.0));
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
+    const int ex = (__double2hiint(nt) >> 20) - 1022;
+    int bk = ((ex + 1) >> 1) - 1;
+    bk = __builtin_amdgcn_readfirstlane(bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk));
+    const int j = lane & 31;
+    const bool bot = lane >= 32, up = (lane & 16) != 0;
+    const double s = g_poles[bk][0][j], sp1 = 1.0 + s, wj = g_poles[bk][1][j];
+    const int h0 = bot ? H : 0;
+    const double* dd = S.d + h0;
+    const double* ee = S.e + h0;
+    double* cc = S.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
+    double* c1 = S.c[1] + h0;
+    double* P = poles + (size_t)zl * NP * NP;
+    double* pa = P + h0 * 32 + j;  // tau (first 1/gamma); + NP 32: G_ii (first z/gamma)
+    double* pg = pa + NP * 32;
+    double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
+#pragma unroll 1
+    for (int t = 0; t < H; t += 8) {
+      double dv[8], ev[8], cv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        dv[i] = dd[t + i];
+        ev[i] = ee[t + i];
+        cv[i] = cc[t + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
+        z1 = fma(tau, z1, cv[i]);
+        pa[(t + i) * 32] = q;
+        pg[(t + i) * 32] = z1 * q;
+        tau = -ev[i] * q;
+        e2 = ev[i] * ev[i];
+      }
+    }
+    double G, x;
+    {
+      const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+      const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+      const double eh = S.e[H - 1];
+      G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+      x = G * fma(-eh * qb, zb, zh);
+      if (!bot) {
+        P[4 * NP * 32 + j] = wj;
+        P[4 * NP * 32 + 32 + j] = G;
+      }
+    }
+#pragma unroll 1
+    for (int t = H - 16; t >= 0; t -= 16) {
+      double r[16], g[16];  // 1/gamma and z/gamma, then tau and G_ii
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        r[i] = pa[(t + i) * 32];
+        g[i] = pg[(t + i) * 32];
+      }
+#pragma unroll
+      for (int h = 1; h >= 0; --h) {
+        double tv[8];
+#pragma unroll
+        for (int i = 7; i >= 0; --i) {
+          const int k = 8 * h + i;
+          double rr = -ee[t + k] * r[k];
+          const double gn = fma(rr * rr, G, r[k]), xn = fma(rr, x, g[k]);
+          const bool mid = k == 15 && !bot && t == H - 16;  // row h itself
+          G = mid ? G : gn;
+          x = mid ? x : xn;
+          rr = mid ? 1.0 : rr;
+          r[k] = rr;
+          g[k] = G;
+          tv[i] = wj * fma(-s, x, c1[t + k]);
+          if (j == 31) cc[t + k] = x;
+        }
+        // sums over the poles, as in k_func
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
+          tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
+        }
+        if (lc == 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) c1[t + 8 * h + (up ? 4 : 0) + i] = tv[i];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        pa[(t + i) * 32] = r[i];
+        pg[(t + i) * 32] = g[i];
+      }
+      // towards the middle edge of the tile: alpha, beta
+      double pi = 1.0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        g[i] *= pi;
+        pi *= r[i];
+      }
+#pragma unroll
+      for (int i = 14; i >= 0; --i) r[i] *= r[i + 1];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        pa[2 * NP * 32 + (t + i) * 32] = r[i];
+        pg[2 * NP * 32 + (t + i) * 32] = g[i];
+      }
+    }
+  } else {
+    for (int b = wave - 1; b < nblk; b += 3) {
+      const int k = 16 * b + lc;
+      // V^T V packed into the block's place, then column by column replaced
+      d4 g = {0.0, 0.0, 0.0, 0.0};
+      for (int k0 = 4 * b; k0 < NP / 4; k0 += 4) {
+        double xv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xv[u] = *reflector256(V, k, 4 * (k0 + u) + lr);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double xm = (k < N - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
+          g = mfma_f64(xm, xm, g);
+        }
+      }
+      const double tk = *reflector256(V, k, k);
+      const double tau = k < N - 2 ? tk : 0.0;
+      double* gs = S.tp + b * 136;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (lr + 4 * r <= lc) gs[lc * (lc + 1) / 2 + lr + 4 * r] = g[r];
+      lds_fence();
+      double tr[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        double sm = 0.0;
+#pragma unroll
+        for (int q = 0; q < j; ++q) sm = fma(tr[q], gs[j * (j + 1) / 2 + q], sm);
+        const double tj = readlane_d(tau, j);
+        tr[j] = lane < j ? -tj * sm : (lane == j ? tj : 0.0);
+        lds_fence();
+        if (lane <= j) gs[j * (j + 1) / 2 + lane] = tr[j];
+      }
+      lds_fence();
+    }
+  }
+  lds_barrier();
+  {
+    const int k = step_row<NP>(tid);
+    S.v[0][tid] = S.c[0][k];
+    S.v[1][tid] = S.c[1][k];
+  }
+  for (int e = tid; e < nblk * 136; e += 256) tblk[(size_t)zl * NP * NP + e] = S.tp[e];
+  // [a, v] = Q [x, y]: thread (pj, pr) has rows pr + 16 e of reflector pj of a block
+  const int pj = tid >> 4, pr = tid & 15;
+  double pf[16];
+  auto load_block = [&](int b) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) pf[e] = *reflector256(V, 16 * b + pj, pr + 16 * e);
+  };
+  if (nblk > 0) load_block(nblk - 1);
+  lds_barrier();
+#pragma unroll 1
+  for (int b = nblk - 1; b >= 0; --b) {
+    const int k = 16 * b + pj;
+    double g0 = 0.0, g1 = 0.0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      pf[e] = (k < N - 2 && pr + 16 * e > k) ? pf[e] : 0.0;
+      g0 = fma(pf[e], S.v[0][pr + 16 * e], g0);
+      g1 = fma(pf[e], S.v[1][pr + 16 * e], g1);
+    }
+    g0 = row_sum16(g0);
+    g1 = row_sum16(g1);
+    if (pr == 0) {
+      S.g[0][pj] = g0;
+      S.g[1][pj] = g1;
+    }
+    lds_barrier();
+    // t = T_b g (row pj of T_b, column pr)
+    const double tv = pj <= pr ? S.tp[b * 136 + pr * (pr + 1) / 2 + pj] : 0.0;
+    const double t0 = row_sum16(tv * S.g[0][pr]), t1 = row_sum16(tv * S.g[1][pr]);
+    if (pr == 0) {
+      S.t[0][pj] = t0;
+      S.t[1][pj] = t1;
+    }
+    lds_barrier();
+    // thread r: row r of [x, y] less V t
+    double s0 = S.v[0][tid], s1 = S.v[1][tid];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const double vv = 16 * b + c < N - 2 && tid > 16 * b + c ? *reflector256(V, 16 * b + c, tid) : 0.0;
+      s0 = fma(-vv, S.t[0][c], s0);
+      s1 = fma(-vv, S.t[1][c], s1);
+    }
+    S.v[0][tid] = s0;
+    S.v[1][tid] = s1;
+    if (b > 0) load_block(b - 1);
+    lds_barrier();
+  }
+  const double ar = S.v[0][tid], vr = S.v[1][tid];
+  const double nv = wave_sum_fast(vr * vr);
+  if (lane == 0) S.red[wave] = nv;
+  lds_barrier();
+  Vz[NP + tid] = ar;
+  Vz[2 * NP + tid] = vr / sqrt((S.red[0] + S.red[1]) + (S.red[2] + S.red[3]));
+  if (ampl && tid < N) ampl[(size_t)z * N + tid] = ar;
+  if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
+}
+
 // R = Y Y^T (and the likelihood's log det M, sum (1 - 1/mu) and b^T a) from
 // the Y = U diag(mu^-1/4) and mu of the Jacobi option, so that one form
 // reaches the transform.
@@ -1350,6 +1610,13 @@ void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st) {
   else
     OAK_SMALL(32);
 #undef OAK_SMALL
+}
+
+// N > 128: the pole arrays to umat, T_b to the rows of ymat that the reduction's
+// trailing block leaves (128 .. 191), a and v.
+void launch_pole256(const ChunkArgs& A, hipStream_t st) {
+  hipLaunchKernelGGL(k_pole256, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,
+                     A.dvec, A.evec, A.umat, A.ymat + 128 * 256, A.vec, A.ampl, A.err);
 }
 
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {

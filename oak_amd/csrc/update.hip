@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256, NP == 32 ? 3 : 4) void k_update_small(int64_t 
 // holds column s of T - and its four waves take the strips in turn.  The k
 // index of the MFMA steps is permuted within pairs (lane group kk covers k =
 // 8 p + 2 kk and the next), so that one LDS read of two entries serves two
-//  Bound by the reads and writes of the ensemble: 64 800 zones of 121 rows,
+// steps.  Bound by the reads and writes of the ensemble: 64 800 zones of 121 rows,
 // N = 64, 8.0 GB and 2.1 GB of M^-1/2, 2.67 ms.  With T from a kernel of its own,
 // a spilling product that waited for each load and the mean in a pass before,
 // these took 1.6, 10.5 and 0.7 ms.

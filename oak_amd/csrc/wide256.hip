@@ -12,24 +12,19 @@
 //                  register tiles over 512 threads, one workgroup per zone:
 //                  496 tiles hold columns 8..255, and columns 0..7 sit in
 //                  LDS for the seven steps that change them; steps 128..253
-//                  on the trailing 128 x 128 block by k_tridiag<128>.
-//   k_formq256     Q = H_0 ... H_253 in blocked compact-WY form on MFMA (the
-//                  scheme of k_formq128 on a 256 x 64 slice), four workgroups
-//                  per zone, one 64-column block of Q each.
-//   tridiag.hip    k_tql (QL on (d, e), rotations logged), k_tql_apply256
-//                  (the rotations on the rows of Q in registers, two threads
-//                  a row) and k_eigvec_epi: eigenvalues, U, a, v and Y.
-//   k_tmat256      T = (Y Y^T) Omega on MFMA, four workgroups per zone, one
-//                  64-row block of T each.
+//                  by k_tridiag_lower<128> and <64>.
+//   funcm.hip      k_pole256: the rational approximation's solves, a and v.
+//   k_qapply256    Q F, then Q (Q F)^T = M^-1/2 and Omega, the reflectors in
+//                  compact-WY blocks on MFMA, four workgroups per zone, one
+//                  64-column block each.
 //   k_update256    out = S [T | a] for the zone's rows, eight workgroups per
 //                  zone (one 32-column block of T each) on one XCD.
 // The operations are those of the N <= 128 path (rrsqrt.F90:100-190 and the
 // post-processing of assimilation.F90:3299-3363); only the split of the work
-// and the order of the partial sums differ.  k_tridiag_lower<128> (the same
-// lower-triangle reduction at NP = 128, steps 0..63) also serves the
-// N = 128 path as its reduction options 3 and 4 (launch_tridiag_lower128),
-// k_tridiag_lower<64, true> the trailing block of option 4 and the whole
-// reduction at NP = 64 (with k_formq64 for Q).
+// and the order of the partial sums differ.  k_tridiag_lower<128> and <64> also
+// serve N = 65..128, k_tridiag_lower<64> alone N = 33..64.
+#include <algorithm>
+
 #include "analysis.hpp"
 #include "common.hpp"
 #include "eigen_common.hpp"
@@ -303,10 +298,9 @@ __global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* _
 // i+1 as it stands before the update is published by its tile column (or
 // the LDS block), and every wave forms its updated value itself.  Two
 // barriers per step.  Steps 0..127 run here; the trailing 128 x 128 block
-// then goes to the NP = 128 kernels (fewer registers, two to four zones per
-// CU through the late, latency-bound steps; launch_tridiag256_tail).
-// Output as k_tridiag: reflector i in row i of qmat (tau_i in entry i), T
-// reversed (d'_k = d_{255-k}).
+// then goes to the NP = 128 and 64 kernels (fewer registers, four and eight
+// zones per CU through the late, latency-bound steps).
+// Output: reflector i in row i of qmat (tau_i in entry i), d and e.
 // ---------------------------------------------------------------------------
 template <int NP>
 struct TriLowerLds {
@@ -621,10 +615,8 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   }
   // the trailing block [H, NP)^2 after step H - 1 (the tiles of tile rows and
   // columns >= H / 8; both triangles) to the rows from H of the zone's
-  // reflector block: NP = 256, as a dense H x H matrix that the NP = 128
-  // kernels reduce (launch_tridiag256_tail); NP = 128, as row r, column
-  // c - H of rows H.. (the layout k_tridiag<128, 1> leaves for
-  // k_tridiag<128, 2>)
+  // reflector block: NP = 256, as a dense H x H matrix; NP = 128, as row r,
+  // column c - H of rows H..
   if (has_u) {
 #pragma unroll
     for (int q = 0; q < NV; ++q)
@@ -661,7 +653,6 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
         if (tr != tc) blk[(size_t)(c0 - H + jj) * LDO + (r0 - H + ii)] = a[ii][jj];
       }
   }
-  if (NP == 256 && t == 0) ev[-A.dstep] = 0.0;  // e_255 of the reversed order
 }
 
 // NP = 128: steps 0..63 on the lower-triangle tiles (two waves, four zones
@@ -685,141 +676,6 @@ void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st) {
   hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
 }
 
-// ---------------------------------------------------------------------------
-// Q = H_0 H_1 ... H_253 from the reflectors in the rows of qmat (row k: v_k,
-// tau_k in entry k), accumulated backwards in blocks of 16 in compact WY
-// form (LAPACK dlarft / dlarfb): H_k0 ... H_k0+15 = I - Vb Tb Vb^T and
-// Q <- Q - Vb (Tb (Vb^T Q)), on v_mfma_f64_16x16x4f64.  Workgroup y of a
-// zone forms columns 64 y .. 64 y + 63 of Q (they depend on no other
-// columns): wave w holds tile column J = 4 y + w in its accumulators, 16
-// tiles of 16 x 16; block b touches tile rows and columns >= b only.  Q goes
-// to umat with its columns reversed, as the QL kernels expect.
-// ---------------------------------------------------------------------------
-struct FormQ256Lds {
-  static constexpr int LV = 17;  // padded row of Vb and Tb
-  double vb[2][256 * LV];        // Vb[r][j]: row r of reflector k0 + j
-  double tb[2][16 * LV];         // Tb
-  double g[16 * LV];             // Vb^T Vb
-  double tau[2][16];
-};
-
-__global__ __launch_bounds__(256, 2) void k_formq256(int64_t z0, const int32_t* __restrict__ zorder,
-                                                  const int64_t* __restrict__ sel_ptr,
-                                                  const double* __restrict__ qmat,
-                                                  double* __restrict__ umat) {
-  constexpr int NP = NPW, NB = 16, LV = FormQ256Lds::LV;
-  __shared__ FormQ256Lds S;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;
-  if (sel_ptr[z + 1] == sel_ptr[z]) return;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int lr = lane >> 4, lc = lane & 15;
-  const double* V = qmat + (size_t)zl * NP * NP;
-  double* U = umat + (size_t)zl * NP * NP;
-  const int J = 4 * (int)blockIdx.y + wave;  // the wave's tile column
-  d4 q[16];
-#pragma unroll
-  for (int I = 0; I < 16; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) q[I][r] = (I == J && lr + 4 * r == lc) ? 1.0 : 0.0;
-  // thread t moves reflector pj = t / 16 of a block, rows pr + 16 e (e < 16)
-  const int pj = t >> 4, pr = t & 15;
-  double pf[16];
-  // reflectors 0..127 are rows of the zone's block; 128..253 (from the NP =
-  // 128 kernels) are rows 0..125 of the 128 x 128 block at row 192, for
-  // rows 128..255 of Q
-  const double* V2 = V + (size_t)192 * NP;
-  auto load_block = [&](int b) {
-    const int k = 16 * b + pj;
-    if (k < NP / 2) {
-      const double* src = V + (size_t)k * NP + pr;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) pf[e] = src[16 * e];
-    } else if (k < NP - 2) {
-      const double* src = V2 + (size_t)(k - NP / 2) * (NP / 2) + pr;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) pf[e] = e < 8 ? 0.0 : src[16 * (e - 8)];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) pf[e] = 0.0;
-    }
-  };
-  load_block(NB - 1);
-  for (int b = NB - 1; b >= 0; --b) {
-    const int buf = b & 1;
-    double* vb = S.vb[buf];
-    double* tb = S.tb[buf];
-    {
-      const int k = 16 * b + pj;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = pr + 16 * e;
-        vb[r * LV + pj] = r == k ? 0.0 : pf[e];
-        if (r == k) S.tau[buf][pj] = pf[e];
-      }
-    }
-    if (b > 0) load_block(b - 1);
-    lds_barrier();
-    // wave 0: G = Vb^T Vb (rows >= 16 b), then Tb column by column:
-    // Tb[j][j] = tau_j, Tb[0:j, j] = -tau_j Tb[0:j, 0:j] G[0:j, j]
-    if (wave == 0) {
-      d4 g = {0.0, 0.0, 0.0, 0.0};
-      for (int kk = 4 * b; kk < 64; ++kk) {
-        const double xv = vb[(4 * kk + lr) * LV + lc];
-        g = mfma_f64(xv, xv, g);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S.g[(lr + 4 * r) * LV + lc] = g[r];
-      __builtin_amdgcn_wave_barrier();
-      if (lane < 16) {
-        double trr[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          asm volatile("" ::: "memory");  // G column by column, not all loads at once
-          double s = 0.0;
-#pragma unroll
-          for (int k = 0; k < j; ++k) s = fma(trr[k], S.g[k * LV + j], s);
-          const double tj = S.tau[buf][j];
-          trr[j] = lane < j ? -tj * s : (lane == j ? tj : 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) tb[lane * LV + j] = trr[j];
-      }
-    }
-    // W = Vb^T Q[:, J]
-    d4 w = {0.0, 0.0, 0.0, 0.0};
-    if (J >= b) {
-#pragma unroll
-      for (int I = 0; I < 16; ++I)
-        if (I >= b) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk)
-            w = mfma_f64(vb[(16 * I + 4 * kk + lr) * LV + lc], q[I][kk], w);
-        }
-    }
-    lds_barrier();  // Tb
-    // W' = -Tb W;  Q[I][J] += Vb[I rows] W'
-    if (J >= b) {
-      d4 wp = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) wp = mfma_f64(-tb[lc * LV + 4 * kk + lr], w[kk], wp);
-#pragma unroll
-      for (int I = 0; I < 16; ++I)
-        if (I >= b) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk)
-            q[I] = mfma_f64(vb[(16 * I + lc) * LV + 4 * kk + lr], wp[kk], q[I]);
-        }
-    }
-  }
-#pragma unroll
-  for (int I = 0; I < 16; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      U[(size_t)(16 * I + lr + 4 * r) * NP + (NP - 1 - (16 * J + lc))] = q[I][r];
-}
-
 // NP = 64 (33 <= N <= 64, and the observation-space zones of N = 128: ones =
 // -1): the whole reduction on one wave per zone, of the steps that the order
 // (N, or the zone's observations) has.
@@ -830,140 +686,271 @@ void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// T = (Y Y^T) Omega (the operator of k_tmat: Omega = RotateVector(w, v) as
-// the identity plus a rank-structured term), rows 64 y .. 64 y + 63 in
-// workgroup y: wave w forms tile row I = 4 y + w of Y Y^T (16 tiles in its
-// accumulators, Y staged through LDS 16 columns at a time, the next block
-// loaded while the current one is multiplied), then its rows' products with
-// the vectors of Omega, then T.  Zones without observations
-// get T = I.
+// T = R Omega, R = Q F Q^T, F = T^-1/2, in two passes of the same kernel, each
+// with the reflectors applied from the left in blocks of 16 in compact WY form
+// (LAPACK dlarft / dlarfb; T_b from k_pole256):
+//   STEP 1: F from the pole arrays, Y = Q F to mat
+//   STEP 2: Y^T, R = Q Y^T, and Omega applied to its columns: X[s][c] = T[c][s]
+// Workgroup y of a zone has columns 64 y .. 64 y + 63 (they depend on no
+// other columns): wave w tile column J = 4 y + w, 16 tiles of 16 x 16 in its
+// accumulators; tiles and blocks of the padding are left out.  The reflector
+// block passes through LDS, double-buffered, the next one loaded while the
+// current one is applied; one barrier per block.  Two workgroups a CU.
+// Bound by the MFMAs, 2 x 17 400 of 16 x 16 x 4 per zone: 16 200 zones take 15.7
+// and 15.6 ms, the MFMAs alone 7.5 each.  With k_pole256 (4.4 ms) they replace Q
+// formed explicitly, QL iterations, the rotations on Q, an epilogue and Y Y^T,
+// which took 107 ms.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 2) void k_tmat256(int64_t z0, const int32_t* __restrict__ zorder,
-                                                 int N, const int64_t* __restrict__ sel_ptr,
-                                                 const double* __restrict__ umat,
-                                                 double* __restrict__ mat,
-                                                 const double* __restrict__ vec) {
-  constexpr int NP = NPW, KC = 16, LY = KC + 1;
-  __shared__ double Yc[2][NP * LY];
+struct QApplyLds {
+  static constexpr int LV = 17;  // padded row of Vb
+  double vb[2][NPW * LV];        // Vb[r][j]: row r of reflector 16 b + j
+  double tb[2][16 * LV];         // T_b
+  double v[NPW];
+};
+
+template <int STEP>
+__global__ __launch_bounds__(256, 2) void k_qapply256(int64_t z0, const int32_t* __restrict__ zorder,
+                                                      int N, const int64_t* __restrict__ sel_ptr,
+                                                      const double* __restrict__ qmat,
+                                                      const double* __restrict__ tblk,
+                                                      double* __restrict__ mat,
+                                                      double* __restrict__ umat,
+                                                      const double* __restrict__ vec) {
+  constexpr int NP = NPW, NB = 16, LV = QApplyLds::LV;
+  __shared__ QApplyLds S;
   const int zl = blockIdx.x;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
-  double* T = mat + (size_t)zl * NP * NP;
-  const int rb = blockIdx.y;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const int lr = lane >> 4, lc = lane & 15;
+  const int J = 4 * (int)blockIdx.y + wave;  // the wave's tile column
+  double* X = umat + (size_t)zl * NP * NP;
   if (sel_ptr[z + 1] == sel_ptr[z]) {
-    for (int e = threadIdx.x; e < 64 * NP; e += 256) {
-      const int r = 64 * rb + e / NP, c = e % NP;
-      T[(size_t)r * NP + c] = r == c ? 1.0 : 0.0;
-    }
+    if (STEP == 2)
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          X[(size_t)(16 * I + lr + 4 * r) * NP + 16 * J + lc] = I == J && lr + 4 * r == lc ? 1.0 : 0.0;
     return;
   }
-  const double* Yz = umat + (size_t)zl * NP * NP;
-  const double* v = vec + (size_t)zl * 4 * NP + 2 * NP;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int li = lane & 15, kk = lane >> 4;
-  const int I = 4 * rb + wave;
-  d4 acc[16];
+  const double* V = qmat + (size_t)zl * NP * NP;
+  double* Y = mat + (size_t)zl * NP * NP;
+  const int nt = (N + 15) >> 4, nblk = N > 2 ? (N + 13) >> 4 : 0;
+  // the lower half's columns see the tile rows mirrored (k_func): f[I] is
+  // tile row I or NB - 1 - I
+  const bool low = STEP == 1 && J >= NB / 2;
+  auto row_of = [&](int I) { return low ? NB - 1 - I : I; };
+  d4 f[NB];
 #pragma unroll
-  for (int J = 0; J < 16; ++J) acc[J] = d4{0, 0, 0, 0};
-  // columns k0 .. k0 + 15 of Y in LDS buffer (k0 / 16) % 2; thread e holds
-  // 16 values of the next block (rows e / 16 + 16 u, column e % 16) in
-  // registers while the current block is multiplied
-  double yn[16];
-  auto load_y = [&](int k0) {
+  for (int I = 0; I < NB; ++I) f[I] = d4{0.0, 0.0, 0.0, 0.0};
+  if (J < nt) {
+    if constexpr (STEP == 1) {
+      const double* P = umat + (size_t)zl * NP * NP;
+      const double* wp = P + 4 * NP * 32;
+      const double* al = P + 2 * NP * 32;
+      const double* be = P + 3 * NP * 32;
+      const int Js = low ? NB - 1 - J : J;
+      auto tile_of = [&](int r) { return r < NB / 2 ? r : NB / 2 + NB - 1 - r; };
+      auto load4 = [&](const double* a, int row, int h, double* o) {
+        const double2* p = reinterpret_cast<const double2*>(a + (size_t)row * 32 + 8 * lr + 4 * h);
+        const double2 x0 = p[0], x1 = p[1];
+        o[0] = x0.x;
+        o[1] = x0.y;
+        o[2] = x1.x;
+        o[3] = x1.y;
+      };
+      const int crow = 16 * tile_of(J) + (low ? 15 - lc : lc);
+      double w[8];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) yn[u] = Yz[(size_t)(threadIdx.x / KC + 16 * u) * NP + k0 + threadIdx.x % KC];
-  };
-  auto store_y = [&](int b) {
+      for (int q = 0; q < 8; ++q) w[q] = wp[8 * lr + q];
+      // the tile on the diagonal: outwards from each column's diagonal entry
+      // for the lane's eight poles, then the transpose (as in k_func)
+      d4 fd;
+      {
+        double g[8];
+        load4(P + NP * 32, crow, 0, g);
+        load4(P + NP * 32, crow, 1, g + 4);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) Yc[b][(threadIdx.x / KC + 16 * u) * LY + threadIdx.x % KC] = yn[u];
-  };
-  load_y(0);
-  store_y(0);
-  __syncthreads();
-  for (int k0 = 0; k0 < NP; k0 += KC) {
-    const int b = (k0 / KC) & 1;
-    if (k0 + KC < NP) load_y(k0 + KC);
-    asm volatile("" ::: "memory");  // compiler barrier: keeps the loads above here
-    const double* Yb = Yc[b];
+        for (int q = 0; q < 8; ++q) g[q] *= w[q];
+        const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
+        d4 us = {0.0, 0.0, 0.0, 0.0}, ut;
 #pragma unroll
-    for (int k4 = 0; k4 < KC; k4 += 4) {
-      const double av = Yb[(16 * I + li) * LY + k4 + kk];
+        for (int i = 15; i >= 0; --i) {
+          if (i % 4 == 3) asm volatile("" ::: "memory");
+          double r[8];
+          load4(P, 16 * tile_of(J) + i, 0, r);
+          load4(P, 16 * tile_of(J) + i, 1, r + 4);
 #pragma unroll
-      for (int J = 0; J < 16; ++J) acc[J] = mfma_f64(av, Yb[(16 * J + li) * LY + k4 + kk], acc[J]);
-    }
-    if (k0 + KC < NP) store_y(b ^ 1);
-    __syncthreads();
-  }
-  // register q of lane l: row 16 I + l/16 + 4 q, column 16 J + l%16
-  const double wN = 1.0 / sqrt((double)N);
-  const double vN = v[N - 1];
-  const double sgv = vN >= 0 ? 1.0 : -1.0;
-  const double alv = -1.0 / (fabs(vN) + 1.0);
-  const double alw = -1.0 / (wN + 1.0);
-  double vw = 0;  // v~ . w~
-  for (int s = 0; s < N - 1; ++s) vw = fma(v[s], wN, vw);
-  double vl[16];
+          for (int q = 0; q < 8; ++q) g[q] *= i < lcs ? r[q] : 1.0;
+          const double sm = sum_xor32(
+              sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+          us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+        }
 #pragma unroll
-  for (int J = 0; J < 16; ++J) {
-    const int c = 16 * J + li;
-    vl[J] = c < N ? v[c] : 0.0;
-  }
+        for (int r = 0; r < 4; ++r) {
+          ut[r] = low ? us[3 - r] : us[r];
+          fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+        }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    // u0 = T0[r][N-1], u1 = T0 v, u2 = T0 w~, u3 = T0 z_v
-    double u0 = 0.0, u1 = 0.0, u2 = 0.0, u3 = 0.0;
-#pragma unroll
-    for (int J = 0; J < 16; ++J) {
-      const int c = 16 * J + li;
-      const double tt = acc[J][q];
-      u0 += c == N - 1 ? tt : 0.0;
-      u1 = fma(tt, vl[J], u1);
-      u2 = fma(tt, c < N - 1 ? wN : 0.0, u2);
-      u3 = fma(tt, vl[J] + (c == N - 1 ? sgv : 0.0), u3);
-    }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      u0 += shfl_xor_d(u0, o);
-      u1 += shfl_xor_d(u1, o);
-      u2 += shfl_xor_d(u2, o);
-      u3 += shfl_xor_d(u3, o);
-    }
-    const int r = 16 * I + kk + 4 * q;
-#pragma unroll
-    for (int J = 0; J < 16; ++J) {
-      const int s = 16 * J + li;
-      double tt = acc[J][q];
-      if (s < N) {
-        const double ws = wN;
-        const double zw = wN + (s == N - 1 ? 1.0 : 0.0);
-        const double vt = (s < N - 1) ? vl[J] : 0.0;
-        if (s == N - 1) tt -= u0;
-        tt += u1 * ws + alw * u2 * zw + alv * u3 * vt + alv * alw * vw * u3 * zw;
+        for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
       }
-      T[(size_t)r * NP + s] = tt;
+      double B[8];
+      auto column = [&](const double* a) {
+        load4(a, crow, 0, B);
+        load4(a, crow, 1, B + 4);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) B[q] *= w[q];
+      };
+      auto tile = [&](const double* a, int I) {
+        const int rI = row_of(I), t16 = 16 * tile_of(rI);
+        d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          double av[4], edge[4];
+          load4(a, t16 + (rI < NB / 2 ? lc : 15 - lc), h, av);
+          load4(al, t16, h, edge);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            acc = mfma_f64(av[q], B[4 * h + q], acc);
+            B[4 * h + q] *= edge[q];
+          }
+        }
+        return acc;
+      };
+      column(be);
+#pragma unroll
+      for (int I = NB / 2 - 2; I >= 0; --I)  // outside
+        if (I < Js && row_of(I) < nt) f[I] = tile(al, I);
+      column(al);
+#pragma unroll
+      for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
+        if (I == NB / 2) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) B[q] *= wp[32 + 8 * lr + q];
+        }
+        if (I > Js && row_of(I) < nt) f[I] = tile(I < NB / 2 ? be : al, I);
+      }
+#pragma unroll
+      for (int I = 0; I < NB / 2; ++I)
+        if (I == Js) f[I] = fd;
+    } else {
+      // Y^T: tile (J, I) of Y, transposed by a product with the identity (exact)
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+        if (I < nt) {
+          d4 y;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) y[r] = Y[(size_t)(16 * J + lr + 4 * r) * NP + 16 * I + lc];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) f[I] = mfma_f64(y[r], 4 * r + lr == lc ? 1.0 : 0.0, f[I]);
+        }
     }
   }
+  if (STEP == 2) S.v[t] = t < N ? vec[(size_t)zl * 4 * NP + 2 * NP + t] : 0.0;
+  // thread t moves reflector pj of a block, rows pr + 16 e, and entry t of T_b
+  const int pj = t >> 4, pr = t & 15;
+  double pf[16], pt = 0.0;
+  auto load_block = [&](int b) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) pf[e] = *reflector256(V, 16 * b + pj, pr + 16 * e);
+    pt = tblk[(size_t)zl * NP * NP + b * 136 + (pj <= pr ? pr * (pr + 1) / 2 + pj : 0)];
+  };
+  if (nblk > 0) load_block(nblk - 1);
+#pragma unroll 1
+  for (int b = nblk - 1; b >= 0; --b) {
+    double* vb = S.vb[b & 1];
+    double* tb = S.tb[b & 1];
+    const int k = 16 * b + pj;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int r = pr + 16 * e;
+      vb[r * LV + pj] = (k < N - 2 && r > k) ? pf[e] : 0.0;
+    }
+    tb[pj * LV + pr] = pj <= pr ? -pt : 0.0;
+    if (b > 0) load_block(b - 1);
+    lds_barrier();
+    if (J >= nt) continue;
+    d4 w = {0.0, 0.0, 0.0, 0.0}, wp = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+      const int rI = row_of(I);
+      if (rI >= b && rI < nt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w = mfma_f64(vb[(16 * rI + 4 * q + lr) * LV + lc], f[I][q], w);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) wp = mfma_f64(tb[lc * LV + 4 * q + lr], w[q], wp);
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+      const int rI = row_of(I);
+      if (rI >= b && rI < nt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) f[I] = mfma_f64(vb[(16 * rI + lc) * LV + 4 * q + lr], wp[q], f[I]);
+    }
+  }
+  if (STEP == 1) {
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Y[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = f[I][r];
+    return;
+  }
+  // X = (R Omega)^T from the columns of the symmetric R (k_tmat's formula):
+  // column c = 16 J + lc, rows s = 16 I + lr + 4 r
+  lds_barrier();
+  const double wN = 1.0 / sqrt((double)N), vN = S.v[N - 1], sgv = vN >= 0 ? 1.0 : -1.0;
+  const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0);
+  double vw = 0.0, u1 = 0.0, u2 = 0.0, u0 = 0.0;
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int s = 16 * I + lr + 4 * r;
+      const double vs = S.v[s];
+      vw += s < N - 1 ? vs : 0.0;
+      u1 = fma(f[I][r], vs, u1);
+      u2 += s < N - 1 ? f[I][r] : 0.0;
+      u0 += s == N - 1 ? f[I][r] : 0.0;
+    }
+  vw = wN * sum_xor32(sum_xor16(vw));
+  u0 = sum_xor32(sum_xor16(u0));
+  u1 = sum_xor32(sum_xor16(u1));
+  u2 = wN * sum_xor32(sum_xor16(u2));
+  const double u3 = fma(sgv, u0, u1);
+  const double c1 = u1 * wN, c2 = alw * u2 + alv * alw * vw * u3, c3 = alv * u3;
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int s = 16 * I + lr + 4 * r;
+      const double zw = s == N - 1 ? wN + 1.0 : wN, vt = s < N - 1 ? S.v[s] : 0.0;
+      const double x = s == N - 1 ? 0.0 : f[I][r];
+      X[(size_t)s * NP + 16 * J + lc] = s < N ? x + (c1 + c2 * zw + c3 * vt) : x;
+    }
 }
 
 // ---------------------------------------------------------------------------
-// Update: out = S_z [T | a] for the zone's rows, transposed on the MFMA as in
-// k_update (A = [T|a]^T from LDS, B = S_z^T from global).  Workgroup g:
-// zone 8 (g / 64) + g % 8 of the chunk, columns 32 cb .. 32 cb + 31 of T with
-// cb = (g / 8) % 8, so the eight workgroups of a zone land on one XCD (the
-// dispatcher deals workgroups to the XCDs in turn) and share its L2 for the
-// zone's rows of S; 68 KB of LDS each, two per CU.  The members of the next
-// 8 k-steps are loaded while those of the current 8 are multiplied.  Each workgroup forms
-// S a itself (bit-identical in all eight), for the mean and the clamp.
-//   MODE 0: xa = xf + Sf a, Sa = Sf T            (rrsqrt.F90:151,185,463)
-//   MODE 1: Sf = (E - xbar)/sqrt(N-1) on the fly; xa = xbar + clamp(Sf a);
-//           Ea = xa + sqrt(N-1) * (inflation * Sf T)  (assimilation.F90:3301-3320)
-// TE is the type of S and out (double, or float on the mixed path).
+// Update (update.hip's MODEs) for the zone's rows, transposed on the MFMA.
+// Workgroup g: zone 8 (g / 64) + g % 8 of the chunk, columns 32 cb .. 32 cb + 31
+// of T with cb = (g / 8) % 8, so the eight workgroups of a zone land on one XCD
+// (the dispatcher deals workgroups to the XCDs in turn) and share its L2 for
+// the zone's rows of S; 68 KB of LDS each, two per CU.  A strip's members are
+// all in registers before the product, which gives the mean of the state
+// without a pass of its own; the factors sqrt(N-1) cancel (update.hip).  Each
+// workgroup forms S a itself (bit-identical in all eight), for the mean and the
+// clamp.  The k index is permuted within pairs of MFMA steps as in k_update64.
+// 16 200 zones of 161 rows, FP32 members: 9.6 ms (18 with a mean from a pass of
+// its own, a division per element and a third of the MFMAs on the increment).
+// TE is the type of S and out (double, or float on the mixed path); the
+// products are in FP64.
 // ---------------------------------------------------------------------------
 template <int MODE, typename TE>
 __global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
                                                    const int32_t* __restrict__ zorder, int N,
                                                    const int64_t* __restrict__ zone_ptr,
-                                                   const double* __restrict__ mat,
+                                                   const double* __restrict__ umat,
                                                    const double* __restrict__ vec,
                                                    const double* __restrict__ X0,
                                                    const TE* __restrict__ S, int64_t ldS,
@@ -972,92 +959,93 @@ __global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
                                                    double maxcorr,
                                                    const double* __restrict__ maxcorr_v) {
 #pragma clang fp contract(off)
-  constexpr int NP = NPW, CB = 32, NCB = NP / CB, NBc = CB / 16, LW = CB + 1;
-  __shared__ double Ws[NP * LW];
-  __shared__ double as[NP];
+  constexpr int NP = NPW, CB = 32, NCB = NP / CB, NBc = CB / 16, LW = NP + 2, Q = NP / 4;
+  __shared__ __attribute__((aligned(16))) double Ws[CB * LW];
+  __shared__ __attribute__((aligned(16))) double as[NP];
   const int g = blockIdx.x;
   const int zl = (g / (8 * NCB)) * 8 + (g & 7), cb = (g >> 3) % NCB;
-  if (zl >= nzc) return;
+  if (zl >= nzc || CB * cb >= N) return;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
   const int64_t i0 = zone_ptr[z];
   const int64_t sz = zone_ptr[z + 1] - i0;
   if (sz <= 0) return;
-  const double* T = mat + (size_t)zl * NP * NP;
-  const double* a = vec + (size_t)zl * 4 * NP + NP;
-  copy_batched<16>(threadIdx.x, NP * CB, 256,
-                   [&](int e) { return T[(size_t)(e / CB) * NP + CB * cb + e % CB]; },
-                   [&](int e, double t) { Ws[(e / CB) * LW + e % CB] = t; });
-  as[threadIdx.x] = a[threadIdx.x];
-  __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int li = lane & 15, kk = lane >> 4;
+  const double* X = umat + (size_t)zl * NP * NP + (size_t)CB * cb * NP;  // X[s][k] = T[k][s]
+  const double* a = vec + (size_t)zl * 4 * NP + NP;
+  copy_batched<16>(threadIdx.x, NP * CB, 256, [&](int e) { return X[e]; },
+                   [&](int e, double t) { Ws[(e / NP) * LW + e % NP] = t; });
+  as[threadIdx.x] = MODE == 1 ? a[threadIdx.x] / scaling : a[threadIdx.x];
+  auto k_of = [&](int q) { return 8 * (q >> 1) + 2 * kk + (q & 1); };
+  lds_barrier();
+  const double* lw = Ws + li * LW + 2 * kk;
   for (int64_t rb = 16 * wave; rb < sz; rb += 64) {
+    const bool rok = rb + li < sz;
+    const int64_t row = i0 + (rok ? rb + li : 0);
+    TE b[Q];
+    {
+      // pairs of members on, the last ones clamped to a member that exists
+      const TE* p = S + row + (int64_t)(2 * kk) * ldS;
+#pragma unroll
+      for (int q = 0; q < Q; q += 2) {
+        b[q] = p[k_of(q) < N ? 0 : -(int64_t)k_of(q) * ldS];
+        b[q + 1] = p[k_of(q + 1) < N ? ldS : -(int64_t)k_of(q) * ldS];
+        p += 8 * ldS;
+        __builtin_amdgcn_sched_barrier(0);  // addresses as they are needed
+      }
+    }
+    double x0 = 0.0, dx = 0.0;
+    if (MODE == 1) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) x0 += k_of(q) < N ? (double)b[q] : 0.0;
+      x0 = sum_xor32(sum_xor16(x0)) / N;
+    } else {
+      x0 = X0[row];
+    }
+    // opaque here: the conversions above would else be kept for below, and spill
+#pragma unroll
+    for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(b[q]));
     d4 acc[NBc];
 #pragma unroll
     for (int J = 0; J < NBc; ++J) acc[J] = d4{0, 0, 0, 0};
-    d4 acca = {0, 0, 0, 0};
-    const int64_t row = rb + li;
-    const bool rok = row < sz;
-    const double xb = (MODE == 1 && rok) ? X0[i0 + row] : 0.0;
-    // the members of 8 k-steps at a time, the next 8 loaded while the
-    // current ones are multiplied (a load per step, waited for at once,
-    // would expose the memory latency 64 times)
-    auto load8 = [&](int k0, TE* raw) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int kc = k0 + 4 * u + kk;
-        const bool ok = rok && kc < N;
-        raw[u] = S[ok ? (i0 + row) + (int64_t)kc * ldS : i0];
+    for (int p = 0; p < Q / 2; ++p) {
+      asm volatile("" ::: "memory");  // the reads of later pairs stay below
+      double d[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double s = (double)b[2 * p + h];
+        d[h] = rok && k_of(2 * p + h) < N ? (MODE == 1 ? s - x0 : s) : 0.0;
       }
-    };
-    TE cur[8];
-    load8(0, cur);
-    for (int k0 = 0; k0 < NP; k0 += 32) {
-      TE nxt[8];
-      load8(k0 + 32 < NP ? k0 + 32 : k0, nxt);
-      asm volatile("" ::: "memory");  // compiler barrier: keeps the loads above here
+      const double2 ak = *reinterpret_cast<const double2*>(as + 8 * p + 2 * kk);
+      dx = fma(d[0], ak.x, dx);
+      dx = fma(d[1], ak.y, dx);
+      double2 A[NBc];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int kc = k0 + 4 * u + kk;
-        const bool ok = rok && kc < N;
-        const double sv = (double)cur[u];
-        const double bval = ok ? ((MODE == 1) ? (sv - xb) / scaling : sv) : 0.0;
+      for (int J = 0; J < NBc; ++J) A[J] = *reinterpret_cast<const double2*>(lw + 16 * J * LW + 8 * p);
 #pragma unroll
-        for (int J = 0; J < NBc; ++J) acc[J] = mfma_f64(Ws[kc * LW + 16 * J + li], bval, acc[J]);
-        acca = mfma_f64(li == 0 ? as[kc] : 0.0, bval, acca);
-      }
+      for (int J = 0; J < NBc; ++J) acc[J] = mfma_f64(A[J].x, d[0], acc[J]);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) cur[u] = nxt[u];
+      for (int J = 0; J < NBc; ++J) acc[J] = mfma_f64(A[J].y, d[1], acc[J]);
     }
-    // S a of row (rb + li): column 0 of the a-tile, lanes 0..15, register 0
-    const double dx = shfl_d(acca[0], li);
-    double xar = 0.0;
-    if (rok) {
-      const double x0 = X0[i0 + row];
-      xar = x0 + dx;
-      if (MODE == 1) {
-        const double mc = maxcorr_v ? maxcorr_v[i0 + row] : maxcorr;
-        if (xar - mc > x0) xar = x0 + mc;
-        if (xar < x0 - mc) xar = x0 - mc;
-      }
-      if (MODE == 0 && cb == 0 && kk == 0) xa[i0 + row] = xar;
+    double xar = x0 + sum_xor32(sum_xor16(dx));
+    if (MODE == 1) {
+      const double mc = maxcorr_v ? maxcorr_v[row] : maxcorr;
+      if (xar - mc > x0) xar = x0 + mc;
+      if (xar < x0 - mc) xar = x0 - mc;
     }
+    if (MODE == 0 && rok && cb == 0 && kk == 0) xa[row] = xar;
 #pragma unroll
-    for (int J = 0; J < NBc; ++J) {
+    for (int J = 0; J < NBc; ++J)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int c = CB * cb + 16 * J + kk + 4 * r;
         if (rok && c < N) {
-          double o = acc[J][r];
-          if (MODE == 1) {
-            const double sa = (infl != 1.0) ? infl * o : o;
-            o = xar + sa * scaling;
-          }
-          Out[(i0 + row) + (int64_t)c * ldO] = (TE)o;
+          const double o = acc[J][r], d = infl != 1.0 ? infl * o : o;
+          Out[row + (int64_t)c * ldO] = (TE)(MODE == 1 ? xar + d : o);
         }
       }
-    }
   }
 }
 
@@ -1073,31 +1061,46 @@ void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
                        A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec,
                        A.err);
   if (tm) tm->mark(PH_EIG);
-  const TriArgs tri{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)256 * 256, 256, 256,
-                    A.dvec, A.evec, 1, (int64_t)255 * A.nzc, (int64_t)254 * A.nzc, -(int64_t)A.nzc,
-                    nullptr, 0, 0, 0};
-  hipLaunchKernelGGL((k_tridiag_lower<256>), dim3(A.nzc), dim3(512), 0, st, tri);
-  launch_tridiag256_tail(A, st);
-  hipLaunchKernelGGL(k_formq256, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                     A.ymat, A.umat);
-  launch_ql256(A, st);
-  if (A.mode == 2) return;  // the likelihood has no kernels at this size
+  // the reduction: steps 0..127, then the trailing block (rows 128..191 of
+  // the reflectors' matrix, dense) as launch_tridiag_lower128 does, its
+  // reflectors to rows 192..255
+  constexpr int64_t ZS = (int64_t)256 * 256;
+  TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, ZS, 256, 256, A.dvec, A.evec, 256, 0, 0, 1,
+            A.vec, 4 * 256, 2 * 256, A.N, 256};
+  hipLaunchKernelGGL((k_tridiag_lower<256>), dim3(A.nzc), dim3(512), 0, st, T);
+  T.mat = A.ymat + 128 * 256;
+  T.qmat = A.ymat + 192 * 256;
+  T.ldm = T.ldv = 128;
+  T.d0 = T.e0 = 128;
+  T.vecs = A.vec + 128;
+  T.ones = -1;
+  hipLaunchKernelGGL((k_tridiag_lower<128>), dim3(A.nzc), dim3(128), 0, st, T);
+  T.mat = T.qmat + 64 * 128;
+  T.qmat = T.qmat + 64 * 128 + 64;
+  T.d0 = T.e0 = 192;
+  T.vecs = A.vec + 192;
+  T.n = std::max(A.N - 192, 0);
+  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
+  launch_pole256(A, st);
+  const double* tb = A.ymat + 128 * 256;
+  hipLaunchKernelGGL(k_qapply256<1>, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                     A.ymat, tb, A.mat, A.umat, A.vec);
   if (tm) tm->mark(PH_TMAT);
-  hipLaunchKernelGGL(k_tmat256, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                     A.umat, A.mat, A.vec);
+  hipLaunchKernelGGL(k_qapply256<2>, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                     A.ymat, tb, A.mat, A.umat, A.vec);
   if (tm) tm->mark(PH_UPDATE);
   const unsigned nb = (unsigned)(((A.nzc + 7) / 8) * 64);  // 8 column blocks per zone
   if (A.prec == 1)
     hipLaunchKernelGGL((k_update256<1, float>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0, A.zorder,
-                       A.N, A.zone_ptr, A.mat, A.vec, A.X0, A.S32, A.ldS, A.xa, A.Out32, A.ldO,
+                       A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S32, A.ldS, A.xa, A.Out32, A.ldO,
                        A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   else if (A.mode == 0)
     hipLaunchKernelGGL((k_update256<0, double>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0,
-                       A.zorder, A.N, A.zone_ptr, A.mat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
+                       A.zorder, A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
                        A.ldO, A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   else
     hipLaunchKernelGGL((k_update256<1, double>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0,
-                       A.zorder, A.N, A.zone_ptr, A.mat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
+                       A.zorder, A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
                        A.ldO, A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   if (tm) tm->mark(PH_END);
 }

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("sigma", [0.5, 2e-3])
-@pytest.mark.parametrize("N", [1, 2, 3, 15, 16, 17, 18, 31, 32, 33, 47, 64, 65, 97, 127, 128])
+@pytest.mark.parametrize("N", [1, 2, 3, 15, 16, 17, 18, 31, 32, 33, 47, 64, 65, 97, 127, 128,
+                               129, 144, 145, 192, 193, 194, 200, 255, 256])
 def test_functions_vs_oracle(N, sigma):
     from oak_amd.rrsqrt import loc_analysis_csr
     g = np.random.default_rng(N)
