@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void k_gram(int64_t z0, const int32_t* __re
   const int64_t p = sel_ptr[z + 1] - p0;
   double* M = mat + (size_t)zl * NP * NP;
   double* bv_out = vec + (size_t)zl * 4 * NP;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int kq = lane >> 4, jl = lane & 15;
   if (p == 0) {
     for (int e = threadIdx.x; e < NP * NP; e += 256) M[e] = (e / NP == e % NP) ? 1.0 : 0.0;
@@ -167,58 +167,56 @@ __global__ __launch_bounds__(256, 2) void k_gram(int64_t z0, const int32_t* __re
   double bacc[NB];
 #pragma unroll
   for (int J = 0; J < NB; ++J) bacc[J] = 0;
-  const int64_t nsteps = (p + 3) >> 2;
-  // The steps of a wave (s = wave, wave + 4, ...) are software-pipelined as
-  // in gram128_wave (analysis128.hip): the index and weight two steps ahead
-  // and the gathers of the next step are in flight while a step's MFMAs run;
-  // the step is branch-free, and a compiler barrier keeps the prefetched
-  // loads from being folded into the next iteration.
-  struct Idx {
-    int64_t l;
-    double w;
-    bool ok;
+  // The steps of a wave (s = wave, wave + 4, ...) are software-pipelined: the
+  // index and weight two steps ahead and the gathers of the next step are in
+  // flight while a step's MFMAs run.  MFMA and vector instructions of a SIMD
+  // share its FP64 issue, so every vector instruction of a step (of 640 cycles
+  // of MFMAs at NP = 64) is lost to them: two steps a pass in place of moves
+  // between the stages, 32-bit offsets, and a step past the zone's rows masked
+  // in its weight r alone (it reads the zone's last row).  27 vector instructions
+  // a step for 62 before: N = 64, 64 800 zones of 2990 rows, 18.9 -> 17.8 ms (the
+  // MFMAs alone: 15.6 at the 1.9 GHz that the device holds under them).
+  const int pn = (int)p, nsteps = (pn + 3) >> 2;
+  const int32_t* si = sel_idx + p0;
+  const double* sw = sel_w + p0;
+  struct Stage {
+    unsigned l;
+    double w, rh, inn;
+    TS rv[NB];
   };
   bool bad = false;  // an index outside 0..m-1 (reported once, after the loop)
-  auto fetch_idx = [&](int64_t s) {
-    Idx x;
-    const int64_t q = 4 * s + kq;
-    x.ok = q < p;
-    const int64_t qc = x.ok ? q : p - 1;  // p >= 1 here
-    x.l = sel_idx[p0 + qc];
-    x.w = sel_w[p0 + qc];
-    return x;
+  auto fetch_idx = [&](int s, Stage& x) {
+    const int q = 4 * s + kq;
+    const unsigned qc = q < pn ? q : pn - 1;  // p >= 1 here
+    x.l = si[qc];
+    x.w = sw[qc];
   };
-  auto fetch_row = [&](Idx& x, double& rh, double& inn, TS* rv) {
-    const bool inr = x.l >= 0 && x.l < m;
-    bad = bad | (x.ok & !inr);
-    x.ok = x.ok & inr;
-    x.l = x.ok ? x.l : 0;
-    rh = rho[x.l];
-    inn = innov[x.l];
-    const TS* row = HS + (size_t)x.l * NP + jl;
+  auto fetch_row = [&](Stage& x) {
+    const bool in = x.l < (unsigned)m;
+    bad = bad | !in;
+    const unsigned l = in ? x.l : 0;
+    x.rh = rho[l];
+    x.inn = innov[l];
+    const TS* row = HS + (size_t)l * NP + jl;
 #pragma unroll
-    for (int J = 0; J < NB; ++J) rv[J] = row[16 * J];
+    for (int J = 0; J < NB; ++J) x.rv[J] = row[16 * J];
   };
-  Idx i0 = fetch_idx(wave), i1 = fetch_idx(wave + 4);
-  double rh0, inn0;
-  TS rv0[NB];
-  fetch_row(i0, rh0, inn0, rv0);
-  for (int64_t s = wave; s < nsteps; s += 4) {
-    const Idx i2 = fetch_idx(s + 8);
-    double rh1, inn1;
-    TS rv1[NB];
-    fetch_row(i1, rh1, inn1, rv1);
+  // step s from `c`, whose place then takes the index of step s + 8; the
+  // rows of step s + 4 to `n`
+  auto step = [&](int s, Stage& c, Stage& n) {
+    fetch_row(n);
+    const double w = c.w;
+    fetch_idx(s + 8, c);
     asm volatile("" ::: "memory");  // compiler barrier: keeps the loads above here
-    const bool ok = i0.ok;
-    const double r = ok ? (i0.w * i0.w) * rh0 : 0.0;
-    const double rd = ok ? r * inn0 : 0.0;
+    const double r = 4 * s + kq < pn ? (w * w) * c.rh : 0.0;
+    const double rd = r * c.inn;
     double bv[NB];
 #pragma unroll
-    for (int J = 0; J < NB; ++J) bv[J] = ok ? (double)rv0[J] : 0.0;
+    for (int J = 0; J < NB; ++J) bv[J] = (double)c.rv[J];
     int t = 0;
 #pragma unroll
     for (int I = 0; I < NB; ++I) {
-      double a = r * bv[I];
+      const double a = r * bv[I];
 #pragma unroll
       for (int J = 0; J <= I; ++J) {
         acc[t] = mfma_f64(a, bv[J], acc[t]);
@@ -227,13 +225,17 @@ __global__ __launch_bounds__(256, 2) void k_gram(int64_t z0, const int32_t* __re
     }
 #pragma unroll
     for (int J = 0; J < NB; ++J) bacc[J] = fma(rd, bv[J], bacc[J]);
-    i0 = i1;
-    i1 = i2;
-    rh0 = rh1;
-    inn0 = inn1;
-#pragma unroll
-    for (int J = 0; J < NB; ++J) rv0[J] = rv1[J];
+  };
+  Stage A, B;
+  fetch_idx(wave, A);
+  fetch_idx(wave + 4, B);
+  fetch_row(A);
+  int s = wave;
+  for (; s + 4 < nsteps; s += 8) {
+    step(s, A, B);
+    step(s + 4, B, A);
   }
+  if (s < nsteps) step(s, A, B);
   if (bad) atomicOr(err, OAKG_DERR_IDX);
   // b: sum the four k-groups of the wave, then the waves
 #pragma unroll

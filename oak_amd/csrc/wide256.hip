@@ -33,7 +33,19 @@ namespace oakg {
 
 namespace {
 constexpr int NPW = 256;
+
+// Workgroup g of a launch with `parts` workgroups per zone: zone 8 (g / (8
+// parts)) + g % 8 and part (g / 8) % parts, so that the parts of a zone follow
+// one another on one XCD (workgroups go to the eight XCDs in turn) and share its
+// L2.  A grid with the part in y runs them a whole pass over the zones apart.
+__device__ __forceinline__ bool zone_part(int parts, int nzc, int& zl, int& part) {
+  const int g = blockIdx.x;
+  zl = (g / (8 * parts)) * 8 + (g & 7);
+  part = (g >> 3) % parts;
+  return zl < nzc;
 }
+inline dim3 zone_parts(int parts, int nzc) { return dim3((unsigned)((nzc + 7) / 8 * 8 * parts)); }
+}  // namespace
 
 // ---------------------------------------------------------------------------
 // Gram.  The lower triangle of M in 32 x 32 blocks (2 x 2 tiles of 16 x 16):
@@ -227,7 +239,9 @@ __device__ __forceinline__ void gram256_wave(int X0, int Y0, int X1, int Y1, int
   }
 }
 
-// grid (zones, 4): workgroup y holds wave slots 4 y .. 4 y + 3.  (Giving each
+// grid (zones, 4): workgroup y holds wave slots 4 y .. 4 y + 3, so that
+// neighbouring zones read the same columns of S at a time (49 ms for 16 200 zones
+// of 2100 observations; 55 to 59 with a zone's four workgroups one after another).  (Giving each
 // XCD a contiguous run of zones, so that neighbours share their rows of S in
 // one L2, was slower: the densely observed zones are contiguous too, and
 // their XCDs finish last.)
@@ -243,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* _
                                                     double* __restrict__ vec,
                                                     unsigned* __restrict__ err) {
   constexpr int NP = NPW;
-  const int zl = blockIdx.x;
+  const int zl = blockIdx.x, y = blockIdx.y;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
   const int64_t p0 = sel_ptr[z];
@@ -251,7 +265,6 @@ __global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* _
   double* M = mat + (size_t)zl * NP * NP;
   double* bv_out = vec + (size_t)zl * 4 * NP;
   if (p == 0) {  // M = I (rows 64 y .. 64 y + 63), b = 0
-    const int y = blockIdx.y;
     for (int e = threadIdx.x; e < NP * NP / 4; e += 256) {
       const int g = y * (NP * NP / 4) + e;
       M[g] = (g / NP == g % NP) ? 1.0 : 0.0;
@@ -259,7 +272,7 @@ __global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* _
     if (y == 0) bv_out[threadIdx.x] = 0.0;
     return;
   }
-  const int ws = __builtin_amdgcn_readfirstlane((int)blockIdx.y * 4 + (int)(threadIdx.x >> 6));
+  const int ws = __builtin_amdgcn_readfirstlane(y * 4 + (int)(threadIdx.x >> 6));
   int X0, Y0, X1, Y1;
   if (ws < 12) {
     gram256_offdiag(2 * ws, X0, Y0);
@@ -709,7 +722,8 @@ struct QApplyLds {
 };
 
 template <int STEP>
-__global__ __launch_bounds__(256, 2) void k_qapply256(int64_t z0, const int32_t* __restrict__ zorder,
+__global__ __launch_bounds__(256, 2) void k_qapply256(int nzc, int64_t z0,
+                                                      const int32_t* __restrict__ zorder,
                                                       int N, const int64_t* __restrict__ sel_ptr,
                                                       const double* __restrict__ qmat,
                                                       const double* __restrict__ tblk,
@@ -718,12 +732,13 @@ __global__ __launch_bounds__(256, 2) void k_qapply256(int64_t z0, const int32_t*
                                                       const double* __restrict__ vec) {
   constexpr int NP = NPW, NB = 16, LV = QApplyLds::LV;
   __shared__ QApplyLds S;
-  const int zl = blockIdx.x;
+  int zl, y;
+  if (!zone_part(4, nzc, zl, y)) return;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
   const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const int lr = lane >> 4, lc = lane & 15;
-  const int J = 4 * (int)blockIdx.y + wave;  // the wave's tile column
+  const int J = 4 * y + wave;  // the wave's tile column
   double* X = umat + (size_t)zl * NP * NP;
   if (sel_ptr[z + 1] == sel_ptr[z]) {
     if (STEP == 2)
@@ -933,10 +948,8 @@ __global__ __launch_bounds__(256, 2) void k_qapply256(int64_t z0, const int32_t*
 
 // ---------------------------------------------------------------------------
 // Update (update.hip's MODEs) for the zone's rows, transposed on the MFMA.
-// Workgroup g: zone 8 (g / 64) + g % 8 of the chunk, columns 32 cb .. 32 cb + 31
-// of T with cb = (g / 8) % 8, so the eight workgroups of a zone land on one XCD
-// (the dispatcher deals workgroups to the XCDs in turn) and share its L2 for
-// the zone's rows of S; 68 KB of LDS each, two per CU.  A strip's members are
+// Workgroup cb of a zone's eight has columns 32 cb .. 32 cb + 31 of T; they share
+// an L2 for the zone's rows of S; 68 KB of LDS each, two per CU.  A strip's members are
 // all in registers before the product, which gives the mean of the state
 // without a pass of its own; the factors sqrt(N-1) cancel (update.hip).  Each
 // workgroup forms S a itself (bit-identical in all eight), for the mean and the
@@ -962,9 +975,8 @@ __global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
   constexpr int NP = NPW, CB = 32, NCB = NP / CB, NBc = CB / 16, LW = NP + 2, Q = NP / 4;
   __shared__ __attribute__((aligned(16))) double Ws[CB * LW];
   __shared__ __attribute__((aligned(16))) double as[NP];
-  const int g = blockIdx.x;
-  const int zl = (g / (8 * NCB)) * 8 + (g & 7), cb = (g >> 3) % NCB;
-  if (zl >= nzc || CB * cb >= N) return;
+  int zl, cb;
+  if (!zone_part(NCB, nzc, zl, cb) || CB * cb >= N) return;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
   const int64_t i0 = zone_ptr[z];
@@ -1083,23 +1095,23 @@ void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
   launch_pole256(A, st);
   const double* tb = A.ymat + 128 * 256;
-  hipLaunchKernelGGL(k_qapply256<1>, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                     A.ymat, tb, A.mat, A.umat, A.vec);
+  hipLaunchKernelGGL(k_qapply256<1>, zone_parts(4, A.nzc), dim3(256), 0, st, A.nzc, A.z0, A.zorder, A.N,
+                     A.sel_ptr, A.ymat, tb, A.mat, A.umat, A.vec);
   if (tm) tm->mark(PH_TMAT);
-  hipLaunchKernelGGL(k_qapply256<2>, dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                     A.ymat, tb, A.mat, A.umat, A.vec);
+  hipLaunchKernelGGL(k_qapply256<2>, zone_parts(4, A.nzc), dim3(256), 0, st, A.nzc, A.z0, A.zorder, A.N,
+                     A.sel_ptr, A.ymat, tb, A.mat, A.umat, A.vec);
   if (tm) tm->mark(PH_UPDATE);
-  const unsigned nb = (unsigned)(((A.nzc + 7) / 8) * 64);  // 8 column blocks per zone
+  const dim3 nb = zone_parts(8, A.nzc);
   if (A.prec == 1)
-    hipLaunchKernelGGL((k_update256<1, float>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0, A.zorder,
+    hipLaunchKernelGGL((k_update256<1, float>), nb, dim3(256), 0, st, A.nzc, A.z0, A.zorder,
                        A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S32, A.ldS, A.xa, A.Out32, A.ldO,
                        A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   else if (A.mode == 0)
-    hipLaunchKernelGGL((k_update256<0, double>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0,
+    hipLaunchKernelGGL((k_update256<0, double>), nb, dim3(256), 0, st, A.nzc, A.z0,
                        A.zorder, A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
                        A.ldO, A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   else
-    hipLaunchKernelGGL((k_update256<1, double>), dim3(nb), dim3(256), 0, st, A.nzc, A.z0,
+    hipLaunchKernelGGL((k_update256<1, double>), nb, dim3(256), 0, st, A.nzc, A.z0,
                        A.zorder, A.N, A.zone_ptr, A.umat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out,
                        A.ldO, A.scaling, A.infl, A.maxcorr, A.maxcorr_v);
   if (tm) tm->mark(PH_END);
