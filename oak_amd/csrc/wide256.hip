@@ -3,10 +3,9 @@
 // A zone's 256 x 256 matrix is 512 KB in FP64: it fits neither the
 // registers of one workgroup nor its LDS, where the N <= 128 kernels keep
 // a zone whole, so each phase splits it its own way:
-//   k_gram256      M = I + S~^T S~ and b = S~^T R^-1 d: 16 waves per zone
-//                  (four workgroups), each over all local observations for
-//                  two or three 32 x 32 blocks of the lower triangle
-//                  (v_mfma_f64_16x16x4f64).
+//   k_gram256      M = I + S~^T S~ and b = S~^T R^-1 d: eight waves per zone,
+//                  each over all local observations for one or two 64 x 64
+//                  blocks of the lower triangle (v_mfma_f64_16x16x4f64).
 //   k_tridiag_lower<256>  Householder reduction to tridiagonal form (lower, as
 //                  dsytd2), steps 0..127, with the lower triangle in 8 x 8
 //                  register tiles over 512 threads, one workgroup per zone:
@@ -48,214 +47,172 @@ inline dim3 zone_parts(int parts, int nzc) { return dim3((unsigned)((nzc + 7) / 
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Gram.  The lower triangle of M in 32 x 32 blocks (2 x 2 tiles of 16 x 16):
-// 28 off-diagonal blocks (4 tiles) and 8 diagonal ones (3 tiles), dealt to
-// 16 wave slots per zone (four workgroups): slots 0..11 two off-diagonal
-// blocks each (8 tiles), slots 12..15 one off-diagonal and two diagonal
-// blocks (10 tiles), which also form b for the columns of their diagonal
-// blocks (all 256 together).  Every wave runs over all the zone's
-// observations, four per MFMA step, with the next step's gathers in flight
-// (the scheme of k_gram); at about 200 registers two waves share a SIMD, so
-// one wave's gathers and VALU work overlap another's MFMAs.
+// Gram.  The lower triangle of M in 64 x 64 blocks: a wave (a workgroup of its
+// own) per off-diagonal block (16 tiles of 16 x 16), two for the four diagonal
+// ones (two each, 20 tiles), which also form b for their columns.  Every wave
+// runs over all the zone's observations, four per MFMA step, pipelined as in
+// k_gram; a block's tile J holds its columns 4 j + J, so that a lane's four
+// columns are one 16-byte load.  The MFMAs share the issue with the vector
+// instructions: large blocks keep these few (a conversion and half a product
+// per MFMA).  grid (zones, 8): neighbouring zones read the same columns of S at
+// a time (with a zone's parts one after another it took a fifth longer).
+// 16 200 zones of 2100 observations, FP32: 37.9 ms (32 x 32 blocks: 49; the
+// MFMAs alone 31 at 2.4 GHz).
 // ---------------------------------------------------------------------------
-// off-diagonal block k (0..27) of the 8 x 8 block grid: (bi, bj), bi > bj
-__device__ __forceinline__ void gram256_offdiag(int k, int& bi, int& bj) {
-  int i = 1;
-  while (k >= i) {
-    k -= i;
-    ++i;
-  }
-  bi = i;
-  bj = k;
-}
-
-// MIX = false: off-diagonal blocks (X0, Y0) and (X1, Y1); MIX = true:
-// off-diagonal block (X0, Y0) and diagonal blocks X1 and Y1.  The lane's
-// values u[4 h + 2 s + k] = row[32 B + 16 k + jl] with B = (h ? (s ? Y1 : X1)
-// : (s ? Y0 : X0)).
-template <typename TS, bool MIX>
-__device__ __forceinline__ void gram256_wave(int X0, int Y0, int X1, int Y1, int64_t p0, int64_t p,
+template <typename TS, bool DIAG>
+__device__ __forceinline__ void gram256_wave(int X, int Y, int64_t p0, int pn,
                                              const int32_t* __restrict__ sel_idx,
-                                             const double* __restrict__ sel_w, int64_t m,
+                                             const double* __restrict__ sel_w, unsigned m,
                                              const double* __restrict__ rho,
                                              const double* __restrict__ innov,
                                              const TS* __restrict__ HS, double* __restrict__ M,
-                                             double* __restrict__ bv_out,
-                                             unsigned* __restrict__ err) {
-  constexpr int NP = NPW;
-  constexpr int NT = MIX ? 10 : 8;
+                                             double* __restrict__ bv_out, unsigned* __restrict__ err) {
+  constexpr int NP = NPW, NT = DIAG ? 20 : 16;
+  typedef TS TS4 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, kq = lane >> 4, jl = lane & 15;
   d4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = d4{0, 0, 0, 0};
-  double bacc[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) bacc[k] = 0.0;
-  const int64_t nsteps = (p + 3) >> 2;
-  struct Idx {
-    int64_t l;
-    double w;
-    bool ok;
+  double bacc[DIAG ? 8 : 1] = {};
+  const int nsteps = (pn + 3) >> 2;
+  const int32_t* si = sel_idx + p0;
+  const double* sw = sel_w + p0;
+  struct Stage {
+    unsigned l;
+    double w, rh, inn;
+    TS4 x, y;  // columns 64 X + 4 jl .. and 64 Y + 4 jl ..
   };
   bool bad = false;  // an index outside 0..m-1 (reported once, after the loop)
-  auto fetch_idx = [&](int64_t s) {
-    Idx x;
-    const int64_t q = 4 * s + kq;
-    x.ok = q < p;
-    const int64_t qc = x.ok ? q : p - 1;  // p >= 1 here
-    x.l = sel_idx[p0 + qc];
-    x.w = sel_w[p0 + qc];
-    return x;
+  auto fetch_idx = [&](int s, Stage& a) {
+    const int q = 4 * s + kq;
+    const unsigned qc = q < pn ? q : pn - 1;  // p >= 1 here
+    a.l = si[qc];
+    a.w = sw[qc];
   };
-  const int c0 = 32 * X0 + jl, c1 = 32 * Y0 + jl, c2 = 32 * X1 + jl, c3 = 32 * Y1 + jl;
-  auto fetch_row = [&](Idx& x, double& rh, double& inn, TS* rv) {
-    const bool inr = x.l >= 0 && x.l < m;
-    bad = bad | (x.ok & !inr);
-    x.ok = x.ok & inr;
-    x.l = x.ok ? x.l : 0;
-    rh = rho[x.l];
-    inn = innov[x.l];
-    const TS* row = HS + (size_t)x.l * NP;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      rv[k] = row[c0 + 16 * k];
-      rv[2 + k] = row[c1 + 16 * k];
-      rv[4 + k] = row[c2 + 16 * k];
-      rv[6 + k] = row[c3 + 16 * k];
-    }
+  const TS* hx = HS + 64 * X + 4 * jl;
+  const TS* hy = HS + 64 * Y + 4 * jl;
+  auto fetch_row = [&](Stage& a) {
+    const bool in = a.l < m;
+    bad = bad | !in;
+    const unsigned l = in ? a.l : 0;
+    a.rh = rho[l];
+    if (DIAG) a.inn = innov[l];
+    a.x = *reinterpret_cast<const TS4*>(hx + (size_t)l * NP);
+    a.y = *reinterpret_cast<const TS4*>(hy + (size_t)l * NP);
   };
-  Idx i0 = fetch_idx(0), i1 = fetch_idx(1);
-  double rh0, inn0;
-  TS rv0[8];
-  fetch_row(i0, rh0, inn0, rv0);
-  for (int64_t s = 0; s < nsteps; ++s) {
-    const Idx i2 = fetch_idx(s + 2);
-    double rh1, inn1;
-    TS rv1[8];
-    fetch_row(i1, rh1, inn1, rv1);
+  auto step = [&](int s, Stage& c, Stage& n) {
+    fetch_row(n);
+    const double w = c.w;
+    fetch_idx(s + 2, c);
     asm volatile("" ::: "memory");  // compiler barrier: keeps the loads above here
-    const bool ok = i0.ok;
-    const double r = ok ? (i0.w * i0.w) * rh0 : 0.0;
-    const double rd = ok ? r * inn0 : 0.0;
-    double bv[8];
+    const double r = 4 * s + kq < pn ? (w * w) * c.rh : 0.0;
+    double x[4], y[4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) bv[k] = ok ? (double)rv0[k] : 0.0;
-    int t = 0;
-#pragma unroll
-    for (int I = 0; I < 2; ++I) {  // off-diagonal block (X0, Y0)
-      const double a = r * bv[I];
-#pragma unroll
-      for (int J = 0; J < 2; ++J) {
-        acc[t] = mfma_f64(a, bv[2 + J], acc[t]);
-        ++t;
-      }
+    for (int k = 0; k < 4; ++k) {
+      x[k] = (double)c.x[k];
+      y[k] = (double)c.y[k];
     }
-    if constexpr (MIX) {  // diagonal blocks X1 and Y1
+    int t = 0;
+    if constexpr (DIAG) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int I = 0; I < 2; ++I) {
-          const double a = r * bv[4 + 2 * h + I];
+        for (int I = 0; I < 4; ++I) {
+          const double a = r * (h ? y[I] : x[I]);
 #pragma unroll
           for (int J = 0; J <= I; ++J) {
-            acc[t] = mfma_f64(a, bv[4 + 2 * h + J], acc[t]);
+            acc[t] = mfma_f64(a, h ? y[J] : x[J], acc[t]);
             ++t;
           }
         }
+      const double rd = r * c.inn;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) bacc[k] = fma(rd, bv[4 + k], bacc[k]);
-    } else {  // off-diagonal block (X1, Y1)
+      for (int k = 0; k < 4; ++k) {
+        bacc[k] = fma(rd, x[k], bacc[k]);
+        bacc[(DIAG ? 4 : 0) + k] = fma(rd, y[k], bacc[(DIAG ? 4 : 0) + k]);
+      }
+    } else {
 #pragma unroll
-      for (int I = 0; I < 2; ++I) {
-        const double a = r * bv[4 + I];
+      for (int I = 0; I < 4; ++I) {
+        const double a = r * x[I];
 #pragma unroll
-        for (int J = 0; J < 2; ++J) {
-          acc[t] = mfma_f64(a, bv[6 + J], acc[t]);
+        for (int J = 0; J < 4; ++J) {
+          acc[t] = mfma_f64(a, y[J], acc[t]);
           ++t;
         }
       }
     }
-    i0 = i1;
-    i1 = i2;
-    rh0 = rh1;
-    inn0 = inn1;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) rv0[k] = rv1[k];
-  }
-  if (bad) atomicOr(err, OAKG_DERR_IDX);
-  if constexpr (MIX) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      bacc[k] += shfl_xor_d(bacc[k], 16);
-      bacc[k] += shfl_xor_d(bacc[k], 32);
-    }
-    if (lane < 16) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) bv_out[32 * (k < 2 ? X1 : Y1) + 16 * (k & 1) + lane] = bacc[k];
-    }
-  }
-  // tile (gi0, gj0): register q of lane l is C[l/16 + 4q][l%16]; a diagonal
-  // tile writes its lower half into both triangles, so that M is exactly
-  // symmetric
-  auto put = [&](int gi0, int gj0, const d4& c, bool dtile) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = kq + 4 * q, j = jl;
-      if (!dtile || i >= j) {
-        const int gi = gi0 + i, gj = gj0 + j;
-        const double v = c[q] + (gi == gj ? 1.0 : 0.0);
-        M[(size_t)gi * NP + gj] = v;
-        M[(size_t)gj * NP + gi] = v;
-      }
-    }
   };
-  int t = 0;
+  Stage A, B;
+  fetch_idx(0, A);
+  fetch_idx(1, B);
+  fetch_row(A);
+  int s = 0;
+  for (; s + 1 < nsteps; s += 2) {
+    step(s, A, B);
+    step(s + 1, B, A);
+  }
+  if (s < nsteps) step(s, A, B);
+  if (bad) atomicOr(err, OAKG_DERR_IDX);
+  // element (i, j) of tile (I, J): row 64 X + 4 i + I, column 64 Y + 4 j + J; i =
+  // kq + 4 q in register q, j = jl
+  if constexpr (DIAG) {
 #pragma unroll
-  for (int I = 0; I < 2; ++I)
-#pragma unroll
-    for (int J = 0; J < 2; ++J) {
-      put(32 * X0 + 16 * I, 32 * Y0 + 16 * J, acc[t], false);
-      ++t;
+    for (int k = 0; k < 8; ++k) {
+      const double b = sum_xor32(sum_xor16(bacc[k]));
+      if (lane < 16) bv_out[64 * (k < 4 ? X : Y) + 4 * lane + (k & 3)] = b;
     }
-  if constexpr (MIX) {
+    // a diagonal block's tile gives both triangles (of a tile (I, I) its own
+    // lower half), so that M is exactly symmetric
+    int t = 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int I = 0; I < 2; ++I)
+      for (int I = 0; I < 4; ++I)
 #pragma unroll
         for (int J = 0; J <= I; ++J) {
-          const int B = h ? Y1 : X1;
-          put(32 * B + 16 * I, 32 * B + 16 * J, acc[t], I == J);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int i = kq + 4 * q, j = jl;
+            if (I != J || i >= j) {
+              const int gi = 64 * (h ? Y : X) + 4 * i + I, gj = 64 * (h ? Y : X) + 4 * j + J;
+              const double v = acc[t][q] + (gi == gj ? 1.0 : 0.0);
+              M[(size_t)gi * NP + gj] = v;
+              M[(size_t)gj * NP + gi] = v;
+            }
+          }
           ++t;
         }
   } else {
 #pragma unroll
-    for (int I = 0; I < 2; ++I)
+    for (int q = 0; q < 4; ++q) {
+      const int gi = 64 * X + 4 * (kq + 4 * q), gj = 64 * Y + 4 * jl;
 #pragma unroll
-      for (int J = 0; J < 2; ++J) {
-        put(32 * X1 + 16 * I, 32 * Y1 + 16 * J, acc[t], false);
-        ++t;
+      for (int I = 0; I < 4; ++I) {
+        d4 v, u;
+#pragma unroll
+        for (int J = 0; J < 4; ++J) {
+          v[J] = acc[4 * I + J][q];
+          u[J] = acc[4 * J + I][q];
+        }
+        *reinterpret_cast<d4*>(M + (size_t)(gi + I) * NP + gj) = v;
+        *reinterpret_cast<d4*>(M + (size_t)(gj + I) * NP + gi) = u;
       }
+    }
   }
 }
 
-// grid (zones, 4): workgroup y holds wave slots 4 y .. 4 y + 3, so that
-// neighbouring zones read the same columns of S at a time (49 ms for 16 200 zones
-// of 2100 observations; 55 to 59 with a zone's four workgroups one after another).  (Giving each
-// XCD a contiguous run of zones, so that neighbours share their rows of S in
-// one L2, was slower: the densely observed zones are contiguous too, and
-// their XCDs finish last.)
 template <typename TS>
-__global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* __restrict__ zorder,
-                                                    const int64_t* __restrict__ sel_ptr,
-                                                    const int32_t* __restrict__ sel_idx,
-                                                    const double* __restrict__ sel_w, int64_t m,
-                                                    const double* __restrict__ rho,
-                                                    const double* __restrict__ innov,
-                                                    const TS* __restrict__ HS,
-                                                    double* __restrict__ mat,
-                                                    double* __restrict__ vec,
-                                                    unsigned* __restrict__ err) {
+__global__ __launch_bounds__(64, 2) void k_gram256(int64_t z0, const int32_t* __restrict__ zorder,
+                                                   const int64_t* __restrict__ sel_ptr,
+                                                   const int32_t* __restrict__ sel_idx,
+                                                   const double* __restrict__ sel_w, int64_t m,
+                                                   const double* __restrict__ rho,
+                                                   const double* __restrict__ innov,
+                                                   const TS* __restrict__ HS,
+                                                   double* __restrict__ mat,
+                                                   double* __restrict__ vec,
+                                                   unsigned* __restrict__ err) {
   constexpr int NP = NPW;
   const int zl = blockIdx.x, y = blockIdx.y;
   const int64_t z = zone_at(zorder, z0 + zl);
@@ -264,27 +221,21 @@ __global__ __launch_bounds__(256, 2) void k_gram256(int64_t z0, const int32_t* _
   const int64_t p = sel_ptr[z + 1] - p0;
   double* M = mat + (size_t)zl * NP * NP;
   double* bv_out = vec + (size_t)zl * 4 * NP;
-  if (p == 0) {  // M = I (rows 64 y .. 64 y + 63), b = 0
-    for (int e = threadIdx.x; e < NP * NP / 4; e += 256) {
-      const int g = y * (NP * NP / 4) + e;
+  if (p == 0) {  // M = I (rows 32 y .. 32 y + 31), b = 0
+    for (int e = threadIdx.x; e < NP * NP / 8; e += 64) {
+      const int g = y * (NP * NP / 8) + e;
       M[g] = (g / NP == g % NP) ? 1.0 : 0.0;
     }
-    if (y == 0) bv_out[threadIdx.x] = 0.0;
+    if (threadIdx.x < 32) bv_out[32 * y + threadIdx.x] = 0.0;
     return;
   }
-  const int ws = __builtin_amdgcn_readfirstlane(y * 4 + (int)(threadIdx.x >> 6));
-  int X0, Y0, X1, Y1;
-  if (ws < 12) {
-    gram256_offdiag(2 * ws, X0, Y0);
-    gram256_offdiag(2 * ws + 1, X1, Y1);
-    gram256_wave<TS, false>(X0, Y0, X1, Y1, p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bv_out,
+  if (y < 6) {
+    const int X = y < 1 ? 1 : (y < 3 ? 2 : 3), Y = y - (y < 1 ? 0 : (y < 3 ? 1 : 3));
+    gram256_wave<TS, false>(X, Y, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M, bv_out,
                             err);
   } else {
-    gram256_offdiag(24 + (ws - 12), X0, Y0);
-    X1 = 2 * (ws - 12);
-    Y1 = X1 + 1;
-    gram256_wave<TS, true>(X0, Y0, X1, Y1, p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bv_out,
-                           err);
+    gram256_wave<TS, true>(2 * (y - 6), 2 * (y - 6) + 1, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho,
+                           innov, HS, M, bv_out, err);
   }
 }
 
@@ -1065,11 +1016,11 @@ __global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   if (tm) tm->mark(PH_GRAM);
   if (A.prec == 1)
-    hipLaunchKernelGGL((k_gram256<float>), dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder,
+    hipLaunchKernelGGL((k_gram256<float>), dim3(A.nzc, 8), dim3(64), 0, st, A.z0, A.zorder,
                        A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.mat, A.vec,
                        A.err);
   else
-    hipLaunchKernelGGL((k_gram256<double>), dim3(A.nzc, 4), dim3(256), 0, st, A.z0, A.zorder,
+    hipLaunchKernelGGL((k_gram256<double>), dim3(A.nzc, 8), dim3(64), 0, st, A.z0, A.zorder,
                        A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec,
                        A.err);
   if (tm) tm->mark(PH_EIG);
