@@ -94,10 +94,6 @@ struct ChunkArgs {
   int32_t* sweeps;
   // 0 = one-sided Jacobi, 1 = Householder tridiagonalisation + functions of T
   int eig_method;
-  unsigned* persist_wq;     // NP = 128: work counter of the persistent Gram (NULL: one
-                            // workgroup per zone)
-  int persist_item;         // its scheduling: 1 a zone per workgroup, 0 each wave its quarter
-  int persist_grid;         // its workgroups (persist_grid128)
   double *dvec, *evec;      // tridiagonal, NP per zone
   unsigned* err;
   double tol;
@@ -150,9 +146,6 @@ void launch_prep_ens(int NP, const PrepEnsArgs& A, hipStream_t st);
 void launch_chunk(int NP, const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 // NP = 128 in two parts (Gram + eigensolve, then transform + update), so
 // that the zones solved in observation space can run in between
-// Workgroups of the persistent Gram that fit on the current device at once
-// (0 when the runtime cannot say).
-int persist_grid128();
 void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 // zones with 1 <= p < 64 at NP = 128 in observation space (dual.hip): A has
@@ -161,6 +154,8 @@ void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_dual128(const ChunkArgs& A, int N, double* ymat128, double* vec128, double* ampl,
                     hipStream_t st, PhaseTimer* tm);
 void launch_chunk128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
+// NP = 128, 256 (gram_blocks.hip)
+void launch_gram_blocks(int NP, const ChunkArgs& A, hipStream_t st);
 // NP = 256 (wide256.hip): the whole chunk
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_pole256(const ChunkArgs& A, hipStream_t st);

@@ -2,9 +2,7 @@
 // the same steps as analysis.hip (rrsqrt.F90:100-190), with kernels shaped
 // for a 128 x 128 ensemble-space matrix.
 //
-//   k_gram128  M = I + S^T diag(r) S on v_mfma_f64_16x16x4f64 (S stored FP64, or
-//              FP32 for the mixed path): 36 lower tiles,
-//              wave w owns tile rows {w, 7-w} (9 tiles each, no cross-wave sum)
+//   gram_blocks.hip  M = I + S^T diag(r) S
 //   k_eig128   block one-sided Jacobi: each wave holds two 16-column blocks of
 //              all 128 rows (2 rows per lane, 64 doubles in registers); a sweep
 //              runs the 120 intra-block pairs of its blocks, then 7 block
@@ -25,257 +23,6 @@ namespace oakg {
 constexpr int P128 = 128;
 
 // ---------------------------------------------------------------------------
-// Gram matrix, NP = 128
-// ---------------------------------------------------------------------------
-template <int W, typename TS>
-__device__ __forceinline__ void gram128_wave(int64_t p0, int64_t p, const int32_t* __restrict__ sel_idx,
-                                             const double* __restrict__ sel_w, int64_t m,
-                                             const double* __restrict__ rho,
-                                             const double* __restrict__ innov,
-                                             const TS* __restrict__ HS, double* __restrict__ M,
-                                             double* __restrict__ bout, unsigned* __restrict__ err,
-                                             int lane) {
-  constexpr int IA = W, IB = 7 - W;
-  const int kq = lane >> 4, jl = lane & 15;
-  d4 accA[IA + 1], accB[IB + 1];
-#pragma unroll
-  for (int J = 0; J <= IA; ++J) accA[J] = d4{0, 0, 0, 0};
-#pragma unroll
-  for (int J = 0; J <= IB; ++J) accB[J] = d4{0, 0, 0, 0};
-  double bacc[8];
-#pragma unroll
-  for (int J = 0; J < 8; ++J) bacc[J] = 0;
-  const int64_t nsteps = (p + 3) >> 2;
-  // Each step's gathers hang on a load (index -> rho, innov and the row of
-  // S), so the steps are software-pipelined: the index and weight of step
-  // s + 2 and the gathers of step s + 1 are in flight while the MFMAs of step
-  // s run (same arithmetic as one step at a time).  The step is branch-free
-  // (indices past the zone's rows and invalid ones are clamped to valid
-  // entries and their values dropped), so that the compiler keeps the loads
-  // where they are issued instead of sinking them to their use.
-  struct Idx {
-    int64_t l;
-    double w;
-    bool ok;
-  };
-  bool bad = false;  // an index outside 0..m-1 (reported once, after the loop)
-  auto fetch_idx = [&](int64_t s) {
-    Idx x;
-    const int64_t q = 4 * s + kq;
-    x.ok = q < p;
-    const int64_t qc = x.ok ? q : p - 1;  // p >= 1 here
-    x.l = sel_idx[p0 + qc];
-    x.w = sel_w[p0 + qc];
-    return x;
-  };
-  // columns 16 J + jl, J = 0..7, stored contiguously (hs_col<128>); row 0
-  // stands in for a step past the zone's rows (its values are dropped)
-  auto fetch_row = [&](Idx& x, double& rh, double& inn, TS* rv) {
-    const bool inr = x.l >= 0 && x.l < m;
-    bad = bad | (x.ok & !inr);
-    x.ok = x.ok & inr;
-    x.l = x.ok ? x.l : 0;
-    rh = rho[x.l];
-    inn = innov[x.l];
-    const TS* row = HS + (size_t)x.l * P128 + 8 * jl;
-    if constexpr (sizeof(TS) == 4) {
-      const float4 u0 = reinterpret_cast<const float4*>(row)[0];
-      const float4 u1 = reinterpret_cast<const float4*>(row)[1];
-      rv[0] = u0.x; rv[1] = u0.y; rv[2] = u0.z; rv[3] = u0.w;
-      rv[4] = u1.x; rv[5] = u1.y; rv[6] = u1.z; rv[7] = u1.w;
-    } else {
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const double2 u = reinterpret_cast<const double2*>(row)[h];
-        rv[2 * h] = u.x;
-        rv[2 * h + 1] = u.y;
-      }
-    }
-  };
-  Idx i0 = fetch_idx(0), i1 = fetch_idx(1);
-  double rh0, inn0;
-  TS rv0[8];
-  fetch_row(i0, rh0, inn0, rv0);
-  for (int64_t s = 0; s < nsteps; ++s) {
-    const Idx i2 = fetch_idx(s + 2);
-    double rh1, inn1;
-    TS rv1[8];
-    fetch_row(i1, rh1, inn1, rv1);
-    // a compiler barrier (no instruction): without it the loads above, whose
-    // only use is the next iteration, are folded into one load at the top
-    // of the loop and the pipeline is gone
-    asm volatile("" ::: "memory");
-    // step s
-    const bool ok = i0.ok;
-    const double r = ok ? (i0.w * i0.w) * rh0 : 0.0;
-    const double rd = ok ? r * inn0 : 0.0;
-    double bv[8];
-#pragma unroll
-    for (int J = 0; J < 8; ++J) bv[J] = ok ? (double)rv0[J] : 0.0;
-    const double aA = r * bv[IA], aB = r * bv[IB];
-#pragma unroll
-    for (int J = 0; J <= IA; ++J) accA[J] = mfma_f64(aA, bv[J], accA[J]);
-#pragma unroll
-    for (int J = 0; J <= IB; ++J) accB[J] = mfma_f64(aB, bv[J], accB[J]);
-    if (W == 0) {
-#pragma unroll
-      for (int J = 0; J < 8; ++J) bacc[J] = fma(rd, bv[J], bacc[J]);
-    }
-    i0 = i1;
-    i1 = i2;
-    rh0 = rh1;
-    inn0 = inn1;
-#pragma unroll
-    for (int J = 0; J < 8; ++J) rv0[J] = rv1[J];
-  }
-  if (bad) atomicOr(err, OAKG_DERR_IDX);
-  auto store = [&](int I, int J, const d4& acc) {
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int i = (lane >> 4) + 4 * rr, j = lane & 15;
-      const int gi = 16 * I + i, gj = 16 * J + j;
-      if (I != J || i >= j) {
-        const double mv = acc[rr] + (gi == gj ? 1.0 : 0.0);
-        M[gi * P128 + gj] = mv;
-        M[gj * P128 + gi] = mv;
-      }
-    }
-  };
-#pragma unroll
-  for (int J = 0; J <= IA; ++J) store(IA, J, accA[J]);
-#pragma unroll
-  for (int J = 0; J <= IB; ++J) store(IB, J, accB[J]);
-  if (W == 0) {
-#pragma unroll
-    for (int J = 0; J < 8; ++J) {
-      bacc[J] += shfl_xor_d(bacc[J], 16);
-      bacc[J] += shfl_xor_d(bacc[J], 32);
-    }
-    if (lane < 16) {
-#pragma unroll
-      for (int J = 0; J < 8; ++J) bout[16 * J + lane] = bacc[J];
-    }
-  }
-}
-
-template <typename TS>
-__global__ __launch_bounds__(256, 2) void k_gram128(int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
-                                                 const int32_t* __restrict__ sel_idx,
-                                                 const double* __restrict__ sel_w, int64_t m,
-                                                 const double* __restrict__ rho,
-                                                 const double* __restrict__ innov,
-                                                 const TS* __restrict__ HS,
-                                                 double* __restrict__ mat, double* __restrict__ vec,
-                                                 unsigned* __restrict__ err) {
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;  // the zone is solved by the other pipeline
-  const int64_t p0 = sel_ptr[z];
-  const int64_t p = sel_ptr[z + 1] - p0;
-  double* M = mat + (size_t)zl * P128 * P128;
-  double* bout = vec + (size_t)zl * 4 * P128;
-  if (p == 0) {
-    for (int e = threadIdx.x; e < P128 * P128; e += 256) M[e] = (e / P128 == e % P128) ? 1.0 : 0.0;
-    for (int e = threadIdx.x; e < P128; e += 256) bout[e] = 0.0;
-    return;
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  switch (wave) {
-    case 0: gram128_wave<0, TS>(p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bout, err, lane); break;
-    case 1: gram128_wave<1, TS>(p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bout, err, lane); break;
-    case 2: gram128_wave<2, TS>(p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bout, err, lane); break;
-    default: gram128_wave<3, TS>(p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bout, err, lane); break;
-  }
-}
-
-// The same Gram as a persistent kernel: a fixed grid takes zones from work
-// counters in the order of the zone loop until the chunk is done.  Wave w of
-// a workgroup always computes quarter w of a zone's tiles (the quarters need
-// no common barrier), so the quarter is fixed per wave and its tile loop is
-// compiled alone.  WG: the workgroup takes one zone for its four waves from
-// counter 0 (the zone broadcast through LDS); else each wave takes the next
-// zone of its own quarter from counter w.  The counters are cleared by the
-// caller (a fill kernel) before each launch; every wave leaves its loop once
-// the zone it reads passes the chunk (with WG all four waves read the same
-// value, so they pass the same number of barriers).
-constexpr int kPersistBlocksPerCU = 2;  // the register bound the kernel is compiled for
-
-__global__ void k_clear_wq(unsigned* wq) {
-  if (threadIdx.x < 4) wq[threadIdx.x] = 0u;
-}
-
-template <int W, typename TS, bool WG>
-__device__ __forceinline__ void gram128_persist_loop(int64_t z0, const int32_t* __restrict__ zorder,
-                                                     int nzc, unsigned* __restrict__ counter,
-                                                     unsigned* sh_item,
-                                                     const int64_t* __restrict__ sel_ptr,
-                                                     const int32_t* __restrict__ sel_idx,
-                                                     const double* __restrict__ sel_w, int64_t m,
-                                                     const double* __restrict__ rho,
-                                                     const double* __restrict__ innov,
-                                                     const TS* __restrict__ HS,
-                                                     double* __restrict__ mat,
-                                                     double* __restrict__ vec,
-                                                     unsigned* __restrict__ err, int lane) {
-  auto zone = [&](unsigned item) {
-    const int64_t z = zone_at(zorder, z0 + (int64_t)item);
-    if (z < 0) return;  // the zone is solved by the other pipeline
-    const int64_t p0 = sel_ptr[z];
-    const int64_t p = sel_ptr[z + 1] - p0;
-    double* M = mat + (size_t)item * P128 * P128;
-    double* bout = vec + (size_t)item * 4 * P128;
-    if (p == 0) {  // identity: rows 32 W .. 32 W + 31; b from quarter 0
-      for (int e = lane; e < 32 * P128; e += 64) {
-        const int r = 32 * W + e / P128, c = e % P128;
-        M[r * P128 + c] = r == c ? 1.0 : 0.0;
-      }
-      if (W == 0)
-        for (int e = lane; e < P128; e += 64) bout[e] = 0.0;
-      return;
-    }
-    gram128_wave<W, TS>(p0, p, sel_idx, sel_w, m, rho, innov, HS, M, bout, err, lane);
-  };
-  if constexpr (WG) {
-    // wave 0 takes the zone; the first barrier publishes it (the store is
-    // waited for before the barrier), the second keeps the slot until every
-    // wave has read it
-    for (;;) {
-      if (W == 0 && lane == 0) *sh_item = atomicAdd(counter, 1u);
-      __syncthreads();
-      const unsigned item = *sh_item;
-      __syncthreads();
-      if (item >= (unsigned)nzc) break;  // the same value in every wave
-      zone(item);
-    }
-  } else {
-    for (;;) {
-      unsigned item = 0;
-      if (lane == 0) item = atomicAdd(counter + W, 1u);
-      item = __builtin_amdgcn_readfirstlane(item);
-      if (item >= (unsigned)nzc) break;
-      zone(item);
-    }
-  }
-}
-
-template <typename TS, bool WG>
-__global__ __launch_bounds__(256, kPersistBlocksPerCU) void k_gram128_persist(
-    int64_t z0, const int32_t* __restrict__ zorder, int nzc, unsigned* __restrict__ counter,
-    const int64_t* __restrict__ sel_ptr, const int32_t* __restrict__ sel_idx,
-    const double* __restrict__ sel_w, int64_t m, const double* __restrict__ rho,
-    const double* __restrict__ innov, const TS* __restrict__ HS, double* __restrict__ mat,
-    double* __restrict__ vec, unsigned* __restrict__ err) {
-  __shared__ unsigned sh_item;
-  // the wave index as a scalar: each wave runs one branch, with no exec mask
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  switch (wave) {
-    case 0: gram128_persist_loop<0, TS, WG>(z0, zorder, nzc, counter, &sh_item, sel_ptr, sel_idx, sel_w, m, rho, innov, HS, mat, vec, err, lane); break;
-    case 1: gram128_persist_loop<1, TS, WG>(z0, zorder, nzc, counter, &sh_item, sel_ptr, sel_idx, sel_w, m, rho, innov, HS, mat, vec, err, lane); break;
-    case 2: gram128_persist_loop<2, TS, WG>(z0, zorder, nzc, counter, &sh_item, sel_ptr, sel_idx, sel_w, m, rho, innov, HS, mat, vec, err, lane); break;
-    default: gram128_persist_loop<3, TS, WG>(z0, zorder, nzc, counter, &sh_item, sel_ptr, sel_idx, sel_w, m, rho, innov, HS, mat, vec, err, lane); break;
-  }
-}
-
 // Block one-sided Jacobi, NP = 128
 // ---------------------------------------------------------------------------
 struct Eig128Lds {
@@ -965,44 +712,9 @@ __global__ __launch_bounds__(256, 2) void k_xform128f(int64_t z0, const int32_t*
   }
 }
 
-int persist_grid128() {
-  // the occupancy the launch bounds guarantee (the runtime's occupancy
-  // query reports one workgroup per CU for these 256-VGPR waves)
-  int dev = 0, ncu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  return kPersistBlocksPerCU * ncu;
-}
-
 void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   if (tm) tm->mark(PH_GRAM);
-  if (A.persist_wq) {
-    hipLaunchKernelGGL(k_clear_wq, dim3(1), dim3(64), 0, st, A.persist_wq);
-    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(A.persist_grid, A.nzc));
-    const dim3 g(grid), b(256);
-    if (A.prec == 1 && A.persist_item == 1)
-      hipLaunchKernelGGL((k_gram128_persist<float, true>), g, b, 0, st, A.z0, A.zorder, A.nzc,
-                         A.persist_wq, A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32,
-                         A.mat, A.vec, A.err);
-    else if (A.prec == 1)
-      hipLaunchKernelGGL((k_gram128_persist<float, false>), g, b, 0, st, A.z0, A.zorder, A.nzc,
-                         A.persist_wq, A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32,
-                         A.mat, A.vec, A.err);
-    else if (A.persist_item == 1)
-      hipLaunchKernelGGL((k_gram128_persist<double, true>), g, b, 0, st, A.z0, A.zorder, A.nzc,
-                         A.persist_wq, A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS,
-                         A.mat, A.vec, A.err);
-    else
-      hipLaunchKernelGGL((k_gram128_persist<double, false>), g, b, 0, st, A.z0, A.zorder, A.nzc,
-                         A.persist_wq, A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS,
-                         A.mat, A.vec, A.err);
-  } else if (A.prec == 1)
-    hipLaunchKernelGGL(k_gram128<float>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.mat, A.vec, A.err);
-  else
-    hipLaunchKernelGGL(k_gram128<double>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.sel_ptr,
-                       A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec, A.err);
+  launch_gram_blocks(128, A, st);
   if (tm) tm->mark(PH_EIG);
   if (A.eig_method == 1) {
     launch_func(128, A, false, st);

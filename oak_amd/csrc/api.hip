@@ -475,7 +475,8 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * MP * MP + 6 * MP) +
                           (dual_lt ? sizeof(double) * ((size_t)2 * PD * PD + 4 * PD) : 0);
   const size_t budget = c->ws_budget;
-  const int nslot = (!c->timing && !c->arena && nz >= 4096) ? c->tune_slots : 1;
+  // one kernel a zone has nothing to overlap with the next chunk's
+  const int nslot = (!c->timing && !c->arena && !chol && nz >= 4096) ? c->tune_slots : 1;
   int64_t zc = std::max<int64_t>(1, (int64_t)(budget / (per_zone * nslot)));
   zc = std::min<int64_t>(zc, 1 << 20);
   if (nslot > 1) zc = std::min<int64_t>(zc, (nz + nslot - 1) / nslot);  // a chunk per slot
@@ -526,16 +527,6 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     vec_d = (double*)wsget(c, Workspace::VEC_D, sizeof(double) * (size_t)4 * PD * zs);
     if (!zord_p || !zord_d || !mat_d || !ymat_d || !vec_d) check(c, hipErrorOutOfMemory, "workspace");
   }
-  // work counters of the persistent Gram, one per slot on its own 256 B
-  const int persist_item = c->tune_persist == 2 ? 1 : 0;
-  const int persist_grid =
-      NP == 128 && c->tune_persist != 0 && !c->arena && nz > 0 ? persist_grid128() : 0;
-  const bool persist = persist_grid > 0;
-  unsigned* wq = nullptr;
-  if (persist) {
-    wq = (unsigned*)wsget(c, Workspace::PERSIST_WQ, (size_t)256 * OAKG_PIPE_SLOTS);
-    if (!wq) check(c, hipErrorOutOfMemory, "workspace");
-  }
   // streams and events of the pipeline, created before any capture
   if (nslot > 1) {
     if (!c->ev_fork) check(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming), "event");
@@ -555,7 +546,7 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     struct Key {
       ChunkArgs base;
       int64_t nz, zc;
-      int NP, nslot, func, order, dual_lt, persist;
+      int NP, nslot, func, order, dual_lt;
       const void* buf[16];
       hipStream_t stream;
     } kk;
@@ -568,9 +559,8 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     kk.func = func;
     kk.order = order;
     kk.dual_lt = dual_lt;
-    kk.persist = persist ? 1 + persist_item : 0;
     const void* bufs[16] = {mat,  ymat,   vec,    dvec,   evec,  sweeps_all,
-                            zorder, zord_p, zord_d, mat_d, ymat_d, vec_d, wq,  umat};
+                            zorder, zord_p, zord_d, mat_d, ymat_d, vec_d, umat};
     memcpy(kk.buf, bufs, sizeof bufs);
     kk.stream = c->stream;
     key.assign((const char*)&kk, (const char*)&kk + sizeof kk);
@@ -638,9 +628,6 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
     A.eig_method = func ? 1 : 0;
     A.dvec = dvec ? dvec + zo * NP : nullptr;
     A.evec = evec ? evec + zo * NP : nullptr;
-    A.persist_wq = persist ? wq + (size_t)64 * sl : nullptr;
-    A.persist_item = persist_item;
-    A.persist_grid = persist_grid;
     PhaseTimer* tm = c->timing ? &c->timer : nullptr;
     if (dual_lt) {
       // ensemble-space zones, then observation-space zones (writing their

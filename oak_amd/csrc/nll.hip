@@ -179,12 +179,16 @@ void launch_nll_adjoint(int NP, const ChunkArgs& A, hipStream_t st) {
 // to it, as rrsqrt.F90:137 clamps the eigenvalues.
 //
 // A wave per zone (WPZ = 1), so that all phases of other zones run beside the
-// serial elimination of one, or four that share the observations (WPZ = 4, the
-// elimination by the first) when there are fewer zones than SIMDs.  Bound by
+// serial elimination of one; four that share the observations (WPZ = 4, the
+// elimination by the first) for zones with kShareRows of them or more.  The
+// zone's own count decides, so that its sums keep their order in every schedule;
+// each of the two launches skips the other's zones.  Bound by
 // the MFMAs and the elimination's FP64 issue.  65 536 zones, N = 32, 41
 // observations each: 0.69 ms, where the eigensolve by QL, its rotations and the
 // adjoint by vector FMAs took 5.9 ms.
 // ---------------------------------------------------------------------------
+constexpr int kShareRows = 512;
+
 template <int NP, int WPZ>
 __global__ __launch_bounds__(64 * WPZ, 2) void k_nll_chol(
     int64_t z0, const int32_t* __restrict__ zorder, const int64_t* __restrict__ sel_ptr,
@@ -201,6 +205,7 @@ __global__ __launch_bounds__(64 * WPZ, 2) void k_nll_chol(
   const int64_t z = zone_at(zorder, z0 + blockIdx.x);
   const int64_t p0 = sel_ptr[z], p = sel_ptr[z + 1] - p0;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
+  if ((p >= kShareRows) != (WPZ > 1)) return;  // the other launch's
   if (p == 0) {
     if (threadIdx.x == 0) Jz[z] = gL[z] = gA[z] = 0.0;
     return;
@@ -457,18 +462,14 @@ __global__ __launch_bounds__(64 * WPZ, 2) void k_nll_chol(
   }
 }
 
-// Four waves a zone below one zone per SIMD of the device (1024): the waves
-// would have a SIMD each anyway, and a zone's observations are shared.
 void launch_nll_chol(int NP, const ChunkArgs& A, hipStream_t st) {
 #define OAK_CHOL(P, WPZ)                                                                           \
   hipLaunchKernelGGL((k_nll_chol<P, WPZ>), dim3(A.nzc), dim3(64 * WPZ), 0, st, A.z0, A.zorder,     \
                      A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.corr, A.infl,     \
                      A.nll_J, A.nll_gL, A.nll_gA, A.nll_gth, A.err)
 #define OAK_CHOL_N(P) \
-  if (A.nzc < 1024)   \
-    OAK_CHOL(P, 4);   \
-  else                \
-    OAK_CHOL(P, 1)
+  OAK_CHOL(P, 4);     \
+  OAK_CHOL(P, 1)
   switch (NP) {
     case 16: OAK_CHOL_N(16); break;
     case 32: OAK_CHOL_N(32); break;

@@ -3,9 +3,7 @@
 // A zone's 256 x 256 matrix is 512 KB in FP64: it fits neither the
 // registers of one workgroup nor its LDS, where the N <= 128 kernels keep
 // a zone whole, so each phase splits it its own way:
-//   k_gram256      M = I + S~^T S~ and b = S~^T R^-1 d: eight waves per zone,
-//                  each over all local observations for one or two 64 x 64
-//                  blocks of the lower triangle (v_mfma_f64_16x16x4f64).
+//   gram_blocks.hip  M = I + S~^T S~ and b = S~^T R^-1 d, eight workgroups.
 //   k_tridiag_lower<256>  Householder reduction to tridiagonal form (lower, as
 //                  dsytd2), steps 0..127, with the lower triangle in 8 x 8
 //                  register tiles over 512 threads, one workgroup per zone:
@@ -45,199 +43,6 @@ __device__ __forceinline__ bool zone_part(int parts, int nzc, int& zl, int& part
 }
 inline dim3 zone_parts(int parts, int nzc) { return dim3((unsigned)((nzc + 7) / 8 * 8 * parts)); }
 }  // namespace
-
-// ---------------------------------------------------------------------------
-// Gram.  The lower triangle of M in 64 x 64 blocks: a wave (a workgroup of its
-// own) per off-diagonal block (16 tiles of 16 x 16), two for the four diagonal
-// ones (two each, 20 tiles), which also form b for their columns.  Every wave
-// runs over all the zone's observations, four per MFMA step, pipelined as in
-// k_gram; a block's tile J holds its columns 4 j + J, so that a lane's four
-// columns are one 16-byte load.  The MFMAs share the issue with the vector
-// instructions: large blocks keep these few (a conversion and half a product
-// per MFMA).  grid (zones, 8): neighbouring zones read the same columns of S at
-// a time (with a zone's parts one after another it took a fifth longer).
-// 16 200 zones of 2100 observations, FP32: 37.9 ms (32 x 32 blocks: 49; the
-// MFMAs alone 31 at 2.4 GHz).
-// ---------------------------------------------------------------------------
-template <typename TS, bool DIAG>
-__device__ __forceinline__ void gram256_wave(int X, int Y, int64_t p0, int pn,
-                                             const int32_t* __restrict__ sel_idx,
-                                             const double* __restrict__ sel_w, unsigned m,
-                                             const double* __restrict__ rho,
-                                             const double* __restrict__ innov,
-                                             const TS* __restrict__ HS, double* __restrict__ M,
-                                             double* __restrict__ bv_out, unsigned* __restrict__ err) {
-  constexpr int NP = NPW, NT = DIAG ? 20 : 16;
-  typedef TS TS4 __attribute__((ext_vector_type(4)));
-  const int lane = threadIdx.x & 63, kq = lane >> 4, jl = lane & 15;
-  d4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = d4{0, 0, 0, 0};
-  double bacc[DIAG ? 8 : 1] = {};
-  const int nsteps = (pn + 3) >> 2;
-  const int32_t* si = sel_idx + p0;
-  const double* sw = sel_w + p0;
-  struct Stage {
-    unsigned l;
-    double w, rh, inn;
-    TS4 x, y;  // columns 64 X + 4 jl .. and 64 Y + 4 jl ..
-  };
-  bool bad = false;  // an index outside 0..m-1 (reported once, after the loop)
-  auto fetch_idx = [&](int s, Stage& a) {
-    const int q = 4 * s + kq;
-    const unsigned qc = q < pn ? q : pn - 1;  // p >= 1 here
-    a.l = si[qc];
-    a.w = sw[qc];
-  };
-  const TS* hx = HS + 64 * X + 4 * jl;
-  const TS* hy = HS + 64 * Y + 4 * jl;
-  auto fetch_row = [&](Stage& a) {
-    const bool in = a.l < m;
-    bad = bad | !in;
-    const unsigned l = in ? a.l : 0;
-    a.rh = rho[l];
-    if (DIAG) a.inn = innov[l];
-    a.x = *reinterpret_cast<const TS4*>(hx + (size_t)l * NP);
-    a.y = *reinterpret_cast<const TS4*>(hy + (size_t)l * NP);
-  };
-  auto step = [&](int s, Stage& c, Stage& n) {
-    fetch_row(n);
-    const double w = c.w;
-    fetch_idx(s + 2, c);
-    asm volatile("" ::: "memory");  // compiler barrier: keeps the loads above here
-    const double r = 4 * s + kq < pn ? (w * w) * c.rh : 0.0;
-    double x[4], y[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      x[k] = (double)c.x[k];
-      y[k] = (double)c.y[k];
-    }
-    int t = 0;
-    if constexpr (DIAG) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int I = 0; I < 4; ++I) {
-          const double a = r * (h ? y[I] : x[I]);
-#pragma unroll
-          for (int J = 0; J <= I; ++J) {
-            acc[t] = mfma_f64(a, h ? y[J] : x[J], acc[t]);
-            ++t;
-          }
-        }
-      const double rd = r * c.inn;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        bacc[k] = fma(rd, x[k], bacc[k]);
-        bacc[(DIAG ? 4 : 0) + k] = fma(rd, y[k], bacc[(DIAG ? 4 : 0) + k]);
-      }
-    } else {
-#pragma unroll
-      for (int I = 0; I < 4; ++I) {
-        const double a = r * x[I];
-#pragma unroll
-        for (int J = 0; J < 4; ++J) {
-          acc[t] = mfma_f64(a, y[J], acc[t]);
-          ++t;
-        }
-      }
-    }
-  };
-  Stage A, B;
-  fetch_idx(0, A);
-  fetch_idx(1, B);
-  fetch_row(A);
-  int s = 0;
-  for (; s + 1 < nsteps; s += 2) {
-    step(s, A, B);
-    step(s + 1, B, A);
-  }
-  if (s < nsteps) step(s, A, B);
-  if (bad) atomicOr(err, OAKG_DERR_IDX);
-  // element (i, j) of tile (I, J): row 64 X + 4 i + I, column 64 Y + 4 j + J; i =
-  // kq + 4 q in register q, j = jl
-  if constexpr (DIAG) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const double b = sum_xor32(sum_xor16(bacc[k]));
-      if (lane < 16) bv_out[64 * (k < 4 ? X : Y) + 4 * lane + (k & 3)] = b;
-    }
-    // a diagonal block's tile gives both triangles (of a tile (I, I) its own
-    // lower half), so that M is exactly symmetric
-    int t = 0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int I = 0; I < 4; ++I)
-#pragma unroll
-        for (int J = 0; J <= I; ++J) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int i = kq + 4 * q, j = jl;
-            if (I != J || i >= j) {
-              const int gi = 64 * (h ? Y : X) + 4 * i + I, gj = 64 * (h ? Y : X) + 4 * j + J;
-              const double v = acc[t][q] + (gi == gj ? 1.0 : 0.0);
-              M[(size_t)gi * NP + gj] = v;
-              M[(size_t)gj * NP + gi] = v;
-            }
-          }
-          ++t;
-        }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int gi = 64 * X + 4 * (kq + 4 * q), gj = 64 * Y + 4 * jl;
-#pragma unroll
-      for (int I = 0; I < 4; ++I) {
-        d4 v, u;
-#pragma unroll
-        for (int J = 0; J < 4; ++J) {
-          v[J] = acc[4 * I + J][q];
-          u[J] = acc[4 * J + I][q];
-        }
-        *reinterpret_cast<d4*>(M + (size_t)(gi + I) * NP + gj) = v;
-        *reinterpret_cast<d4*>(M + (size_t)(gj + I) * NP + gi) = u;
-      }
-    }
-  }
-}
-
-template <typename TS>
-__global__ __launch_bounds__(64, 2) void k_gram256(int64_t z0, const int32_t* __restrict__ zorder,
-                                                   const int64_t* __restrict__ sel_ptr,
-                                                   const int32_t* __restrict__ sel_idx,
-                                                   const double* __restrict__ sel_w, int64_t m,
-                                                   const double* __restrict__ rho,
-                                                   const double* __restrict__ innov,
-                                                   const TS* __restrict__ HS,
-                                                   double* __restrict__ mat,
-                                                   double* __restrict__ vec,
-                                                   unsigned* __restrict__ err) {
-  constexpr int NP = NPW;
-  const int zl = blockIdx.x, y = blockIdx.y;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;
-  const int64_t p0 = sel_ptr[z];
-  const int64_t p = sel_ptr[z + 1] - p0;
-  double* M = mat + (size_t)zl * NP * NP;
-  double* bv_out = vec + (size_t)zl * 4 * NP;
-  if (p == 0) {  // M = I (rows 32 y .. 32 y + 31), b = 0
-    for (int e = threadIdx.x; e < NP * NP / 8; e += 64) {
-      const int g = y * (NP * NP / 8) + e;
-      M[g] = (g / NP == g % NP) ? 1.0 : 0.0;
-    }
-    if (threadIdx.x < 32) bv_out[32 * y + threadIdx.x] = 0.0;
-    return;
-  }
-  if (y < 6) {
-    const int X = y < 1 ? 1 : (y < 3 ? 2 : 3), Y = y - (y < 1 ? 0 : (y < 3 ? 1 : 3));
-    gram256_wave<TS, false>(X, Y, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M, bv_out,
-                            err);
-  } else {
-    gram256_wave<TS, true>(2 * (y - 6), 2 * (y - 6) + 1, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho,
-                           innov, HS, M, bv_out, err);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Householder reduction of M (lower, as dsytd2: H_i x = beta e_1 for the
@@ -1015,14 +820,7 @@ __global__ __launch_bounds__(256, 2) void k_update256(int nzc, int64_t z0,
 // ---------------------------------------------------------------------------
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   if (tm) tm->mark(PH_GRAM);
-  if (A.prec == 1)
-    hipLaunchKernelGGL((k_gram256<float>), dim3(A.nzc, 8), dim3(64), 0, st, A.z0, A.zorder,
-                       A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS32, A.mat, A.vec,
-                       A.err);
-  else
-    hipLaunchKernelGGL((k_gram256<double>), dim3(A.nzc, 8), dim3(64), 0, st, A.z0, A.zorder,
-                       A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, A.HS, A.mat, A.vec,
-                       A.err);
+  launch_gram_blocks(256, A, st);
   if (tm) tm->mark(PH_EIG);
   // the reduction: steps 0..127, then the trailing block (rows 128..191 of
   // the reflectors' matrix, dense) as launch_tridiag_lower128 does, its

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 def test_functions_vs_oracle(N, sigma):
     from oak_amd.rrsqrt import loc_analysis_csr
     g = np.random.default_rng(N)
-    p = np.array([0, 1, 2, 3, max(N - 1, 1), N, N + 1, 3 * N, 150])
+    p = np.array([0, 1, 2, 3, max(N - 1, 1), N, N + 1, 3 * N, 150, 511, 512, 600])
     m = int(p.max())
     nz = len(p)
     zone_ptr = np.cumsum(np.r_[0, 1 + np.arange(nz) % 3])

@@ -1,6 +1,6 @@
-"""The likelihood's kernel for N <= 64 at the ensemble sizes where its tiles end
-and with one and four waves per zone (1600 and 100 zones, some without
-observations), against the dense FP64 reference.  Needs an MI355X."""
+"""The likelihood's kernel for N <= 64 at the ensemble sizes where its tiles end,
+for zones with no, few and so many observations (700) that four waves share
+them, against the dense FP64 reference.  Needs an MI355X."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +10,7 @@ from tests.nll_ref import nll_reference, selection
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,m", [(10, 70), (40, 90)])
+@pytest.mark.parametrize("nx,m", [(10, 70), (40, 90), (6, 700)])
 @pytest.mark.parametrize("N", [2, 16, 17, 32, 33, 48, 64])
 def test_nll_vs_reference(N, nx, m):
     from oak_amd import synth
