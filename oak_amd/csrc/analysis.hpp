@@ -64,7 +64,7 @@ struct PrepEnsArgs {
   const double *yo, *rmse2;
   const uint8_t* excl;
   double scaling;
-  double *xbar, *HEc, *HS, *innov, *rho;
+  double *HEc, *HS, *innov, *rho;
   unsigned* err;
   // mixed precision (FP32 state): E32, Hshift32 in, HS32 out
   const float* E32;
@@ -99,7 +99,7 @@ struct ChunkArgs {
   double tol;
   int max_sweeps;
   int zone_rows;     // mean rows of a zone
-  const double* X0;  // xf (mode 0) or xbar (mode 1, N = 65..128)
+  const double* X0;  // xf (mode 0)
   const double* S;   // Sf (mode 0) or E (mode 1)
   int64_t ldS;
   double* xa;   // mode 0
@@ -171,10 +171,12 @@ void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st);
 void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st);
 // the same M^-1/2 from the Jacobi option's eigenvectors
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
+// NP = 128: what Omega adds to M^-1/2, for k_update128
+void launch_omega_rows128(const ChunkArgs& A, hipStream_t st);
 // pole table of the current device
 hipError_t init_poles(int device);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
-// N <= 64 (update.hip): T from mat (N <= 32) or M^-1/2 from ymat
+// N <= 128 (update.hip): T from mat (N <= 32) or M^-1/2 from ymat
 void launch_update(int NP, const ChunkArgs& A, hipStream_t st);
 // N <= 64: Gram, factor and adjoint in one; N > 64: the adjoint after the eigensolve
 void launch_nll_chol(int NP, const ChunkArgs& A, hipStream_t st);

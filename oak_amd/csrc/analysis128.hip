@@ -8,9 +8,8 @@
 //              runs the 120 intra-block pairs of its blocks, then 7 block
 //              rounds (round-robin over the 8 blocks) of 16 cross-block rounds;
 //              blocks move between waves through the zone's scratch matrix
-//   funcm.hip  M^-1/2, a and v from the tridiagonal form (default)
-//   k_xform128 T = M^-1/2 Omega formed in LDS and the update Ea = xa + Sf T
-//              run from it (FP64 MFMA; FP32 MFMA for FP32 members)
+//   funcm.hip  the transform, a and v from the tridiagonal form (default)
+//   update.hip the update Ea = xa + Sf T
 #include <type_traits>
 
 #include <algorithm>
@@ -329,389 +328,6 @@ __global__ __launch_bounds__(256) void k_eig128(int64_t z0, const int32_t* __res
   if (tid == 0) sweeps_out[zl] = sweeps;
 }
 
-// ---------------------------------------------------------------------------
-// Transform and update fused, NP = 128, FP64: T = M^-1/2 Omega is formed in
-// LDS and out = Sf_z T, xa = x0 + Sf_z a run from it, so T never goes through
-// HBM.  One workgroup per zone (the 128 x 128 block fills the LDS):
-//   1. M^-1/2 -> LDS (row stride LDT: the MFMA operand reads, 16 rows x 4
-//      consecutive doubles per instruction, hit distinct banks)
-//   2. the Omega correction (the rank-structured formula of k_tmat in
-//      analysis.hip), applied in place; the buffer then holds X[s][r] = T[r][s]
-//   3. the update (Out^T strip = X Sf_strip^T) with the A operand X read
-//      from LDS and each wave's first strip of Sf loaded during steps 1-2
-// ---------------------------------------------------------------------------
-constexpr int LDT = P128 + 2;
-
-struct XformLds {
-  double t[P128 * LDT];
-  double u[4][P128];   // quarter sums of T v
-  double w[4][P128];   // quarter sums of T over the first N-1 entries
-  double v[P128];
-  double a[P128 + 2];  // a, then v.w~
-};
-
-template <int MODE, typename TE>
-__global__ __launch_bounds__(512) void k_xform128(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
-                                                  const int64_t* __restrict__ zone_ptr,
-                                                  const double* __restrict__ ymat,
-                                                  const double* __restrict__ vec,
-                                                  const double* __restrict__ X0,
-                                                  const TE* __restrict__ S, int64_t ldS,
-                                                  double* __restrict__ xa, TE* __restrict__ Out,
-                                                  int64_t ldO, double scaling, double infl,
-                                                  double maxcorr,
-                                                  const double* __restrict__ maxcorr_v) {
-#pragma clang fp contract(off)
-  // FP64 state, update on FP64 MFMA (MODE 0: locAnalysis with Sf given,
-  // MODE 1: ensemble); FP32 members run in k_xform128f.
-  constexpr bool F32 = std::is_same<TE, float>::value;
-  static_assert(!F32, "FP32 state runs in k_xform128f");
-  __shared__ XformLds L;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int li = lane & 15, kk = lane >> 4;
-  const int64_t i0 = zone_ptr[z];
-  const int64_t sz = zone_ptr[z + 1] - i0;
-  // The k index of the MFMA steps is permuted within pairs of steps: in
-  // steps 2p and 2p+1 lane group kk covers k = 8p + 2kk and 8p + 2kk + 1, so
-  // one 16-byte LDS read gives a lane both A operands.  B uses the same map.
-  // Sf values of strip rb: b[q] = Sf[rb + li][k(q)], k(q) = 8 (q/2) + 2 kk + q%2,
-  // loaded raw from clamped addresses; the selection and centring are
-  // applied where the values are first used, so the loads stay in flight
-  TE b[P128 / 4];
-  double x0 = 0.0;
-  auto load_strip = [&](int64_t rb) {
-    const int64_t row = rb + li;
-    const int64_t rr = i0 + (row < sz ? row : 0);
-    x0 = X0[rr];
-#pragma unroll
-    for (int q = 0; q < P128 / 4; ++q) {
-      const int k = 8 * (q >> 1) + 2 * kk + (q & 1);
-      b[q] = S[rr + (int64_t)(k < N ? k : 0) * ldS];
-    }
-  };
-  const double* Vz = vec + (size_t)zl * 4 * P128;
-  if (tid < P128) L.a[tid] = Vz[P128 + tid];
-  else if (tid < 2 * P128) L.v[tid - P128] = tid - P128 < N ? Vz[2 * P128 + tid - P128] : 0.0;
-  if (sel_ptr[z + 1] == sel_ptr[z]) {
-    // no observations: T = I (a = 0), the update copies the forecast anomalies
-    for (int e = tid; e < P128 * P128; e += 512) L.t[(e >> 7) * LDT + (e & 127)] = (e >> 7) == (e & 127);
-    if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-  } else {
-    // M^-1/2 is stored to LDS first, then the wave's first strip of Sf is
-    // loaded; the barriers of this kernel order LDS only, so the Sf loads
-    // stay in flight while the transform is formed
-    const double2* R2 = reinterpret_cast<const double2*>(ymat + (size_t)zl * P128 * P128);
-#pragma unroll
-    for (int it = 0; it < P128 * P128 / 1024; ++it) {
-      const int e = tid + 512 * it;
-      *reinterpret_cast<double2*>(L.t + (e >> 6) * LDT + 2 * (e & 63)) = R2[e];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-    // Omega = v w^T + P(v) P(w)^T (rrsqrt.F90:737-756, matoper.F90:509-535)
-    // applied on the right of the symmetric T (as k_tmat in analysis.hip).
-    // With w = 1/sqrt(N) 1,
-    // alpha_v = -1/(|v_N| + 1), alpha_w = -1/(1/sqrt(N) + 1), row r of T Omega is
-    //   x[s] = T[r][s] - [s = N-1] T[r][N-1] + wN (T v)_r
-    //          + (alpha_w U2 + alpha_v alpha_w (v.w~) U3) zw[s] + alpha_v U3 vt[s]
-    // with U2 = wN sum_{q<N-1} T[r][q], U3 = (T v)_r + sign(v_N) T[r][N-1],
-    // zw[s] = wN + [s = N-1], vt[s] = v[s] for s < N-1 (0 at N-1); the row
-    // sums are read as column sums of the symmetric T.
-    const double wN = 1.0 / sqrt((double)N);
-    const double vN = L.v[N - 1];
-    const double sgv = vN >= 0 ? 1.0 : -1.0;
-    const double alv = -1.0 / (fabs(vN) + 1.0);
-    const double alw = -1.0 / (wN + 1.0);
-    {
-      const int r = tid & 127, h = tid >> 7;  // quarter h of the column
-      double su = 0, sw = 0;
-#pragma unroll 8
-      for (int q = 32 * h; q < 32 * h + 32; ++q) {
-        const double tq = L.t[q * LDT + r];
-        su = fma(tq, L.v[q], su);
-        sw += q < N - 1 ? tq : 0.0;
-      }
-      L.u[h][r] = su;
-      L.w[h][r] = sw;
-    }
-    if (wave == 0) {
-      double s = 0;
-      for (int q = lane; q < N - 1; q += 64) s = fma(L.v[q], wN, s);
-      s = wave_sum_fast(s);
-      if (lane == 0) L.a[P128] = s;
-    }
-    lds_barrier();
-    const int r = tid & 127;
-    const double u0 = L.t[(N - 1) * LDT + r];
-    const double u1 = (L.u[0][r] + L.u[1][r]) + (L.u[2][r] + L.u[3][r]);
-    const double u2 = wN * ((L.w[0][r] + L.w[1][r]) + (L.w[2][r] + L.w[3][r]));
-    const double u3 = u1 + sgv * u0;
-    const double vw = L.a[P128];
-    const double c1 = u1 * wN;
-    const double c2 = alw * u2 + alv * alw * vw * u3;
-    const double c3 = alv * u3;
-    // X[s][r] = (T Omega)[r][s], in place (T symmetric: T[r][s] = t[s][r])
-#pragma unroll 4
-    for (int s = tid >> 7; s < N; s += 4) {
-      const double zw = s == N - 1 ? wN + 1.0 : wN;
-      const double vt = s < N - 1 ? L.v[s] : 0.0;
-      double x = L.t[s * LDT + r];
-      if (s == N - 1) x -= u0;
-      x += c1 + c2 * zw + c3 * vt;
-      L.t[s * LDT + r] = x;
-    }
-    lds_barrier();
-  }
-  // out = Sf_z T: Out^T strip = T^T Sf_strip^T, A operand X[16 J + li][k]
-  const double* xr = L.t + li * LDT + 2 * kk;
-  for (int64_t rb = 16 * wave; rb < sz; rb += 128) {
-    if (rb != 16 * wave) load_strip(rb);
-    const int64_t row = rb + li;
-    const bool rok = row < sz;
-    double dxp = 0.0;
-#pragma unroll
-    for (int q = 0; q < P128 / 4; ++q) {
-      const bool ok = rok && (8 * (q >> 1) + 2 * kk + (q & 1)) < N;
-      b[q] = ok ? ((MODE == 1) ? (b[q] - x0) / scaling : b[q]) : 0.0;
-    }
-#pragma unroll
-    for (int p = 0; p < P128 / 8; ++p) {
-      const double2 ak = *reinterpret_cast<const double2*>(L.a + 8 * p + 2 * kk);
-      dxp = fma(b[2 * p], ak.x, dxp);
-      dxp = fma(b[2 * p + 1], ak.y, dxp);
-    }
-    dxp += shfl_xor_d(dxp, 16);
-    dxp += shfl_xor_d(dxp, 32);
-    double xar = x0 + dxp;
-    if (MODE == 1) {
-      const double mc = (maxcorr_v && rok) ? maxcorr_v[i0 + row] : maxcorr;
-      if (xar - mc > x0) xar = x0 + mc;
-      if (xar < x0 - mc) xar = x0 - mc;
-    }
-    if (MODE == 0 && rok && kk == 0) xa[i0 + row] = xar;
-    // two passes over the output tiles (4 each) keep the accumulators small
-#pragma unroll 1
-    for (int h = 0; h < 2; ++h) {
-      const double* xh = xr + 64 * h * LDT;
-      d4 acc[4];
-#pragma unroll
-      for (int J = 0; J < 4; ++J) acc[J] = d4{0, 0, 0, 0};
-#pragma unroll
-      for (int p = 0; p < P128 / 8; ++p) {
-        // keeps the compiler from hoisting the reads of later pairs; the
-        // other wave on the SIMD covers the read latency
-        asm volatile("" ::: "memory");
-        double2 A[4];
-#pragma unroll
-        for (int J = 0; J < 4; ++J) A[J] = *reinterpret_cast<const double2*>(xh + 16 * J * LDT + 8 * p);
-#pragma unroll
-        for (int J = 0; J < 4; ++J) acc[J] = mfma_f64(A[J].x, b[2 * p], acc[J]);
-#pragma unroll
-        for (int J = 0; J < 4; ++J) acc[J] = mfma_f64(A[J].y, b[2 * p + 1], acc[J]);
-      }
-      if (rok) {
-#pragma unroll
-        for (int J = 0; J < 4; ++J) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int col = 64 * h + 16 * J + kk + 4 * r;
-            if (col < N) {
-              double o = acc[J][r];
-              if (MODE == 1) {
-                const double sa = (infl != 1.0) ? infl * o : o;
-                o = xar + sa * scaling;
-              }
-              Out[(i0 + row) + (int64_t)col * ldO] = o;
-            }
-          }
-        }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same for FP32 members (mixed precision): M^-1/2, rounded to FP32 where
-// it was formed, is staged in LDS and T Omega kept in FP32, the operand
-// precision of the FP32 update that consumes it (the Omega row sums and xa =
-// x0 + Sf a stay in FP64).  The buffers take 74 KB, so two zones share a CU;
-// four waves per zone.
-//   FP32 MFMA layout: A (16x4) lane l holds A[l % 16][l / 16], B (4x16)
-//   B[l / 16][l % 16], D (16x16) register r holds D[4 (l / 16) + r][l % 16].
-// ---------------------------------------------------------------------------
-constexpr int LDF = P128 + 4;
-
-struct XformLdsF {
-  float t[P128 * LDF];
-  double u[2][P128];   // half sums of T v
-  double w[2][P128];   // half sums of T over the first N-1 entries
-  double v[P128];
-  double a[P128 + 2];  // a / scaling, then v.w~
-};
-
-__global__ __launch_bounds__(256, 2) void k_xform128f(int64_t z0, const int32_t* __restrict__ zorder, int N, const int64_t* __restrict__ sel_ptr,
-                                                   const int64_t* __restrict__ zone_ptr,
-                                                   const double* __restrict__ ymat,
-                                                   const double* __restrict__ vec,
-                                                   const double* __restrict__ X0,
-                                                   const float* __restrict__ S, int64_t ldS,
-                                                   float* __restrict__ Out, int64_t ldO,
-                                                   double scaling, double infl, double maxcorr,
-                                                   const double* __restrict__ maxcorr_v) {
-#pragma clang fp contract(off)
-  __shared__ XformLdsF L;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int li = lane & 15, kk = lane >> 4;
-  const int64_t i0 = zone_ptr[z];
-  const int64_t sz = zone_ptr[z + 1] - i0;
-  // k permuted within pairs of MFMA steps (as in k_xform128): in steps 2p and
-  // 2p+1 lane group kk covers k = 8p + 2kk and 8p + 2kk + 1
-  float b[P128 / 4];
-  double x0 = 0.0;
-  auto load_strip = [&](int64_t rb) {
-    const int64_t row = rb + li;
-    const int64_t rr = i0 + (row < sz ? row : 0);
-    x0 = X0[rr];
-#pragma unroll
-    for (int q = 0; q < P128 / 4; ++q) {
-      const int k = 8 * (q >> 1) + 2 * kk + (q & 1);
-      b[q] = S[rr + (int64_t)(k < N ? k : 0) * ldS];
-    }
-  };
-  const double* Vz = vec + (size_t)zl * 4 * P128;
-  if (tid < P128) L.a[tid] = Vz[P128 + tid] / scaling;
-  else L.v[tid - P128] = tid - P128 < N ? Vz[2 * P128 + tid - P128] : 0.0;
-  if (sel_ptr[z + 1] == sel_ptr[z]) {
-    // no observations: T = I (a = 0), the update copies the forecast anomalies
-    for (int e = tid; e < P128 * P128; e += 256)
-      L.t[(e >> 7) * LDF + (e & 127)] = (e >> 7) == (e & 127) ? 1.0f : 0.0f;
-    if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-  } else {
-    // M^-1/2 as k_func and k_dual_lift leave it for this path, in FP32
-    const float4* R4 = reinterpret_cast<const float4*>(ymat + (size_t)zl * P128 * P128);
-    float4 rv[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) rv[u] = R4[tid + 256 * u];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = tid + 256 * u;
-      *reinterpret_cast<float4*>(L.t + (e >> 5) * LDF + 4 * (e & 31)) = rv[u];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (sz > 0) load_strip(16 * wave);
-    lds_barrier();
-    // Omega on the right of the symmetric T, as in k_xform128 (row sums read
-    // as column sums, accumulated in FP64)
-    const double wN = 1.0 / sqrt((double)N);
-    const double vN = L.v[N - 1];
-    const double sgv = vN >= 0 ? 1.0 : -1.0;
-    const double alv = -1.0 / (fabs(vN) + 1.0);
-    const double alw = -1.0 / (wN + 1.0);
-    {
-      const int r = tid & 127, h = tid >> 7;  // half h of the column
-      double su = 0, sw = 0;
-#pragma unroll 8
-      for (int q = 64 * h; q < 64 * h + 64; ++q) {
-        const double tq = L.t[q * LDF + r];
-        su = fma(tq, L.v[q], su);
-        sw += q < N - 1 ? tq : 0.0;
-      }
-      L.u[h][r] = su;
-      L.w[h][r] = sw;
-    }
-    if (wave == 0) {
-      double s = 0;
-      for (int q = lane; q < N - 1; q += 64) s = fma(L.v[q], wN, s);
-      s = wave_sum_fast(s);
-      if (lane == 0) L.a[P128] = s;
-    }
-    lds_barrier();
-    const int r = tid & 127;
-    const double u0 = L.t[(N - 1) * LDF + r];
-    const double u1 = L.u[0][r] + L.u[1][r];
-    const double u2 = wN * (L.w[0][r] + L.w[1][r]);
-    const double u3 = u1 + sgv * u0;
-    const double vw = L.a[P128];
-    const double c1 = u1 * wN;
-    const double c2 = alw * u2 + alv * alw * vw * u3;
-    const double c3 = alv * u3;
-    // X[s][r] = (T Omega)[r][s], in place (T symmetric: T[r][s] = t[s][r])
-#pragma unroll 4
-    for (int s = tid >> 7; s < N; s += 2) {
-      const double zw = s == N - 1 ? wN + 1.0 : wN;
-      const double vt = s < N - 1 ? L.v[s] : 0.0;
-      double x = L.t[s * LDF + r];
-      if (s == N - 1) x -= u0;
-      x += c1 + c2 * zw + c3 * vt;
-      L.t[s * LDF + r] = (float)x;
-    }
-    lds_barrier();
-  }
-  // out = Sf_z T: Out^T strip = T^T Sf_strip^T (as the FP32 branch of k_xform128)
-  const float* xr = L.t + li * LDF + 2 * kk;
-  const double sc_infl = scaling * infl;
-  const float inv = (float)(1.0 / scaling);
-  for (int64_t rb = 16 * wave; rb < sz; rb += 64) {
-    if (rb != 16 * wave) load_strip(rb);
-    const int64_t row = rb + li;
-    const bool rok = row < sz;
-    const float xb = (float)x0;
-    double dxp = 0.0;
-#pragma unroll
-    for (int q = 0; q < P128 / 4; ++q) {
-      const int kc = 8 * (q >> 1) + 2 * kk + (q & 1);
-      const bool ok = rok && kc < N;
-      const float ev = b[q];
-      if (ok) dxp = fma((double)ev - x0, L.a[kc], dxp);
-      b[q] = ok ? (ev - xb) * inv : 0.0f;
-    }
-    dxp += shfl_xor_d(dxp, 16);
-    dxp += shfl_xor_d(dxp, 32);
-    double xar = x0 + dxp;
-    const double mc = (maxcorr_v && rok) ? maxcorr_v[i0 + row] : maxcorr;
-    if (xar - mc > x0) xar = x0 + mc;
-    if (xar < x0 - mc) xar = x0 - mc;
-#pragma unroll 1
-    for (int h = 0; h < 2; ++h) {
-      const float* xh = xr + 64 * h * LDF;
-      f4 acc[4];
-#pragma unroll
-      for (int J = 0; J < 4; ++J) acc[J] = f4{0, 0, 0, 0};
-#pragma unroll
-      for (int p = 0; p < P128 / 8; ++p) {
-        asm volatile("" ::: "memory");
-        float2 A[4];
-#pragma unroll
-        for (int J = 0; J < 4; ++J) A[J] = *reinterpret_cast<const float2*>(xh + 16 * J * LDF + 8 * p);
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          acc[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[J].x, b[2 * p], acc[J], 0, 0, 0);
-#pragma unroll
-        for (int J = 0; J < 4; ++J)
-          acc[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[J].y, b[2 * p + 1], acc[J], 0, 0, 0);
-      }
-      if (rok) {
-#pragma unroll
-        for (int J = 0; J < 4; ++J) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int col = 64 * h + 16 * J + 4 * kk + r;
-            if (col < N)
-              Out[(i0 + row) + (int64_t)col * ldO] = (float)(xar + sc_infl * (double)acc[J][r]);
-          }
-        }
-      }
-    }
-  }
-}
-
 void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   if (tm) tm->mark(PH_GRAM);
   launch_gram_blocks(128, A, st);
@@ -732,20 +348,10 @@ void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
     if (tm) tm->mark(PH_END);
     return;
   }
-  // transform and update in one kernel (the timer books it as the update)
+  if (tm) tm->mark(PH_TMAT);
+  launch_omega_rows128(A, st);
   if (tm) tm->mark(PH_UPDATE);
-  if (A.prec == 1)
-    hipLaunchKernelGGL(k_xform128f, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                       A.zone_ptr, A.ymat, A.vec, A.X0, A.S32, A.ldS, A.Out32, A.ldO, A.scaling,
-                       A.infl, A.maxcorr, A.maxcorr_v);
-  else if (A.mode == 0)
-    hipLaunchKernelGGL((k_xform128<0, double>), dim3(A.nzc), dim3(512), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                       A.zone_ptr, A.ymat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out, A.ldO, A.scaling,
-                       A.infl, A.maxcorr, A.maxcorr_v);
-  else
-    hipLaunchKernelGGL((k_xform128<1, double>), dim3(A.nzc), dim3(512), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
-                       A.zone_ptr, A.ymat, A.vec, A.X0, A.S, A.ldS, A.xa, A.Out, A.ldO, A.scaling,
-                       A.infl, A.maxcorr, A.maxcorr_v);
+  launch_update(128, A, st);
   if (tm) tm->mark(PH_END);
 }
 

@@ -977,10 +977,6 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     const double* dval = stage(c, Workspace::H_VAL, H->val, H->nnz, dev);
     const T* dHs = stage(c, Workspace::H_SHIFT, Hshift, m, dev);
     const double* dmc = stage(c, Workspace::MAXCORR, maxc_elem, n, dev);
-    // the mean of the state: the update forms it from its own rows but for N = 65..128
-    const bool own_mean = NP <= 64 || NP == 256;
-    double* xbar = own_mean ? nullptr
-                            : (double*)wsget(c, Workspace::XBAR, sizeof(double) * std::max<int64_t>(n, 1));
     double* HEc = (double*)wsget(c, Workspace::HEC, sizeof(double) * std::max<int64_t>(m, 1) * N);
     double* HS = nullptr;
     float* HS32 = nullptr;
@@ -990,7 +986,7 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
       HS = (double*)wsget(c, Workspace::HS, sizeof(double) * std::max<int64_t>(m, 1) * NP);
     double* innov = (double*)wsget(c, Workspace::INNOV, sizeof(double) * std::max<int64_t>(m, 1));
     double* rho = (double*)wsget(c, Workspace::RHO, sizeof(double) * std::max<int64_t>(m, 1));
-    if ((!own_mean && !xbar) || !HEc || !(mixed ? (void*)HS32 : (void*)HS) || !innov || !rho)
+    if (!HEc || !(mixed ? (void*)HS32 : (void*)HS) || !innov || !rho)
       check(c, hipErrorOutOfMemory, "workspace");
     const double scaling = sqrt((double)N - 1.0);
     PrepEnsArgs P{};
@@ -1005,7 +1001,6 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     P.rmse2 = g.od.rmse2;
     P.excl = g.od.excluded;
     P.scaling = scaling;
-    P.xbar = xbar;
     P.HEc = HEc;
     P.HS = HS;
     P.HS32 = HS32;
@@ -1044,7 +1039,6 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     A.err = c->d_err;
     A.tol = c->jacobi_tol > 0 ? c->jacobi_tol : 4.0 * NP * 2.220446049250313e-16;
     A.max_sweeps = c->max_sweeps;
-    A.X0 = xbar;
     A.ldS = ld_e;
     A.xa = nullptr;
     A.ldO = ld_ea;
@@ -1223,7 +1217,6 @@ int ensemble_report_impl(oakg_ctx* c, const oakg_obs* obs, const oakg_csr* H, co
     P.rmse2 = g.od.rmse2;
     P.excl = g.od.excluded;
     P.scaling = sqrt((double)N - 1.0);
-    P.xbar = nullptr;  // the state mean is not needed
     P.HEc = HEc;
     P.HS = HS;
     P.HS32 = HS32;

@@ -15,8 +15,8 @@
 // (1 - x^-1/2) / (x - 1) and (x^1/2 - 1) / (x - 1) written without the
 // cancellation at x -> 1).  I + G runs through the NP = 64 reduction and
 // k_func with the weights of f and h (funcm.hip), and k_dual_lift writes a,
-// the normalised M^1/2 1_N and M^-1/2 into the zone's NP = 128 slots, as
-// k_func leaves them for the other zones.  The work per zone drops from that
+// the normalised M^1/2 1_N = v, M^-1/2 and its products with 1_N and v into the
+// zone's NP = 128 slots, as k_func leaves them for the other zones.  The work per zone drops from that
 // of a 128 x 128 reduction to a 64 x 64 one plus two products of 128 x p with
 // p x p and p x 128.
 //
@@ -26,6 +26,7 @@
 //   k_dual_lift   a, M^1/2 1_N, M^-1/2 from f(I + G) and the two vectors
 #include "analysis.hpp"
 #include "common.hpp"
+#include "eigen_common.hpp"
 
 namespace oakg {
 
@@ -179,6 +180,7 @@ __global__ __launch_bounds__(256, 2) void k_dual_lift(int64_t z0, const int32_t*
       }
   }
   TS* R = reinterpret_cast<TS*>(ymat + (size_t)zl * NPP * NPP);
+  double s0 = 0.0, s1 = 0.0;  // M^-1/2 1_N of the wave's columns
 #pragma unroll 1
   for (int I = 0; I < 8; ++I) {
     d4 x0 = {0.0, 0.0, 0.0, 0.0}, x1 = {0.0, 0.0, 0.0, 0.0};
@@ -195,10 +197,15 @@ __global__ __launch_bounds__(256, 2) void k_dual_lift(int64_t z0, const int32_t*
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = 16 * I + lr + 4 * r, c0 = 16 * wave + lc, c1 = c0 + 64;
-      R[(size_t)row * NPP + c0] = (TS)((row == c0 ? 1.0 : 0.0) - x0[r]);
-      R[(size_t)row * NPP + c1] = (TS)((row == c1 ? 1.0 : 0.0) - x1[r]);
+      const double y0 = (row == c0 ? 1.0 : 0.0) - x0[r], y1 = (row == c1 ? 1.0 : 0.0) - x1[r];
+      R[(size_t)row * NPP + c0] = (TS)y0;
+      R[(size_t)row * NPP + c1] = (TS)y1;
+      s0 += row < N ? y0 : 0.0;
+      s1 += row < N ? y1 : 0.0;
     }
   }
+  s0 = sum_xor32(sum_xor16(s0));
+  s1 = sum_xor32(sum_xor16(s1));
   double* V = vec + (size_t)zl * 4 * NPP;
   // a, M^1/2 1_N (rows i < 128, threads 0..127; the other waves add zeros)
   const int i = tid;
@@ -212,10 +219,14 @@ __global__ __launch_bounds__(256, 2) void k_dual_lift(int64_t z0, const int32_t*
   }
   const double ss = wave_sum_fast(vr * vr);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
+  if (lr == 0) {
+    V[16 * wave + lc] = s0;
+    V[16 * wave + lc + 64] = s1;
+  }
   lds_barrier();
   if (tid < NPP) {
     const double nv = (red[0] + red[1]) + (red[2] + red[3]);
-    V[i] = 0.0;
+    V[3 * NPP + i] = i < N ? 1.0 / sqrt(nv) : 0.0;  // M^-1/2 v
     V[NPP + i] = ar;
     V[2 * NPP + i] = vr / sqrt(nv);
     if (ampl && i < N) ampl[(size_t)z * N + i] = ar;

@@ -77,4 +77,61 @@ __device__ __forceinline__ const double* reflector256(const double* V, int k, in
   return k < 128 ? V + k * 256 + r : V + 192 * 256 + (k - 128) * 128 + (r < 128 ? 0 : r - 128);
 }
 
+// T = R Omega (below) with R v = kappa 1, kappa = 1 / |M^1/2 1|, and R 1 known: row c
+// of T is T[c][s] = R[c][s] + p_c + q_c v_s for s < N - 1, and T[c][N-1] = p_c + l_c
+// (the names as below: p = c1 + c2 wN, q = c3, l = c2).
+struct OmegaRow {
+  double p, q, l;
+};
+__device__ __forceinline__ OmegaRow omega_row(int N, double kappa, double r1, double rN, double vN,
+                                              double vsum) {
+  const double wN = 1.0 / sqrt((double)N);
+  const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0);
+  const double u2 = wN * (r1 - rN), u3 = vN >= 0 ? kappa + rN : kappa - rN;
+  const double c2 = alw * u2 + alv * alw * (wN * vsum) * u3;
+  return OmegaRow{fma(c2, wN, kappa * wN), alv * u3, c2};
+}
+
+// T = R Omega for the symmetric R = M^-1/2, Omega = RotateVector(w, v) with w =
+// 1/sqrt(N) 1 (rrsqrt.F90:185, 737-745; perpSpace matoper.F90:509-535) as the
+// identity and rank-one terms, applied to the columns of R that a wave holds in
+// MFMA tiles: f[I][r] is R[row(I, r)][c] for the lane's column c and, over the
+// four lane groups, all rows.  It becomes X[s][c] = T[c][s]:
+//   T[c][s] = R[c][s] (0 at s = N-1) + u1 wN + (alpha_w u2 + alpha_v alpha_w (v.w~)
+//             u3) zw_s + alpha_v u3 vt_s,  u1 = (R v)_c, u2 = (R w~)_c, u3 = u1 +
+//             sign(v_N) R[c][N-1], zw = w + e_{N-1}, vt = v (0 at N-1), w~ = w (0 at
+//             N-1), alpha_v = -1/(|v_N|+1), alpha_w = -1/(wN+1)
+template <int NT, typename Row>
+__device__ __forceinline__ void omega_columns(d4 (&f)[NT], int N, const double* v, Row row) {
+  const double wN = 1.0 / sqrt((double)N), vN = v[N - 1], sgv = vN >= 0 ? 1.0 : -1.0;
+  const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0);
+  double vw = 0.0, u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+  for (int I = 0; I < NT; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int s = row(I, r);
+      const double vs = s < N ? v[s] : 0.0, x = f[I][r];
+      vw += s < N - 1 ? vs : 0.0;
+      u1 = fma(x, vs, u1);
+      u2 += s < N - 1 ? x : 0.0;
+      u0 += s == N - 1 ? x : 0.0;
+    }
+  vw = wN * sum_xor32(sum_xor16(vw));
+  u0 = sum_xor32(sum_xor16(u0));
+  u1 = sum_xor32(sum_xor16(u1));
+  u2 = wN * sum_xor32(sum_xor16(u2));
+  const double u3 = fma(sgv, u0, u1);
+  const double c1 = u1 * wN, c2 = alw * u2 + alv * alw * vw * u3, c3 = alv * u3;
+#pragma unroll
+  for (int I = 0; I < NT; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int s = row(I, r);
+      const double zw = s == N - 1 ? wN + 1.0 : wN, vt = s < N - 1 ? v[s] : 0.0;
+      const double x = s == N - 1 ? 0.0 : f[I][r];
+      f[I][r] = s < N ? x + (c1 + c2 * zw + c3 * vt) : x;
+    }
+}
+
 }  // namespace oakg

@@ -151,7 +151,7 @@ hipError_t init_poles(int device) {
 // DUAL (observation-space zones, dual.hip): F with the weights w / (1 + s),
 // i.e. x -> 1 / (x + sqrt x), and y with w s / (1 + s), x -> 1 / (1 + sqrt x);
 // v is left as Q y.  LIKE: also log det M, sum (1 - 1/mu) and b^T a (slot 3 of
-// vec) for the likelihood.  TR is the type R is stored in (float for the FP32 update
+// vec) for the likelihood; else, at NP = 128, R 1 and R v in slots 0 and 3.  TR is the type R is stored in (float for the FP32 update
 // of the mixed path).
 // ---------------------------------------------------------------------------
 template <int NP>
@@ -715,6 +715,13 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       R[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = (TR)f[I][r];
+  if (!DUAL && !LIKE && NP == 128) {  // R 1 (k_update128)
+    double rs = 0.0;
+#pragma unroll
+    for (int I = 0; I < NB; ++I) rs += (f[I][0] + f[I][1]) + (f[I][2] + f[I][3]);
+    rs = sum_xor32(sum_xor16(rs));
+    if (lr == 0) Vz[16 * J + lc] = rs;
+  }
   lds_barrier();
   if (tid < NP) {
     double nv = 0.0;
@@ -727,6 +734,8 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     const double ar = S.c[0][tid], vr = S.c[1][tid];
     Vz[NP + tid] = ar;
     Vz[2 * NP + tid] = DUAL ? vr : vr / sqrt(nv);
+    // R v = 1 / |M^1/2 1|
+    if (!DUAL && !LIKE && NP == 128) Vz[3 * NP + tid] = tid < N ? 1.0 / sqrt(nv) : 0.0;
     if (ampl && tid < N) ampl[(size_t)z * N + tid] = ar;
     if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
   }
@@ -1571,6 +1580,61 @@ __global__ __launch_bounds__(256) void k_yyt(int64_t z0, const int32_t* __restri
   }
 }
 
+// R 1 and R v in slots 0 and 3 of vec, as k_func leaves them at NP = 128 (R is
+// symmetric: a thread per column).
+template <int NP, typename TR>
+__global__ __launch_bounds__(NP) void k_row_sums(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                 const int64_t* __restrict__ sel_ptr,
+                                                 const double* __restrict__ ymat, double* vec) {
+  const int zl = blockIdx.x, c = threadIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  if (z < 0 || sel_ptr[z + 1] == sel_ptr[z]) return;
+  const TR* R = reinterpret_cast<const TR*>(ymat + (size_t)zl * NP * NP);
+  double* Vz = vec + (size_t)zl * 4 * NP;
+  double s1 = 0.0, sv = 0.0;
+  for (int s = 0; s < N; ++s) {
+    const double x = (double)R[(size_t)s * NP + c];
+    s1 += x;
+    sv = fma(x, Vz[2 * NP + s], sv);
+  }
+  Vz[c] = s1;
+  Vz[3 * NP + c] = sv;
+}
+
+// What Omega adds to the rows of R (OmegaRow), from R 1, R v and row N - 1 of R: p
+// and q in place of the first two, row N - 1 of (R Omega)^T in that of the last.
+template <int NP, typename TR>
+__global__ __launch_bounds__(NP) void k_omega_rows(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                   const int64_t* __restrict__ sel_ptr, double* ymat,
+                                                   double* vec) {
+  __shared__ double red[NP / 64];
+  const int zl = blockIdx.x, c = threadIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  if (z < 0 || sel_ptr[z + 1] == sel_ptr[z]) return;
+  TR* last = reinterpret_cast<TR*>(ymat + (size_t)zl * NP * NP) + (size_t)(N - 1) * NP + c;
+  double* Vz = vec + (size_t)zl * 4 * NP;
+  const double r1 = Vz[c], kv = Vz[3 * NP + c], rN = (double)*last, vN = Vz[2 * NP + N - 1];
+  const double s = wave_sum_fast(c < N - 1 ? Vz[2 * NP + c] : 0.0);
+  if ((c & 63) == 0) red[c >> 6] = s;
+  __syncthreads();
+  double sv = 0.0;
+#pragma unroll
+  for (int w = 0; w < NP / 64; ++w) sv += red[w];
+  const OmegaRow o = omega_row(N, kv, r1, rN, vN, sv);
+  Vz[c] = o.p;
+  Vz[3 * NP + c] = o.q;
+  *last = (TR)(o.p + o.l);
+}
+
+void launch_omega_rows128(const ChunkArgs& A, hipStream_t st) {
+  if (A.prec == 1)
+    hipLaunchKernelGGL((k_omega_rows<128, float>), dim3(A.nzc), dim3(128), 0, st, A.z0, A.zorder, A.N,
+                       A.sel_ptr, A.ymat, A.vec);
+  else
+    hipLaunchKernelGGL((k_omega_rows<128, double>), dim3(A.nzc), dim3(128), 0, st, A.z0, A.zorder, A.N,
+                       A.sel_ptr, A.ymat, A.vec);
+}
+
 // The reduction (wide256.hip) and the functions of T for a chunk at NP = 64
 // or 128 (dual: the observation-space zones).
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
@@ -1630,6 +1694,13 @@ void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {
   else
     OAK_YYT(128, double);
 #undef OAK_YYT
+  if (NP == 64 || A.mode == 2) return;
+  if (A.prec == 1)
+    hipLaunchKernelGGL((k_row_sums<128, float>), g, dim3(128), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                       A.ymat, A.vec);
+  else
+    hipLaunchKernelGGL((k_row_sums<128, double>), g, dim3(128), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                       A.ymat, A.vec);
 }
 
 }  // namespace oakg

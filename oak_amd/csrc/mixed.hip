@@ -5,7 +5,6 @@
 // eigenvalue functions (1+lambda)^-1 and (1+lambda)^-1/2, the transform T,
 // the innovation scaling and the accumulation of S^T R^-1 S stay in FP64.
 //
-//   k_state_mean_f32   xbar (FP64 sums of FP32 members)
 //   k_spmm_obs<float>  HE = H E + Hshift (FP64 accumulation)
 //   k_obs_anom_f32     HS = (HE - ybar)/sqrt(N-1) stored FP32, innov/rho FP64
 //   k_gram<NP, float>  (analysis.hip / analysis128.hip) M = I + S^T diag(r) S
@@ -17,7 +16,7 @@
 //                      spread (T ~ I); with |C| up to ~1e5 (precise SSH
 //                      observations) that is ~1e-3 of the spread.  Rounding
 //                      S itself perturbs those directions only at second order.
-//   update             (update.hip for N <= 64; k_xform128f for NP = 128)
+//   update             (update.hip for N <= 128)
 //                      Ea = xa + sqrt(N-1) infl (Sf T) on v_mfma_f32_16x16x4f32
 //                      with T rounded to FP32; xa = xbar + clamp(Sf a) in FP64
 //                      (the FP32 sum of N terms Sf_k a_k cancels strongly)
@@ -26,35 +25,6 @@
 #include "spmm.hpp"
 
 namespace oakg {
-
-__global__ void k_state_mean_f32(int64_t n, int N, const float* __restrict__ E, int64_t ld,
-                                 double* __restrict__ xbar) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0;
-  for (int k = 0; k < N; ++k) s += (double)E[i + (int64_t)k * ld];
-  xbar[i] = s / N;
-}
-
-// The same with four consecutive elements per thread (16-byte loads; E 16-byte
-// aligned, ld and n multiples of 4): a quarter of the load instructions, the
-// same sums.
-__global__ void k_state_mean_f32x4(int64_t n4, int N, const float4* __restrict__ E4, int64_t ld4,
-                                   double* __restrict__ xbar) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n4) return;
-  double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  for (int k = 0; k < N; ++k) {
-    const float4 v = E4[i + (int64_t)k * ld4];
-    s0 += (double)v.x;
-    s1 += (double)v.y;
-    s2 += (double)v.z;
-    s3 += (double)v.w;
-  }
-  double2* x2 = reinterpret_cast<double2*>(xbar + 4 * i);
-  x2[0] = make_double2(s0 / N, s1 / N);
-  x2[1] = make_double2(s2 / N, s3 / N);
-}
 
 template <int NP, int TR>
 __global__ __launch_bounds__(256) void k_obs_anom_f32(int64_t m, int N, const double* __restrict__ HEc,
@@ -101,14 +71,6 @@ static inline unsigned nblk32(int64_t n, int b) { return (unsigned)((n + b - 1) 
 
 template <int NP>
 static void prep_ens_f32_t(const PrepEnsArgs& A, hipStream_t st) {
-  if (A.xbar) {  // NULL: observation side only (the report)
-    if ((uintptr_t)A.E32 % 16 == 0 && A.ldE % 4 == 0 && A.n % 4 == 0)
-      hipLaunchKernelGGL(k_state_mean_f32x4, dim3(nblk32(A.n / 4, 256)), dim3(256), 0, st, A.n / 4,
-                         A.N, reinterpret_cast<const float4*>(A.E32), A.ldE / 4, A.xbar);
-    else
-      hipLaunchKernelGGL(k_state_mean_f32, dim3(nblk32(A.n, 256)), dim3(256), 0, st, A.n, A.N,
-                         A.E32, A.ldE, A.xbar);
-  }
   if (A.m == 0) return;
   hipLaunchKernelGGL(k_spmm_obs<float>, dim3(spmm_blocks(A.m, A.N)), dim3(256), 0, st, A.m, A.n, A.N,
                      A.row_ptr, A.col, A.val, A.E32, A.ldE, A.Hshift32, A.HEc, A.err);

@@ -1,4 +1,4 @@
-// The update of a zone's rows for N <= 64:
+// The update of a zone's rows for N <= 128:
 //   MODE 0 (locAnalysis): xa = xf + Sf a, Sa = Sf T   (rrsqrt.F90:151,185,463)
 //   MODE 1 (ensemble): Sf = (E - xbar)/sqrt(N-1) with xbar the members' mean;
 //     xa = xbar + clamp(Sf a); Ea = xa + sqrt(N-1) (inflation Sf T)
@@ -32,6 +32,30 @@ __device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// The lane's members k(q) = 8 (q / 2) + 2 kk + q % 2 of a row, those past N
+// replaced by the first; the addresses are formed as they are needed (all at
+// once they spill), and the values made opaque, so that their conversions for
+// the mean are not kept for the product.
+template <int Q, typename TE>
+__device__ __forceinline__ void load_members(TE (&b)[Q], const TE* S, int64_t row, int64_t ldS, int kk,
+                                             int N) {
+  const TE* p = S + row + (int64_t)(2 * kk) * ldS;
+  const TE* first = S + row;
+#pragma unroll
+  for (int q = 0; q < Q; q += 2) {
+    const int k = 4 * q + 2 * kk;
+    b[q] = *(k < N ? p : first);
+    b[q + 1] = *(k + 1 < N ? p + ldS : first);
+    p += 8 * ldS;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <int Q, typename TE>
+__device__ __forceinline__ void opaque(TE (&b)[Q]) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(b[q]));
+}
+
 // What the rows of a strip share: the row's mean (or xf), the clamp and the
 // column of the increment.  b: the lane's members k(q) of row `row`, replaced
 // by the anomalies; as: a (MODE 0) or a / sqrt(N-1).  Returns xa.
@@ -45,11 +69,13 @@ __device__ __forceinline__ double strip_head(TE (&b)[Q], int N, K k, As as, bool
 #pragma unroll
     for (int q = 0; q < Q; ++q) x0 += k(q) < N ? (double)b[q] : 0.0;
     x0 = sum_xor32(sum_xor16(x0)) / N;
+    opaque(b);
   } else {
     x0 = X0[row];
   }
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
+    if (q % 4 == 0) asm volatile("" ::: "memory");  // a piece by piece
     double d = MODE == 1 ? (double)b[q] - x0 : (double)b[q];
     d = rok && k(q) < N ? d : 0.0;
     dx = fma(d, as(q), dx);
@@ -65,10 +91,10 @@ __device__ __forceinline__ double strip_head(TE (&b)[Q], int N, K k, As as, bool
 }
 
 template <int MODE, typename TE>
-__device__ __forceinline__ TE out_value(TE o, double xar, double infl) {
+__device__ __forceinline__ TE out_value(double o, double xar, double infl) {
 #pragma clang fp contract(off)
-  if (MODE == 0) return o;
-  const double d = infl != 1.0 ? infl * (double)o : (double)o;
+  if (MODE == 0) return (TE)o;
+  const double d = infl != 1.0 ? infl * o : o;
   return (TE)(xar + d);
 }
 
@@ -263,6 +289,133 @@ __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* 
   }
 }
 
+// 65 <= N <= 128: R = M^-1/2 (FP32 for FP32 members) from ymat, 32 rows at a time
+// through LDS in two buffers - the whole would leave one workgroup a CU with its
+// loads, products and stores one after another - while each of eight waves keeps
+// a strip of 16 rows; the next rows are in flight during a product, and the
+// four waves on a SIMD belong to two workgroups.  The product is with R; row k of T
+// is row k of R plus p_k + q_k v (OmegaRow, in slots 0 and 3 of vec), so a row of
+// Sf adds its products with p and q; row N - 1 in ymat is that of T^T already.
+// 64 800 zones of 121 rows, N = 128: 8.6 ms FP64, 4.15 FP32 (T whole in LDS, and a
+// pass for the mean: 9.3 + 1.35 and 4.85 + 0.7).  Omega on the way to LDS cost 0.7 to
+// 1.2 ms more, in k_func's registers 3.4 ms of spills there.
+template <int MODE, typename TE>
+__global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                      const int64_t* __restrict__ sel_ptr,
+                                                      const int64_t* __restrict__ zone_ptr,
+                                                      const double* __restrict__ ymat,
+                                                      const double* __restrict__ vec,
+                                                      const double* __restrict__ X0,
+                                                      const TE* __restrict__ S, int64_t ldS,
+                                                      double* __restrict__ xa, TE* __restrict__ Out,
+                                                      int64_t ldO, double scaling, double infl,
+                                                      double maxcorr,
+                                                      const double* __restrict__ maxcorr_v) {
+  constexpr int NP = 128, Q = NP / 4, CB = 32, LD = sizeof(TE) == 4 ? NP + 4 : NP + 2;
+  typedef TE TE2 __attribute__((ext_vector_type(2)));
+  typedef TE TEV __attribute__((ext_vector_type(16 / sizeof(TE))));
+  constexpr int EV = 16 / sizeof(TE), NV = 8 / EV;  // 16-byte pieces of a thread's 8 entries
+  __shared__ __attribute__((aligned(16))) TE L[2][CB * LD];
+  __shared__ __attribute__((aligned(16))) double as[NP], p[NP], q[NP], v[NP];
+  const int zl = blockIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  const int64_t i0 = zone_ptr[z], sz = zone_ptr[z + 1] - i0;
+  if (sz <= 0) return;
+  const int tid = threadIdx.x;
+  const bool active = sel_ptr[z + 1] > sel_ptr[z];  // else T = I, a = 0
+  const TE* X = reinterpret_cast<const TE*>(ymat + (size_t)zl * NP * NP);
+  const double* Vz = vec + (size_t)zl * 4 * NP;
+  if (tid < NP) {
+    const double a = Vz[NP + tid];
+    as[tid] = MODE == 1 ? a / scaling : a;
+    p[tid] = active ? Vz[tid] : 0.0;
+    q[tid] = active ? Vz[3 * NP + tid] : 0.0;
+    v[tid] = active ? Vz[2 * NP + tid] : 0.0;
+  }
+  // thread t moves entries 8 (t % 16) .. + 7 of row t / 16 of a block
+  TEV st[NV];
+  auto fetch = [&](int h, int t) {
+    const int sr = t >> 4, sc = 8 * (t & 15);
+#pragma unroll
+    for (int w = 0; w < NV; ++w)
+      st[w] = *reinterpret_cast<const TEV*>(X + (size_t)(CB * h + sr) * NP + sc + EV * w);
+    if (!active)
+#pragma unroll
+      for (int w = 0; w < NV; ++w)
+#pragma unroll
+        for (int i = 0; i < EV; ++i) st[w][i] = CB * h + sr == sc + EV * w + i ? (TE)1 : (TE)0;
+  };
+  auto put = [&](int h, int t) {
+    const int sr = t >> 4, sc = 8 * (t & 15);
+#pragma unroll
+    for (int w = 0; w < NV; ++w) *reinterpret_cast<TEV*>(L[h & 1] + sr * LD + sc + EV * w) = st[w];
+  };
+  const int nh = (N + CB - 1) / CB;
+  for (int64_t r0 = 0; r0 < sz; r0 += 128) {
+    // the thread index opaque in each pass: loads, addresses and predicates made
+    // from it would else be formed ahead of the loop, and spill
+    int tp = threadIdx.x;
+    asm volatile("" : "+v"(tp));
+    const int wave = __builtin_amdgcn_readfirstlane(tp >> 6), li = tp & 15, kk = (tp >> 4) & 3;
+    auto k_of = [&](int q) { return 8 * (q >> 1) + 2 * kk + (q & 1); };
+    const int64_t rb = r0 + 16 * wave;
+    const bool rok = rb + li < sz;
+    const int64_t row = i0 + (rok ? rb + li : 0);
+    TE b[Q];
+    if (rb < sz) load_members(b, S, row, ldS, kk, N);
+    fetch(0, tp);
+    put(0, tp);
+    lds_barrier();
+    double xar = 0.0, gp = 0.0, gq = 0.0;
+    if (rb < sz) {
+      xar = strip_head<Q, MODE>(b, N, k_of, [&](int q) { return as[k_of(q)]; }, rok, row, X0, maxcorr,
+                                maxcorr_v);
+      if (MODE == 0 && rok && kk == 0) xa[row] = xar;
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (i % 4 == 0) asm volatile("" ::: "memory");  // the vectors piece by piece
+        gp = fma((double)b[i], p[k_of(i)], gp);
+        gq = fma((double)b[i], q[k_of(i)], gq);
+      }
+      gp = sum_xor32(sum_xor16(gp));
+      gq = sum_xor32(sum_xor16(gq));
+      opaque(b);
+    }
+#pragma unroll 1
+    for (int h = 0; h < nh; ++h) {
+      int tq = threadIdx.x;
+      asm volatile("" : "+v"(tq));
+      const int li = tq & 15, kk = (tq >> 4) & 3;
+      if (h + 1 < nh) fetch(h + 1, tq);
+      if (rb < sz) {
+        const TE* lt = L[h & 1] + li * LD + 2 * kk;
+        vec4<TE> acc[2] = {};
+#pragma unroll
+        for (int g = 0; g < Q / 2; ++g) {
+          asm volatile("" ::: "memory");  // the reads of later pairs stay below
+          TE2 A[2];
+#pragma unroll
+          for (int J = 0; J < 2; ++J) A[J] = *reinterpret_cast<const TE2*>(lt + 16 * J * LD + 8 * g);
+#pragma unroll
+          for (int J = 0; J < 2; ++J) acc[J] = mfma(A[J].x, b[2 * g], acc[J]);
+#pragma unroll
+          for (int J = 0; J < 2; ++J) acc[J] = mfma(A[J].y, b[2 * g + 1], acc[J]);
+        }
+#pragma unroll
+        for (int J = 0; J < 2; ++J)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int col = CB * h + 16 * J + drow<TE>(kk, r);
+            const double y = (double)acc[J][r] + (col < N - 1 ? fma(gq, v[col], gp) : 0.0);
+            if (rok && col < N) Out[row + (int64_t)col * ldO] = out_value<MODE, TE>(y, xar, infl);
+          }
+      }
+      if (h + 1 < nh) put(h + 1, tq);
+      lds_barrier();
+    }
+  }
+}
+
 // Waves per zone at N <= 32: one for every 32 rows of a mean zone, at most
 // the four of a workgroup (a wave reads the whole of T).
 void launch_update(int NP, const ChunkArgs& A, hipStream_t st) {
@@ -282,6 +435,11 @@ void launch_update(int NP, const ChunkArgs& A, hipStream_t st) {
       break;                                                                                          \
     case 64:                                                                                          \
       hipLaunchKernelGGL((k_update64<MODE, TE>), dim3(A.nzc), blk, 0, st, A.z0, A.zorder, A.N,        \
+                         A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,    \
+                         A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                  \
+      break;                                                                                          \
+    case 128:                                                                                         \
+      hipLaunchKernelGGL((k_update128<MODE, TE>), dim3(A.nzc), dim3(512), 0, st, A.z0, A.zorder, A.N, \
                          A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,    \
                          A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                  \
       break;                                                                                          \

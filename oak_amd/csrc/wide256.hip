@@ -668,38 +668,12 @@ __global__ __launch_bounds__(256, 2) void k_qapply256(int nzc, int64_t z0,
         Y[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = f[I][r];
     return;
   }
-  // X = (R Omega)^T from the columns of the symmetric R (k_tmat's formula):
-  // column c = 16 J + lc, rows s = 16 I + lr + 4 r
   lds_barrier();
-  const double wN = 1.0 / sqrt((double)N), vN = S.v[N - 1], sgv = vN >= 0 ? 1.0 : -1.0;
-  const double alv = -1.0 / (fabs(vN) + 1.0), alw = -1.0 / (wN + 1.0);
-  double vw = 0.0, u1 = 0.0, u2 = 0.0, u0 = 0.0;
+  omega_columns(f, N, S.v, [&](int I, int r) { return 16 * I + lr + 4 * r; });
 #pragma unroll
   for (int I = 0; I < NB; ++I)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int s = 16 * I + lr + 4 * r;
-      const double vs = S.v[s];
-      vw += s < N - 1 ? vs : 0.0;
-      u1 = fma(f[I][r], vs, u1);
-      u2 += s < N - 1 ? f[I][r] : 0.0;
-      u0 += s == N - 1 ? f[I][r] : 0.0;
-    }
-  vw = wN * sum_xor32(sum_xor16(vw));
-  u0 = sum_xor32(sum_xor16(u0));
-  u1 = sum_xor32(sum_xor16(u1));
-  u2 = wN * sum_xor32(sum_xor16(u2));
-  const double u3 = fma(sgv, u0, u1);
-  const double c1 = u1 * wN, c2 = alw * u2 + alv * alw * vw * u3, c3 = alv * u3;
-#pragma unroll
-  for (int I = 0; I < NB; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int s = 16 * I + lr + 4 * r;
-      const double zw = s == N - 1 ? wN + 1.0 : wN, vt = s < N - 1 ? S.v[s] : 0.0;
-      const double x = s == N - 1 ? 0.0 : f[I][r];
-      X[(size_t)s * NP + 16 * J + lc] = s < N ? x + (c1 + c2 * zw + c3 * vt) : x;
-    }
+    for (int r = 0; r < 4; ++r) X[(size_t)(16 * I + lr + 4 * r) * NP + 16 * J + lc] = f[I][r];
 }
 
 // ---------------------------------------------------------------------------
