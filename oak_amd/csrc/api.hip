@@ -475,8 +475,12 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   const size_t per_zone = sizeof(double) * ((size_t)(NP == 256 ? 3 : 2) * MP * MP + 6 * MP) +
                           (dual_lt ? sizeof(double) * ((size_t)2 * PD * PD + 4 * PD) : 0);
   const size_t budget = c->ws_budget;
-  // one kernel a zone has nothing to overlap with the next chunk's
-  const int nslot = (!c->timing && !c->arena && !chol && nz >= 4096) ? c->tune_slots : 1;
+  // Chunks on several streams gain 2 to 6% where the loop takes a millisecond or
+  // more and cost their launches where it takes less (three slots against one:
+  // 4096 zones of N = 16 230 and 184 us, 51 200 zones 800 and 837; 5490 zones of N =
+  // 40 1517 and 1582); one kernel a zone has nothing to overlap with the next's
+  const bool slots = !c->timing && !c->arena && !chol && nz >= 4096 && nz * NP >= ((int64_t)1 << 18);
+  const int nslot = slots ? c->tune_slots : 1;
   int64_t zc = std::max<int64_t>(1, (int64_t)(budget / (per_zone * nslot)));
   zc = std::min<int64_t>(zc, 1 << 20);
   if (nslot > 1) zc = std::min<int64_t>(zc, (nz + nslot - 1) / nslot);  // a chunk per slot
@@ -749,7 +753,6 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
 
   if (c->timing) c->timer.mark(PH_SELECT);
   SelDev sel{};
-  int64_t total = 0;
   if (csr) {
     // caller-supplied selection
     const int64_t* dptr = stage(c, Workspace::U_SEL_PTR, sel_ptr_in, nz + 1, dev);
@@ -772,9 +775,8 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
     sel.ptr = dptr;
     sel.idx = stage(c, Workspace::U_SEL_IDX, sel_idx_in, tot, dev);
     sel.w = stage(c, Workspace::U_SEL_W, sel_w_in, tot, dev);
-    total = tot;
   } else {
-    check(c, run_selection(c->ws, g.zd, g.od, localise, c->stream, c->d_err, c->pinned, sel, &total),
+    check(c, run_selection(c->ws, g.zd, g.od, localise, c->stream, c->d_err, c->pinned, sel, nullptr),
           "selection");
   }
 
@@ -823,7 +825,6 @@ int local_analysis_impl(oakg_ctx* c, const oakg_zones* zones, int64_t nzones_csr
   float ms = 0;
   if (!c->arena) (void)hipEventElapsedTime(&ms, c->ev_t0, c->ev_t1);
   collect_stats(c, nz, sel.ptr, ms);
-  (void)total;
   if (!dev) {
     check(c, hipMemcpy(xa, dxa, sizeof(double) * n, hipMemcpyDeviceToHost), "D2H xa");
     copy_out_2d(c, Sa, ldSa, dSa, n, N, "D2H Sa");
@@ -882,8 +883,7 @@ int local_nll_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, in
   check(c, hipGetLastError(), "prep");
   if (c->timing) c->timer.mark(PH_SELECT);
   SelDev sel{};
-  int64_t total = 0;
-  check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, &total), "selection");
+  check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, nullptr), "selection");
   int32_t* sweeps = (int32_t*)wsget(c, Workspace::SWEEPS, sizeof(int32_t) * std::max<int64_t>(nz, 1));
   if (!sweeps) check(c, hipErrorOutOfMemory, "workspace");
   ChunkArgs A{};
@@ -922,7 +922,6 @@ int local_nll_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, in
   if (nll_zone && nz > 0) check(c, hipMemcpy(nll_zone, Jz, sizeof(double) * nz, k), "copy nll");
   if (!dev && m > 0)
     check(c, hipMemcpy(grad_log_sigma, gth, sizeof(double) * m, hipMemcpyDeviceToHost), "D2H");
-  (void)total;
   return OAKG_OK;
 }
 
@@ -1018,8 +1017,7 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     check(c, hipGetLastError(), "prep");
     if (c->timing) c->timer.mark(PH_SELECT);
     SelDev sel{};
-    int64_t total = 0;
-    check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, &total), "selection");
+    check(c, run_selection(c->ws, g.zd, g.od, 1, c->stream, c->d_err, c->pinned, sel, nullptr), "selection");
     T* dEa = dev ? Ea : (T*)wsget(c, Workspace::OUT_S, sizeof(T) * std::max<int64_t>(n, 1) * N);
     const int64_t ld_ea = dev ? ldEa : n;
     int32_t* sweeps = (int32_t*)wsget(c, Workspace::SWEEPS, sizeof(int32_t) * std::max<int64_t>(nz, 1));
