@@ -74,12 +74,17 @@ inline dim3 zone_parts(int parts, int nzc) { return dim3((unsigned)((nzc + 7) / 
 template <int NP>
 struct TriLowerLds {
   static constexpr int PR = (tri_rx(NP - 1) + 2) & ~1;  // padded length of a row vector
+  // distance of the slots of part: a wave writes its column sums into the slots
+  // of 8 and more consecutive tile rows at the same place, so an odd distance puts
+  // these on different banks (at 144 for NP = 128 and 288 for 256, multiples of 16,
+  // conflicts were half of all LDS cycles)
+  static constexpr int PS = NP == 64 ? 77 : tri_rx(NP - 1) + 3;
   static constexpr int NW = NP == 256 ? 8 : (NP == 128 ? 2 : 1);  // waves of the workgroup
   static constexpr int NRW = NP / 64;                  // row waves
   double colw[NW][PR];     // each wave's copy of v
   double pub[2][PR];       // column i+1 before step i's update (double-buffered)
   double pw[2][PR];        // p (double-buffered)
-  double part[NP / 8][PR]; // slot s of row r: its partial sum of A v
+  double part[NP / 8][PS]; // slot s of row r: its partial sum of A v
   double l0[NP][9];        // columns 0..7 of every row (steps 0..6)
   double hp[NRW][8];       // the row waves' shares of (A v)_0..7 (steps 0..6)
   double red[2][NRW];      // the row waves' shares of v^T p (double-buffered)
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   const int64_t zstride = A.zstride;
   const int ldm = A.ldm, ldv = A.ldv;
   using L = TriLowerLds<NP>;
-  constexpr int NH = NP / 64, PR = L::PR, H = NP / 2, NB = NP / 8;
+  constexpr int NH = NP / 64, H = NP / 2, NB = NP / 8;
   constexpr int NT = (NB - 1) * NB / 2;  // register tiles (tile columns 1..NB-1)
   constexpr int BS = 64 * L::NW;         // threads
   __shared__ L S;
@@ -154,7 +159,7 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
 #pragma unroll
     for (int c = 0; c < 8; ++c) S.l0[row][c] = M[(size_t)row * ldm + c];
   }
-  for (int e = t; e < NB * PR; e += BS) (&S.part[0][0])[e] = 0.0;
+  for (int e = t; e < NB * L::PS; e += BS) (&S.part[0][0])[e] = 0.0;
   double x[NH];
 #pragma unroll
   for (int h = 0; h < NH; ++h) x[h] = M[(size_t)(lane + 64 * h) * ldm];  // column 0 (M symmetric)
@@ -197,8 +202,24 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
         const int r = lane + 64 * h;
         if (r >= i + 2) s = fma(x[h], x[h], s);
       }
-      s = wave_sum_d(s);
       const int ia = i + 1;
+      // with it x^T u over the same rows (v^T u = scal x^T u + u_{i+1}): the
+      // sums' latencies overlap
+      double su[NV];
+      if (has_u) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+          su[q] = 0.0;
+#pragma unroll
+          for (int h = 0; h < NH; ++h)
+            if (lane + 64 * h >= i + 2) su[q] = fma(x[h], u[q][h], su[q]);
+        }
+        s = wave_sum_d(s);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) su[q] = wave_sum_d(su[q]);
+      } else {
+        s = wave_sum_d(s);
+      }
       const double alpha = readlane_d(pick(ia >> 6), ia & 63);
       const double di = readlane_d(pick(i >> 6), i & 63);
       beta = alpha;
@@ -242,23 +263,24 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
       if (has_u) {
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
-          double su = 0.0;
+          double ua = u[q][0];
 #pragma unroll
-          for (int h = 0; h < NH; ++h) su = fma(v[h], u[q][h], su);
-          su = tau * wave_sum_d(su);
+          for (int h = 1; h < NH; ++h) ua = (ia >> 6) == h ? u[q][h] : ua;
+          const double f = -tau * fma(scal, su[q], readlane_d(ua, ia & 63));
 #pragma unroll
-          for (int h = 0; h < NH; ++h) u[q][h] = fma(-su, v[h], u[q][h]);
+          for (int h = 0; h < NH; ++h) u[q][h] = fma(f, v[h], u[q][h]);
         }
       }
     }
-    // partial sums of the tiles (zeros from a tile outside the trailing block)
+    // partial sums of the tiles (zeros, once, from a tile that left the trailing
+    // block)
     const bool act = own && (c0 + 7 > i);
     double vR[8], vC[8];
 #pragma unroll
     for (int jj = 0; jj < 8; ++jj) vC[jj] = col[C0 + jj];
 #pragma unroll
     for (int ii = 0; ii < 8; ++ii) vR[ii] = col[R0 + ii];
-    if (own) {
+    if (own && c0 + 8 > i) {
 #pragma unroll
       for (int ii = 0; ii < 8; ++ii) {
         double ps = 0.0;
@@ -318,11 +340,15 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
     // p = tau A v and the row waves' shares of v^T p
     if (row >= 0) {
       const int rowx = tri_rx(row);
-      double s4[4];
+      double s4[4] = {};
+      // the slots of a row of the trailing block below the first live tile
+      // column are zeros
 #pragma unroll
-      for (int q = 0; q < 4; ++q) s4[q] = S.part[q][rowx];
+      for (int q0 = 0; q0 < NB; q0 += 4)
+        if (8 * q0 + 32 > i) {
 #pragma unroll
-      for (int q = 4; q < NB; ++q) s4[q & 3] += S.part[q][rowx];
+          for (int q = 0; q < 4; ++q) s4[q] += S.part[q0 + q][rowx];
+        }
       double s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
       if (i < 7 && row < 8) {
         if constexpr (NP == 256)
