@@ -159,6 +159,32 @@ void launch_gram_blocks(int NP, const ChunkArgs& A, hipStream_t st);
 // NP = 256 (wide256.hip): the whole chunk
 void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm);
 void launch_pole256(const ChunkArgs& A, hipStream_t st);
+// A Householder reduction (wide256.hip, tridiag64.hip).  zstride, ldm and ldv: the
+// distance between the zones' matrices and the leading dimensions of M and of
+// the reflector rows (NP for a zone's own block; a trailing block sits inside
+// the zone's reflector block).
+// vecs (NULL: none): the zone's vectors (stride zvec) to which the reflectors
+// are applied as they are formed, entries 0 .. NP-1 (b, giving Q^T b) and
+// c1 .. c1 + NP-1 (1_N for ones >= 0: row r < ones is 1; else as found).
+struct TriArgs {
+  int64_t z0;
+  const int32_t* zorder;
+  const int64_t* sel_ptr;
+  const double* mat;
+  double* qmat;
+  int64_t zstride;
+  int ldm, ldv;
+  // d_i of zone zl at dvec[zl dz + d0 + i dstep], e_i at evec[zl dz + e0 + i dstep]
+  double *dvec, *evec;
+  int64_t dz, d0, e0, dstep;
+  double* vecs;
+  int zvec, c1, ones;
+  // k_tridiag64: order of the matrix (the rows from it on are the identity's); -1:
+  // the zone's observation count
+  int n;
+};
+// up to 64 rows (tridiag64.hip): every step
+void launch_tridiag64(const TriArgs& T, int nzc, hipStream_t st);
 // Householder reductions on the lower triangle (wide256.hip): d, e, the
 // reflectors, and Q^T b and Q^T 1_N (ones = N; -1: the vector in slot 2) in
 // place of b and slot 2 of vec

@@ -9,7 +9,7 @@
 //                  register tiles over 512 threads, one workgroup per zone:
 //                  496 tiles hold columns 8..255, and columns 0..7 sit in
 //                  LDS for the seven steps that change them; steps 128..253
-//                  by k_tridiag_lower<128> and <64>.
+//                  by k_tridiag_lower<128> and k_tridiag64.
 //   funcm.hip      k_pole256: the rational approximation's solves, a and v.
 //   k_qapply256    Q F, then Q (Q F)^T = M^-1/2 and Omega, the reflectors in
 //                  compact-WY blocks on MFMA, four workgroups per zone, one
@@ -18,8 +18,8 @@
 //                  zone (one 32-column block of T each) on one XCD.
 // The operations are those of the N <= 128 path (rrsqrt.F90:100-190 and the
 // post-processing of assimilation.F90:3299-3363); only the split of the work
-// and the order of the partial sums differ.  k_tridiag_lower<128> and <64> also
-// serve N = 65..128, k_tridiag_lower<64> alone N = 33..64.
+// and the order of the partial sums differ.  k_tridiag_lower<128> and k_tridiag64
+// also serve N = 65..128, k_tridiag64 alone N = 33..64.
 #include <algorithm>
 
 #include "analysis.hpp"
@@ -67,7 +67,7 @@ inline dim3 zone_parts(int parts, int nzc) { return dim3((unsigned)((nzc + 7) / 
 // i+1 as it stands before the update is published by its tile column (or
 // the LDS block), and every wave forms its updated value itself.  Two
 // barriers per step.  Steps 0..127 run here; the trailing 128 x 128 block
-// then goes to the NP = 128 and 64 kernels (fewer registers, four and eight
+// then goes to the kernels for 128 and 64 rows (fewer registers, four and twelve
 // zones per CU through the late, latency-bound steps).
 // Output: reflector i in row i of qmat (tau_i in entry i), d and e.
 // ---------------------------------------------------------------------------
@@ -78,8 +78,8 @@ struct TriLowerLds {
   // of 8 and more consecutive tile rows at the same place, so an odd distance puts
   // these on different banks (at 144 for NP = 128 and 288 for 256, multiples of 16,
   // conflicts were half of all LDS cycles)
-  static constexpr int PS = NP == 64 ? 77 : tri_rx(NP - 1) + 3;
-  static constexpr int NW = NP == 256 ? 8 : (NP == 128 ? 2 : 1);  // waves of the workgroup
+  static constexpr int PS = tri_rx(NP - 1) + 3;
+  static constexpr int NW = NP == 256 ? 8 : 2;           // waves of the workgroup
   static constexpr int NRW = NP / 64;                  // row waves
   double colw[NW][PR];     // each wave's copy of v
   double pub[2][PR];       // column i+1 before step i's update (double-buffered)
@@ -90,36 +90,8 @@ struct TriLowerLds {
   double red[2][NRW];      // the row waves' shares of v^T p (double-buffered)
 };
 
-// FULL = false: steps 0 .. NP/2 - 1, then the trailing block is handed on
-// (below); FULL = true: every step, and the trailing 2 x 2 block gives the
-// last two d and the last e (e_{NP-1} is left to the caller).  zstride, ldm
-// and ldv: the distance between the zones' matrices and the leading
-// dimensions of M and of the reflector rows (NP for a zone's own block; the
-// N = 128 trailing block, reduced by k_tridiag_lower<64, true>, sits in rows
-// 64.. of the zone's NP = 128 block).
-// vecs (NULL: none): the zone's vectors (stride zvec) to which the reflectors
-// are applied as they are formed, entries 0 .. NP-1 (b, giving Q^T b) and
-// c1 .. c1 + NP-1 (1_N for ones >= 0: row r < ones is 1; else as found).
-struct TriArgs {
-  int64_t z0;
-  const int32_t* zorder;
-  const int64_t* sel_ptr;
-  const double* mat;
-  double* qmat;
-  int64_t zstride;
-  int ldm, ldv;
-  // d_i of zone zl at dvec[zl dz + d0 + i dstep], e_i at evec[zl dz + e0 + i dstep]
-  double *dvec, *evec;
-  int64_t dz, d0, e0, dstep;
-  double* vecs;
-  int zvec, c1, ones;
-  // FULL: order of the matrix (the rows from it on are the identity's); -1: the
-  // zone's observation count
-  int n;
-};
-
-template <int NP, bool FULL = false>
-__global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tridiag_lower(TriArgs A) {
+template <int NP>
+__global__ __launch_bounds__(NP == 256 ? 512 : 128) void k_tridiag_lower(TriArgs A) {
   const double* __restrict__ mat = A.mat;
   double* __restrict__ qmat = A.qmat;
   const int64_t zstride = A.zstride;
@@ -163,20 +135,15 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   double x[NH];
 #pragma unroll
   for (int h = 0; h < NH; ++h) x[h] = M[(size_t)(lane + 64 * h) * ldm];  // column 0 (M symmetric)
-  // the vectors: vector q in the registers of wave q % NW (one wave: both)
-  constexpr int NV = L::NW > 1 ? 1 : 2;
-  double u[NV][NH];
-  double* uz = A.vecs ? A.vecs + (size_t)zl * A.zvec : nullptr;
+  // the vectors: vector q in the registers of wave q
+  double u[NH];
+  double* uz = A.vecs ? A.vecs + (size_t)zl * A.zvec + (wave ? A.c1 : 0) : nullptr;
   const bool has_u = A.vecs && wave < 2;
   if (has_u) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      const bool second = (NV == 2 ? q : wave) == 1;
-#pragma unroll
-      for (int h = 0; h < NH; ++h) {
-        const int r = lane + 64 * h;
-        u[q][h] = second && A.ones >= 0 ? (r < A.ones ? 1.0 : 0.0) : uz[(second ? A.c1 : 0) + r];
-      }
+    for (int h = 0; h < NH; ++h) {
+      const int r = lane + 64 * h;
+      u[h] = wave && A.ones >= 0 ? (r < A.ones ? 1.0 : 0.0) : uz[r];
     }
   }
   __syncthreads();
@@ -187,8 +154,7 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
     return v;
   };
   double* col = S.colw[wave];
-  const int n = FULL ? (A.n >= 0 ? A.n : (int)(A.sel_ptr[z + 1] - A.sel_ptr[z])) : NP;
-  for (int i = 0; i < (FULL ? n - 2 : H); ++i) {
+  for (int i = 0; i < H; ++i) {
     const int b = i & 1;
     double* pw = S.pw[b];
     double* pub = S.pub[b];
@@ -205,18 +171,13 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
       const int ia = i + 1;
       // with it x^T u over the same rows (v^T u = scal x^T u + u_{i+1}): the
       // sums' latencies overlap
-      double su[NV];
+      double su = 0.0;
       if (has_u) {
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-          su[q] = 0.0;
-#pragma unroll
-          for (int h = 0; h < NH; ++h)
-            if (lane + 64 * h >= i + 2) su[q] = fma(x[h], u[q][h], su[q]);
-        }
+        for (int h = 0; h < NH; ++h)
+          if (lane + 64 * h >= i + 2) su = fma(x[h], u[h], su);
         s = wave_sum_d(s);
-#pragma unroll
-        for (int q = 0; q < NV; ++q) su[q] = wave_sum_d(su[q]);
+        su = wave_sum_d(su);
       } else {
         s = wave_sum_d(s);
       }
@@ -261,15 +222,12 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
         }
       }
       if (has_u) {
+        double ua = u[0];
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-          double ua = u[q][0];
+        for (int h = 1; h < NH; ++h) ua = (ia >> 6) == h ? u[h] : ua;
+        const double f = -tau * fma(scal, su, readlane_d(ua, ia & 63));
 #pragma unroll
-          for (int h = 1; h < NH; ++h) ua = (ia >> 6) == h ? u[q][h] : ua;
-          const double f = -tau * fma(scal, su[q], readlane_d(ua, ia & 63));
-#pragma unroll
-          for (int h = 0; h < NH; ++h) u[q][h] = fma(f, v[h], u[q][h]);
-        }
+        for (int h = 0; h < NH; ++h) u[h] = fma(f, v[h], u[h]);
       }
     }
     // partial sums of the tiles (zeros, once, from a tile that left the trailing
@@ -353,10 +311,8 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
       if (i < 7 && row < 8) {
         if constexpr (NP == 256)
           s = (S.hp[0][row] + S.hp[1][row]) + (S.hp[2][row] + S.hp[3][row]);
-        else if constexpr (NP == 128)
-          s = S.hp[0][row] + S.hp[1][row];
         else
-          s = S.hp[0][row];
+          s = S.hp[0][row] + S.hp[1][row];
       }
       const double pr = row > i ? tau * s : 0.0;
       pw[rowx] = pr;
@@ -367,13 +323,10 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
     lds_barrier();
     // A -= v w^T + w v^T, w = p + K v, K = -tau/2 v^T p
     double vpt;
-    if constexpr (NP == 256) {
+    if constexpr (NP == 256)
       vpt = (S.red[b][0] + S.red[b][1]) + (S.red[b][2] + S.red[b][3]);
-    } else if constexpr (NP == 128) {
+    else
       vpt = S.red[b][0] + S.red[b][1];
-    } else {
-      vpt = S.red[b][0];
-    }
     const double K = -0.5 * tau * vpt;
     if (act) {
       double wC[8];
@@ -414,28 +367,7 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
   // column c - H of rows H..
   if (has_u) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q)
-#pragma unroll
-      for (int h = 0; h < NH; ++h)
-        uz[((NV == 2 ? q : wave) == 1 ? A.c1 : 0) + lane + 64 * h] = u[q][h];
-  }
-  if constexpr (FULL) {
-    // rows n - 2 and n - 1 (x: column n - 2), then the identity's
-    static_assert(!FULL || NP == 64, "one wave: lane r has row r");
-    if (lane == n - 2) dv[lane * A.dstep] = x[0];
-    if (lane == n - 1) {
-      if (n >= 2) ev[(n - 2) * A.dstep] = x[0];
-      if (n <= 8) dv[lane * A.dstep] = S.l0[lane][lane];
-    }
-    if (n > 8 && own && tr == tc && tc == (n - 1) >> 3) {
-      double dn = a[0][0];
-#pragma unroll
-      for (int jj = 1; jj < 8; ++jj) dn = jj == ((n - 1) & 7) ? a[jj][jj] : dn;
-      dv[(n - 1) * A.dstep] = dn;
-    }
-    if (lane >= n) dv[lane * A.dstep] = 1.0;
-    if (lane >= n - 1 && lane < NP - 1) ev[lane * A.dstep] = 0.0;
-    return;
+    for (int h = 0; h < NH; ++h) uz[lane + 64 * h] = u[h];
   }
   constexpr int LDO = NP == 256 ? H : NP;
   if (own && tc >= H / 8) {
@@ -452,8 +384,7 @@ __global__ __launch_bounds__(NP == 256 ? 512 : (NP == 128 ? 128 : 64)) void k_tr
 
 // NP = 128: steps 0..63 on the lower-triangle tiles (two waves, four zones
 // per CU); then the trailing 64 x 64 block (rows 64.., columns 0..63 of the
-// zone's reflector block) in full by k_tridiag_lower<64> (one wave per zone,
-// eight zones per CU): its reflectors go to columns 64..127 of the same rows
+// zone's reflector block) in full by k_tridiag64 (one wave per zone): its reflectors go to columns 64..127 of the same rows
 // (their columns 0..63 keep the block's values, which k_func masks: a
 // reflector is zero up to its own index), its d, e and vector entries to
 // 64..127.  As one kernel on full 8 x 8 tiles (four waves, two zones per CU)
@@ -468,7 +399,7 @@ void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st) {
   T.vecs = A.vec + 64;
   T.ones = -1;
   T.n = ones - 64;
-  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
+  launch_tridiag64(T, A.nzc, st);
 }
 
 // NP = 64 (33 <= N <= 64, and the observation-space zones of N = 128: ones =
@@ -477,7 +408,7 @@ void launch_tridiag_lower128(const ChunkArgs& A, int ones, hipStream_t st) {
 void launch_tridiag_lower64(const ChunkArgs& A, int ones, hipStream_t st) {
   const TriArgs T{A.z0, A.zorder, A.sel_ptr, A.mat, A.ymat, (int64_t)64 * 64, 64, 64,
                   A.dvec, A.evec, 64, 0, 0, 1, A.vec, 4 * 64, 2 * 64, ones, ones};
-  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
+  launch_tridiag64(T, A.nzc, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -841,7 +772,7 @@ void launch_chunk256(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   T.d0 = T.e0 = 192;
   T.vecs = A.vec + 192;
   T.n = std::max(A.N - 192, 0);
-  hipLaunchKernelGGL((k_tridiag_lower<64, true>), dim3(A.nzc), dim3(64), 0, st, T);
+  launch_tridiag64(T, A.nzc, st);
   launch_pole256(A, st);
   const double* tb = A.ymat + 128 * 256;
   hipLaunchKernelGGL(k_qapply256<1>, zone_parts(4, A.nzc), dim3(256), 0, st, A.nzc, A.z0, A.zorder, A.N,
