@@ -238,26 +238,33 @@ __global__ __launch_bounds__(NP == 256 ? 512 : 128) void k_tridiag_lower(TriArgs
     for (int jj = 0; jj < 8; ++jj) vC[jj] = col[C0 + jj];
 #pragma unroll
     for (int ii = 0; ii < 8; ++ii) vR[ii] = col[R0 + ii];
+    // (one branch around all sums: their chains of dependent multiply-adds
+    // interleave)
     if (own && c0 + 8 > i) {
+      if (act) {
+        double ps[8];
 #pragma unroll
-      for (int ii = 0; ii < 8; ++ii) {
-        double ps = 0.0;
-        if (act) {
+        for (int ii = 0; ii < 8; ++ii) ps[ii] = a[ii][0] * vC[0];
 #pragma unroll
-          for (int jj = 0; jj < 8; ++jj) ps = fma(a[ii][jj], vC[jj], ps);
+        for (int jj = 1; jj < 8; ++jj)
+#pragma unroll
+          for (int ii = 0; ii < 8; ++ii) ps[ii] = fma(a[ii][jj], vC[jj], ps[ii]);
+#pragma unroll
+        for (int ii = 0; ii < 8; ++ii) S.part[tc][R0 + ii] = ps[ii];
+        if (tr != tc) {
+          double cs[8];
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) cs[jj] = a[0][jj] * vR[0];
+#pragma unroll
+          for (int ii = 1; ii < 8; ++ii)
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj) cs[jj] = fma(a[ii][jj], vR[ii], cs[jj]);
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) S.part[tr][C0 + jj] = cs[jj];
         }
-        S.part[tc][R0 + ii] = ps;
-      }
-      if (tr != tc) {
+      } else {
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-          double cs = 0.0;
-          if (act) {
-#pragma unroll
-            for (int ii = 0; ii < 8; ++ii) cs = fma(a[ii][jj], vR[ii], cs);
-          }
-          S.part[tr][C0 + jj] = cs;
-        }
+        for (int k = 0; k < 8; ++k) S.part[tc][R0 + k] = S.part[tr][C0 + k] = 0.0;
       }
       // column i+1 before this step's update, from its tile column
       if (tc == ((i + 1) >> 3)) {
