@@ -79,8 +79,10 @@ def flops_model(N, counts, zone_sizes, dual_lt=0):
                                        S^T R^-1 d)
       eig    9 N^3                    (symmetric eigensolve with vectors,
                                        Golub & Van Loan's count for
-                                       tridiagonalisation + QL)
-      trans  N^2 (N + 1) + 10 N^2     (T = Y Y^T Omega: the symmetric
+                                       tridiagonalisation + QL, also
+                                       where the functions come without
+                                       eigenvectors)
+      trans  N^2 (N + 1) + 10 N^2     (T = M^-1/2 Omega: the symmetric
                                        product Y Y^T and Omega applied as its
                                        rank-structured correction; OAK's dense
                                        form, RotateVector + three N x N GEMMs,
@@ -309,9 +311,9 @@ def phase_rooflines(F, phase, mixed, N=128):
     eigensolve (FP64), the transform and update (FP32 MFMA on the mixed path,
     FP64 otherwise)."""
     work = {"gram": F["gram"], "eig": F["eig"], "tmat": F["trans"], "update": F["update"]}
-    if phase["tmat"] == 0.0:  # N > 64: transform and update in one kernel
-        work["update"] += work["tmat"]
-        del work["tmat"]
+    if N <= 128:  # M^-1/2 comes from the eigensolve's kernels
+        phase = dict(phase, eig=phase["eig"] + phase["tmat"])
+        work["eig"] += work.pop("tmat")
     out = {}
     for k, w in work.items():
         if phase[k] <= 0:
@@ -329,43 +331,35 @@ def roofline(F, phase, mixed, eig_name, config, N):
     of the arithmetic it runs on (FP32 MFMA for the mixed contractions, FP64
     otherwise)."""
     work = {"gram": F["gram"], "eig": F["eig"], "tmat": F["trans"], "update": F["update"]}
-    # N > 64: transform and update run in one kernel, booked as the update
-    fused = phase["tmat"] == 0.0
-    if fused:
-        work["update"] += work["tmat"]
+    if N <= 128:  # M^-1/2 comes from the eigensolve's kernels
+        phase = dict(phase, eig=phase["eig"] + phase["tmat"])
+        work["eig"] += work.pop("tmat")
     kern = max(work, key=lambda k: phase[k])
-    gk = "k_gram256" if N > 128 else ("k_gram128" if N > 64 else "k_gram")
+    gk = "k_gram_blocks<%d>" % (256 if N > 128 else 128) if N > 64 else "k_gram"
+    uk = "k_update128" if N > 64 else ("k_update64" if N > 32 else "k_update_small")
     names = {
-        "gram": ("%s<float> (S^T R^-1 S from FP32 S, v_mfma_f64_16x16x4f64)" % gk if mixed else
+        "gram": ("%s (S^T R^-1 S from FP32 S, v_mfma_f64_16x16x4f64)" % gk if mixed else
                  "%s (S^T R^-1 S, v_mfma_f64_16x16x4f64)" % gk),
         "eig": eig_name,
-        "tmat": "k_tmat (T = Y Y^T Omega, v_mfma_f64_16x16x4f64)",
-        "update": ("k_update_f32 (Ea = xa + A' W, v_mfma_f32_16x16x4f32)" if mixed else
-                   "k_update (Ea = xa + A' W, v_mfma_f64_16x16x4f64)"),
+        "update": (uk + " (Ea = xa + A' T, v_mfma_f32_16x16x4f32)" if mixed else
+                   uk + " (Ea = xa + A' T, v_mfma_f64_16x16x4f64)"),
     }
     if N > 128:
-        names["tmat"] = "k_tmat256 (T = Y Y^T Omega, v_mfma_f64_16x16x4f64)"
+        names["tmat"] = "k_qapply256<2> (T = Q (Q F)^T Omega, v_mfma_f64_16x16x4f64)"
         names["update"] = ("k_update256 (Ea = xa + A' T from FP32 members on "
                            "v_mfma_f64_16x16x4f64)" if mixed else
                            "k_update256 (Ea = xa + A' T, v_mfma_f64_16x16x4f64)")
-    if fused:
-        names["update"] = ("k_xform128f (T = Y Y^T Omega in LDS on v_mfma_f32_16x16x4f32, then "
-                           "Ea = xa + A' T on v_mfma_f32_16x16x4f32)" if mixed else
-                           "k_xform128 (T = Y Y^T Omega in LDS on v_mfma_f64_16x16x4f64, then "
-                           "Ea = xa + A' T on v_mfma_f64_16x16x4f64)")
     peak = PEAK_FP32_MFMA if (mixed and N <= 128 and kern == "update") else PEAK_FP64
     ach = work[kern] / (phase[kern] * 1e-3)
     return {"bound": "mfma", "kernel": names[kern], "achieved": ach / 1e12, "peak": peak / 1e12,
             "unit": "TFLOP/s", "frac": ach / peak, "traffic": phase_traffic(kern, mixed, config)}
 
 
-# the kernels of each phase at N > 64 (the observation-space bucket's
-# kernels and the Jacobi fallback passes included)
-PHASE_KERNELS = {"eig": ["k_tridiag", "k_tridiag_lower", "k_formq128", "k_tql", "k_tql_apply128",
-                         "k_eig128", "k_tql_apply", "k_tql_apply64", "k_formq64", "k_eigvec_epi",
-                         "k_eig", "k_dual_lift"],
-                 "gram": ["k_gram128", "k_gram128_persist", "k_dual_gram"],
-                 "update": ["k_xform128", "k_xform128f"]}
+# the kernels of each phase at 64 < N <= 128 (the observation-space bucket's
+# included)
+PHASE_KERNELS = {"eig": ["k_tridiag_lower", "k_tridiag64", "k_func", "k_omega_rows", "k_dual_lift"],
+                 "gram": ["k_gram_blocks", "k_dual_gram"],
+                 "update": ["k_update128"]}
 
 
 def phase_traffic(kern, mixed, config):
@@ -474,7 +468,7 @@ def main():
                     help="default: both for config 2 (the headline: mixed timed against FP64), "
                          "mixed for config 4 (FP32 members), fp64 otherwise")
     ap.add_argument("--eig", default="ql", choices=["ql", "jacobi"],
-                    help="eigensolver: tridiagonal QL (default) or one-sided Jacobi")
+                    help="eigensolver: tridiagonal form (default) or one-sided Jacobi")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--serial", action="store_true",
                     help="run every step with phase timing (zone chunks in order on one stream), "
@@ -514,17 +508,15 @@ def main():
     g, H, Hshift, yo, rmse2 = device_inputs(DP, device)
     print("# generated %s in %.1f s" % (desc, time.time() - t0), file=sys.stderr, flush=True)
     n, N = DP.E.shape
-    eig_name = (("k_tridiag_lower<256>+k_tridiag<128>+k_formq256+k_tql+k_tql_apply256+k_eigvec_epi (Householder on "
-                 "register tiles, Q in blocked WY form on FP64 MFMA, implicit QL, rotations on "
-                 "rows in registers, eigenvector epilogue; FP64)" if N > 128 else
-                 "k_tridiag_lower<128>+k_tridiag_lower<64>+k_formq128+k_tql+k_tql_apply128 "
-                 "(Householder on the lower triangle, Q in "
-                 "blocked WY form on FP64 MFMA, implicit QL, eigenvector epilogue; FP64), with "
-                 "the zones of p < 64 through k_tridiag_lower<64>+k_formq64+k_tql+k_tql_apply64+"
-                 "k_eigvec_epi at 64 "
+    eig_name = (("k_tridiag_lower<256>+k_tridiag_lower<128>+k_tridiag64+k_pole256+k_qapply256 (Householder "
+                 "on register tiles, M^-1/2 of the tridiagonal form as a rational function, Q applied "
+                 "in blocked WY form on FP64 MFMA; FP64)" if N > 128 else
+                 "k_tridiag_lower<128>+k_tridiag64+k_func<128> (Householder on the lower triangle, "
+                 "M^-1/2 of the tridiagonal form as a rational function, Q applied in blocked WY "
+                 "form on FP64 MFMA; FP64), with the zones of p < 64 through k_tridiag64+k_func<64> "
                  "and k_dual_lift" if N > 64 else
-                 "k_tridiag_lower<64>+k_formq64+k_tql+k_tql_apply64+k_eigvec_epi (Householder on "
-                 "the lower triangle + implicit QL, FP64; k_tridiag below N = 33)")
+                 "k_tridiag64+k_func<64> (Householder with a row per lane, M^-1/2 of the tridiagonal "
+                 "form as a rational function; FP64; k_tridiag_small+k_func_small up to N = 32)")
                 if args.eig == "ql" else "k_eig (one-sided Jacobi, FP64)")
     eig_id = OAKG_EIG_QL if args.eig == "ql" else OAKG_EIG_JACOBI
     res = {}

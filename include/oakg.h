@@ -58,7 +58,7 @@ extern "C" {
 #define OAKG_EHIP 3   /* HIP runtime error                                          */
 #define OAKG_ENOMEM 4 /* device allocation failed                                   */
 #define OAKG_EUNSUP 5 /* configuration not supported (e.g. N above the maximum)     */
-#define OAKG_ECONV 6  /* eigensolver did not finish a zone (N > 128: no fallback)   */
+#define OAKG_ECONV 6  /* eigensolver did not finish a zone (no longer returned)     */
 
 #define OAKG_FP64 0  /* plain FP64 path                                             */
 #define OAKG_MIXED 1 /* FP32/BF16 contractions, FP64 eigensolve                     */
@@ -112,7 +112,7 @@ typedef struct {
   int64_t obs_selected;    /* sum over zones of the local observation count p_z  */
   int64_t pmax;            /* largest p_z                                        */
   int32_t sweeps_max;      /* most Jacobi sweeps used by one zone                */
-  int32_t eig_fallbacks;   /* zones the QL eigensolver left to Jacobi            */
+  int32_t eig_fallbacks;   /* always 0 (the default solver does not iterate)     */
   double ms_total;         /* device time of the whole call                      */
   /* device time per phase, recorded only with oakg_set_timing(ctx, 1):
      prep (H·E, anomalies), select, gram (S^T R^-1 S), eig (eigensolve),
@@ -129,7 +129,8 @@ int oakg_create(oakg_ctx** ctx, int device, int precision);
 int oakg_destroy(oakg_ctx* ctx);
 const char* oakg_last_error(const oakg_ctx* ctx);
 /* Launch on this HIP stream (hipStream_t) instead of the default stream.
-   With 4096 zones or more (and phase timing off) the zone chunks also run on
+   With 4096 zones or more, and a quarter of a million matrix rows over all
+   zones, (and phase timing off) the zone chunks also run on
    internal non-blocking streams of the context (default priority; two with
    the default OAKG_TUNE_SLOTS),
    ordered after the work already on `stream` and joined back into it by
@@ -140,19 +141,20 @@ int oakg_set_stream(oakg_ctx* ctx, void* stream);
 int oakg_set_timing(oakg_ctx* ctx, int on);
 /* Eigensolver of the N x N ensemble-space matrix (OAK calls LAPACK dsyev,
    matoper_inc.F90:986-1005):
-     OAKG_EIG_QL      Householder tridiagonalisation + implicit QL (default;
-                      zones where QL fails fall back to Jacobi)
-     OAKG_EIG_JACOBI  one-sided Jacobi for every zone                        */
+     OAKG_EIG_QL      Householder tridiagonalisation, then M^-1/2 and M^-1 of the
+                      tridiagonal form as sums of shifted solves, without
+                      eigenvectors (default)
+     OAKG_EIG_JACOBI  one-sided Jacobi for every zone (N <= 128)             */
 #define OAKG_EIG_JACOBI 0
 #define OAKG_EIG_QL 1
 int oakg_set_eigensolver(oakg_ctx* ctx, int method);
 int oakg_get_stats(oakg_ctx* ctx, oakg_stats* out);
 /* Tuning knobs of the zone loop (each zone is computed alone, so every
- * setting but OAKG_TUNE_DUAL and OAKG_TUNE_TRIDIAG_SPLIT = 2, 3, 4 gives the same
- * bits; those two give the same analysis to rounding):
+ * setting but OAKG_TUNE_DUAL gives the same bits; that one gives the same
+ * analysis to rounding):
  *   OAKG_TUNE_SLOTS       zone chunks in flight on as many streams (1..4,
- *                         default 3; from 4096 zones, phase timing off)
- *   OAKG_TUNE_QL_ZONES    zones per wave of the QL kernel (4, 8, 16, 32; 16)
+ *                         default 3; see oakg_set_stream)
+ *   OAKG_TUNE_QL_ZONES    4, 8, 16 or 32: kept, without effect
  *   OAKG_TUNE_GRAPH       1: the zone loop (Gram, eigensolve, transform,
  *                         update of every chunk, on all its streams) is
  *                         captured in a HIP graph on first use and replayed
@@ -163,28 +165,14 @@ int oakg_get_stats(oakg_ctx* ctx, oakg_stats* out);
  *                         count (quarter-octave buckets; every zone chunk
  *                         gets the same mix), the heaviest first; 0: in
  *                         zone order (default)
- *   OAKG_TUNE_TRIDIAG_SPLIT  1: at N > 64 the Householder reduction runs as
- *                         two kernels (the first half of the steps, then the
- *                         rest with fewer registers and more zones per CU);
- *                         2: three kernels, the middle quarter of the steps
- *                         on 6 x 6 register tiles (sums grouped differently);
- *                         3: two kernels, the first with the lower triangle
- *                         only (half the registers per zone, four zones per
- *                         CU; sums grouped differently); 4: as 3, the second
- *                         on the lower triangle as well (one wave per zone);
- *                         0: one kernel (default)
+ *   OAKG_TUNE_TRIDIAG_SPLIT  0..4: kept, without effect
  *   OAKG_TUNE_DUAL        at N > 64, zones with 1 <= p < value local
  *                         observations (value 16, 32 or 64; 0 = off, the
  *                         default) are solved in the p x p observation space:
  *                         G = S~ S~^T instead of M = I + S~^T S~, which have
  *                         the same nonzero spectrum.  The analysis is the
  *                         same to rounding (not bit for bit).
- *   OAKG_TUNE_PERSIST     at N > 64, the Gram kernel as a persistent grid
- *                         (two workgroups per CU) taking zones from work
- *                         counters in the zone loop's order: 2 a zone per
- *                         workgroup, 1 each wave the next zone of its
- *                         quarter of the tiles; 0: a workgroup per zone
- *                         (default)
+ *   OAKG_TUNE_PERSIST     0..2: kept, without effect
  * oakg_get_tuning also reads OAKG_TUNE_GRAPH_REPLAYS / _CAPTURES (counts). */
 #define OAKG_TUNE_SLOTS 1
 #define OAKG_TUNE_QL_ZONES 2

@@ -196,11 +196,10 @@ class Context:
 
     def set_tuning(self, slots=None, ql_zones=None, graph=None, order=None, tri_split=None,
                    dual=None, persist=None):
-        """Zone chunks in flight, zones per QL wave, HIP-graph replay of the
-        zone loop, zones ordered by observation count, the N > 64 Householder
-        reduction as two kernels, zones with fewer than `dual` observations
-        solved in observation space, the N > 64 Gram as a persistent kernel
-        (oakg_set_tuning)."""
+        """Zone chunks in flight, HIP-graph replay of the zone loop, zones
+        ordered by observation count, zones with fewer than `dual`
+        observations solved in observation space; ql_zones, tri_split and
+        persist are kept but choose nothing (oakg_set_tuning)."""
         L = load()
         for key, v in ((OAKG_TUNE_SLOTS, slots), (OAKG_TUNE_QL_ZONES, ql_zones),
                        (OAKG_TUNE_GRAPH, graph), (OAKG_TUNE_ORDER, order),

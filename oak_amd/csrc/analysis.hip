@@ -3,13 +3,14 @@
 //   k_gram    C = S^T diag(r) S and b = S^T (r o d) on v_mfma_f64_16x16x4f64,
 //             stored as M = I + C (rrsqrt.F90:135, 142; r = w^2/rmse^2,
 //             covariance.F90:612-619)
-//   k_eig     one-sided (Hestenes) Jacobi on M, one matrix row per lane held in
+//   k_eig     one-sided (Hestenes) Jacobi on M (option), one matrix row per lane in
 //             registers; columns converge to x_j = mu_j u_j with mu = 1 + lambda
 //             (the eigen-decomposition of rrsqrt.F90:136-140).  Epilogue builds
 //             a = (I+C)^-1 b (rrsqrt.F90:142), v ~ (I+C)^1/2 1 (:176-177) and
 //             Y = X diag(mu^-5/4) with Y Y^T = (I+C)^-1/2
 //   k_tmat    T = (I+C)^-1/2 Omega, Omega = RotateVector(w, v) (rrsqrt.F90:185,
-//             737-745; perpSpace matoper.F90:509-535) as identity + rank-5 terms
+//             737-745; perpSpace matoper.F90:509-535) as identity + rank-5 terms, after
+//             k_eig at N <= 32 (else update.hip, funcm.hip)
 // The Householder path and the update (Sf T, Sf a) are in funcm.hip and update.hip.
 #include "analysis.hpp"
 #include "common.hpp"
@@ -313,8 +314,7 @@ __global__ __launch_bounds__(256) void k_eig(int64_t z0, const int32_t* __restri
                                              double* __restrict__ ampl,
                                              int32_t* __restrict__ sweeps_out,
                                              unsigned* __restrict__ err, double tol,
-                                             int max_sweeps,
-                                             const int32_t* __restrict__ only) {
+                                             int max_sweeps) {
   constexpr int GPW = 64 / NP;
   constexpr int H = NP / 2;
   __shared__ EigLds<NP> lds[4];
@@ -322,15 +322,13 @@ __global__ __launch_bounds__(256) void k_eig(int64_t z0, const int32_t* __restri
   EigLds<NP>& L = lds[wave];
   const int grp = lane / NP, r = lane % NP, gb = grp * NP;
   const int zl = (blockIdx.x * 4 + wave) * GPW + grp;
-  // with `only`, zones whose flag has no bit in 3 are left untouched
-  bool valid = zl < nzc && (!only || (only[zl] & 3));
+  bool valid = zl < nzc;
   int64_t z = valid ? zone_at(zorder, z0 + zl) : 0;
   if (z < 0) {  // solved by the other pipeline
     valid = false;
     z = 0;
   }
-  // a wave with no zone to solve leaves at once (the fallback pass visits
-  // every zone and redoes only the flagged ones); the waves share no barrier
+  // a wave with no zone to solve leaves at once; the waves share no barrier
   if (__ballot(valid) == 0) return;
   const bool active = valid && (sel_ptr[z + 1] > sel_ptr[z]);
   const double* M = mat + (size_t)(valid ? zl : 0) * NP * NP;
@@ -597,7 +595,7 @@ static void eig_t(const ChunkArgs& A, hipStream_t st) {
   } else {
     hipLaunchKernelGGL(k_eig<NP>, dim3(nblk(A.nzc, 4 * GPW)), dim3(256), 0, st, A.z0, A.zorder, A.nzc,
                        A.N, A.sel_ptr, A.mat, A.ymat, A.vec, A.ampl, A.sweeps, A.err, A.tol,
-                       A.max_sweeps, (const int32_t*)nullptr);
+                       A.max_sweeps);
     if (NP == 64) launch_yyt(NP, A, st);
   }
 }

@@ -1,5 +1,5 @@
 // FP64 per-zone analysis for ensembles of 65..128 members (NP = 128):
-// the same steps as analysis.hip (rrsqrt.F90:100-190), with kernels shaped
+// the steps of the smaller ones (rrsqrt.F90:100-190), with kernels shaped
 // for a 128 x 128 ensemble-space matrix.
 //
 //   gram_blocks.hip  M = I + S^T diag(r) S
@@ -344,7 +344,7 @@ void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
 void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
   if (A.mode == 2) {  // innovation likelihood: adjoint instead of transform + update
     if (tm) tm->mark(PH_UPDATE);
-    launch_nll_adjoint(128, A, st);
+    launch_nll_adjoint128(A, st);
     if (tm) tm->mark(PH_END);
     return;
   }

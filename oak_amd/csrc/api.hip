@@ -55,7 +55,7 @@ struct oakg_ctx {
   size_t ws_budget = (size_t)8 << 30;  // chunk workspace of one zone loop (all slots)
   double jacobi_tol = 0;  // 0 = default for the precision
   int max_sweeps = 40;
-  int eig_method = 1;     // 1 = tridiagonal QL (default), 0 = one-sided Jacobi
+  int eig_method = 1;     // 1 = tridiagonal form (default), 0 = one-sided Jacobi
   // last call, for the lazily copied per-zone counts
   int64_t last_nz = 0;
   const int64_t* last_sel_ptr = nullptr;
@@ -64,13 +64,14 @@ struct oakg_ctx {
   // internal streams of the chunk pipeline (default priority) and their events
   hipStream_t aux[OAKG_PIPE_SLOTS - 1] = {};
   hipEvent_t ev_fork = nullptr, ev_join[OAKG_PIPE_SLOTS - 1] = {};
-  // tuning knobs (oakg_set_tuning): zone chunks in flight, zones per QL wave
+  // tuning knobs (oakg_set_tuning): zone chunks in flight; ql_zw, tri_split and
+  // persist are kept for oakg_get_tuning and choose nothing
   int tune_slots = 3;
   int tune_ql_zw = 16;
   int tune_order = 0;  // 1: zones ordered by observation count (k_zone_order)
-  int tune_tri_split = 0;  // 1: N = 128 Householder reduction as two launches
+  int tune_tri_split = 0;
   int tune_dual = 0;  // N = 128: zones with 1 <= p < tune_dual solved in observation space
-  int tune_persist = 0;  // N = 128: the Gram as a persistent kernel (2 zone per workgroup, 1 per wave)
+  int tune_persist = 0;
   // the zone loop captured in a HIP graph and replayed while its launches
   // (kernel arguments, buffers, streams) stay the same
   bool graph = false;
@@ -102,8 +103,7 @@ __global__ void k_fill_f64(double* p, int64_t n, double v) {
 }
 // Per-call statistics to the host (pinned memory, read after a
 // synchronisation): [0] error bits, [1] zones with p > 0, [2] sum p, [3] max
-// p, [4] max sweeps, [5] zones handed to a fallback.  The workgroups add up in
-// the error block (integers, so in any order); the last one publishes.
+// p, [4] max sweeps.  The workgroups add up in the error block (integers, so in any order); the last one publishes.
 __global__ __launch_bounds__(256) void k_call_stats(int64_t nz, const int64_t* __restrict__ sel_ptr,
                                                     const int32_t* __restrict__ sweeps, unsigned* err,
                                                     int64_t* __restrict__ out) {
@@ -134,7 +134,6 @@ __global__ __launch_bounds__(256) void k_call_stats(int64_t nz, const int64_t* _
       return (int64_t)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     out[0] = (int64_t)__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    out[5] = (int64_t)__hip_atomic_load(err + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     out[1] = get(sums);
     out[2] = nz > 0 ? sel_ptr[nz] - sel_ptr[0] : 0;
     out[3] = get(sums + 1);
@@ -406,13 +405,12 @@ void finish_call(oakg_ctx* c, int64_t nz, const int64_t* sel_ptr, const int32_t*
                      c->pinned);
   check(c, hipGetLastError(), "stats launch");
   check(c, hipStreamSynchronize(c->stream), "sync");
-  int64_t h[6];
-  for (int i = 0; i < 6; ++i) h[i] = ((volatile int64_t*)c->pinned)[i];
+  int64_t h[5];
+  for (int i = 0; i < 5; ++i) h[i] = ((volatile int64_t*)c->pinned)[i];
   c->stats.zones_analysed = h[1];
   c->stats.obs_selected = h[2];
   c->stats.pmax = h[3];
   c->stats.sweeps_max = (int32_t)h[4];
-  c->stats.eig_fallbacks = (int32_t)h[5];
   const unsigned herr = (unsigned)h[0];
   if (herr & OAKG_DERR_RMSE) arg_fail(c, "observation error variance rmse^2 <= 0 or not finite");
   if (herr & OAKG_DERR_IDX) arg_fail(c, "index out of range in H or in the selection");
@@ -457,8 +455,8 @@ void materialize_counts(oakg_ctx* c) {
 // Runs the chunked zone loop (gram, eigensolve, tmat, update) for all zones.
 // Without phase timing, consecutive chunks rotate over the caller's stream
 // and OAKG_PIPE_SLOTS - 1 internal streams, each with its own part of the
-// chunk workspace, so that the tail of one chunk's kernels (the QL sweeps of
-// its slowest zones, above all) overlaps the next chunks' work.  The streams are
+// chunk workspace, so that the tail of one chunk's kernels overlaps the next
+// chunks' work.  The streams are
 // joined by events before the call continues.  With phase timing the chunks
 // run in order on the caller's stream (the timer's events are on that stream).
 // Returns whether the zones' Jacobi sweeps are in sweeps_all.

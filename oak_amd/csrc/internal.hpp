@@ -13,8 +13,8 @@ namespace oakg {
 constexpr int kMaxCells = 1 << 22;  // cap of the observation bin grid
 
 // Words of a context's error block, all zero at the start of a call: [0] error
-// bits, [1] eigensolver fallbacks, the arrival counters of the kernels whose
-// last workgroup joins the parts, and their sums (int64, from kSyncSums on).
+// bits, [1] unused, the arrival counters of the kernels whose last workgroup
+// joins the parts, and their sums (int64, from kSyncSums on).
 constexpr int kSyncGeo = 2, kSyncStats = 3, kSyncSums = 4, kSyncWords = 10;
 
 

@@ -48,9 +48,7 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
                                                      double* __restrict__ gL,
                                                      double* __restrict__ gA,
                                                      double* __restrict__ gth) {
-  constexpr int KPL = NP > 64 ? NP / 64 : 1;  // vector entries per lane
-  constexpr bool YLDS = NP <= 64;
-  __shared__ double Ys[YLDS ? NP * NP : 1];
+  constexpr int KPL = NP / 64;  // vector entries per lane
   __shared__ double sw[4][NP];
   __shared__ double red[4][3];
   const int zl = blockIdx.x;
@@ -67,20 +65,11 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
     return;
   }
   const double* V = vec + (size_t)zl * 4 * NP;
-  const double* Yg = ymat + (size_t)zl * NP * NP;
-  if (YLDS) {
-    copy_batched<16>(tid, NP * NP, 256, [&](int e) { return Yg[e]; },
-                     [&](int e, double x) { Ys[e] = x; });
-    __syncthreads();
-  }
-  const double* Y = YLDS ? Ys : Yg;
-  double ak[KPL], wk[KPL];
+  const double* Y = ymat + (size_t)zl * NP * NP;  // M^-1/2: u = |M^-1/2 s|^2
+  double ak[KPL];
 #pragma unroll
   for (int c = 0; c < KPL; ++c) {
-    const int k = lane + 64 * c;
-    ak[c] = k < NP ? V[NP + k] : 0.0;
-    // NP >= 64: Y is M^-1/2, u = |M^-1/2 s|^2; else u = sum_k mu_k^-1/2 (Y^T s)_k^2
-    wk[c] = NP >= 64 ? 1.0 : (k < NP ? 1.0 / sqrt(V[3 * NP + k]) : 0.0);
+    ak[c] = V[NP + lane + 64 * c];
   }
   const double Lz = corr[z];
   double accL = 0.0, accR = 0.0, accLog = 0.0;
@@ -93,8 +82,8 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
 #pragma unroll
     for (int c = 0; c < KPL; ++c) {
       const int j = lane + 64 * c;
-      const double s = j < NP ? srow[hs_col<NP>(j)] : 0.0;
-      if (j < NP) sw[wave][j] = s;
+      const double s = srow[hs_col<NP>(j)];
+      sw[wave][j] = s;
       t = fma(s, ak[c], t);
     }
     __builtin_amdgcn_wave_barrier();
@@ -103,11 +92,9 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
 #pragma unroll
     for (int c = 0; c < KPL; ++c) {
       const int k = lane + 64 * c;
-      if (k < NP) {
-        double y = 0.0;
-        for (int j = 0; j < NP; ++j) y = fma(Y[(size_t)j * NP + k], sw[wave][j], y);
-        u = fma(wk[c] * y, y, u);
-      }
+      double y = 0.0;
+      for (int j = 0; j < NP; ++j) y = fma(Y[(size_t)j * NP + k], sw[wave][j], y);
+      u = fma(y, y, u);
     }
     u = nll_wave_sum(u);
     __builtin_amdgcn_wave_barrier();
@@ -128,20 +115,11 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
   }
   __syncthreads();
   if (wave == 0) {
-    // sum_k log mu_k, sum_k (1 - 1/mu_k), a^T a, b^T a over the NP entries
-    // (padding entries have mu = 1, a = b = 0)
-    double slog = 0, sinv = 0, aa = 0, ba = 0;
-    for (int k = lane; k < NP; k += 64) {
-      const double mu = NP >= 64 ? 1.0 : V[3 * NP + k], ak2 = V[NP + k];
-      slog += log(mu);
-      sinv += 1.0 - 1.0 / mu;
-      aa = fma(ak2, ak2, aa);
-      ba = fma(V[k], ak2, ba);
-    }
-    slog = NP >= 64 ? V[3 * NP] : nll_wave_sum(slog);
-    sinv = NP >= 64 ? V[3 * NP + 1] : nll_wave_sum(sinv);
+    // sum_k log mu_k, sum_k (1 - 1/mu_k) and b^T a from k_func; a^T a
+    double aa = 0;
+    for (int k = lane; k < NP; k += 64) aa = fma(V[NP + k], V[NP + k], aa);
     aa = nll_wave_sum(aa);
-    ba = NP >= 64 ? V[3 * NP + 2] : nll_wave_sum(ba);
+    const double slog = V[3 * NP], sinv = V[3 * NP + 1], ba = V[3 * NP + 2];
     if (lane == 0) {
       const double sL = ((red[0][0] + red[1][0]) + red[2][0]) + red[3][0];
       const double sR = ((red[0][1] + red[1][1]) + red[2][1]) + red[3][1];
@@ -153,15 +131,10 @@ __global__ __launch_bounds__(256) void k_nll_adjoint(int64_t z0, const int32_t* 
   }
 }
 
-void launch_nll_adjoint(int NP, const ChunkArgs& A, hipStream_t st) {
-#define OAK_NLL(P)                                                                                \
-  hipLaunchKernelGGL(k_nll_adjoint<P>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,       \
-                     A.sel_idx, A.sel_w, A.rho, A.innov, A.HS, A.ymat, A.vec, A.corr, A.infl,     \
-                     A.nll_J, A.nll_gL, A.nll_gA, A.nll_gth)
-  switch (NP) {
-    case 128: OAK_NLL(128); break;
-  }
-#undef OAK_NLL
+void launch_nll_adjoint128(const ChunkArgs& A, hipStream_t st) {
+  hipLaunchKernelGGL(k_nll_adjoint<128>, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
+                     A.sel_idx, A.sel_w, A.rho, A.innov, A.HS, A.ymat, A.vec, A.corr, A.infl,
+                     A.nll_J, A.nll_gL, A.nll_gA, A.nll_gth);
 }
 
 // ---------------------------------------------------------------------------

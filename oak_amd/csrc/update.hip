@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* 
       v[tid] = tid < N ? Vz[2 * NP + tid] : 0.0;
     }
     lds_barrier();
-    // (analysis.hip's k_tmat): with zw = w + e_{N-1}, vt = v but 0 at N - 1,
+    // (k_tmat): with zw = w + e_{N-1}, vt = v but 0 at N - 1,
     // T[r][s] = R[r][s] (0 at s = N-1) + u1 w + (alpha_w u2 + alpha_v alpha_w
     // (v.w~) u3) zw_s + alpha_v u3 vt_s, u1 = (R v)_r, u2 = (R w~)_r, u3 = u1 +
     // sign(v_N) R[r][N-1]
