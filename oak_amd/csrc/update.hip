@@ -296,8 +296,8 @@ __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* 
 // four waves on a SIMD belong to two workgroups.  The product is with R; row k of T
 // is row k of R plus p_k + q_k v (OmegaRow, in slots 0 and 3 of vec), so a row of
 // Sf adds its products with p and q; row N - 1 in ymat is that of T^T already.
-// 64 800 zones of 121 rows, N = 128: 8.6 ms FP64, 4.15 FP32 (T whole in LDS, and a
-// pass for the mean: 9.3 + 1.35 and 4.85 + 0.7).  Omega on the way to LDS cost 0.7 to
+// 64 800 zones of 121 rows, N = 128: 7.5 ms FP64 (27 GB moved: 3.7 TB/s), 4.1 FP32
+// (T whole in LDS, and a pass for the mean: 9.3 + 1.35 and 4.85 + 0.7).  Omega on the way to LDS cost 0.7 to
 // 1.2 ms more, in k_func's registers 3.4 ms of spills there.
 template <int MODE, typename TE>
 __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t* __restrict__ zorder, int N,
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
   constexpr int NP = 128, Q = NP / 4, CB = 32, LD = sizeof(TE) == 4 ? NP + 4 : NP + 2;
   typedef TE TE2 __attribute__((ext_vector_type(2)));
   typedef TE TEV __attribute__((ext_vector_type(16 / sizeof(TE))));
-  constexpr int EV = 16 / sizeof(TE), NV = 8 / EV;  // 16-byte pieces of a thread's 8 entries
+  constexpr int EV = 16 / sizeof(TE), NV = 4 / EV;  // 16-byte pieces of a thread's 4 entries
   __shared__ __attribute__((aligned(16))) TE L[2][CB * LD];
   __shared__ __attribute__((aligned(16))) double as[NP], p[NP], q[NP], v[NP];
   const int zl = blockIdx.x;
@@ -332,10 +332,12 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
     q[tid] = active ? Vz[3 * NP + tid] : 0.0;
     v[tid] = active ? Vz[2 * NP + tid] : 0.0;
   }
-  // thread t moves entries 8 (t % 16) .. + 7 of row t / 16 of a block
+  // thread t moves entries 4 (t % 16) .. + 3 of each half of row t / 16 of a
+  // block, a half at a time: with both in registers beside the strip, the FP64
+  // kernel spilled (34 GB moved instead of 27, 8.4 ms)
   TEV st[NV];
-  auto fetch = [&](int h, int t) {
-    const int sr = t >> 4, sc = 8 * (t & 15);
+  auto fetch = [&](int h, int t, int half) {
+    const int sr = t >> 4, sc = 4 * (t & 15) + 64 * half;
 #pragma unroll
     for (int w = 0; w < NV; ++w)
       st[w] = *reinterpret_cast<const TEV*>(X + (size_t)(CB * h + sr) * NP + sc + EV * w);
@@ -345,10 +347,11 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
 #pragma unroll
         for (int i = 0; i < EV; ++i) st[w][i] = CB * h + sr == sc + EV * w + i ? (TE)1 : (TE)0;
   };
-  auto put = [&](int h, int t) {
-    const int sr = t >> 4, sc = 8 * (t & 15);
+  auto put = [&](int h, int t, int half) {
+    const int sr = t >> 4, sc = 4 * (t & 15) + 64 * half;
 #pragma unroll
-    for (int w = 0; w < NV; ++w) *reinterpret_cast<TEV*>(L[h & 1] + sr * LD + sc + EV * w) = st[w];
+    for (int w = 0; w < NV; ++w)
+      *reinterpret_cast<TEV*>(L[h & 1] + sr * LD + sc + EV * w) = st[w];
   };
   const int nh = (N + CB - 1) / CB;
   for (int64_t r0 = 0; r0 < sz; r0 += 128) {
@@ -362,9 +365,11 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
     const bool rok = rb + li < sz;
     const int64_t row = i0 + (rok ? rb + li : 0);
     TE b[Q];
+    fetch(0, tp, 0);
     if (rb < sz) load_members(b, S, row, ldS, kk, N);
-    fetch(0, tp);
-    put(0, tp);
+    put(0, tp, 0);
+    fetch(0, tp, 1);
+    put(0, tp, 1);
     lds_barrier();
     double xar = 0.0, gp = 0.0, gq = 0.0;
     if (rb < sz) {
@@ -386,12 +391,13 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
       int tq = threadIdx.x;
       asm volatile("" : "+v"(tq));
       const int li = tq & 15, kk = (tq >> 4) & 3;
-      if (h + 1 < nh) fetch(h + 1, tq);
-      if (rb < sz) {
-        const TE* lt = L[h & 1] + li * LD + 2 * kk;
-        vec4<TE> acc[2] = {};
+      if (h + 1 < nh) fetch(h + 1, tq, 0);
+      const TE* lt = L[h & 1] + li * LD + 2 * kk;
+      vec4<TE> acc[2] = {};
+      auto product = [&](int half) {
 #pragma unroll
-        for (int g = 0; g < Q / 2; ++g) {
+        for (int e = 0; e < Q / 4; ++e) {
+          const int g = half * (Q / 4) + e;
           asm volatile("" ::: "memory");  // the reads of later pairs stay below
           TE2 A[2];
 #pragma unroll
@@ -401,6 +407,14 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
 #pragma unroll
           for (int J = 0; J < 2; ++J) acc[J] = mfma(A[J].y, b[2 * g + 1], acc[J]);
         }
+      };
+      if (rb < sz) product(0);
+      if (h + 1 < nh) {
+        put(h + 1, tq, 0);
+        fetch(h + 1, tq, 1);
+      }
+      if (rb < sz) {
+        product(1);
 #pragma unroll
         for (int J = 0; J < 2; ++J)
 #pragma unroll
@@ -410,7 +424,7 @@ __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t*
             if (rok && col < N) Out[row + (int64_t)col * ldO] = out_value<MODE, TE>(y, xar, infl);
           }
       }
-      if (h + 1 < nh) put(h + 1, tq);
+      if (h + 1 < nh) put(h + 1, tq, 1);
       lds_barrier();
     }
   }
