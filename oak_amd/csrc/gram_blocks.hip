@@ -27,6 +27,9 @@ namespace {
 // the MFMAs alone 31 at 2.4 GHz).  64 800 zones of N = 128, 14 million rows in
 // all: 5.65 ms (a wave per two tile rows, all columns loaded by each: 6.6; with
 // kSplitRows 256 and 128: 5.8 and 6.1, 0.01 ms less for 5760 zones of 271 rows).
+// What is padding is left out: at N <= 128 the tile rows of the last block beyond
+// the members (NL of them hold some), above the
+// blocks without members (5760 zones of N = 100, whole analysis 3.57 -> 3.51 ms).
 constexpr int kGramSplit = 4, kSplitRows = 512;
 
 template <int NP>
@@ -34,7 +37,7 @@ __device__ __forceinline__ int block_col(int X, int J, int j) {
   return 64 * X + (NP == 128 ? 16 * J + j : 4 * j + J);
 }
 
-template <int NP, typename TS, bool DIAG, int SPLIT>
+template <int NP, typename TS, bool DIAG, int SPLIT, int NL>
 __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
                                              const int32_t* __restrict__ sel_idx,
                                              const double* __restrict__ sel_w, unsigned m,
@@ -42,7 +45,7 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
                                              const double* __restrict__ innov,
                                              const TS* __restrict__ HS, double* __restrict__ M,
                                              double* __restrict__ bv_out, unsigned* __restrict__ err) {
-  constexpr int NT = DIAG ? 20 : 16;
+  constexpr int NT = DIAG ? 10 + NL * (NL + 1) / 2 : 4 * NL;
   typedef TS TS4 __attribute__((ext_vector_type(4)));
   const int part = SPLIT > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int lane = threadIdx.x & 63, kq = lane >> 4, jl = lane & 15;
@@ -93,7 +96,7 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int I = 0; I < 4; ++I) {
+        for (int I = 0; I < (h ? NL : 4); ++I) {
           const double a = r * (h ? y[I] : x[I]);
 #pragma unroll
           for (int J = 0; J <= I; ++J) {
@@ -105,11 +108,11 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         bacc[k] = fma(rd, x[k], bacc[k]);
-        bacc[(DIAG ? 4 : 0) + k] = fma(rd, y[k], bacc[(DIAG ? 4 : 0) + k]);
+        if (k < NL) bacc[(DIAG ? 4 : 0) + k] = fma(rd, y[k], bacc[(DIAG ? 4 : 0) + k]);
       }
     } else {
 #pragma unroll
-      for (int I = 0; I < 4; ++I) {
+      for (int I = 0; I < NL; ++I) {
         const double a = r * x[I];
 #pragma unroll
         for (int J = 0; J < 4; ++J) {
@@ -179,7 +182,7 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
             const int i = kq + 4 * q, j = jl;
             if (I != J || i >= j) {
               const int gi = block_col<NP>(h ? Y : X, I, i), gj = block_col<NP>(h ? Y : X, J, j);
-              const double v = acc[t][q] + (gi == gj ? 1.0 : 0.0);
+              const double v = (t < NT ? acc[t < NT ? t : 0][q] : 0.0) + (gi == gj ? 1.0 : 0.0);
               M[(size_t)gi * NP + gj] = v;
               M[(size_t)gj * NP + gi] = v;
             }
@@ -194,8 +197,9 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int gi = block_col<NP>(X, I, kq + 4 * q), gj = block_col<NP>(Y, J, jl);
-          M[(size_t)gi * NP + gj] = acc[4 * I + J][q];
-          M[(size_t)gj * NP + gi] = acc[4 * I + J][q];
+          const double v = I < NL ? acc[I < NL ? 4 * I + J : 0][q] : 0.0;
+          M[(size_t)gi * NP + gj] = v;
+          M[(size_t)gj * NP + gi] = v;
         }
   } else {
     // four columns (rows of the mirrored block) of a lane are consecutive
@@ -219,8 +223,8 @@ __device__ __forceinline__ void gram_block(int X, int Y, int64_t p0, int pn,
 
 }  // namespace
 
-template <int NP, typename TS, int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT, 2) void k_gram_blocks(int64_t z0,
+template <int NP, typename TS, int SPLIT, int NL>
+__global__ __launch_bounds__(64 * SPLIT, 2) void k_gram_blocks(int64_t z0, int N,
                                                               const int32_t* __restrict__ zorder,
                                                               const int64_t* __restrict__ sel_ptr,
                                                               const int32_t* __restrict__ sel_idx,
@@ -252,35 +256,52 @@ __global__ __launch_bounds__(64 * SPLIT, 2) void k_gram_blocks(int64_t z0,
   }
   if (y < NOFF) {
     const int X = y < 1 ? 1 : (y < 3 ? 2 : 3), Y = y - (y < 1 ? 0 : (y < 3 ? 1 : 3));
-    gram_block<NP, TS, false, SPLIT>(X, Y, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M,
+    if (64 * X >= N) {  // padding
+      for (int e = threadIdx.x; e < 64 * 64; e += 64 * SPLIT) {
+        const int i = 64 * X + (e >> 6), j = 64 * Y + (e & 63);
+        M[(size_t)i * NP + j] = M[(size_t)j * NP + i] = 0.0;
+      }
+      return;
+    }
+    gram_block<NP, TS, false, SPLIT, NL>(X, Y, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M,
                                      bv_out, err);
   } else {
     const int X = 2 * (y - NOFF);
-    gram_block<NP, TS, true, SPLIT>(X, X + 1, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M,
+    gram_block<NP, TS, true, SPLIT, NL>(X, X + 1, p0, (int)p, sel_idx, sel_w, (unsigned)m, rho, innov, HS, M,
                                     bv_out, err);
   }
 }
 
-template <int NP, typename TS>
+template <int NP, typename TS, int NL>
 static void gram_blocks_t(const ChunkArgs& A, const TS* HS, hipStream_t st) {
   constexpr int NBL = NP / 64, PARTS = NBL * (NBL - 1) / 2 + NBL / 2;
   const dim3 grid(A.nzc, PARTS);
-  hipLaunchKernelGGL((k_gram_blocks<NP, TS, kGramSplit>), grid, dim3(64 * kGramSplit), 0, st, A.z0,
+  hipLaunchKernelGGL((k_gram_blocks<NP, TS, kGramSplit, NL>), grid, dim3(64 * kGramSplit), 0, st, A.z0, A.N,
                      A.zorder, A.sel_ptr, A.sel_idx, A.sel_w, A.m, A.rho, A.innov, HS, A.mat, A.vec,
                      A.err);
-  hipLaunchKernelGGL((k_gram_blocks<NP, TS, 1>), grid, dim3(64), 0, st, A.z0, A.zorder, A.sel_ptr,
+  hipLaunchKernelGGL((k_gram_blocks<NP, TS, 1, NL>), grid, dim3(64), 0, st, A.z0, A.N, A.zorder, A.sel_ptr,
                      A.sel_idx, A.sel_w, A.m, A.rho, A.innov, HS, A.mat, A.vec, A.err);
+}
+
+template <typename TS>
+static void gram128_t(const ChunkArgs& A, const TS* HS, hipStream_t st) {
+  switch ((A.N - 49) / 16) {  // 65..80, ..96, ..112, ..128 members
+    case 1: gram_blocks_t<128, TS, 1>(A, HS, st); break;
+    case 2: gram_blocks_t<128, TS, 2>(A, HS, st); break;
+    case 3: gram_blocks_t<128, TS, 3>(A, HS, st); break;
+    default: gram_blocks_t<128, TS, 4>(A, HS, st); break;
+  }
 }
 
 void launch_gram_blocks(int NP, const ChunkArgs& A, hipStream_t st) {
   if (NP == 128 && A.prec == 1)
-    gram_blocks_t<128, float>(A, A.HS32, st);
+    gram128_t<float>(A, A.HS32, st);
   else if (NP == 128)
-    gram_blocks_t<128, double>(A, A.HS, st);
+    gram128_t<double>(A, A.HS, st);
   else if (A.prec == 1)
-    gram_blocks_t<256, float>(A, A.HS32, st);
+    gram_blocks_t<256, float, 4>(A, A.HS32, st);
   else
-    gram_blocks_t<256, double>(A, A.HS, st);
+    gram_blocks_t<256, double, 4>(A, A.HS, st);
 }
 
 }  // namespace oakg
