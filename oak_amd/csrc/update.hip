@@ -174,8 +174,8 @@ __global__ __launch_bounds__(256, NP == 32 ? 3 : 4) void k_update_small(int64_t 
 // steps.  Bound by the reads and writes of the ensemble: 64 800 zones of 121 rows,
 // N = 64, 8.0 GB and 2.1 GB of M^-1/2, 2.67 ms.  With T from a kernel of its own,
 // a spilling product that waited for each load and the mean in a pass before,
-// these took 1.6, 10.5 and 0.7 ms.
-template <int MODE, typename TE>
+// these took 1.6, 10.5 and 0.7 ms.  NB tile rows and columns hold members.
+template <int MODE, typename TE, int NB>
 __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                      const int64_t* __restrict__ sel_ptr,
                                                      const int64_t* __restrict__ zone_ptr,
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* 
                                                      int64_t ldO, double scaling, double infl,
                                                      double maxcorr,
                                                      const double* __restrict__ maxcorr_v) {
-  constexpr int NP = 64, NB = NP / 16, Q = NP / 4;
+  constexpr int NP = 64, Q = 4 * NB;
   constexpr int LD = sizeof(TE) == 4 ? NP + 4 : NP + 2;  // reads of 16 rows on distinct banks
   typedef TE TE2 __attribute__((ext_vector_type(2)));
   __shared__ __attribute__((aligned(16))) TE L[NP * LD];
@@ -448,9 +448,14 @@ void launch_update(int NP, const ChunkArgs& A, hipStream_t st) {
                          A.infl, A.maxcorr, A.maxcorr_v);                                             \
       break;                                                                                          \
     case 64:                                                                                          \
-      hipLaunchKernelGGL((k_update64<MODE, TE>), dim3(A.nzc), blk, 0, st, A.z0, A.zorder, A.N,        \
-                         A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,    \
-                         A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                  \
+      if (A.N <= 48)                                                                                  \
+        hipLaunchKernelGGL((k_update64<MODE, TE, 3>), dim3(A.nzc), blk, 0, st, A.z0, A.zorder, A.N,   \
+                           A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,  \
+                           A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                \
+      else                                                                                            \
+        hipLaunchKernelGGL((k_update64<MODE, TE, 4>), dim3(A.nzc), blk, 0, st, A.z0, A.zorder, A.N,   \
+                           A.sel_ptr, A.zone_ptr, A.ymat, A.vec, A.X0, SRC, A.ldS, A.xa, DST, A.ldO,  \
+                           A.scaling, A.infl, A.maxcorr, A.maxcorr_v);                                \
       break;                                                                                          \
     case 128:                                                                                         \
       hipLaunchKernelGGL((k_update128<MODE, TE>), dim3(A.nzc), dim3(512), 0, st, A.z0, A.zorder, A.N, \
