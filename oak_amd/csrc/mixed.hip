@@ -7,7 +7,7 @@
 //
 //   k_spmm_obs<float>  HE = H E + Hshift (FP64 accumulation)
 //   k_obs_anom_f32     HS = (HE - ybar)/sqrt(N-1) stored FP32, innov/rho FP64
-//   k_gram<NP, float>  (analysis.hip / analysis128.hip) M = I + S^T diag(r) S
+//   k_gram<NP, float>  (analysis.hip; gram_blocks.hip) M = I + S^T diag(r) S
 //                      from the FP32 S on FP64 MFMA: products of FP32 values
 //                      are exact in FP64, so only the rounding of S to FP32
 //                      remains.  An FP32-accumulated Gram has errors of size

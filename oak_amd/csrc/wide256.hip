@@ -77,7 +77,8 @@ struct TriLowerLds {
   // distance of the slots of part: a wave writes its column sums into the slots
   // of 8 and more consecutive tile rows at the same place, so an odd distance puts
   // these on different banks (at 144 for NP = 128 and 288 for 256, multiples of 16,
-  // conflicts were half of all LDS cycles)
+  // conflicts were half of all LDS cycles: 16 200 zones of N = 256, 32.5 ms for
+  // 27.1)
   static constexpr int PS = tri_rx(NP - 1) + 3;
   static constexpr int NW = NP == 256 ? 8 : 2;           // waves of the workgroup
   static constexpr int NRW = NP / 64;                  // row waves
