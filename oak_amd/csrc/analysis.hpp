@@ -95,6 +95,7 @@ struct ChunkArgs {
   // 0 = one-sided Jacobi, 1 = Householder tridiagonalisation + functions of T
   int eig_method;
   double *dvec, *evec;      // tridiagonal, NP per zone
+  const double* poles;      // the rational approximation's table (poles.hpp)
   unsigned* err;
   double tol;
   int max_sweeps;
@@ -199,8 +200,6 @@ void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st);
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st);
 // NP = 128: what Omega adds to M^-1/2, for k_update128
 void launch_omega_rows128(const ChunkArgs& A, hipStream_t st);
-// pole table of the current device
-hipError_t init_poles(int device);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
 // N <= 128 (update.hip): T from mat (N <= 32) or M^-1/2 from ymat
 void launch_update(int NP, const ChunkArgs& A, hipStream_t st);

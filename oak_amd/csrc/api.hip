@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "internal.hpp"
 #include "interp.hpp"
+#include "poles.hpp"
 
 #ifndef OAKG_PIPE_SLOTS
 #define OAKG_PIPE_SLOTS 4  // at most this many zone chunks in flight on as many streams
@@ -60,6 +61,7 @@ struct oakg_ctx {
   int64_t last_nz = 0;
   const int64_t* last_sel_ptr = nullptr;
   int64_t* pinned = nullptr;  // host memory the device writes small results to
+  double* poles = nullptr;    // device copy of pole_table(), owned by the context
   bool counts_ready = true;
   // internal streams of the chunk pipeline (default priority) and their events
   hipStream_t aux[OAKG_PIPE_SLOTS - 1] = {};
@@ -463,6 +465,7 @@ void materialize_counts(oakg_ctx* c) {
 bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_all) {
   // the likelihood at N <= 64 keeps nothing per zone (nll.hip); else the
   // functions of T (N > 128 with either method) or the Jacobi option
+  base.poles = c->poles;
   const bool chol = base.mode == 2 && NP <= 64;
   const bool func = (c->eig_method == 1 || NP == 256) && !chol;
   const int MP = chol ? 1 : NP;  // matrices MP x MP and vectors of MP entries per zone
@@ -1526,7 +1529,6 @@ int oakg_create(oakg_ctx** out, int device, int precision) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || device < 0 || device >= ndev) return OAKG_EHIP;
   if (hipSetDevice(device) != hipSuccess) return OAKG_EHIP;
-  if (init_poles(device) != hipSuccess) return OAKG_EHIP;
   oakg_ctx* c = new (std::nothrow) oakg_ctx;
   if (!c) return OAKG_ENOMEM;
   c->device = device;
@@ -1534,6 +1536,19 @@ int oakg_create(oakg_ctx** out, int device, int precision) {
   if (hipHostMalloc((void**)&c->pinned, 64, hipHostMallocDefault) != hipSuccess) {
     delete c;
     return OAKG_ENOMEM;
+  }
+  const std::vector<double>& pt = pole_table();
+  const size_t pb = sizeof(double) * pt.size();
+  if (hipMalloc(&c->poles, pb) != hipSuccess) {
+    (void)hipHostFree(c->pinned);
+    delete c;
+    return OAKG_ENOMEM;
+  }
+  if (hipMemcpy(c->poles, pt.data(), pb, hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipHostFree(c->pinned);
+    (void)hipFree(c->poles);
+    delete c;
+    return OAKG_EHIP;
   }
   // chunk workspace: a quarter of the device memory, between 8 and 64 GiB
   // (larger chunks leave fewer part-filled rounds of workgroups at the end
@@ -1574,6 +1589,7 @@ int oakg_destroy(oakg_ctx* c) {
   if (c->ev_t1) (void)hipEventDestroy(c->ev_t1);
   if (c->d_err) (void)hipFree(c->d_err);
   if (c->pinned) (void)hipHostFree(c->pinned);
+  if (c->poles) (void)hipFree(c->poles);
   c->ws.release();
   delete c;
   return OAKG_OK;

@@ -32,98 +32,15 @@
 // ms of the eigensolve of 64 800 zones at N = 128.
 #include <math.h>
 
-#include <mutex>
 #include <type_traits>
 #include <utility>
 
 #include "analysis.hpp"
 #include "common.hpp"
 #include "eigen_common.hpp"
+#include "poles.hpp"
 
 namespace oakg {
-
-namespace {
-
-constexpr int kPoles = 31;    // lane 31 of the pole wave carries s = 0 (T itself)
-constexpr int kBuckets = 25;  // kappa = 4, 16, ... 4^25
-
-// [bucket][0: s, 1: w][pole]; pole 31: s = 0, w = 0
-__device__ double g_poles[kBuckets][2][32];
-
-// Poles and weights for [1, kappa], in extended precision.  With k =
-// kappa^-1/2 the zeros and poles are -c_j, c_j = sc^2(j K' / 62) (modulus
-// k' = sqrt(1 - k^2)), by the descending Landen transformation for the lower
-// half and c_{62-j} = kappa / c_j for the upper one.
-void zolotarev(long double kappa, double* s, double* w) {
-  constexpr int K = kPoles;
-  const long double k = 1.0L / sqrtl(kappa);
-  long double a[24], c[24];
-  int n = 0;
-  a[0] = 1.0L;
-  c[0] = sqrtl(1.0L - k * k);
-  long double b = k;
-  while (n < 22 && fabsl(c[n]) > 1e-20L * a[n]) {
-    a[n + 1] = (a[n] + b) / 2;
-    c[n + 1] = (a[n] - b) / 2;
-    b = sqrtl(a[n] * b);
-    ++n;
-  }
-  const long double Kp = 2.0L * atanl(1.0L) / a[n];  // (pi / 2) / AGM(1, k)
-  long double cj[2 * K];
-  for (int j = 1; j <= K; ++j) {
-    long double phi = ldexpl(a[n] * (j * Kp / (2 * K)), n);
-    for (int i = n; i >= 1; --i) phi = (phi + asinl(c[i] * sinl(phi) / a[i])) / 2;
-    const long double t = tanl(phi);
-    cj[j] = t * t;
-  }
-  cj[K] = sqrtl(kappa);
-  for (int j = K + 1; j < 2 * K; ++j) cj[j] = kappa / cj[2 * K - j];
-  long double wl[K];
-  for (int l = 0; l < K; ++l) {
-    long double v = 1.0L;
-    for (int i = 0; i < K; ++i) {
-      if (i < K - 1) v *= cj[2 * i + 2] - cj[2 * l + 1];
-      if (i != l) v /= cj[2 * i + 1] - cj[2 * l + 1];
-    }
-    wl[l] = v;
-  }
-  // the relative error equioscillates: scale to its midpoint
-  long double lo = 1e30L, hi = 0.0L;
-  for (int g = 0; g <= 2000; ++g) {
-    const long double x = powl(kappa, g / 2000.0L);
-    long double f = 0.0L;
-    for (int l = 0; l < K; ++l) f += wl[l] / (x + cj[2 * l + 1]);
-    f *= sqrtl(x);
-    lo = fminl(lo, f);
-    hi = fmaxl(hi, f);
-  }
-  for (int l = 0; l < K; ++l) {
-    s[l] = (double)cj[2 * l + 1];
-    w[l] = (double)(wl[l] * 2.0L / (lo + hi));
-  }
-  s[K] = 0.0;
-  w[K] = 0.0;
-}
-
-std::mutex g_pole_mu;
-bool g_pole_done[64] = {};
-
-}  // namespace
-
-// Fills the current device's table (once per device, before any launch).
-hipError_t init_poles(int device) {
-  std::lock_guard<std::mutex> lock(g_pole_mu);
-  if (device >= 0 && device < 64 && g_pole_done[device]) return hipSuccess;
-  static double host[kBuckets][2][32];
-  long double kappa = 1.0L;
-  for (int b = 0; b < kBuckets; ++b) {
-    kappa *= 4.0L;
-    zolotarev(kappa, host[b][0], host[b][1]);
-  }
-  const hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(g_poles), host, sizeof host);
-  if (e == hipSuccess && device >= 0 && device < 64) g_pole_done[device] = true;
-  return e;
-}
 
 // ---------------------------------------------------------------------------
 // R, a and v of a zone, one workgroup per zone, NP/16 waves:
@@ -206,6 +123,7 @@ __device__ __forceinline__ void load_poles4(const double* arr, int r, int k4, do
 template <int NP, bool DUAL, bool LIKE, typename TR>
 __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ sel_ptr,
+                                                    const double* __restrict__ ptab,
                                                     double* __restrict__ qmat,
                                                     const double* __restrict__ dvec,
                                                     const double* __restrict__ evec,
@@ -257,8 +175,8 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     // lanes 0..31 rows 0 .. NP/2 - 1 downwards, lanes 32..63 the rest upwards
     const int j = lane & 31;
     const bool bot = lane >= 32;
-    const double s = g_poles[bk][0][j], sp1 = 1.0 + s;
-    double wj = g_poles[bk][1][j];
+    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s;
+    double wj = ptab[bk * kPoleSet + 32 + j];
     if (DUAL) wj = wj * s / sp1;
     const int h0 = bot ? NP / 2 : 0;
     const double* dd = S.p.d + h0;
@@ -430,8 +348,8 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     load_poles4(arr, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(o[4]));
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      double w = g_poles[bk][1][8 * lr + q];
-      if (DUAL) w = w / (1.0 + g_poles[bk][0][8 * lr + q]);
+      double w = ptab[bk * kPoleSet + 32 + 8 * lr + q];
+      if (DUAL) w = w / (1.0 + ptab[bk * kPoleSet + 8 * lr + q]);
       o[q] *= w;
     }
   };
@@ -896,6 +814,7 @@ struct FuncSmallLds {
 template <int NP>
 __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                       const int64_t* __restrict__ sel_ptr,
+                                                      const double* __restrict__ ptab,
                                                       const double* __restrict__ qmat,
                                                       const double* __restrict__ dvec,
                                                       const double* __restrict__ evec,
@@ -952,7 +871,7 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
   const int jx = (j & ~1) ^ (H == 8 && bot ? 16 : 0);
   auto at = [&](int i) { return i * 32 + (jx ^ (2 * i)) + (j & 1); };
   {
-    const double s = g_poles[bk][0][j], sp1 = 1.0 + s, wj = g_poles[bk][1][j];
+    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s, wj = ptab[bk * kPoleSet + 32 + j];
     double* cc = S.p.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
     double* c1 = S.p.c[1] + h0;
     double qv[H], zv[H], ev[H];
@@ -1016,7 +935,7 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
   // eight poles a lane, the other one by a product with the identity ----
   double w8[8];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) w8[q] = g_poles[bk][1][8 * lr + q];
+  for (int q = 0; q < 8; ++q) w8[q] = ptab[bk * kPoleSet + 32 + 8 * lr + q];
   d4 f[NB][NB];
 #pragma unroll
   for (int J = 0; J < NB; ++J) {
@@ -1294,6 +1213,7 @@ struct PoleLds {
 
 __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ sel_ptr,
+                                                    const double* __restrict__ ptab,
                                                     const double* __restrict__ qmat,
                                                     const double* __restrict__ dvec,
                                                     const double* __restrict__ evec, double* poles,
@@ -1336,7 +1256,7 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
     bk = __builtin_amdgcn_readfirstlane(bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk));
     const int j = lane & 31;
     const bool bot = lane >= 32, up = (lane & 16) != 0;
-    const double s = g_poles[bk][0][j], sp1 = 1.0 + s, wj = g_poles[bk][1][j];
+    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s, wj = ptab[bk * kPoleSet + 32 + j];
     const int h0 = bot ? H : 0;
     const double* dd = S.d + h0;
     const double* ee = S.e + h0;
@@ -1640,7 +1560,7 @@ void launch_omega_rows128(const ChunkArgs& A, hipStream_t st) {
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
 #define OAK_FUNC(P, D, LK, TR)                                                                     \
   hipLaunchKernelGGL((k_func<P, D, LK, TR>), dim3(A.nzc), dim3(4 * P), 0, st, A.z0, A.zorder, A.N, \
-                     A.sel_ptr, A.ymat, A.dvec, A.evec, A.vec, A.ampl, A.err)
+                     A.sel_ptr, A.poles, A.ymat, A.dvec, A.evec, A.vec, A.ampl, A.err)
   if (NP == 64) {
     launch_tridiag_lower64(A, dual ? -1 : A.N, st);
     if (dual)
@@ -1667,7 +1587,7 @@ void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st) {
                        A.z0, A.zorder, A.nzc, A.N, A.sel_ptr, A.mat, A.ymat, A.dvec, A.evec,       \
                        A.vec);                                                                     \
     hipLaunchKernelGGL(k_func_small<P>, dim3(A.nzc), dim3(64), 0, st, A.z0, A.zorder, A.N,         \
-                       A.sel_ptr, A.ymat, A.dvec, A.evec, A.mat, A.vec, A.ampl, A.err);            \
+                       A.sel_ptr, A.poles, A.ymat, A.dvec, A.evec, A.mat, A.vec, A.ampl, A.err);            \
   } while (0)
   if (NP == 16)
     OAK_SMALL(16);
@@ -1679,8 +1599,8 @@ void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st) {
 // N > 128: the pole arrays to umat, T_b to the rows of ymat that the reduction's
 // trailing block leaves (128 .. 191), a and v.
 void launch_pole256(const ChunkArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL(k_pole256, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.ymat,
-                     A.dvec, A.evec, A.umat, A.ymat + 128 * 256, A.vec, A.ampl, A.err);
+  hipLaunchKernelGGL(k_pole256, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.poles,
+                     A.ymat, A.dvec, A.evec, A.umat, A.ymat + 128 * 256, A.vec, A.ampl, A.err);
 }
 
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {
