@@ -77,6 +77,14 @@ __device__ __forceinline__ const double* reflector256(const double* V, int k, in
   return k < 128 ? V + k * 256 + r : V + 192 * 256 + (k - 128) * 128 + (r < 128 ? 0 : r - 128);
 }
 
+// What k_pole256 leaves for the products that form F at N > 128, in doubles of a
+// zone: the arrays of a block of poles (in a matrix of their own), and, after T_b,
+// the weights and G_hh of each block or the 256 weights of the eigenvectors, and
+// the number of blocks (0: eigenvectors).
+struct PoleSet256 {
+  static constexpr int kArrays = 4 * 256 * 32, kWeights = 16 * 136, kCount = kWeights + 256;
+};
+
 // T = R Omega (below) with R v = kappa 1, kappa = 1 / |M^1/2 1|, and R 1 known: row c
 // of T is T[c][s] = R[c][s] + p_c + q_c v_s for s < N - 1, and T[c][N-1] = p_c + l_c
 // (the names as below: p = c1 + c2 wN, q = c3, l = c2).

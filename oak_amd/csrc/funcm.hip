@@ -1,17 +1,16 @@
 // The matrix functions of M = I + C that the analysis needs, from its
-// tridiagonal form M = Q T Q^T (N > 32), without eigenvectors:
+// tridiagonal form M = Q T Q^T, without eigenvectors:
 //
 //   R = M^-1/2                 (rrsqrt.F90:185; the transform is R Omega)
 //   a = M^-1 b                 (rrsqrt.F90:142)
 //   v = M^1/2 1 / |M^1/2 1|    (rrsqrt.F90:176-177)
 //
 // x^-1/2 on [1, kappa] is Zolotarev's best rational approximation in partial
-// fractions, sum_j w_j / (x + s_j) with 31 poles -s_j < 0 (N. J. Higham,
-// "Functions of Matrices", 2008, section 5.2; J. van den Eshof et al., Comput.
-// Phys. Commun. 146, 2002; N. Hale, N. J. Higham and L. N. Trefethen, SIAM J.
-// Numer. Anal. 46, 2008).  Its relative error is 5e-16 at kappa = 1e6 and
-// grows to 1e-7 at 1e15, four orders below the eps kappa by which rounding C
-// moves M^-1/2 in any case.  Then
+// fractions, sum_j w_j / (x + s_j) with poles -s_j < 0 (N. J. Higham, "Functions
+// of Matrices", 2008, section 5.2; J. van den Eshof et al., Comput. Phys. Commun.
+// 146, 2002), for kappa above a bound of T's spectrum: 31 poles, a lane each, up
+// to kappa = 2^20, 63 in two blocks one after the other up to 2^44, to 4.3e-16
+// either way (poles.hpp).  Then
 //
 //   T^-1/2 = sum_j w_j (T + s_j)^-1,  T^1/2 c = sum_j w_j (c - s_j (T + s_j)^-1 c)
 //
@@ -25,13 +24,20 @@
 //
 // for m the neighbour of i towards the middle and every k at or beyond m.
 // T >= I (M is I plus a positive semidefinite matrix), so every exact pivot is
-// at least 1 + s: a pivot that rounding leaves below is set to it, as
-// rrsqrt.F90:137 clamps the eigenvalues.  One lane per pole and half runs the
-// recurrences, NP/2 rows in and NP/2 rows out; a QL iteration with its ~1.1
-// N^2 plane rotations on the rows of Q, which this replaces, took 22 of the 45
-// ms of the eigensolve of 64 800 zones at N = 128.
+// at least 1 + s: a pivot that rounding leaves below is set to it.  One lane per
+// pole and half runs the recurrences, NP/2 rows in and NP/2 rows out; a QL
+// iteration with its ~1.1 N^2 plane rotations on the rows of Q, which this
+// replaces, took 22 of the 45 ms of the eigensolve of 64 800 zones at N = 128.
+//
+// Above kappa = 2^44 rounding C has moved T's small eigenvalues by a part of 1 and
+// more.  A zone with fewer such precise observations than members can be
+// indefinite, bounded pivots are no bound on G then (Sa came out up to 1e266 off),
+// and only the eigenvalues can be cut off at 1 as rrsqrt.F90:137 does: these zones
+// take QL (ql_functions) in the kernel that meets them.
 #include <math.h>
+#include <stddef.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -41,6 +47,197 @@
 #include "poles.hpp"
 
 namespace oakg {
+
+// ---------------------------------------------------------------------------
+// Zones beyond the poles: eigenvalues and eigenvectors of T by implicit QL
+// (A. Dubrulle, R. S. Martin and J. H. Wilkinson, Numer. Math. 12, 1968), a sweep's
+// rotations by the last wave while a thread per row applies the sweep before.
+// Called by the NT threads of a workgroup; Z: NP x NP in LDS or global memory, row k
+// of it eigenvector k.
+// T comes with its rows in reverse: the reduction leaves the strongly observed
+// directions in the first rows, and QL wants the large entries last (with them first,
+// the small eigenvalues came out ten times less accurate).
+// Negligible couplings are those below the rounding of the largest entries, too: with
+// fewer observations than members the reduction leaves no others after some rows, and
+// QL is soon done.  Bound by the chain of the 1.1 NP^2 rotations otherwise, and at N > 64
+// by the rows of Z through the caches.  4096 zones of N = 128 with 256 observations of
+// a ten millionth of the spread: 29 ms with the reduction, with 32 of them 6.1 (two
+// blocks of poles 5.5, one 2.2; QL over the lanes of a wave, a zone each, took 9.5 and
+// 3.5 in all).
+// ---------------------------------------------------------------------------
+template <int NP>
+struct QlLds {
+  double d[NP], e[NP];     // T, last row first (e_i couples i and i + 1); then the weights of F in e
+  double c[2][NP];         // cosines of two sweeps; then Z^T u in c[0] and s[0]
+  double u[2][NP];         // Q^T b, Q^T 1; then x, y
+  double s[2][NP];         // sines
+  int range[2][2];         // the sweeps' first and last row; -1: no sweep
+};
+
+// Largest |d| + |e| of T below 2^ex (of a finite T; 1025 for infinities).
+__device__ __forceinline__ int exponent_above(double nt) { return (__double2hiint(nt) >> 20) - 1022; }
+
+// The next sweep's rotations (one wave, every lane the same numbers).
+template <int NP>
+__device__ __forceinline__ void ql_sweep(QlLds<NP>& S, double tiny, int buf) {
+  const int lane = threadIdx.x & 63;
+  // the first coupling lo that is not negligible, and the first after it that is
+  int lo = -1, hi = -1;
+  for (int b = 0; b < NP && hi < 0; b += 64) {
+    const int i = b + lane;
+    const bool live = i < NP - 1 && fabs(S.e[i < NP ? i : 0]) >
+                                        fmax(0x1p-53 * (fabs(S.d[i < NP ? i : 0]) + fabs(S.d[i < NP - 1 ? i + 1 : 0])), tiny);
+    const unsigned long long on = __ballot(live);
+    unsigned long long off = ~on;
+    if (lo < 0) {
+      if (on == 0) continue;
+      const int t = __ffsll((long long)on) - 1;
+      lo = b + t;
+      off &= ~((2ull << t) - 1ull);
+    }
+    if (off != 0) hi = b + __ffsll((long long)off) - 1;
+  }
+  if (lo >= 0) {
+    const double dl = S.d[lo], el = S.e[lo];
+    double dn = S.d[hi], di = S.d[hi - 1], ei = S.e[hi - 1];  // rows i + 1 and i
+    double g = (S.d[lo + 1] - dl) / (2.0 * el);
+    g = dn - dl + el / (g + copysign(sqrt(fma(g, g, 1.0)), g));
+    double s = 1.0, c = 1.0, p = 0.0;
+    for (int i = hi - 1; i >= lo; --i) {
+      const int nx = i > lo ? i - 1 : lo;
+      const double dx = S.d[nx], ex = S.e[nx];  // the next row's, ahead of the chain
+      const double f = s * ei, b = c * ei, hh = fma(f, f, g * g);
+      const bool turns = hh > 0x1p-900;  // else no rotation
+      const double rn = rsqrt_acc(turns ? hh : 1.0);
+      s = turns ? f * rn : 0.0;
+      c = turns ? g * rn : 1.0;
+      S.e[i + 1] = turns ? hh * rn : 0.0;
+      g = dn - p;
+      const double q = fma(di - g, s, 2.0 * c * b);
+      p = s * q;
+      S.d[i + 1] = g + p;
+      g = fma(c, q, -b);
+      S.c[buf][i] = c;
+      S.s[buf][i] = s;
+      dn = di;
+      di = dx;
+      ei = ex;
+    }
+    S.d[lo] = dl - p;
+    S.e[lo] = g;
+    S.e[hi] = 0.0;
+  }
+  if (lane == 0) {
+    S.range[buf][0] = lo;
+    S.range[buf][1] = hi;
+  }
+}
+
+template <int NP, int NT, bool DUAL, bool LIKE>
+__device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z, double* like) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const bool leads = wave == NT / 64 - 1;
+  if (tid < NP)
+    for (int k = 0; k < NP; ++k) Z[(size_t)k * NP + tid] = k == NP - 1 - tid ? 1.0 : 0.0;
+  // couplings that are rounding of the largest entries: with as many members as
+  // observations and more the reduction leaves only those after some rows
+  const double tiny = 0x1p-53 * nt;
+  if (leads) ql_sweep<NP>(S, tiny, 0);
+  __syncthreads();
+  // two sweeps an eigenvalue are usual; the bound ends any other case
+#pragma unroll 1
+  for (int sweep = 0; sweep < 40 * NP; ++sweep) {
+    const int buf = sweep & 1, lo = S.range[buf][0], hi = S.range[buf][1];
+    if (lo < 0) break;
+    if (leads) ql_sweep<NP>(S, tiny, buf ^ 1);
+    if (tid < NP) {
+      // eight rows at a time, with the next eight (clamped to lo) in flight
+      constexpr int Q = 8;
+      auto at = [&](int i) { return i > lo ? i : lo; };
+      double zc = Z[(size_t)hi * NP + tid], zi[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) zi[q] = Z[(size_t)at(hi - 1 - q) * NP + tid];
+#pragma unroll 1
+      for (int i0 = hi - 1; i0 >= lo; i0 -= Q) {
+        double zn[Q], c[Q], s[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          zn[q] = Z[(size_t)at(i0 - Q - q) * NP + tid];
+          c[q] = S.c[buf][at(i0 - q)];
+          s[q] = S.s[buf][at(i0 - q)];
+        }
+        if (i0 - Q + 1 >= lo) {
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            Z[(size_t)(i0 - q + 1) * NP + tid] = fma(s[q], zi[q], c[q] * zc);
+            zc = fma(c[q], zi[q], -s[q] * zc);
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+            if (i0 - q >= lo) {
+              Z[(size_t)(i0 - q + 1) * NP + tid] = fma(s[q], zi[q], c[q] * zc);
+              zc = fma(c[q], zi[q], -s[q] * zc);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) zi[q] = zn[q];
+      }
+      Z[(size_t)lo * NP + tid] = zc;
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  // Z^T u, a wave per eigenvector, times the functions of mu = max(lambda, 1)
+  double slog = 0.0, sinv = 0.0, sba = 0.0;
+#pragma unroll 1
+  for (int k = wave; k < NP; k += NT / 64) {
+    double t0 = 0.0, t1 = 0.0;
+    for (int r = lane; r < NP; r += 64) {
+      const double zr = Z[(size_t)k * NP + r];
+      t0 = fma(zr, S.u[0][r], t0);
+      t1 = fma(zr, S.u[1][r], t1);
+    }
+    t0 = wave_sum_fast(t0);
+    t1 = wave_sum_fast(t1);
+    const double mu = S.d[k] < 1.0 ? 1.0 : S.d[k], sq = sqrt(mu);
+    if (lane == 0) {
+      S.c[0][k] = t0 / mu;
+      S.s[0][k] = DUAL ? t1 / (1.0 + sq) : t1 * sq;
+      S.e[k] = DUAL ? 1.0 / (mu + sq) : 1.0 / sq;
+    }
+    if (LIKE) {
+      slog += log(mu);
+      sinv += 1.0 - 1.0 / mu;
+      sba = fma(t0 / mu, t0, sba);
+    }
+  }
+  __syncthreads();
+  if (LIKE) {  // the waves' shares (u is still wanted: through d)
+    if (lane == 0) {
+      S.d[3 * wave] = slog;
+      S.d[3 * wave + 1] = sinv;
+      S.d[3 * wave + 2] = sba;
+    }
+    __syncthreads();
+    if (tid < 3) {
+      double t = 0.0;
+      for (int w = 0; w < NT / 64; ++w) t += S.d[3 * w + tid];
+      like[tid] = t;
+    }
+  }
+  if (tid < NP) {
+    double x = 0.0, y = 0.0;
+    for (int k = 0; k < NP; ++k) {
+      const double zk = Z[(size_t)k * NP + tid];
+      x = fma(zk, S.c[0][k], x);
+      y = fma(zk, S.s[0][k], y);
+    }
+    S.u[0][tid] = x;
+    S.u[1][tid] = y;
+  }
+  __syncthreads();
+}
 
 // ---------------------------------------------------------------------------
 // R, a and v of a zone, one workgroup per zone, NP/16 waves:
@@ -92,10 +289,12 @@ struct FuncLds {
       double g[2][16];        // V^T [x, y]
       double t[2][16];        // T_b V^T [x, y]
     } m;
+    QlLds<NP> q;
   };
   double tp[NB * 136];  // T_b, packed by columns (upper triangles)
   double c[2][NP];      // x, y; then a, v
-  int bucket;
+  double bound;         // of T's spectrum
+  int first, count;     // the blocks of poles; count 0: QL
 };
 
 // place of row r in the elimination order, and back
@@ -120,219 +319,42 @@ __device__ __forceinline__ void load_poles4(const double* arr, int r, int k4, do
   }
 }
 
-template <int NP, bool DUAL, bool LIKE, typename TR>
-__global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
-                                                    const int64_t* __restrict__ sel_ptr,
-                                                    const double* __restrict__ ptab,
-                                                    double* __restrict__ qmat,
-                                                    const double* __restrict__ dvec,
-                                                    const double* __restrict__ evec,
-                                                    double* __restrict__ vec, double* __restrict__ ampl,
-                                                    unsigned* __restrict__ err) {
+// DEEP false: a zone of one block of poles (else false is returned); true: one of two
+// or of none.
+template <int NP, bool DUAL, bool LIKE, typename TR, bool DEEP>
+__device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int N, int64_t cnt_obs,
+                                          const double* __restrict__ ptab, double* __restrict__ qmat,
+                                          const double* __restrict__ dvec,
+                                          const double* __restrict__ evec,
+                                          double* __restrict__ mat, double* __restrict__ vec,
+                                          double* __restrict__ ampl, unsigned* __restrict__ err) {
   using L = FuncLds<NP>;
   constexpr int NB = L::NB, LV = L::LV;
   constexpr int TPR = NP / 4, ER = 4;  // threads per reflector of a block, rows of each
-  __shared__ L S;
-  const int zl = blockIdx.x;
-  const int64_t z = zone_at(zorder, z0 + zl);
-  if (z < 0) return;  // the zone is solved by the other pipeline
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane >> 4, lc = lane & 15;
   double* Vz = vec + (size_t)zl * 4 * NP;
-  if (sel_ptr[z + 1] == sel_ptr[z]) {  // no observations: a = 0
-    if (tid < NP) Vz[NP + tid] = 0.0;
-    return;
-  }
   double* V = qmat + (size_t)zl * NP * NP;
   // order of M (the rest is the identity): the tiles and reflector blocks that
   // reach it take part
-  const int n = DUAL ? (int)(sel_ptr[z + 1] - sel_ptr[z]) : N;
+  const int n = DUAL ? (int)cnt_obs : N;
   const int nt = (n + 15) >> 4, nblk = n > 2 ? (n + 13) >> 4 : 0;
-  if (tid < NP) {
-    const int k = step_row<NP>(tid);
-    S.p.d[k] = dvec[(size_t)zl * NP + tid];
-    S.p.e[k] = evec[(size_t)zl * NP + (tid < NP / 2 ? tid : tid - 1)];
-    S.p.c[0][k] = Vz[tid];
-    S.p.c[1][k] = Vz[2 * NP + tid];
-  }
+  auto load_t = [&]() {
+    if (tid < NP) {
+      const int k = step_row<NP>(tid);
+      S.p.d[k] = dvec[(size_t)zl * NP + tid];
+      S.p.e[k] = evec[(size_t)zl * NP + (tid < NP / 2 ? tid : tid - 1)];
+      S.p.c[0][k] = Vz[tid];
+      S.p.c[1][k] = Vz[2 * NP + tid];
+    }
+  };
+  load_t();
   lds_barrier();
-  if (wave == 0) {
-    // ---- pivots and solves, one lane per pole ----
-    double nt = 0.0;  // Gershgorin bound of T
-#pragma unroll
-    for (int h = 0; h < NP / 64; ++h) {
-      const int k = lane + 64 * h;  // k's outer neighbour couples through e of k - 1
-      nt = fmax(nt, fabs(S.p.d[k]) + fabs(S.p.e[k]) + (k % (NP / 2) ? fabs(S.p.e[k - 1]) : 0.0));
-    }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
-    // smallest kappa = 4^(bucket+1) >= nt (nt < 2^ex); any nt gives a row of the table
-    const int ex = (__double2hiint(nt) >> 20) - 1022;
-    int bk = ((ex + 1) >> 1) - 1;
-    bk = bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk);
-    bk = __builtin_amdgcn_readfirstlane(bk);
-    if (lane == 0) S.bucket = bk;
-    // lanes 0..31 rows 0 .. NP/2 - 1 downwards, lanes 32..63 the rest upwards
-    const int j = lane & 31;
-    const bool bot = lane >= 32;
-    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s;
-    double wj = ptab[bk * kPoleSet + 32 + j];
-    if (DUAL) wj = wj * s / sp1;
-    const int h0 = bot ? NP / 2 : 0;
-    const double* dd = S.p.d + h0;
-    const double* ee = S.p.e + h0;
-    double* cc = S.p.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
-    double* c1 = S.p.c[1] + h0;
-    double* aa = S.p.a + h0 * 32;
-    double* gg = S.p.g + h0 * 32;
-    // position of the lane's pole in the row of step 16 t + i (i constant)
-    auto at = [&](int t, int i) { return (16 * t + i) * 32 + ((j & ~1) ^ (2 * i)) + (j & 1); };
-    double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
-#pragma unroll 1
-    for (int t = 0; t < NB / 2; ++t) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        asm volatile("" ::: "memory");  // the reads of eight rows at a time
-        double dv[8], ev[8], cv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int k = 16 * t + 8 * h + i;
-          dv[i] = dd[k];
-          ev[i] = ee[k];
-          cv[i] = cc[k];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
-          z1 = fma(tau, z1, cv[i]);
-          aa[at(t, 8 * h + i)] = q;
-          gg[at(t, 8 * h + i)] = z1 * q;
-          tau = -ev[i] * q;
-          e2 = ev[i] * ev[i];
-        }
-      }
-    }
-    // the middle: q, z1 of rows h (top lanes) and h + 1 (bottom lanes);
-    // 1 / G_hh = gamma_h - e_h^2 / gamma_{h+1}, x_h = G_hh (z_h + tau_{h+1} z_{h+1})
-    double G, x;
-    {
-      const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
-      const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
-      const double eh = S.p.e[NP / 2 - 1];
-      G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
-      x = G * fma(-eh * qb, zb, zh);
-      if (!bot) S.p.d[j] = G;
-    }
-    double slog = LIKE && !bot ? -log(G) : 0.0, sinv = 0.0, sba = 0.0;
-#pragma unroll 1
-    for (int t = NB / 2 - 1; t >= 0; --t) {
-#pragma unroll
-      for (int h = 1; h >= 0; --h) {
-        asm volatile("" ::: "memory");
-        double iv[8], zi[8], ev[8], tv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int k = 16 * t + 8 * h + i;
-          iv[i] = aa[at(t, 8 * h + i)];
-          zi[i] = gg[at(t, 8 * h + i)];
-          ev[i] = ee[k];
-          tv[i] = c1[k];
-        }
-#pragma unroll
-        for (int i = 7; i >= 0; --i) {
-          double r = -ev[i] * iv[i];
-          const double gn = fma(r * r, G, iv[i]), xn = fma(r, x, zi[i]);
-          if (h == 1 && i == 7) {
-            // row h itself: G and x as they are, and 1 for tau
-            const bool mid = !bot && t == NB / 2 - 1;
-            if (LIKE) slog -= mid ? 0.0 : log(iv[i]);
-            G = mid ? G : gn;
-            x = mid ? x : xn;
-            r = mid ? 1.0 : r;
-          } else {
-            if (LIKE) slog -= log(iv[i]);
-            G = gn;
-            x = xn;
-          }
-          aa[at(t, 8 * h + i)] = r;
-          gg[at(t, 8 * h + i)] = G;
-          tv[i] = DUAL ? wj * x : wj * fma(-s, x, tv[i]);
-          if (LIKE) {
-            sinv += 1.0 - G;
-            sba = fma(S.p.c[0][h0 + 16 * t + 8 * h + i], x, sba);
-          }
-          if (j == 31) cc[16 * t + 8 * h + i] = x;
-        }
-        // sums over the poles: of each 32 lanes the lower 16 keep steps 0..3
-        // of the eight, the upper 16 steps 4..7
-        const bool up = (lane & 16) != 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
-          tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
-        }
-        if (lc == 0) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) c1[16 * t + 8 * h + (up ? 4 : 0) + i] = tv[i];
-        }
-      }
-    }
-    if (LIKE) {  // log det M, sum (1 - 1/mu) and b^T a
-      slog += shfl_xor_d(slog, 32);
-      sinv += shfl_xor_d(sinv, 32);
-      sba += shfl_xor_d(sba, 32);
-      if (lane == 31) {
-        Vz[3 * NP] = slog;
-        Vz[3 * NP + 1] = sinv;
-        Vz[3 * NP + 2] = sba;
-      }
-    }
-  } else {
-    // ---- T_b of the reflector blocks ----
-    for (int b = wave - 1; b < nblk; b += NB - 1) {
-      const int k = 16 * b + lc;
-      const double* src = V + (size_t)k * NP;
-      d4 g = {0.0, 0.0, 0.0, 0.0};
-      for (int k0 = 4 * b; k0 < 4 * nt; k0 += 4) {
-        double xv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) xv[u] = src[4 * (k0 + u) + lr];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const double xm = (k < n - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
-          g = mfma_f64(xm, xm, g);
-        }
-      }
-      const double tk = src[k];
-      const double tau = k < n - 2 ? tk : 0.0;
-      // V^T V packed into the block's place, then column by column replaced:
-      // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j]
-      double* gs = S.tp + b * 136;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (lr + 4 * r <= lc) gs[lc * (lc + 1) / 2 + lr + 4 * r] = g[r];
-      __builtin_amdgcn_wave_barrier();
-      double tr[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        asm volatile("" ::: "memory");  // column by column, not all loads at once
-        double sm = 0.0;
-#pragma unroll
-        for (int q = 0; q < j; ++q) sm = fma(tr[q], gs[j * (j + 1) / 2 + q], sm);
-        const double tj = readlane_d(tau, j);
-        tr[j] = lane < j ? -tj * sm : (lane == j ? tj : 0.0);
-        __builtin_amdgcn_wave_barrier();
-        if (lane <= j) gs[j * (j + 1) / 2 + lane] = tr[j];
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
-  lds_barrier();
-  // ---- F = T^-1/2, tile column J (waves w and w + 4 share a SIMD: the
+  // F = T^-1/2, tile column J (waves w and w + 4 share a SIMD: the
   // columns J and NB - 1 - J, whose updates add up alike).  The columns of the
   // lower half see the rows mirrored: f[I] is tile row I or NB - 1 - I, so that
   // I < Js lie outside the wave's own tile, Js < I < NB/2 towards the middle
-  // and the rest beyond it ----
+  // and the rest beyond it
   const int J = wave < NB / 2 ? wave : NB + NB / 2 - 1 - wave;
   const bool low = J >= NB / 2;
   const int Js = low ? NB - 1 - J : J;
@@ -340,126 +362,357 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
   // place of tile row r in the pole arrays (elimination order)
   auto tile_of = [&](int r) { return r < NB / 2 ? r : NB / 2 + NB - 1 - r; };
   d4 f[NB];
-  // column lc of tile J from arr, times the weights of the lane's eight poles
-  auto column_factors = [&](const double* arr, double (&o)[8]) {
-    const int bk = S.bucket;
-    const int row = 16 * tile_of(J) + (low ? 15 - lc : lc);
-    load_poles4(arr, row, 2 * lr, reinterpret_cast<double(&)[4]>(o[0]));
-    load_poles4(arr, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(o[4]));
+  double* Fz = mat + (size_t)zl * NP * NP;  // M is no longer needed
+#pragma unroll 1
+  for (int batch = 0;; ++batch) {
+    if (wave == 0) {
+      // ---- pivots and solves, one lane per pole ----
+      int blk = 0, cnt = 1;
+      if (batch == 0) {
+        double nt = 0.0;  // Gershgorin bound of T
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      double w = ptab[bk * kPoleSet + 32 + 8 * lr + q];
-      if (DUAL) w = w / (1.0 + ptab[bk * kPoleSet + 8 * lr + q]);
-      o[q] *= w;
+        for (int h = 0; h < NP / 64; ++h) {
+          const int k = lane + 64 * h;  // k's outer neighbour couples through e of k - 1
+          nt = fmax(nt, fabs(S.p.d[k]) + fabs(S.p.e[k]) + (k % (NP / 2) ? fabs(S.p.e[k - 1]) : 0.0));
+        }
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
+        const int ex = __builtin_amdgcn_readfirstlane(exponent_above(nt));
+        const PoleBlocks pb = pole_blocks(ex > 1024 ? 0 : ex);  // infinities end as NaN in a
+        blk = pb.first;
+        cnt = pb.count;
+        if (lane == 0) {
+          S.bound = nt;
+          S.first = blk;
+          S.count = cnt;
+        }
+        if (!DEEP && cnt != 1) cnt = 0;
+      } else {
+        blk = __builtin_amdgcn_readfirstlane(S.first + batch);
+      }
+      if (cnt != 0) {
+        // lanes 0..31 rows 0 .. NP/2 - 1 downwards, lanes 32..63 the rest upwards
+        const int j = lane & 31;
+        const bool bot = lane >= 32;
+        const bool tl = j == 31 && batch == 0;  // the lane of T itself
+        const double s = ptab[blk * kPoleBlock + j], sp1 = 1.0 + s;
+        double wj = ptab[blk * kPoleBlock + 32 + j];
+        if (DUAL) wj = wj * s / sp1;
+        const int h0 = bot ? NP / 2 : 0;
+        const double* dd = S.p.d + h0;
+        const double* ee = S.p.e + h0;
+        double* cc = S.p.c[tl ? 0 : 1] + h0;  // the lane's right-hand side
+        double* c1 = S.p.c[1] + h0;
+        double* aa = S.p.a + h0 * 32;
+        double* gg = S.p.g + h0 * 32;
+        // position of the lane's pole in the row of step 16 t + i (i constant)
+        auto at = [&](int t, int i) { return (16 * t + i) * 32 + ((j & ~1) ^ (2 * i)) + (j & 1); };
+        double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
+#pragma unroll 1
+        for (int t = 0; t < NB / 2; ++t) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            asm volatile("" ::: "memory");  // the reads of eight rows at a time
+            double dv[8], ev[8], cv[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const int k = 16 * t + 8 * h + i;
+              dv[i] = dd[k];
+              ev[i] = ee[k];
+              cv[i] = cc[k];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
+              z1 = fma(tau, z1, cv[i]);
+              aa[at(t, 8 * h + i)] = q;
+              gg[at(t, 8 * h + i)] = z1 * q;
+              tau = -ev[i] * q;
+              e2 = ev[i] * ev[i];
+            }
+          }
+        }
+        // the middle: q, z1 of rows h (top lanes) and h + 1 (bottom lanes);
+        // 1 / G_hh = gamma_h - e_h^2 / gamma_{h+1}, x_h = G_hh (z_h + tau_{h+1} z_{h+1})
+        double G, x;
+        {
+          const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+          const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+          const double eh = S.p.e[NP / 2 - 1];
+          G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+          x = G * fma(-eh * qb, zb, zh);
+          if (!bot) S.p.d[j] = G;
+        }
+        double slog = LIKE && !bot ? -log(G) : 0.0, sinv = 0.0, sba = 0.0;
+#pragma unroll 1
+        for (int t = NB / 2 - 1; t >= 0; --t) {
+#pragma unroll
+          for (int h = 1; h >= 0; --h) {
+            asm volatile("" ::: "memory");
+            double iv[8], zi[8], ev[8], tv[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const int k = 16 * t + 8 * h + i;
+              iv[i] = aa[at(t, 8 * h + i)];
+              zi[i] = gg[at(t, 8 * h + i)];
+              ev[i] = ee[k];
+              tv[i] = c1[k];
+            }
+#pragma unroll
+            for (int i = 7; i >= 0; --i) {
+              double r = -ev[i] * iv[i];
+              const double gn = fma(r * r, G, iv[i]), xn = fma(r, x, zi[i]);
+              if (h == 1 && i == 7) {
+                // row h itself: G and x as they are, and 1 for tau
+                const bool mid = !bot && t == NB / 2 - 1;
+                if (LIKE) slog -= mid ? 0.0 : log(iv[i]);
+                G = mid ? G : gn;
+                x = mid ? x : xn;
+                r = mid ? 1.0 : r;
+              } else {
+                if (LIKE) slog -= log(iv[i]);
+                G = gn;
+                x = xn;
+              }
+              aa[at(t, 8 * h + i)] = r;
+              gg[at(t, 8 * h + i)] = G;
+              tv[i] = DUAL ? wj * x : wj * fma(-s, x, tv[i]);
+              if (LIKE) {
+                sinv += 1.0 - G;
+                sba = fma(S.p.c[0][h0 + 16 * t + 8 * h + i], x, sba);
+              }
+              if (tl) cc[16 * t + 8 * h + i] = x;
+            }
+            // sums over the poles: of each 32 lanes the lower 16 keep steps 0..3
+            // of the eight, the upper 16 steps 4..7
+            const bool up = (lane & 16) != 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
+              tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
+            }
+            if (lc == 0) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) c1[16 * t + 8 * h + (up ? 4 : 0) + i] = tv[i];
+            }
+          }
+        }
+        if (LIKE) {  // log det M, sum (1 - 1/mu) and b^T a
+          slog += shfl_xor_d(slog, 32);
+          sinv += shfl_xor_d(sinv, 32);
+          sba += shfl_xor_d(sba, 32);
+          if (lane == 31 && batch == 0) {
+            Vz[3 * NP] = slog;
+            Vz[3 * NP + 1] = sinv;
+            Vz[3 * NP + 2] = sba;
+          }
+        }
+      }
+    } else if (batch == 0) {
+      // ---- T_b of the reflector blocks ----
+      for (int b = wave - 1; b < nblk; b += NB - 1) {
+        const int k = 16 * b + lc;
+        const double* src = V + (size_t)k * NP;
+        d4 g = {0.0, 0.0, 0.0, 0.0};
+        for (int k0 = 4 * b; k0 < 4 * nt; k0 += 4) {
+          double xv[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) xv[u] = src[4 * (k0 + u) + lr];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const double xm = (k < n - 2 && 4 * (k0 + u) + lr > k) ? xv[u] : 0.0;
+            g = mfma_f64(xm, xm, g);
+          }
+        }
+        const double tk = src[k];
+        const double tau = k < n - 2 ? tk : 0.0;
+        // V^T V packed into the block's place, then column by column replaced:
+        // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j]
+        double* gs = S.tp + b * 136;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (lr + 4 * r <= lc) gs[lc * (lc + 1) / 2 + lr + 4 * r] = g[r];
+        __builtin_amdgcn_wave_barrier();
+        double tr[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          asm volatile("" ::: "memory");  // column by column, not all loads at once
+          double sm = 0.0;
+#pragma unroll
+          for (int q = 0; q < j; ++q) sm = fma(tr[q], gs[j * (j + 1) / 2 + q], sm);
+          const double tj = readlane_d(tau, j);
+          tr[j] = lane < j ? -tj * sm : (lane == j ? tj : 0.0);
+          __builtin_amdgcn_wave_barrier();
+          if (lane <= j) gs[j * (j + 1) / 2 + lane] = tr[j];
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
     }
-  };
-  d4 fd = {0.0, 0.0, 0.0, 0.0};  // the diagonal tile
-  {
-    // lane (lr, lc) runs column lc outwards from its diagonal entry for its
-    // eight poles; the sums over the poles reach every lr, which keeps rows
-    // lr + 4 r of that triangle (i: the rows in elimination order)
-    double g[8];
-    column_factors(S.p.g, g);
-    d4 us;
-    const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
+    lds_barrier();
+    if (!DEEP && S.count != 1) return false;
+    if (DEEP && S.count == 0) break;
+    // F = T^-1/2: what the blocks before this one gave
+    if (batch > 0) {
 #pragma unroll
-    for (int i = 15; i >= 0; --i) {
-      if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f[I][r] = Fz[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc];
+    } else {
+#pragma unroll
+      for (int I = 0; I < NB; ++I) f[I] = d4{0.0, 0.0, 0.0, 0.0};
+    }
+    // column lc of tile J from arr, times the weights of the lane's eight poles
+    auto column_factors = [&](const double* arr, double (&o)[8]) {
+      const int blk = S.first + batch;
+      const int row = 16 * tile_of(J) + (low ? 15 - lc : lc);
+      load_poles4(arr, row, 2 * lr, reinterpret_cast<double(&)[4]>(o[0]));
+      load_poles4(arr, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(o[4]));
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        double w = ptab[blk * kPoleBlock + 32 + 8 * lr + q];
+        if (DUAL) w = w / (1.0 + ptab[blk * kPoleBlock + 8 * lr + q]);
+        o[q] *= w;
+      }
+    };
+    d4 fd = {0.0, 0.0, 0.0, 0.0};  // the diagonal tile
+    {
+      // lane (lr, lc) runs column lc outwards from its diagonal entry for its
+      // eight poles; the sums over the poles reach every lr, which keeps rows
+      // lr + 4 r of that triangle (i: the rows in elimination order)
+      double g[8];
+      column_factors(S.p.g, g);
+      d4 us;
+      const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
+#pragma unroll
+      for (int i = 15; i >= 0; --i) {
+        if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          double r[4];
+          load_poles4(S.p.a, 16 * tile_of(J) + i, 2 * lr + h, r);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? r[q] : 1.0;
+        }
+        const double sm =
+            sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+        if (i % 4 == 3) us[i / 4] = 0.0;
+        us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+      }
+      // the other triangle: the transpose by a product with the identity (exact)
+      d4 ut;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        ut[r] = low ? us[3 - r] : us[r];
+        fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+    }
+    if (tid < NP) {
+      const int k = step_row<NP>(tid);
+      if (batch == 0) S.c[0][tid] = S.p.c[0][k];
+      S.c[1][tid] = S.p.c[1][k] + (batch == 0 ? 0.0 : S.c[1][tid]);
+    }
+    lds_barrier();
+    // towards the middle edge of a row's tile: alpha = tau_i ... (row i to the
+    // edge), beta = G_ii times the tau between the outer edge and row i
+    if (tid < 32 * NB) {
+      const int t = tid >> 5, j = tid & 31;
+      double r[16], g[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int at = pole_at(16 * t + i, j);
+        r[i] = S.p.a[at];
+        g[i] = S.p.g[at];
+      }
+      double pi = 1.0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        g[i] *= pi;
+        pi *= r[i];
+      }
+#pragma unroll
+      for (int i = 14; i >= 0; --i) r[i] *= r[i + 1];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int at = pole_at(16 * t + i, j);
+        S.p.a[at] = r[i];
+        S.p.g[at] = g[i];
+      }
+    }
+    lds_barrier();
+    // off the diagonal: rows from arr, columns in B, both relative to the tile
+    // edges (alpha of a tile's outermost row is the tile's whole product); four
+    // poles at a time keep the operands few
+    auto tile = [&](const double* arr, int I, double (&B)[8], d4 acc) {
+      const int rI = row_of(I), t16 = 16 * tile_of(rI);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        double r[4];
-        load_poles4(S.p.a, 16 * tile_of(J) + i, 2 * lr + h, r);
+        double av[4], edge[4];
+        load_poles4(arr, t16 + (rI < NB / 2 ? lc : 15 - lc), 2 * lr + h, av);
+        load_poles4(S.p.a, t16, 2 * lr + h, edge);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? r[q] : 1.0;
+        for (int q = 0; q < 4; ++q) {
+          acc = mfma_f64(av[q], B[4 * h + q], acc);
+          B[4 * h + q] *= edge[q];
+        }
+        asm volatile("" ::: "memory");
       }
-      const double sm =
-          sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
-      if (i % 4 == 3) us[i / 4] = 0.0;
-      us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
-    }
-    // the other triangle: the transpose by a product with the identity (exact)
-    d4 ut;
+      return acc;
+    };
+    {
+      double B[8];
+      column_factors(S.p.g, B);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ut[r] = low ? us[3 - r] : us[r];
-      fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
-    }
+      for (int I = NB / 2 - 2; I >= 0; --I)  // outside
+        if (I < Js && J < nt && row_of(I) < nt) f[I] = tile(S.p.a, I, B, f[I]);
+      column_factors(S.p.a, B);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
-  }
-  if (tid < NP) {
-    const int k = step_row<NP>(tid);
-    S.c[0][tid] = S.p.c[0][k];
-    S.c[1][tid] = S.p.c[1][k];
-  }
-  lds_barrier();
-  // towards the middle edge of a row's tile: alpha = tau_i ... (row i to the
-  // edge), beta = G_ii times the tau between the outer edge and row i
-  if (tid < 32 * NB) {
-    const int t = tid >> 5, j = tid & 31;
-    double r[16], g[16];
+      for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
+        if (I == NB / 2) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int at = pole_at(16 * t + i, j);
-      r[i] = S.p.a[at];
-      g[i] = S.p.g[at];
-    }
-    double pi = 1.0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      g[i] *= pi;
-      pi *= r[i];
-    }
-#pragma unroll
-    for (int i = 14; i >= 0; --i) r[i] *= r[i + 1];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int at = pole_at(16 * t + i, j);
-      S.p.a[at] = r[i];
-      S.p.g[at] = g[i];
-    }
-  }
-  lds_barrier();
-  // off the diagonal: rows from arr, columns in B, both relative to the tile
-  // edges (alpha of a tile's outermost row is the tile's whole product); four
-  // poles at a time keep the operands few
-  auto tile = [&](const double* arr, int I, double (&B)[8]) {
-    const int rI = row_of(I), t16 = 16 * tile_of(rI);
-    d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      double av[4], edge[4];
-      load_poles4(arr, t16 + (rI < NB / 2 ? lc : 15 - lc), 2 * lr + h, av);
-      load_poles4(S.p.a, t16, 2 * lr + h, edge);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        acc = mfma_f64(av[q], B[4 * h + q], acc);
-        B[4 * h + q] *= edge[q];
+          for (int q = 0; q < 8; ++q) B[q] *= S.p.d[8 * lr + q];
+        }
+        if (I > Js && J < nt && row_of(I) < nt) f[I] = tile(I < NB / 2 ? S.p.g : S.p.a, I, B, f[I]);
       }
-      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int I = 0; I < NB / 2; ++I)
+        if (I == Js) f[I] += fd;
     }
-    return acc;
-  };
-  {
-    double B[8];
-    column_factors(S.p.g, B);
+    if (!DEEP || batch + 1 >= S.count) break;
+    // another block: F so far to memory, d and Q^T 1 again
 #pragma unroll
-    for (int I = NB / 2 - 2; I >= 0; --I)  // outside
-      if (I < Js) f[I] = J < nt && row_of(I) < nt ? tile(S.p.a, I, B) : d4{0.0, 0.0, 0.0, 0.0};
-    column_factors(S.p.a, B);
+    for (int I = 0; I < NB; ++I)
 #pragma unroll
-    for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
-      if (I == NB / 2) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) B[q] *= S.p.d[8 * lr + q];
-      }
-      if (I > Js)
-        f[I] = J < nt && row_of(I) < nt ? tile(I < NB / 2 ? S.p.g : S.p.a, I, B)
-                                        : d4{0.0, 0.0, 0.0, 0.0};
+      for (int r = 0; r < 4; ++r) Fz[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = f[I][r];
+    lds_barrier();
+    load_t();
+    lds_barrier();
+  }
+  if (DEEP && S.count == 0) {
+    // F, x and y from the eigenvectors, which go where M was
+    const double bound = S.bound;
+    if (tid < NP) {
+      S.q.d[NP - 1 - tid] = dvec[(size_t)zl * NP + tid];
+      S.q.e[tid] = tid < NP - 1 ? evec[(size_t)zl * NP + NP - 2 - tid] : 0.0;
+      S.q.u[0][tid] = Vz[tid];
+      S.q.u[1][tid] = Vz[2 * NP + tid];
+    }
+    __syncthreads();
+    ql_functions<NP, 4 * NP, DUAL, LIKE>(S.q, bound, Fz, Vz + 3 * NP);
+    if (tid < NP) {
+      S.c[0][tid] = S.q.u[0][tid];
+      S.c[1][tid] = S.q.u[1][tid];
     }
 #pragma unroll
-    for (int I = 0; I < NB / 2; ++I)
-      if (I == Js) f[I] = fd;
+    for (int I = 0; I < NB; ++I) f[I] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int k = 0; k < NP; k += 4) {
+      const double* zk = Fz + (size_t)(k + lr) * NP + lc;
+      const double b = S.q.e[k + lr] * zk[16 * J];
+#pragma unroll
+      for (int I = 0; I < NB; ++I) f[I] = mfma_f64(zk[16 * row_of(I)], b, f[I]);
+    }
   }
   // ---- R = Q F Q^T, [a, v] = Q [x, y] ----
   // thread t moves reflector pj of a block, rows pr + TPR e (loaded whole,
@@ -657,6 +910,51 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     if (ampl && tid < N) ampl[(size_t)z * N + tid] = ar;
     if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
   }
+  return true;
+}
+
+// The workgroup's LDS: one variable for k_func and for deep_zone, which it calls.
+template <int NP>
+__device__ __forceinline__ FuncLds<NP>& func_lds() {
+  __shared__ FuncLds<NP> S;
+  return S;
+}
+
+// A function of its own: inside k_func its loops made the tiles of every zone spill, and
+// as kernels after k_func they cost 50 us of 1.2 ms at 5490 zones of N = 40 in waiting
+// for a place on the device.
+template <int NP, bool DUAL, bool LIKE, typename TR>
+__device__ __attribute__((noinline)) void deep_zone(int zl, int64_t z, int N, int64_t cnt,
+                                                    const double* ptab, double* qmat, const double* dvec,
+                                                    const double* evec, double* mat, double* vec,
+                                                    double* ampl, unsigned* err) {
+  func_zone<NP, DUAL, LIKE, TR, true>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl,
+                                      err);
+}
+
+template <int NP, bool DUAL, bool LIKE, typename TR>
+__global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
+                                                    const int64_t* __restrict__ sel_ptr,
+                                                    const double* __restrict__ ptab,
+                                                    double* __restrict__ qmat,
+                                                    const double* __restrict__ dvec,
+                                                    const double* __restrict__ evec,
+                                                    double* __restrict__ mat,
+                                                    double* __restrict__ vec, double* __restrict__ ampl,
+                                                    unsigned* __restrict__ err) {
+  const int zl = blockIdx.x;
+  const int64_t z = zone_at(zorder, z0 + zl);
+  if (z < 0) return;  // the zone is solved by the other pipeline
+  const int64_t cnt = sel_ptr[z + 1] - sel_ptr[z];
+  if (cnt == 0) {  // no observations: a = 0
+    if (threadIdx.x < NP) vec[(size_t)zl * 4 * NP + NP + threadIdx.x] = 0.0;
+    return;
+  }
+  if (!func_zone<NP, DUAL, LIKE, TR, false>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec,
+                                            ampl, err)) {
+    lds_barrier();
+    deep_zone<NP, DUAL, LIKE, TR>(zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl, err);
+  }
 }
 
 // ===========================================================================
@@ -808,11 +1106,15 @@ struct FuncSmallLds {
       double t[NB][16 * 17];  // V^T V, then T_b
       double v[NP];
     } m;
+    struct {
+      QlLds<NP> q;
+      double z[NP * NP];  // its eigenvectors
+    };
   };
 };
 
 template <int NP>
-__global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t* __restrict__ zorder, int N,
+__global__ __launch_bounds__(64, NP == 16 ? 3 : 2) void k_func_small(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                       const int64_t* __restrict__ sel_ptr,
                                                       const double* __restrict__ ptab,
                                                       const double* __restrict__ qmat,
@@ -835,12 +1137,14 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
     return;
   }
   const double* V = qmat + (size_t)zl * NP * NP;
+  const double dl = lane < NP ? dvec[(size_t)zl * NP + lane] : 0.0;
+  const double u0 = lane < NP ? Vz[lane] : 0.0, u1 = lane < NP ? Vz[2 * NP + lane] : 0.0;
   if (lane < NP) {
     const int k = step_row<NP>(lane);
-    S.p.d[k] = dvec[(size_t)zl * NP + lane];
+    S.p.d[k] = dl;
     S.p.e[k] = evec[(size_t)zl * NP + (lane < H ? lane : lane - 1)];
-    S.p.c[0][k] = Vz[lane];
-    S.p.c[1][k] = Vz[2 * NP + lane];
+    S.p.c[0][k] = u0;
+    S.p.c[1][k] = u1;
   }
   // reflector 16 b + lc, rows 4 q + lr (zero up to row k, none past N - 3)
   double va[NB][NP / 4], tau[NB];
@@ -859,154 +1163,220 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
     nt = fabs(S.p.d[lane]) + fabs(S.p.e[lane]) + (lane % H ? fabs(S.p.e[lane - 1]) : 0.0);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
-  const int ex = (__double2hiint(nt) >> 20) - 1022;
-  int bk = ((ex + 1) >> 1) - 1;
-  bk = __builtin_amdgcn_readfirstlane(bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk));
-  double alpha[H], gh;  // alpha of the lane's rows and pole; G_hh
-  const int j = lane & 31;
-  const bool bot = lane >= 32;
-  const int h0 = bot ? H : 0;
-  double* aa = S.p.a + h0 * 32;
-  double* gg = S.p.g + h0 * 32;
-  const int jx = (j & ~1) ^ (H == 8 && bot ? 16 : 0);
-  auto at = [&](int i) { return i * 32 + (jx ^ (2 * i)) + (j & 1); };
-  {
-    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s, wj = ptab[bk * kPoleSet + 32 + j];
-    double* cc = S.p.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
-    double* c1 = S.p.c[1] + h0;
-    double qv[H], zv[H], ev[H];
-    double q = 0.0, z1 = 0.0, t = 0.0, e2 = 0.0;
+  const int ex = __builtin_amdgcn_readfirstlane(exponent_above(nt));
+  const PoleBlocks pb = pole_blocks(ex > 1024 ? 0 : ex);  // infinities end as NaN in a
+  d4 c[NB], f[NB][NB];
+  if (pb.count > 0) {
+#pragma unroll 1
+    for (int batch = 0;; ++batch) {
+      // the thread index made opaque in each pass (as in k_func)
+      int lq = threadIdx.x;
+      asm volatile("" : "+v"(lq));
+      const int lane = lq, lr = lq >> 4, lc = lq & 15;
+      const int j = lane & 31;
+      const bool bot = lane >= 32;
+      const int h0 = bot ? H : 0;
+      double* aa = S.p.a + h0 * 32;
+      double* gg = S.p.g + h0 * 32;
+      const int jx = (j & ~1) ^ (H == 8 && bot ? 16 : 0);
+      auto at = [&](int i) { return i * 32 + (jx ^ (2 * i)) + (j & 1); };
+      double alpha[H], gh;  // alpha of the lane's rows and pole; G_hh
+      const int blk = pb.first + batch;
+      const bool tl = j == 31 && batch == 0;  // the lane of T itself
+      {
+        const double s = ptab[blk * kPoleBlock + j], sp1 = 1.0 + s, wj = ptab[blk * kPoleBlock + 32 + j];
+        double* cc = S.p.c[tl ? 0 : 1] + h0;  // the lane's right-hand side
+        double* c1 = S.p.c[1] + h0;
+        double qv[H], zv[H], ev[H];
+        double q = 0.0, z1 = 0.0, t = 0.0, e2 = 0.0;
 #pragma unroll
-    for (int i = 0; i < H; ++i) {
-      ev[i] = S.p.e[h0 + i];
-      q = rcp_acc(fmax(fma(-e2, q, S.p.d[h0 + i] + s), sp1));
-      z1 = fma(t, z1, cc[i]);
-      qv[i] = q;
-      zv[i] = z1 * q;
-      t = -ev[i] * q;
-      e2 = ev[i] * ev[i];
-    }
-    const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
-    const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
-    const double eh = S.p.e[H - 1];
-    double G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
-    double x = G * fma(-eh * qb, zb, zh), al = 1.0;
-    gh = G;
-    double tv[H];
+        for (int i = 0; i < H; ++i) {
+          ev[i] = S.p.e[h0 + i];
+          q = rcp_acc(fmax(fma(-e2, q, S.p.d[h0 + i] + s), sp1));
+          z1 = fma(t, z1, cc[i]);
+          qv[i] = q;
+          zv[i] = z1 * q;
+          t = -ev[i] * q;
+          e2 = ev[i] * ev[i];
+        }
+        const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+        const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+        const double eh = S.p.e[H - 1];
+        double G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+        double x = G * fma(-eh * qb, zb, zh), al = 1.0;
+        gh = G;
+        double tv[H];
 #pragma unroll
-    for (int i = H - 1; i >= 0; --i) {
-      double rr = -ev[i] * qv[i];
-      const double gn = fma(rr * rr, G, qv[i]), xn = fma(rr, x, zv[i]);
-      const bool mid = i == H - 1 && !bot;  // row h itself
-      G = mid ? G : gn;
-      x = mid ? x : xn;
-      rr = mid ? 1.0 : rr;
-      al *= rr;
-      alpha[i] = al;
-      aa[at(i)] = rr;
-      gg[at(i)] = G;
-      tv[i] = wj * fma(-s, x, c1[i]);
-      if (j == 31) cc[i] = x;
-    }
-    // sums over the poles: of each 32 lanes the lower 16 keep the first half
-    // of the rows, the upper 16 the second
-    const bool up = (lane & 16) != 0;
+        for (int i = H - 1; i >= 0; --i) {
+          double rr = -ev[i] * qv[i];
+          const double gn = fma(rr * rr, G, qv[i]), xn = fma(rr, x, zv[i]);
+          const bool mid = i == H - 1 && !bot;  // row h itself
+          G = mid ? G : gn;
+          x = mid ? x : xn;
+          rr = mid ? 1.0 : rr;
+          al *= rr;
+          alpha[i] = al;
+          aa[at(i)] = rr;
+          gg[at(i)] = G;
+          tv[i] = wj * fma(-s, x, c1[i]);
+          if (tl) cc[i] = x;
+        }
+        // sums over the poles: of each 32 lanes the lower 16 keep the first half
+        // of the rows, the upper 16 the second
+        const bool up = (lane & 16) != 0;
 #pragma unroll
-    for (int i = 0; i < H / 2; ++i) {
-      const double give = up ? tv[i] : tv[i + H / 2], keep = up ? tv[i + H / 2] : tv[i];
-      tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
-    }
-    if (lc == 0) {
+        for (int i = 0; i < H / 2; ++i) {
+          const double give = up ? tv[i] : tv[i + H / 2], keep = up ? tv[i + H / 2] : tv[i];
+          tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
+        }
+        if (lc == 0) {
 #pragma unroll
-      for (int i = 0; i < H / 2; ++i) c1[(up ? H / 2 : 0) + i] = tv[i];
-    }
-  }
-  lds_fence();
-  // [x, y] as columns 0 and 1 of a tile per 16 rows
-  d4 c[NB];
-#pragma unroll
-  for (int I = 0; I < NB; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double t = S.p.c[lc & 1][step_row<NP>(16 * I + lr + 4 * r)];
-      c[I][r] = lc < 2 ? t : 0.0;
-    }
-  // ---- F = T^-1/2: each half's triangle outwards from its diagonal entries,
-  // eight poles a lane, the other one by a product with the identity ----
-  double w8[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) w8[q] = ptab[bk * kPoleSet + 32 + 8 * lr + q];
-  d4 f[NB][NB];
-#pragma unroll
-  for (int J = 0; J < NB; ++J) {
-    // column 16 J + lc is row lcs (elimination order) of half hb
-    const bool hb = NP == 32 ? J == 1 : lc >= 8;
-    const int lcs = hb ? 15 - lc : lc, base = NP == 32 ? 16 * J : (hb ? 8 : 0);
-    double g[8];
-    load_poles4(S.p.g, base + lcs, 2 * lr, reinterpret_cast<double(&)[4]>(g[0]));
-    load_poles4(S.p.g, base + lcs, 2 * lr + 1, reinterpret_cast<double(&)[4]>(g[4]));
-#pragma unroll
-    for (int q = 0; q < 8; ++q) g[q] *= w8[q];
-    const int lrs = hb ? 3 - lr : lr;
-    d4 us = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = H - 1; i >= 0; --i) {
-      if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        double rr[4];
-        load_poles4(S.p.a, base + i, 2 * lr + h, rr);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? rr[q] : 1.0;
+          for (int i = 0; i < H / 2; ++i) c1[(up ? H / 2 : 0) + i] = tv[i];
+        }
       }
-      const double sm =
-          sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
-      us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+      lds_fence();
+      // [x, y] as columns 0 and 1 of a tile per 16 rows
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double t = S.p.c[lc & 1][step_row<NP>(16 * I + lr + 4 * r)];
+          c[I][r] = lc < 2 ? t : 0.0;
+        }
+      // ---- F = T^-1/2: each half's triangle outwards from its diagonal entries,
+      // eight poles a lane, the other one by a product with the identity ----
+      double w8[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w8[q] = ptab[blk * kPoleBlock + 32 + 8 * lr + q];
+#pragma unroll
+      for (int J = 0; J < NB; ++J) {
+        // column 16 J + lc is row lcs (elimination order) of half hb
+        const bool hb = NP == 32 ? J == 1 : lc >= 8;
+        const int lcs = hb ? 15 - lc : lc, base = NP == 32 ? 16 * J : (hb ? 8 : 0);
+        double g[8];
+        load_poles4(S.p.g, base + lcs, 2 * lr, reinterpret_cast<double(&)[4]>(g[0]));
+        load_poles4(S.p.g, base + lcs, 2 * lr + 1, reinterpret_cast<double(&)[4]>(g[4]));
+#pragma unroll
+        for (int q = 0; q < 8; ++q) g[q] *= w8[q];
+        const int lrs = hb ? 3 - lr : lr;
+        d4 us = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = H - 1; i >= 0; --i) {
+          if (i % 4 == 3) asm volatile("" ::: "memory");  // the reads of four rows at a time
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            double rr[4];
+            load_poles4(S.p.a, base + i, 2 * lr + h, rr);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) g[4 * h + q] *= i < lcs ? rr[q] : 1.0;
+          }
+          const double sm =
+              sum_xor32(sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+          us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+        }
+        d4 ut, fd;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          ut[r] = hb ? us[3 - r] : us[r];
+          fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+        f[J][J] = fd;
+      }
+      // the entries between the halves
+      lds_fence();
+#pragma unroll
+      for (int i = 0; i < H; ++i) aa[at(i)] = alpha[i];
+      // G_hh of the poles 8 lr + q (lanes 0..31 hold them)
+      double w8g[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w8g[q] = w8[q] * shfl_d(gh, 8 * lr + q);
+      lds_fence();
+      {
+        double av[NB][8];
+#pragma unroll
+        for (int I = 0; I < NB; ++I) {
+          const int row = step_row<NP>(16 * I + lc);
+          load_poles4(S.p.a, row, 2 * lr, reinterpret_cast<double(&)[4]>(av[I][0]));
+          load_poles4(S.p.a, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(av[I][4]));
+        }
+        if (NP == 32) {
+          f[0][NB - 1] = d4{0.0, 0.0, 0.0, 0.0};
+          f[NB - 1][0] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            f[0][NB - 1] = mfma_f64(av[0][q], av[NB - 1][q] * w8g[q], f[0][NB - 1]);
+            f[NB - 1][0] = mfma_f64(av[NB - 1][q], av[0][q] * w8g[q], f[NB - 1][0]);
+          }
+        } else {
+          d4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+          for (int q = 0; q < 8; ++q) x = mfma_f64(av[0][q], av[0][q] * w8g[q], x);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) f[0][0][r] = (lc < 8) == (r < 2) ? f[0][0][r] : x[r];
+        }
+      }
+      lds_fence();
+      if (batch + 1 == pb.count) break;
+      // another block: this one's F to memory (kept in registers it would cost the
+      // zones of one block their occupancy), x and y to free slots, Q^T 1 again
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * I + lr + 4 * r;
+#pragma unroll
+          for (int J = 0; J < NB; ++J) M[row * NP + 16 * J + lc] = f[I][J][r];
+          if (lc < 2) Vz[(lc ? 1 : 3) * NP + row] = c[I][r];
+        }
+      if (lane < NP) S.p.c[1][step_row<NP>(lane)] = Vz[2 * NP + lane];
+      lds_fence();
     }
-    d4 ut, fd;
+    if (pb.count == 2) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ut[r] = hb ? us[3 - r] : us[r];
-      fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * I + lr + 4 * r;
+#pragma unroll
+          for (int J = 0; J < NB; ++J) f[I][J][r] += M[row * NP + 16 * J + lc];
+          if (lc == 0) c[I][r] = Vz[3 * NP + row];
+          if (lc == 1) c[I][r] += Vz[NP + row];
+        }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
-    f[J][J] = fd;
-  }
-  // the entries between the halves
-  lds_fence();
-#pragma unroll
-  for (int i = 0; i < H; ++i) aa[at(i)] = alpha[i];
-  // G_hh of the poles 8 lr + q (lanes 0..31 hold them)
-  double w8g[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) w8g[q] = w8[q] * shfl_d(gh, 8 * lr + q);
-  lds_fence();
-  {
-    double av[NB][8];
+  } else {
+    // from the eigenvectors
+    if (lane < NP) {
+      S.q.d[NP - 1 - lane] = dl;
+      S.q.e[lane] = lane < NP - 1 ? evec[(size_t)zl * NP + NP - 2 - lane] : 0.0;
+      S.q.u[0][lane] = u0;
+      S.q.u[1][lane] = u1;
+    }
+    __syncthreads();
+    ql_functions<NP, 64, false, false>(S.q, nt, S.z, nullptr);
 #pragma unroll
     for (int I = 0; I < NB; ++I) {
-      const int row = step_row<NP>(16 * I + lc);
-      load_poles4(S.p.a, row, 2 * lr, reinterpret_cast<double(&)[4]>(av[I][0]));
-      load_poles4(S.p.a, row, 2 * lr + 1, reinterpret_cast<double(&)[4]>(av[I][4]));
-    }
-    if (NP == 32) {
-      f[0][NB - 1] = d4{0.0, 0.0, 0.0, 0.0};
-      f[NB - 1][0] = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        f[0][NB - 1] = mfma_f64(av[0][q], av[NB - 1][q] * w8g[q], f[0][NB - 1]);
-        f[NB - 1][0] = mfma_f64(av[NB - 1][q], av[0][q] * w8g[q], f[NB - 1][0]);
+      for (int r = 0; r < 4; ++r) {
+        const double t = S.q.u[lc & 1][16 * I + lr + 4 * r];
+        c[I][r] = lc < 2 ? t : 0.0;
       }
-    } else {
-      d4 x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int q = 0; q < 8; ++q) x = mfma_f64(av[0][q], av[0][q] * w8g[q], x);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) f[0][0][r] = (lc < 8) == (r < 2) ? f[0][0][r] : x[r];
+      for (int J = 0; J < NB; ++J) f[I][J] = d4{0.0, 0.0, 0.0, 0.0};
     }
+#pragma unroll 1
+    for (int k = 0; k < NP; k += 4) {
+      const double* zk = S.z + (k + lr) * NP + lc;
+#pragma unroll
+      for (int J = 0; J < NB; ++J) {
+        const double b = S.q.e[k + lr] * zk[16 * J];
+#pragma unroll
+        for (int I = 0; I < NB; ++I) f[I][J] = mfma_f64(zk[16 * I], b, f[I][J]);
+      }
+    }
+    lds_fence();
   }
-  lds_fence();
   // ---- T_b of the reflector blocks: lane i of row b of the wave has row i;
   // T_b[j][j] = tau_j, T_b[0:j, j] = -tau_j T_b[0:j, 0:j] (V^T V)[0:j, j] ----
 #pragma unroll
@@ -1201,15 +1571,44 @@ __global__ __launch_bounds__(64, 2) void k_func_small(int64_t z0, const int32_t*
 // 1 to 3), then a = Q x and v = Q y / |Q y|.  For the products that form F, per
 // row (in elimination order) and pole: tau and G_ii (the tiles on the
 // diagonal), and alpha and beta relative to the tile edges; `poles` has these
-// four arrays, then the weights and G_hh.  The recurrence
+// four arrays, of one block of poles and then of the other (or the eigenvectors,
+// ql_zone256), tblk, after T_b, the weights and G_hh of each block (or the
+// eigenvectors' weights) and the number of blocks (PoleSet256).  The recurrence
 // leaves 1/gamma and z/gamma of the way in where tau and G go on the way out.
 template <int NP>
 struct PoleLds {
-  double d[NP], e[NP], c[2][NP];  // c: Q^T b, Q^T 1, then x, y (elimination order)
-  double v[2][NP];                // x, y; then a, v
+  union {
+    struct {
+      double d[NP], e[NP], c[2][NP];  // c: Q^T b, Q^T 1, then x, y (elimination order)
+      double v[2][NP];                // x, y; then a, v
+    };
+    QlLds<NP> q;
+  };
+  double bound;  // of T's spectrum
+  int count;
   double tp[NP / 16 * 136];       // T_b, packed
   double g[2][16], t[2][16], red[4];
 };
+
+__device__ __forceinline__ PoleLds<256>& pole_lds() {
+  __shared__ PoleLds<256> S;
+  return S;
+}
+
+// QL for a zone beyond the poles (a function of its own as deep_zone): the
+// eigenvectors to Z.
+__device__ __attribute__((noinline)) void ql_zone256(const double* d, const double* e, const double* Vz,
+                                                     double* Z) {
+  constexpr int NP = 256;
+  PoleLds<NP>& S = pole_lds();
+  const int tid = threadIdx.x;
+  S.q.d[NP - 1 - tid] = d[tid];
+  S.q.e[tid] = tid < NP - 1 ? e[NP - 2 - tid] : 0.0;
+  S.q.u[0][tid] = Vz[tid];
+  S.q.u[1][tid] = Vz[2 * NP + tid];
+  __syncthreads();
+  ql_functions<NP, 256, false, false>(S.q, S.bound, Z, nullptr);
+}
 
 __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ sel_ptr,
@@ -1221,7 +1620,7 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
                                                     double* __restrict__ vec, double* __restrict__ ampl,
                                                     unsigned* __restrict__ err) {
   constexpr int NP = 256, H = NP / 2;
-  __shared__ PoleLds<NP> S;
+  PoleLds<NP>& S = pole_lds();
   const int zl = blockIdx.x;
   const int64_t z = zone_at(zorder, z0 + zl);
   if (z < 0) return;
@@ -1242,6 +1641,8 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
     S.c[1][k] = Vz[2 * NP + tid];
   }
   lds_barrier();
+  double* tz = tblk + (size_t)zl * NP * NP;
+  double* P0 = poles + (size_t)zl * NP * NP;
   if (wave == 0) {
     double nt = 0.0;  // Gershgorin bound of T
 #pragma unroll
@@ -1251,106 +1652,131 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
     }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) nt = fmax(nt, shfl_xor_d(nt, o));
-    const int ex = (__double2hiint(nt) >> 20) - 1022;
-    int bk = ((ex + 1) >> 1) - 1;
-    bk = __builtin_amdgcn_readfirstlane(bk < 0 ? 0 : (bk > kBuckets - 1 ? kBuckets - 1 : bk));
+    const int ex = __builtin_amdgcn_readfirstlane(exponent_above(nt));
+    const PoleBlocks pb = pole_blocks(ex > 1024 ? 0 : ex);  // infinities end as NaN in a
+    if (lane == 0) {
+      S.bound = nt;
+      S.count = pb.count;
+      tz[PoleSet256::kCount] = (double)pb.count;
+    }
     const int j = lane & 31;
     const bool bot = lane >= 32, up = (lane & 16) != 0;
-    const double s = ptab[bk * kPoleSet + j], sp1 = 1.0 + s, wj = ptab[bk * kPoleSet + 32 + j];
-    const int h0 = bot ? H : 0;
-    const double* dd = S.d + h0;
-    const double* ee = S.e + h0;
-    double* cc = S.c[j == 31 ? 0 : 1] + h0;  // the lane's right-hand side
-    double* c1 = S.c[1] + h0;
-    double* P = poles + (size_t)zl * NP * NP;
-    double* pa = P + h0 * 32 + j;  // tau (first 1/gamma); + NP 32: G_ii (first z/gamma)
-    double* pg = pa + NP * 32;
-    double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
+    // block by block, the one with T itself last: y adds up in v
 #pragma unroll 1
-    for (int t = 0; t < H; t += 8) {
-      double dv[8], ev[8], cv[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        dv[i] = dd[t + i];
-        ev[i] = ee[t + i];
-        cv[i] = cc[t + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
-        z1 = fma(tau, z1, cv[i]);
-        pa[(t + i) * 32] = q;
-        pg[(t + i) * 32] = z1 * q;
-        tau = -ev[i] * q;
-        e2 = ev[i] * ev[i];
-      }
-    }
-    double G, x;
-    {
-      const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
-      const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
-      const double eh = S.e[H - 1];
-      G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
-      x = G * fma(-eh * qb, zb, zh);
-      if (!bot) {
-        P[4 * NP * 32 + j] = wj;
-        P[4 * NP * 32 + 32 + j] = G;
-      }
-    }
+    for (int batch = pb.count - 1; batch >= 0; --batch) {
+      const int blk = pb.first + batch;
+      const bool tl = j == 31 && batch == 0;  // the lane of T itself
+      const double s = ptab[blk * kPoleBlock + j], sp1 = 1.0 + s, wj = ptab[blk * kPoleBlock + 32 + j];
+      const int h0 = bot ? H : 0;
+      const double* dd = S.d + h0;
+      const double* ee = S.e + h0;
+      double* cc = S.c[tl ? 0 : 1] + h0;  // the lane's right-hand side
+      double* c1 = S.c[1] + h0;
+      double* P = P0 + batch * PoleSet256::kArrays;
+      double* pa = P + h0 * 32 + j;  // tau (first 1/gamma); + NP 32: G_ii (first z/gamma)
+      double* pg = pa + NP * 32;
+      double q = 0.0, z1 = 0.0, tau = 0.0, e2 = 0.0;
 #pragma unroll 1
-    for (int t = H - 16; t >= 0; t -= 16) {
-      double r[16], g[16];  // 1/gamma and z/gamma, then tau and G_ii
+      for (int t = 0; t < H; t += 8) {
+        double dv[8], ev[8], cv[8];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        r[i] = pa[(t + i) * 32];
-        g[i] = pg[(t + i) * 32];
-      }
-#pragma unroll
-      for (int h = 1; h >= 0; --h) {
-        double tv[8];
-#pragma unroll
-        for (int i = 7; i >= 0; --i) {
-          const int k = 8 * h + i;
-          double rr = -ee[t + k] * r[k];
-          const double gn = fma(rr * rr, G, r[k]), xn = fma(rr, x, g[k]);
-          const bool mid = k == 15 && !bot && t == H - 16;  // row h itself
-          G = mid ? G : gn;
-          x = mid ? x : xn;
-          rr = mid ? 1.0 : rr;
-          r[k] = rr;
-          g[k] = G;
-          tv[i] = wj * fma(-s, x, c1[t + k]);
-          if (j == 31) cc[t + k] = x;
+        for (int i = 0; i < 8; ++i) {
+          dv[i] = dd[t + i];
+          ev[i] = ee[t + i];
+          cv[i] = cc[t + i];
         }
-        // sums over the poles, as in k_func
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
-          tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
-        }
-        if (lc == 0) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) c1[t + 8 * h + (up ? 4 : 0) + i] = tv[i];
+        for (int i = 0; i < 8; ++i) {
+          q = rcp_acc(fmax(fma(-e2, q, dv[i] + s), sp1));
+          z1 = fma(tau, z1, cv[i]);
+          pa[(t + i) * 32] = q;
+          pg[(t + i) * 32] = z1 * q;
+          tau = -ev[i] * q;
+          e2 = ev[i] * ev[i];
         }
       }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        pa[(t + i) * 32] = r[i];
-        pg[(t + i) * 32] = g[i];
+      double G, x;
+      {
+        const double qo = shfl_xor_d(q, 32), zo = shfl_xor_d(z1, 32);
+        const double qh = bot ? qo : q, qb = bot ? q : qo, zh = bot ? zo : z1, zb = bot ? z1 : zo;
+        const double eh = S.e[H - 1];
+        G = rcp_acc(fmax(fma(-eh * qb, eh, rcp_acc(qh)), sp1));
+        x = G * fma(-eh * qb, zb, zh);
+        if (!bot) {
+          tz[PoleSet256::kWeights + 64 * batch + j] = wj;
+          tz[PoleSet256::kWeights + 64 * batch + 32 + j] = G;
+        }
       }
-      // towards the middle edge of the tile: alpha, beta
-      double pi = 1.0;
+#pragma unroll 1
+      for (int t = H - 16; t >= 0; t -= 16) {
+        double r[16], g[16];  // 1/gamma and z/gamma, then tau and G_ii
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        g[i] *= pi;
-        pi *= r[i];
+        for (int i = 0; i < 16; ++i) {
+          r[i] = pa[(t + i) * 32];
+          g[i] = pg[(t + i) * 32];
+        }
+#pragma unroll
+        for (int h = 1; h >= 0; --h) {
+          double tv[8];
+#pragma unroll
+          for (int i = 7; i >= 0; --i) {
+            const int k = 8 * h + i;
+            double rr = -ee[t + k] * r[k];
+            const double gn = fma(rr * rr, G, r[k]), xn = fma(rr, x, g[k]);
+            const bool mid = k == 15 && !bot && t == H - 16;  // row h itself
+            G = mid ? G : gn;
+            x = mid ? x : xn;
+            rr = mid ? 1.0 : rr;
+            r[k] = rr;
+            g[k] = G;
+            tv[i] = wj * fma(-s, x, c1[t + k]);
+            if (tl) cc[t + k] = x;
+          }
+          // sums over the poles, as in k_func
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const double give = up ? tv[i] : tv[i + 4], keep = up ? tv[i + 4] : tv[i];
+            tv[i] = row_sum16(keep + shfl_xor_d(give, 16));
+          }
+          if (lc == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c1[t + 8 * h + (up ? 4 : 0) + i] = tv[i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          pa[(t + i) * 32] = r[i];
+          pg[(t + i) * 32] = g[i];
+        }
+        // towards the middle edge of the tile: alpha, beta
+        double pi = 1.0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          g[i] *= pi;
+          pi *= r[i];
+        }
+#pragma unroll
+        for (int i = 14; i >= 0; --i) r[i] *= r[i + 1];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          pa[2 * NP * 32 + (t + i) * 32] = r[i];
+          pg[2 * NP * 32 + (t + i) * 32] = g[i];
+        }
       }
+      if (pb.count > 1) {
+        // y of both blocks, Q^T 1 again in between
+        lds_fence();
 #pragma unroll
-      for (int i = 14; i >= 0; --i) r[i] *= r[i + 1];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        pa[2 * NP * 32 + (t + i) * 32] = r[i];
-        pg[2 * NP * 32 + (t + i) * 32] = g[i];
+        for (int h = 0; h < NP / 64; ++h) {
+          const int k = lane + 64 * h, r = step_row<NP>(k);
+          if (batch > 0) {
+            S.v[1][k] = S.c[1][k];
+            S.c[1][k] = Vz[2 * NP + r];
+          } else {
+            S.c[1][k] += S.v[1][k];
+          }
+        }
+        lds_fence();
       }
     }
   } else {
@@ -1390,12 +1816,17 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
     }
   }
   lds_barrier();
-  {
+  if (S.count == 0) {  // x and y where v is
+    static_assert(offsetof(PoleLds<NP>, v) == offsetof(PoleLds<NP>, q) + offsetof(QlLds<NP>, u), "");
+    ql_zone256(dvec + (size_t)zl * NP, evec + (size_t)zl * NP, Vz, P0);
+    tz[PoleSet256::kWeights + tid] = S.q.e[tid];
+  } else {
     const int k = step_row<NP>(tid);
-    S.v[0][tid] = S.c[0][k];
-    S.v[1][tid] = S.c[1][k];
+    const double x = S.c[0][k], y = S.c[1][k];
+    S.v[0][tid] = x;
+    S.v[1][tid] = y;
   }
-  for (int e = tid; e < nblk * 136; e += 256) tblk[(size_t)zl * NP * NP + e] = S.tp[e];
+  for (int e = tid; e < nblk * 136; e += 256) tz[e] = S.tp[e];
   // [a, v] = Q [x, y]: thread (pj, pr) has rows pr + 16 e of reflector pj of a block
   const int pj = tid >> 4, pr = tid & 15;
   double pf[16];
@@ -1560,7 +1991,7 @@ void launch_omega_rows128(const ChunkArgs& A, hipStream_t st) {
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
 #define OAK_FUNC(P, D, LK, TR)                                                                     \
   hipLaunchKernelGGL((k_func<P, D, LK, TR>), dim3(A.nzc), dim3(4 * P), 0, st, A.z0, A.zorder, A.N, \
-                     A.sel_ptr, A.poles, A.ymat, A.dvec, A.evec, A.vec, A.ampl, A.err)
+                     A.sel_ptr, A.poles, A.ymat, A.dvec, A.evec, A.mat, A.vec, A.ampl, A.err)
   if (NP == 64) {
     launch_tridiag_lower64(A, dual ? -1 : A.N, st);
     if (dual)
@@ -1596,7 +2027,7 @@ void launch_func_small(int NP, const ChunkArgs& A, hipStream_t st) {
 #undef OAK_SMALL
 }
 
-// N > 128: the pole arrays to umat, T_b to the rows of ymat that the reduction's
+// N > 128: the pole arrays to umat, T_b (and the weights) to the rows of ymat that the reduction's
 // trailing block leaves (128 .. 191), a and v.
 void launch_pole256(const ChunkArgs& A, hipStream_t st) {
   hipLaunchKernelGGL(k_pole256, dim3(A.nzc), dim3(256), 0, st, A.z0, A.zorder, A.N, A.sel_ptr, A.poles,

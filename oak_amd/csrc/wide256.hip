@@ -442,6 +442,132 @@ struct QApplyLds {
   double v[NPW];
 };
 
+// Tile column J of F = T^-1/2 of a zone (k_pole256's arrays in uz, the weights in tz): what
+// one block of poles adds to it.  The lower half's columns see the tile rows
+// mirrored (k_func): f[I] is tile row I or 15 - I.
+__device__ __forceinline__ void add_block256(int J, int nt, int batch, const double* __restrict__ uz,
+                                             const double* __restrict__ tz, d4 (&f)[16]) {
+  constexpr int NP = NPW, NB = 16;
+  const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
+  const bool low = J >= NB / 2;
+  auto row_of = [&](int I) { return low ? NB - 1 - I : I; };
+  const double* P = uz + batch * PoleSet256::kArrays;
+  const double* wp = tz + PoleSet256::kWeights + 64 * batch;
+  const double* al = P + 2 * NP * 32;
+  const double* be = P + 3 * NP * 32;
+  const int Js = low ? NB - 1 - J : J;
+  auto tile_of = [&](int r) { return r < NB / 2 ? r : NB / 2 + NB - 1 - r; };
+  auto load4 = [&](const double* a, int row, int h, double* o) {
+    const double2* p = reinterpret_cast<const double2*>(a + (size_t)row * 32 + 8 * lr + 4 * h);
+    const double2 x0 = p[0], x1 = p[1];
+    o[0] = x0.x;
+    o[1] = x0.y;
+    o[2] = x1.x;
+    o[3] = x1.y;
+  };
+  const int crow = 16 * tile_of(J) + (low ? 15 - lc : lc);
+  double w[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) w[q] = wp[8 * lr + q];
+  // the tile on the diagonal: outwards from each column's diagonal entry
+  // for the lane's eight poles, then the transpose (as in k_func)
+  d4 fd;
+  {
+    double g[8];
+    load4(P + NP * 32, crow, 0, g);
+    load4(P + NP * 32, crow, 1, g + 4);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) g[q] *= w[q];
+    const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
+    d4 us = {0.0, 0.0, 0.0, 0.0}, ut;
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+      if (i % 4 == 3) asm volatile("" ::: "memory");
+      double r[8];
+      load4(P, 16 * tile_of(J) + i, 0, r);
+      load4(P, 16 * tile_of(J) + i, 1, r + 4);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) g[q] *= i < lcs ? r[q] : 1.0;
+      const double sm = sum_xor32(
+          sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
+      us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      ut[r] = low ? us[3 - r] : us[r];
+      fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+  }
+  double B[8];
+  auto column = [&](const double* a) {
+    load4(a, crow, 0, B);
+    load4(a, crow, 1, B + 4);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) B[q] *= w[q];
+  };
+  auto tile = [&](const double* a, int I, d4 acc) {
+    const int rI = row_of(I), t16 = 16 * tile_of(rI);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      double av[4], edge[4];
+      load4(a, t16 + (rI < NB / 2 ? lc : 15 - lc), h, av);
+      load4(al, t16, h, edge);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        acc = mfma_f64(av[q], B[4 * h + q], acc);
+        B[4 * h + q] *= edge[q];
+      }
+    }
+    return acc;
+  };
+  column(be);
+#pragma unroll
+  for (int I = NB / 2 - 2; I >= 0; --I)  // outside
+    if (I < Js && row_of(I) < nt) f[I] = tile(al, I, f[I]);
+  column(al);
+#pragma unroll
+  for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
+    if (I == NB / 2) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) B[q] *= wp[32 + 8 * lr + q];
+    }
+    if (I > Js && row_of(I) < nt) f[I] = tile(I < NB / 2 ? be : al, I, f[I]);
+  }
+#pragma unroll
+  for (int I = 0; I < NB / 2; ++I)
+    if (I == Js) f[I] += fd;
+}
+
+// F of a zone of two blocks of poles, or of the eigenvectors in uz, to Y, tile column J
+// by one wave (a function of its own: its loops would make k_qapply256 spill).
+__device__ __attribute__((noinline)) void deep_f256(int J, int nt, int count, const double* uz,
+                                                    const double* tz, double* Y) {
+  constexpr int NP = NPW, NB = 16;
+  const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
+  auto row_of = [&](int I) { return J >= NB / 2 ? NB - 1 - I : I; };
+  d4 f[NB];
+#pragma unroll
+  for (int I = 0; I < NB; ++I) f[I] = d4{0.0, 0.0, 0.0, 0.0};
+  if (count == 0) {
+#pragma unroll 1
+    for (int k = 0; k < NP; k += 4) {
+      const double* zk = uz + (size_t)(k + lr) * NP + lc;
+      const double b = tz[PoleSet256::kWeights + k + lr] * zk[16 * J];
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+        if (row_of(I) < nt) f[I] = mfma_f64(zk[16 * row_of(I)], b, f[I]);
+    }
+  }
+#pragma unroll 1
+  for (int batch = 0; batch < count; ++batch) add_block256(J, nt, batch, uz, tz, f);
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Y[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = f[I][r];
+}
+
 template <int STEP>
 __global__ __launch_bounds__(256, 2) void k_qapply256(int nzc, int64_t z0,
                                                       const int32_t* __restrict__ zorder,
@@ -482,94 +608,19 @@ __global__ __launch_bounds__(256, 2) void k_qapply256(int nzc, int64_t z0,
   for (int I = 0; I < NB; ++I) f[I] = d4{0.0, 0.0, 0.0, 0.0};
   if (J < nt) {
     if constexpr (STEP == 1) {
-      const double* P = umat + (size_t)zl * NP * NP;
-      const double* wp = P + 4 * NP * 32;
-      const double* al = P + 2 * NP * 32;
-      const double* be = P + 3 * NP * 32;
-      const int Js = low ? NB - 1 - J : J;
-      auto tile_of = [&](int r) { return r < NB / 2 ? r : NB / 2 + NB - 1 - r; };
-      auto load4 = [&](const double* a, int row, int h, double* o) {
-        const double2* p = reinterpret_cast<const double2*>(a + (size_t)row * 32 + 8 * lr + 4 * h);
-        const double2 x0 = p[0], x1 = p[1];
-        o[0] = x0.x;
-        o[1] = x0.y;
-        o[2] = x1.x;
-        o[3] = x1.y;
-      };
-      const int crow = 16 * tile_of(J) + (low ? 15 - lc : lc);
-      double w[8];
+      const double* tz = tblk + (size_t)zl * NP * NP;
+      const double* uz = umat + (size_t)zl * NP * NP;
+      const int count = __builtin_amdgcn_readfirstlane((int)tz[PoleSet256::kCount]);
+      if (count == 1) {
+        add_block256(J, nt, 0, uz, tz, f);
+      } else {
+        deep_f256(J, nt, count, uz, tz, Y);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) w[q] = wp[8 * lr + q];
-      // the tile on the diagonal: outwards from each column's diagonal entry
-      // for the lane's eight poles, then the transpose (as in k_func)
-      d4 fd;
-      {
-        double g[8];
-        load4(P + NP * 32, crow, 0, g);
-        load4(P + NP * 32, crow, 1, g + 4);
+        for (int I = 0; I < NB; ++I)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) g[q] *= w[q];
-        const int lcs = low ? 15 - lc : lc, lrs = low ? 3 - lr : lr;
-        d4 us = {0.0, 0.0, 0.0, 0.0}, ut;
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-          if (i % 4 == 3) asm volatile("" ::: "memory");
-          double r[8];
-          load4(P, 16 * tile_of(J) + i, 0, r);
-          load4(P, 16 * tile_of(J) + i, 1, r + 4);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) g[q] *= i < lcs ? r[q] : 1.0;
-          const double sm = sum_xor32(
-              sum_xor16(((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]))));
-          us[i / 4] = (lrs == (i & 3) && i <= lcs) ? sm : us[i / 4];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ut[r] = low ? us[3 - r] : us[r];
-          fd[r] = 4 * r + lr == lc ? 0.0 : ut[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) fd = mfma_f64(ut[r], 4 * r + lr == lc ? 1.0 : 0.0, fd);
+          for (int r = 0; r < 4; ++r)
+            f[I][r] = Y[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc];
       }
-      double B[8];
-      auto column = [&](const double* a) {
-        load4(a, crow, 0, B);
-        load4(a, crow, 1, B + 4);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) B[q] *= w[q];
-      };
-      auto tile = [&](const double* a, int I) {
-        const int rI = row_of(I), t16 = 16 * tile_of(rI);
-        d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          double av[4], edge[4];
-          load4(a, t16 + (rI < NB / 2 ? lc : 15 - lc), h, av);
-          load4(al, t16, h, edge);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            acc = mfma_f64(av[q], B[4 * h + q], acc);
-            B[4 * h + q] *= edge[q];
-          }
-        }
-        return acc;
-      };
-      column(be);
-#pragma unroll
-      for (int I = NB / 2 - 2; I >= 0; --I)  // outside
-        if (I < Js && row_of(I) < nt) f[I] = tile(al, I);
-      column(al);
-#pragma unroll
-      for (int I = 1; I < NB; ++I) {  // towards the middle, and beyond it
-        if (I == NB / 2) {
-#pragma unroll
-          for (int q = 0; q < 8; ++q) B[q] *= wp[32 + 8 * lr + q];
-        }
-        if (I > Js && row_of(I) < nt) f[I] = tile(I < NB / 2 ? be : al, I);
-      }
-#pragma unroll
-      for (int I = 0; I < NB / 2; ++I)
-        if (I == Js) f[I] = fd;
     } else {
       // Y^T: tile (J, I) of Y, transposed by a product with the identity (exact)
 #pragma unroll

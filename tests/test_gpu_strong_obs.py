@@ -19,8 +19,12 @@ def _functions(St, dt):
     N = St.shape[1]
     U, s, Vt = np.linalg.svd(St, full_matrices=False)
     mu, c = 1.0 + s * s, Vt @ np.ones(N)
-    R = np.eye(N) + Vt.T @ ((1.0 / np.sqrt(mu) - 1.0)[:, None] * Vt)
-    v = np.ones(N) + Vt.T @ ((np.sqrt(mu) - 1.0) * c)
+    # (I - V V^T only where V is not square: its rounding would hide mu^-1/2)
+    full = len(s) == N
+    R = Vt.T @ (((1.0 / np.sqrt(mu) - (0.0 if full else 1.0)))[:, None] * Vt)
+    v = Vt.T @ ((np.sqrt(mu) - (0.0 if full else 1.0)) * c)
+    if not full:
+        R, v = R + np.eye(N), v + np.ones(N)
     T = R @ O.rotate_vector(np.full(N, 1.0 / np.sqrt(N)), v / np.linalg.norm(v))
     return T, Vt.T @ (s / mu * (U.T @ dt)), mu[-1], mu[0]
 
