@@ -203,9 +203,9 @@ void launch_omega_rows128(const ChunkArgs& A, hipStream_t st);
 void launch_prep_ens_f32(int NP, const PrepEnsArgs& A, hipStream_t st);
 // N <= 128 (update.hip): T from mat (N <= 32) or M^-1/2 from ymat
 void launch_update(int NP, const ChunkArgs& A, hipStream_t st);
-// N <= 64: Gram, factor and adjoint in one; N > 64: the adjoint after the eigensolve
+// N <= 64: Gram, factor and adjoint in one; N > 64: factor and adjoint after the Gram
 void launch_nll_chol(int NP, const ChunkArgs& A, hipStream_t st);
-void launch_nll_adjoint128(const ChunkArgs& A, hipStream_t st);
+void launch_nll128(const ChunkArgs& A, hipStream_t st);
 void launch_report(int NP, const ReportArgs& A, hipStream_t st);
 void launch_nll_totals(int64_t nz, const double* Jz, const double* gA, double* out,
                        hipStream_t st);

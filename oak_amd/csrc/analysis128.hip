@@ -342,12 +342,6 @@ void launch_solve128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
 }
 
 void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
-  if (A.mode == 2) {  // innovation likelihood: adjoint instead of transform + update
-    if (tm) tm->mark(PH_UPDATE);
-    launch_nll_adjoint128(A, st);
-    if (tm) tm->mark(PH_END);
-    return;
-  }
   if (tm) tm->mark(PH_TMAT);
   launch_omega_rows128(A, st);
   if (tm) tm->mark(PH_UPDATE);
@@ -356,6 +350,14 @@ void launch_apply128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
 }
 
 void launch_chunk128(const ChunkArgs& A, hipStream_t st, PhaseTimer* tm) {
+  if (A.mode == 2) {  // innovation likelihood and its adjoint
+    if (tm) tm->mark(PH_GRAM);
+    launch_gram_blocks(128, A, st);
+    if (tm) tm->mark(PH_EIG);
+    launch_nll128(A, st);
+    if (tm) tm->mark(PH_END);
+    return;
+  }
   launch_solve128(A, st, tm);
   launch_apply128(A, st, tm);
 }

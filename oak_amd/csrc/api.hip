@@ -463,12 +463,13 @@ void materialize_counts(oakg_ctx* c) {
 // run in order on the caller's stream (the timer's events are on that stream).
 // Returns whether the zones' Jacobi sweeps are in sweeps_all.
 bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_all) {
-  // the likelihood at N <= 64 keeps nothing per zone (nll.hip); else the
-  // functions of T (N > 128 with either method) or the Jacobi option
+  // the likelihood takes a triangular factor with either method, and at N <= 64 keeps
+  // nothing per zone (nll.hip); else the functions of T (N > 128 with either method)
+  // or the Jacobi option
   base.poles = c->poles;
-  const bool chol = base.mode == 2 && NP <= 64;
+  const bool chol = base.mode == 2, one = chol && NP <= 64;
   const bool func = (c->eig_method == 1 || NP == 256) && !chol;
-  const int MP = chol ? 1 : NP;  // matrices MP x MP and vectors of MP entries per zone
+  const int MP = one ? 1 : NP;  // matrices MP x MP and vectors of MP entries per zone
   // zones with 1 <= p < dual_lt in observation space (dual.hip): N > 64, the
   // analysis modes (not the likelihood), not in a no-allocation call
   const int dual_lt = (NP == 128 && func && base.mode != 2 && !c->arena && nz > 0) ? c->tune_dual : 0;
@@ -480,7 +481,7 @@ bool run_zones(oakg_ctx* c, int NP, ChunkArgs base, int64_t nz, int32_t* sweeps_
   // more and cost their launches where it takes less (three slots against one:
   // 4096 zones of N = 16 230 and 184 us, 51 200 zones 800 and 837; 5490 zones of N =
   // 40 1517 and 1582); one kernel a zone has nothing to overlap with the next's
-  const bool slots = !c->timing && !c->arena && !chol && nz >= 4096 && nz * NP >= ((int64_t)1 << 18);
+  const bool slots = !c->timing && !c->arena && !one && nz >= 4096 && nz * NP >= ((int64_t)1 << 18);
   const int nslot = slots ? c->tune_slots : 1;
   int64_t zc = std::max<int64_t>(1, (int64_t)(budget / (per_zone * nslot)));
   zc = std::min<int64_t>(zc, 1 << 20);

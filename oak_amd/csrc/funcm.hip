@@ -133,8 +133,8 @@ __device__ __forceinline__ void ql_sweep(QlLds<NP>& S, double tiny, int buf) {
   }
 }
 
-template <int NP, int NT, bool DUAL, bool LIKE>
-__device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z, double* like) {
+template <int NP, int NT, bool DUAL>
+__device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const bool leads = wave == NT / 64 - 1;
   if (tid < NP)
@@ -189,7 +189,6 @@ __device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z,
   }
   __syncthreads();
   // Z^T u, a wave per eigenvector, times the functions of mu = max(lambda, 1)
-  double slog = 0.0, sinv = 0.0, sba = 0.0;
 #pragma unroll 1
   for (int k = wave; k < NP; k += NT / 64) {
     double t0 = 0.0, t1 = 0.0;
@@ -206,26 +205,8 @@ __device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z,
       S.s[0][k] = DUAL ? t1 / (1.0 + sq) : t1 * sq;
       S.e[k] = DUAL ? 1.0 / (mu + sq) : 1.0 / sq;
     }
-    if (LIKE) {
-      slog += log(mu);
-      sinv += 1.0 - 1.0 / mu;
-      sba = fma(t0 / mu, t0, sba);
-    }
   }
   __syncthreads();
-  if (LIKE) {  // the waves' shares (u is still wanted: through d)
-    if (lane == 0) {
-      S.d[3 * wave] = slog;
-      S.d[3 * wave + 1] = sinv;
-      S.d[3 * wave + 2] = sba;
-    }
-    __syncthreads();
-    if (tid < 3) {
-      double t = 0.0;
-      for (int w = 0; w < NT / 64; ++w) t += S.d[3 * w + tid];
-      like[tid] = t;
-    }
-  }
   if (tid < NP) {
     double x = 0.0, y = 0.0;
     for (int k = 0; k < NP; ++k) {
@@ -264,8 +245,7 @@ __device__ __forceinline__ void ql_functions(QlLds<NP>& S, double nt, double* Z,
 // waves (256 registers) spilled and took 79 us, pivots from one end 66 us.
 // DUAL (observation-space zones, dual.hip): F with the weights w / (1 + s),
 // i.e. x -> 1 / (x + sqrt x), and y with w s / (1 + s), x -> 1 / (1 + sqrt x);
-// v is left as Q y.  LIKE: also log det M, sum (1 - 1/mu) and b^T a (slot 3 of
-// vec) for the likelihood; else, at NP = 128, R 1 and R v in slots 0 and 3.  TR is the type R is stored in (float for the FP32 update
+// v is left as Q y.  At NP = 128, R 1 and R v in slots 0 and 3 of vec.  TR is the type R is stored in (float for the FP32 update
 // of the mixed path).
 // ---------------------------------------------------------------------------
 template <int NP>
@@ -321,7 +301,7 @@ __device__ __forceinline__ void load_poles4(const double* arr, int r, int k4, do
 
 // DEEP false: a zone of one block of poles (else false is returned); true: one of two
 // or of none.
-template <int NP, bool DUAL, bool LIKE, typename TR, bool DEEP>
+template <int NP, bool DUAL, typename TR, bool DEEP>
 __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int N, int64_t cnt_obs,
                                           const double* __restrict__ ptab, double* __restrict__ qmat,
                                           const double* __restrict__ dvec,
@@ -443,7 +423,6 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
           x = G * fma(-eh * qb, zb, zh);
           if (!bot) S.p.d[j] = G;
         }
-        double slog = LIKE && !bot ? -log(G) : 0.0, sinv = 0.0, sba = 0.0;
 #pragma unroll 1
         for (int t = NB / 2 - 1; t >= 0; --t) {
 #pragma unroll
@@ -465,22 +444,16 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
               if (h == 1 && i == 7) {
                 // row h itself: G and x as they are, and 1 for tau
                 const bool mid = !bot && t == NB / 2 - 1;
-                if (LIKE) slog -= mid ? 0.0 : log(iv[i]);
                 G = mid ? G : gn;
                 x = mid ? x : xn;
                 r = mid ? 1.0 : r;
               } else {
-                if (LIKE) slog -= log(iv[i]);
                 G = gn;
                 x = xn;
               }
               aa[at(t, 8 * h + i)] = r;
               gg[at(t, 8 * h + i)] = G;
               tv[i] = DUAL ? wj * x : wj * fma(-s, x, tv[i]);
-              if (LIKE) {
-                sinv += 1.0 - G;
-                sba = fma(S.p.c[0][h0 + 16 * t + 8 * h + i], x, sba);
-              }
               if (tl) cc[16 * t + 8 * h + i] = x;
             }
             // sums over the poles: of each 32 lanes the lower 16 keep steps 0..3
@@ -495,16 +468,6 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
 #pragma unroll
               for (int i = 0; i < 4; ++i) c1[16 * t + 8 * h + (up ? 4 : 0) + i] = tv[i];
             }
-          }
-        }
-        if (LIKE) {  // log det M, sum (1 - 1/mu) and b^T a
-          slog += shfl_xor_d(slog, 32);
-          sinv += shfl_xor_d(sinv, 32);
-          sba += shfl_xor_d(sba, 32);
-          if (lane == 31 && batch == 0) {
-            Vz[3 * NP] = slog;
-            Vz[3 * NP + 1] = sinv;
-            Vz[3 * NP + 2] = sba;
           }
         }
       }
@@ -699,7 +662,7 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
       S.q.u[1][tid] = Vz[2 * NP + tid];
     }
     __syncthreads();
-    ql_functions<NP, 4 * NP, DUAL, LIKE>(S.q, bound, Fz, Vz + 3 * NP);
+    ql_functions<NP, 4 * NP, DUAL>(S.q, bound, Fz);
     if (tid < NP) {
       S.c[0][tid] = S.q.u[0][tid];
       S.c[1][tid] = S.q.u[1][tid];
@@ -886,7 +849,7 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       R[(size_t)(16 * row_of(I) + lr + 4 * r) * NP + 16 * J + lc] = (TR)f[I][r];
-  if (!DUAL && !LIKE && NP == 128) {  // R 1 (k_update128)
+  if (!DUAL && NP == 128) {  // R 1 (k_update128)
     double rs = 0.0;
 #pragma unroll
     for (int I = 0; I < NB; ++I) rs += (f[I][0] + f[I][1]) + (f[I][2] + f[I][3]);
@@ -906,7 +869,7 @@ __device__ __forceinline__ bool func_zone(FuncLds<NP>& S, int zl, int64_t z, int
     Vz[NP + tid] = ar;
     Vz[2 * NP + tid] = DUAL ? vr : vr / sqrt(nv);
     // R v = 1 / |M^1/2 1|
-    if (!DUAL && !LIKE && NP == 128) Vz[3 * NP + tid] = tid < N ? 1.0 / sqrt(nv) : 0.0;
+    if (!DUAL && NP == 128) Vz[3 * NP + tid] = tid < N ? 1.0 / sqrt(nv) : 0.0;
     if (ampl && tid < N) ampl[(size_t)z * N + tid] = ar;
     if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
   }
@@ -923,16 +886,16 @@ __device__ __forceinline__ FuncLds<NP>& func_lds() {
 // A function of its own: inside k_func its loops made the tiles of every zone spill, and
 // as kernels after k_func they cost 50 us of 1.2 ms at 5490 zones of N = 40 in waiting
 // for a place on the device.
-template <int NP, bool DUAL, bool LIKE, typename TR>
+template <int NP, bool DUAL, typename TR>
 __device__ __attribute__((noinline)) void deep_zone(int zl, int64_t z, int N, int64_t cnt,
                                                     const double* ptab, double* qmat, const double* dvec,
                                                     const double* evec, double* mat, double* vec,
                                                     double* ampl, unsigned* err) {
-  func_zone<NP, DUAL, LIKE, TR, true>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl,
+  func_zone<NP, DUAL, TR, true>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl,
                                       err);
 }
 
-template <int NP, bool DUAL, bool LIKE, typename TR>
+template <int NP, bool DUAL, typename TR>
 __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                     const int64_t* __restrict__ sel_ptr,
                                                     const double* __restrict__ ptab,
@@ -950,10 +913,10 @@ __global__ __launch_bounds__(4 * NP, 4) void k_func(int64_t z0, const int32_t* _
     if (threadIdx.x < NP) vec[(size_t)zl * 4 * NP + NP + threadIdx.x] = 0.0;
     return;
   }
-  if (!func_zone<NP, DUAL, LIKE, TR, false>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec,
+  if (!func_zone<NP, DUAL, TR, false>(func_lds<NP>(), zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec,
                                             ampl, err)) {
     lds_barrier();
-    deep_zone<NP, DUAL, LIKE, TR>(zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl, err);
+    deep_zone<NP, DUAL, TR>(zl, z, N, cnt, ptab, qmat, dvec, evec, mat, vec, ampl, err);
   }
 }
 
@@ -1354,7 +1317,7 @@ __global__ __launch_bounds__(64, NP == 16 ? 3 : 2) void k_func_small(int64_t z0,
       S.q.u[1][lane] = u1;
     }
     __syncthreads();
-    ql_functions<NP, 64, false, false>(S.q, nt, S.z, nullptr);
+    ql_functions<NP, 64, false>(S.q, nt, S.z);
 #pragma unroll
     for (int I = 0; I < NB; ++I) {
 #pragma unroll
@@ -1607,7 +1570,7 @@ __device__ __attribute__((noinline)) void ql_zone256(const double* d, const doub
   S.q.u[0][tid] = Vz[tid];
   S.q.u[1][tid] = Vz[2 * NP + tid];
   __syncthreads();
-  ql_functions<NP, 256, false, false>(S.q, S.bound, Z, nullptr);
+  ql_functions<NP, 256, false>(S.q, S.bound, Z);
 }
 
 __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* __restrict__ zorder, int N,
@@ -1884,13 +1847,12 @@ __global__ __launch_bounds__(256, 2) void k_pole256(int64_t z0, const int32_t* _
   if (ar != ar) atomicOr(err, OAKG_DERR_NAN);
 }
 
-// R = Y Y^T (and the likelihood's log det M, sum (1 - 1/mu) and b^T a) from
-// the Y = U diag(mu^-1/4) and mu of the Jacobi option, so that one form
+// R = Y Y^T from the Y = U diag(mu^-1/4) of the Jacobi option, so that one form
 // reaches the transform.
 template <int NP, typename TR>
 __global__ __launch_bounds__(256) void k_yyt(int64_t z0, const int32_t* __restrict__ zorder,
                                              const int64_t* __restrict__ sel_ptr,
-                                             double* __restrict__ ymat, double* __restrict__ vec) {
+                                             double* __restrict__ ymat) {
   constexpr int LD = NP + 1, NB = NP / 16;
   __shared__ double Y[NP * LD];
   const int zl = blockIdx.x;
@@ -1900,19 +1862,6 @@ __global__ __launch_bounds__(256) void k_yyt(int64_t z0, const int32_t* __restri
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane >> 4, lc = lane & 15;
   double* Yz = ymat + (size_t)zl * NP * NP;
-  double* Vz = vec + (size_t)zl * 4 * NP;
-  double slog = 0.0, sinv = 0.0, sba = 0.0;
-  if (wave == 0) {
-    for (int k = lane; k < NP; k += 64) {
-      const double mu = Vz[3 * NP + k];
-      slog += log(mu);
-      sinv += 1.0 - 1.0 / mu;
-      sba = fma(Vz[k], Vz[NP + k], sba);
-    }
-    slog = wave_sum_fast(slog);
-    sinv = wave_sum_fast(sinv);
-    sba = wave_sum_fast(sba);
-  }
   for (int e = tid; e < NP * NP; e += 256) Y[(e / NP) * LD + e % NP] = Yz[e];
   __syncthreads();
   TR* R = reinterpret_cast<TR*>(Yz);
@@ -1923,11 +1872,6 @@ __global__ __launch_bounds__(256) void k_yyt(int64_t z0, const int32_t* __restri
       acc = mfma_f64(Y[(16 * I + lc) * LD + k + lr], Y[(16 * J + lc) * LD + k + lr], acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) R[(size_t)(16 * I + lr + 4 * r) * NP + 16 * J + lc] = (TR)acc[r];
-  }
-  if (tid == 0) {
-    Vz[3 * NP] = slog;
-    Vz[3 * NP + 1] = sinv;
-    Vz[3 * NP + 2] = sba;
   }
 }
 
@@ -1989,23 +1933,21 @@ void launch_omega_rows128(const ChunkArgs& A, hipStream_t st) {
 // The reduction (wide256.hip) and the functions of T for a chunk at NP = 64
 // or 128 (dual: the observation-space zones).
 void launch_func(int NP, const ChunkArgs& A, bool dual, hipStream_t st) {
-#define OAK_FUNC(P, D, LK, TR)                                                                     \
-  hipLaunchKernelGGL((k_func<P, D, LK, TR>), dim3(A.nzc), dim3(4 * P), 0, st, A.z0, A.zorder, A.N, \
+#define OAK_FUNC(P, D, TR)                                                                     \
+  hipLaunchKernelGGL((k_func<P, D, TR>), dim3(A.nzc), dim3(4 * P), 0, st, A.z0, A.zorder, A.N, \
                      A.sel_ptr, A.poles, A.ymat, A.dvec, A.evec, A.mat, A.vec, A.ampl, A.err)
   if (NP == 64) {
     launch_tridiag_lower64(A, dual ? -1 : A.N, st);
     if (dual)
-      OAK_FUNC(64, true, false, double);
+      OAK_FUNC(64, true, double);
     else
-      OAK_FUNC(64, false, false, double);
+      OAK_FUNC(64, false, double);
   } else {
     launch_tridiag_lower128(A, A.N, st);
     if (A.prec == 1)
-      OAK_FUNC(128, false, false, float);
-    else if (A.mode == 2)
-      OAK_FUNC(128, false, true, double);
+      OAK_FUNC(128, false, float);
     else
-      OAK_FUNC(128, false, false, double);
+      OAK_FUNC(128, false, double);
   }
 #undef OAK_FUNC
 }
@@ -2037,7 +1979,7 @@ void launch_pole256(const ChunkArgs& A, hipStream_t st) {
 void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {
   const dim3 g(A.nzc), b(256);
 #define OAK_YYT(P, TR) \
-  hipLaunchKernelGGL((k_yyt<P, TR>), g, b, 0, st, A.z0, A.zorder, A.sel_ptr, A.ymat, A.vec)
+  hipLaunchKernelGGL((k_yyt<P, TR>), g, b, 0, st, A.z0, A.zorder, A.sel_ptr, A.ymat)
   if (NP == 64)
     OAK_YYT(64, double);
   else if (A.prec == 1)
@@ -2045,7 +1987,7 @@ void launch_yyt(int NP, const ChunkArgs& A, hipStream_t st) {
   else
     OAK_YYT(128, double);
 #undef OAK_YYT
-  if (NP == 64 || A.mode == 2) return;
+  if (NP == 64) return;
   if (A.prec == 1)
     hipLaunchKernelGGL((k_row_sums<128, float>), g, dim3(128), 0, st, A.z0, A.zorder, A.N, A.sel_ptr,
                        A.ymat, A.vec);
