@@ -568,7 +568,8 @@ void launch_prep_loc(int NP, const PrepLocArgs& A, hipStream_t st) {
 template <int NP>
 static void prep_ens_t(const PrepEnsArgs& A, hipStream_t st) {
   if (A.m == 0) return;
-  hipLaunchKernelGGL(k_spmm_obs<double>, dim3(spmm_blocks(A.m, A.N)), dim3(256), 0, st, A.m, A.n, A.N,
+  const SpmmGrid g = spmm_grid(A.m, A.N);
+  hipLaunchKernelGGL(k_spmm_obs<double>, dim3(g.x, g.y, g.z), dim3(256), 0, st, A.m, A.n, A.N,
                      A.row_ptr, A.col, A.val, A.E, A.ldE, A.Hshift, A.HEc, A.err);
   constexpr int TR = NP > 128 ? 16 : (NP > 64 ? 32 : 64);
   hipLaunchKernelGGL((k_obs_anom<NP, TR>), dim3(nblk(A.m, TR)), dim3(256), 0, st, A.m, A.N, A.HEc, A.yo,

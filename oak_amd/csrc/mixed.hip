@@ -72,7 +72,8 @@ static inline unsigned nblk32(int64_t n, int b) { return (unsigned)((n + b - 1) 
 template <int NP>
 static void prep_ens_f32_t(const PrepEnsArgs& A, hipStream_t st) {
   if (A.m == 0) return;
-  hipLaunchKernelGGL(k_spmm_obs<float>, dim3(spmm_blocks(A.m, A.N)), dim3(256), 0, st, A.m, A.n, A.N,
+  const SpmmGrid g = spmm_grid(A.m, A.N);
+  hipLaunchKernelGGL(k_spmm_obs<float>, dim3(g.x, g.y, g.z), dim3(256), 0, st, A.m, A.n, A.N,
                      A.row_ptr, A.col, A.val, A.E32, A.ldE, A.Hshift32, A.HEc, A.err);
   constexpr int TR = NP > 128 ? 16 : (NP > 64 ? 32 : 64);
   hipLaunchKernelGGL((k_obs_anom_f32<NP, TR>), dim3(nblk32(A.m, TR)), dim3(256), 0, st, A.m, A.N,

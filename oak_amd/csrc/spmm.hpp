@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "common.hpp"
+#include "spmm_grid.hpp"
 
 namespace oakg {
 
@@ -17,12 +18,7 @@ namespace oakg {
 // of them, which reads the row's indices once for all, and four entries at a
 // time, so that 16 gathers are in flight.  201 000 rows of 4 entries, 100 FP32
 // members: 0.85 ms with a member per grid row and one entry at a time, 0.55 so.
-constexpr int kSpmmMembers = 4;
-
-inline unsigned spmm_blocks(int64_t m, int N) {
-  return 8u * (unsigned)((m + 255) / 256) * (unsigned)((N + 8 * kSpmmMembers - 1) / (8 * kSpmmMembers));
-}
-
+// (grid: spmm_grid)
 template <typename TE>
 __global__ __launch_bounds__(256) void k_spmm_obs(int64_t m, int64_t n, int N,
                                                   const int64_t* __restrict__ row_ptr,
@@ -34,9 +30,8 @@ __global__ __launch_bounds__(256) void k_spmm_obs(int64_t m, int64_t n, int N,
                                                   unsigned* __restrict__ err) {
 #pragma clang fp contract(off)
   constexpr int MB = kSpmmMembers;
-  const unsigned nb = (unsigned)((m + 255) / 256), slot = blockIdx.x >> 3;
-  const int k0 = (int)(8 * MB * (slot / nb) + (blockIdx.x & 7));
-  const int64_t l = (int64_t)(slot % nb) * 256 + threadIdx.x;
+  const int k0 = spmm_member(blockIdx.x, blockIdx.y);
+  const int64_t l = spmm_row(blockIdx.x, blockIdx.z) + threadIdx.x;
   if (k0 >= N || l >= m) return;
   const TE* Ek[MB];
 #pragma unroll
