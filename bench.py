@@ -474,8 +474,8 @@ def main():
                     help="run every step with phase timing (zone chunks in order on one stream), "
                          "as the rocprofv3 kernel summaries are taken")
     ap.add_argument("--tune", action="store_true",
-                    help="autotune the launch shapes (chunks in flight, zones per QL wave, HIP "
-                         "graph) on this workload and store them in oak_amd/tuning.json")
+                    help="autotune the launch shapes (chunks in flight, zone order, HIP graph, "
+                         "observation-space bucket) on this workload and store them in oak_amd/tuning.json")
     ap.add_argument("--calib", action="store_true",
                     help="also run a plain 1 GiB device copy (calibrates rocprof byte counters)")
     ap.add_argument("--calib-only", action="store_true",
@@ -554,8 +554,9 @@ def main():
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f64" if head == "fp64" else "f32 state, f32 MFMA, f64 eigensolve",
         "data": "synthetic (seeded GRF ensembles and observations, random-init, no datasets)",
-        "config": {"workload": "config%d: %s, %s, %s eigensolver" % (
-                       args.config, desc, head, args.eig),
+        "config": {"workload": "config%d: %s, %s, %s" % (
+                       args.config, desc, head,
+                       "one-sided Jacobi" if args.eig == "jacobi" else "tridiagonal form"),
                    "n": int(n), "N": int(N), "m": int(P.m), "zones": int(P.nzones),
                    "mean_p": float(counts.mean()), "median_p": float(np.median(counts)),
                    "max_p": int(counts.max()),

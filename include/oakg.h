@@ -143,8 +143,11 @@ int oakg_set_timing(oakg_ctx* ctx, int on);
    matoper_inc.F90:986-1005):
      OAKG_EIG_QL      Householder tridiagonalisation, then M^-1/2 and M^-1 of the
                       tridiagonal form as sums of shifted solves, without
-                      eigenvectors (default)
-     OAKG_EIG_JACOBI  one-sided Jacobi for every zone (N <= 128)             */
+                      eigenvectors (default); by its eigenvalues, cut off at 1,
+                      in zones whose spectrum reaches beyond 2^44
+     OAKG_EIG_JACOBI  one-sided Jacobi for every zone of an analysis (N <= 128;
+                      above, as OAKG_EIG_QL)
+   The likelihood (oakg_local_nll) takes a triangular factor whichever is set.  */
 #define OAKG_EIG_JACOBI 0
 #define OAKG_EIG_QL 1
 int oakg_set_eigensolver(oakg_ctx* ctx, int method);
@@ -170,7 +173,8 @@ int oakg_get_stats(oakg_ctx* ctx, oakg_stats* out);
  *                         observations (value 16, 32 or 64; 0 = off, the
  *                         default) are solved in the p x p observation space:
  *                         G = S~ S~^T instead of M = I + S~^T S~, which have
- *                         the same nonzero spectrum.  The analysis is the
+ *                         the same nonzero spectrum (OAKG_EIG_QL, N <= 128; not
+ *                         in oakg_local_analysis_csr_noalloc).  The analysis is the
  *                         same to rounding (not bit for bit).
  *   OAKG_TUNE_PERSIST     0..2: kept, without effect
  * oakg_get_tuning also reads OAKG_TUNE_GRAPH_REPLAYS / _CAPTURES (counts). */

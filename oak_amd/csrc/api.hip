@@ -1056,7 +1056,7 @@ int ensemble_impl(oakg_ctx* c, const oakg_zones* zones, const oakg_obs* obs, con
     A.maxcorr = max_correction;
     A.maxcorr_v = dmc;
     A.zone_rows = (int)std::min<int64_t>(n / std::max<int64_t>(nz, 1), INT32_MAX);
-  const bool swept = run_zones(c, NP, A, nz, sweeps);
+    const bool swept = run_zones(c, NP, A, nz, sweeps);
     if (c->timing) c->timer.mark(PH_END);
     check(c, hipEventRecord(c->ev_t1, c->stream), "event");
     finish_call(c, nz, sel.ptr, swept ? sweeps : nullptr);
@@ -1246,10 +1246,9 @@ int ensemble_report_impl(oakg_ctx* c, const oakg_obs* obs, const oakg_csr* H, co
   });
 }
 
-// genObservationOper + packSparseMatrix on the GPU (interp.hip): the box
-// trees and simplex tables are built on the host from the node coordinates
-// (copied back first when they are device arrays), everything per
-// observation runs on the device.
+// genObservationOper + packSparseMatrix on the GPU (interp.hip): the cuts of the box
+// trees and the simplex tables follow from the grids' shapes, on the host; the boxes'
+// bounds and everything per observation are computed on the device.
 int obs_operator_impl(oakg_ctx* c, int32_t nvar, const oakg_grid* grids, int64_t m,
                       const int32_t* obs_var, const double* ox, const double* oy, const double* oz,
                       const double* ot, int64_t* row_ptr, int32_t* col, double* val, int64_t cap,

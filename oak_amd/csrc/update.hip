@@ -296,9 +296,9 @@ __global__ __launch_bounds__(256, 3) void k_update64(int64_t z0, const int32_t* 
 // four waves on a SIMD belong to two workgroups.  The product is with R; row k of T
 // is row k of R plus p_k + q_k v (OmegaRow, in slots 0 and 3 of vec), so a row of
 // Sf adds its products with p and q; row N - 1 in ymat is that of T^T already.
-// 64 800 zones of 121 rows, N = 128: 7.5 ms FP64 (27 GB moved: 3.7 TB/s), 4.1 FP32
-// (T whole in LDS, and a pass for the mean: 9.3 + 1.35 and 4.85 + 0.7).  Omega on the way to LDS cost 0.7 to
-// 1.2 ms more, in k_func's registers 3.4 ms of spills there.
+// 64 800 zones of 121 rows, N = 128: 7.2 ms FP64 (26.9 GB moved: 3.7 TB/s), 4.2 FP32
+// (13.6 GB; T whole in LDS, and a pass for the mean: 9.3 + 1.35 and 4.85 + 0.7).  Omega on
+// the way to LDS cost 0.7 to 1.2 ms more, in k_func's registers 3.4 ms of spills there.
 template <int MODE, typename TE>
 __global__ __launch_bounds__(512, 4) void k_update128(int64_t z0, const int32_t* __restrict__ zorder, int N,
                                                       const int64_t* __restrict__ sel_ptr,
