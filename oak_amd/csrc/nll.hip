@@ -904,11 +904,11 @@ __global__ __launch_bounds__(256, 2) void k_nll_again(int64_t z0, int nzc, int N
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k < nzc) {
     const int64_t z = zone_at(zorder, z0 + k);
-    if (gL[z] != gL[z]) zone[atomicAdd(&n, 1)] = (int)z;
+    if (gL[z] != gL[z]) zone[atomicAdd(&n, 1)] = k;
   }
   lds_barrier();
   for (int i = 0; i < n; ++i) {
-    const int64_t z = zone[i];
+    const int64_t z = zone_at(zorder, z0 + zone[i]);
     const double shift = gA[z];
     const int64_t p0 = sel_ptr[z], p = sel_ptr[z + 1] - p0;
     lds_barrier();
